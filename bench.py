@@ -5,7 +5,7 @@ Workload (default): synthetic config 3 -- 3-D, 4,000,000 points in [0,1]^3,
 128 Gaussian blobs (sigma U[0.005,0.03], Zipf(1.1) sizes) + 3 % uniform
 noise, eps 0.001425, minpts 10 -- the configuration the performance target
 is stated on.  One step = one full clustering of the 4 M points (grid index,
-neighbour counts, seed-list expansion, union-find merge, border, canonical
+neighbour counts, near components, component borders, border points, canonical
 relabel), FP32 distances with FP64 guard-band rechecks, inputs already
 resident in HBM, labels left in HBM.  value = points clustered per second
 over the timed steps.
@@ -117,43 +117,41 @@ def kernel_bytes(st, dim, f32):
              non-empty line its point range (two starts, 8); per candidate
              its coordinates s*D; per cell the core count 4 and mask clear 8;
              per listed core point of a light cell the list entry 4.
-    k_adj    per lane (core point of a light cell): list entry 4, cell_of 4,
-             cell_z 4, fixed-point coordinates 4*D (+ FP64 8*D in the FP64
-             form), the packed rows of the near lines above the cell (5 in
-             3-D, 2 in 2-D); per non-empty near line its first start 4; per
-             cell on it: next start, cell_z, core count (12); per pair test:
-             core flag 1 + coordinates s*D; per core cell the mask 8; per
-             adjacency bit found (half the directed bits, diag[3] / 2, exact
-             when no cell is heavy) the mirror: the row of each cell 8 and
-             the other cell's mask 8.
+    k_adj    per core cell (k_rep's records are written per cell before it:
+             16): list entry 4, its representative 16, the packed rows of the
+             near lines above it (5 in 3-D, 2 in 2-D), its mask 8; per pair
+             tested the other representative 16.
     k_rows   per cell and group of 5 lines: cell_xyz 8, the cell's sort key
              staged 8, five packed rows written 20 (the line-table entries
              of a tile's span and the keys of the extra lines around it are
              not counted: a lower bound).
-    k_expand per popped cell: chain label 4, adjacency mask 8, 9 near rows
-             36; per adjacency bit: the neighbour's label 4 and its claim 4;
+    k_expand with seed lists: per popped cell: chain label 4, near mask 8, 9
+             near rows 36; per bit: the neighbour's label 4 and its claim 4;
              per cell the seeding scan: core count 4 and label 4.
+    k_link   without: per cell: mask 8, own row 4, root 4; per core cell: mask
+             written 8, list entry 4; per joined pair its line's row 4 and
+             the other cell's entry 4.
     s = 4 (fixed point, FP32 form) or 8 (FP64 form)."""
     n, c = st["n_points"], st["n_cells"]
     s = 4 if f32 else 8
     w = st["work"]
-    lines_all = 25 if dim == 3 else 5
+    groups = (25 if dim == 3 else 5) // 5
     upper = 5 if dim == 3 else 2
-    groups = lines_all // 5
-    a = st["n_adj_points"]
+    a, cc = st["n_adj_points"], st["n_core_cells"]
     dg = st["diag"]
     core = (n * (4 + 8 + s * dim + 1) + 20 * w[0] + 8 * w[1] + s * dim * st["pairs_evaluated"] +
             c * (4 + 8) + 4 * a)
-    lane = 12 + 4 * dim + (0 if f32 else 8 * dim) + 4 * upper
-    adj = (a * lane + 4 * w[2] + 12 * w[3] + dg[8] * (1 + s * dim) + 8 * st["n_core_cells"] +
-           16 * (dg[3] // 2))
+    near = cc * (4 + 16 + 4 * upper + 8) + 16 * dg[8] + 16 * c
     rows = c * groups * (8 + 8 + 20)
     expand = dg[0] * (4 + 8 + 36) + dg[3] * 8 + c * 8
-    return {"k_core": core, "k_adj": adj, "k_rows": rows, "k_expand": expand}
+    link = c * (8 + 4 + 4) + cc * (8 + 4) + (dg[3] // 2) * 8
+    out = {"k_core": core, "k_adj": near, "k_rows": rows}
+    out["k_expand" if dg[0] else "k_link"] = expand if dg[0] else link
+    return out
 
 
 KERNEL_TIME = {"k_core": "t_core_ms", "k_adj": "t_adj_ms", "k_rows": "t_rows_ms",
-               "k_expand": "t_expand_ms"}
+               "k_expand": "t_expand_ms", "k_link": "t_expand_ms"}
 
 
 def measured_traffic(workload, precision):
@@ -699,6 +697,8 @@ def main():
     traffic = measured_traffic(args.workload, args.precision)
     kernels = {}
     for k, tk in KERNEL_TIME.items():
+        if k not in kb:
+            continue
         # live HIP events on the library's stream: k_core's from the timed leg
         t_k = float(np.mean([s[tk] for s in (sts if k == "k_core" else sts_ph)]))
         if t_k <= 0:

@@ -30,8 +30,6 @@ namespace {
 
 constexpr int64_t kChunk = 4096;  // points per chunk of bbox / cell-key blocks
 constexpr int kMaxExpandPasses = 100000;
-// heavy cells from which their adjacency pass runs beside the light one
-constexpr long long kHeavyOverlap = 1024;
 
 struct Buf {
   void* p = nullptr;
@@ -49,10 +47,6 @@ struct dclust_handle {
   int device = 0;
   int num_cu = 0;
   hipStream_t stream = nullptr;
-  // second stream (default priority, like the first) for kernels that run
-  // beside the main sequence, and the events that fork and join it
-  hipStream_t stream2 = nullptr;
-  hipEvent_t fork[4] = {};
   hipEvent_t ev[E_N] = {};
   std::vector<Buf> bufs;
   int64_t last_n = -1;
@@ -67,7 +61,6 @@ struct dclust_handle {
   std::vector<uint8_t> prev_sig;   // launch state of the last eager run
   int prev_npass = 0;              // its expansion passes
   long long prev_nlines = 0;       // its neighbour-line count
-  long long prev_nheavy = 0;       // heavy cells of the last run (any kind)
   int prev_sort_passes = 0;        // its radix passes
   hipGraphExec_t gexec = nullptr;  // captured run
   std::vector<uint8_t> gsig;       // launch state it was captured for
@@ -118,11 +111,11 @@ struct dclust_handle {
 namespace {
 
 enum Slot {
-  S_XYZ, S_INST, S_CHUNK, S_BBOX, S_CTL, S_KEY0, S_KEY1, S_VAL0, S_VAL1, S_HIST, S_OFFS,
+  S_XYZ, S_INST, S_CHUNK, S_BBOX, S_CTL, S_KEY, S_VAL, S_HIST, S_OFFS,
   S_DTOT, S_PASS, S_CSTART, S_CKEY, S_CINST, S_CM, S_ROWS, S_CELLOF, S_X0, S_X1, S_X2,
   S_G0, S_G1, S_G2, S_ORIG, S_CORE, S_LABEL, S_PARENT, S_COMPMIN, S_PAIRS, S_Q0, S_Q1,
   S_KEYV, S_FLAG, S_RANK, S_SCAN, S_LABOUT, S_COREOUT, S_PAIRCNT, S_SEGPOS, S_LINES, S_AMASK,
-  S_HEAVY, S_REC, S_RECN, S_CXYZ, S_CCOMP, S_ADJPTS, S_BORDERPTS, S_CORECELLS, S_TUNELAB, S_STAT, S_GLINES,
+  S_REC, S_RECN, S_CXYZ, S_CCOMP, S_BORDERPTS, S_CORECELLS, S_TUNELAB, S_STAT, S_GLINES,
   S_CZ, S_XOFF, S_OS_LABEL, S_OS_STATE, S_OS_SEEDS, S_OS_LEN, S_OS_CONTACT, S_OS_FIRST, S_ROWSFB
 };
 
@@ -217,6 +210,7 @@ float ev_ms(dclust_handle* h, int a, int b) {
 }
 
 struct RunShape {
+  bool chains;  // near components by seed-list expansion (else by union-find)
   int seeds;
   int threads;
   int blocks;
@@ -260,12 +254,20 @@ const ShapeRow* shape_row(int dims, int64_t n) {
   return nullptr;
 }
 
+// Near components: a call that names any value of the expansion's shape
+// (MAX_SEEDS, THREAD_BLOCKS, THREAD_COUNT, EXTRA_COLLISION_SIZE) runs the
+// seed-list expansion with that shape.  A call that leaves them all 0 unites
+// the near graph's pairs in a parallel union-find instead (k_link_*): the
+// expansion's time is the serial rounds of its longest wavefront, 435 us of
+// 2.45 ms on 4 M 3-D points (plus 64 us to merge its chains) and 79 (+ 24) of
+// 358 us on 10 k 2-D points, where the union-find takes 182 and 26 us.
 // Launch shape: explicit parameters win; a call that leaves seed list,
 // workgroup size and workgroup count all at 0 takes the built-in table's
 // shape for its dimension mix and size, other zeros the rule (seed list 1024
 // entries, 256 threads, blocks at resident occupancy, at most 8 per CU).
 RunShape pick_shape(dclust_handle* h, const dclust_params& p, int64_t n, bool f32, int dims) {
   RunShape r;
+  r.chains = p.seed_list_size > 0 || p.blocks > 0 || p.block_threads > 0 || p.extra_collision > 0;
   const ShapeRow* row = (p.seed_list_size == 0 && p.block_threads == 0 && p.blocks == 0)
                             ? shape_row(dims, n)
                             : nullptr;
@@ -354,19 +356,6 @@ hipError_t mark(dclust_handle* h, int e, bool graph, hipStream_t s = nullptr) {
                : hipEventRecord(h->ev[e], s);
 }
 
-// Work on the second stream after everything enqueued so far on the first
-// (fork event k), and the first stream's wait for it (join event k + 1).
-hipError_t fork_second(dclust_handle* h, int k) {
-  hipError_t e = hipEventRecord(h->fork[k], h->stream);
-  if (e == hipSuccess) e = hipStreamWaitEvent(h->stream2, h->fork[k], 0);
-  return e;
-}
-hipError_t join_second(dclust_handle* h, int k) {
-  hipError_t e = hipEventRecord(h->fork[k + 1], h->stream2);
-  if (e == hipSuccess) e = hipStreamWaitEvent(h->stream, h->fork[k + 1], 0);
-  return e;
-}
-
 // Keys, sort, CSR, gather and line table, then the neighbour rows (one
 // stream: the gather fills the device, so running the rows beside it gains
 // nothing).
@@ -388,28 +377,18 @@ void enqueue_head(const Dev& d, int nchunks, hipStream_t s) {
   launch_index_head(d, nchunks, s);
 }
 
-// per-cell state, core flags, near adjacency, seeding segments
+// per-cell state, core flags, near graph, seeding segments
 hipError_t enqueue_core(dclust_handle* h, const Dev& d, const RunShape& shape, bool f32,
                         bool graph) {
   const hipStream_t s = h->stream;
   hipError_t e;
   if ((e = mark(h, E_INDEX, graph)) != hipSuccess) return e;
-  launch_init_run(d, shape.waves, s);
+  launch_init_run(d, shape.chains ? shape.waves : 0, s);
   // the core (neighbour-count) kernel is bracketed by its own events
   if ((e = mark(h, E_CORE0, graph)) != hipSuccess) return e;
   launch_core(d, f32, s);
   if ((e = mark(h, E_CORE, graph)) != hipSuccess) return e;
-  // heavy cells on the second stream beside the light ones when the last
-  // run had many (the fork and join cost more than a near-empty heavy pass
-  // takes); the labels do not depend on it
-  if (h->prev_nheavy >= kHeavyOverlap) {
-    if ((e = fork_second(h, 2)) != hipSuccess) return e;
-    launch_adj_heavy(d, f32, h->num_cu * 16, h->stream2);
-    launch_adj_light(d, f32, s);
-    if ((e = join_second(h, 2)) != hipSuccess) return e;
-  } else {
-    launch_adj(d, f32, h->num_cu * 16, s);
-  }
+  launch_near(d, s);
   if ((e = mark(h, E_ADJ, graph)) != hipSuccess) return e;
   return hipSuccess;
 }
@@ -424,12 +403,19 @@ void enqueue_pass(const Dev& d, const RunShape& shape, int pass, hipStream_t s, 
   if (pass > 0 || check > 0) launch_pass_carry(d, pass, check, s);
 }
 
-// chain merge, far pairs, border points, canonical labels
+// near components by union-find (in place of the expansion passes)
+hipError_t enqueue_link(dclust_handle* h, const Dev& d, bool graph) {
+  launch_link(d, h->stream);
+  return mark(h, E_PASS0, graph);
+}
+
+// chain merge, component borders, border points, canonical labels
 hipError_t enqueue_tail(dclust_handle* h, const Dev& d, bool f32, int grid_cells, bool graph) {
   const hipStream_t s = h->stream;
   hipError_t e;
   if ((e = mark(h, E_EXPAND, graph)) != hipSuccess) return e;
-  launch_merge(d, grid_cells, s);
+  if (d.chains) launch_merge(d, grid_cells, s);
+  launch_comp(d, s);
   if ((e = mark(h, E_MERGE, graph)) != hipSuccess) return e;
   launch_far(d, f32, grid_cells, s);
   if ((e = mark(h, E_FAR, graph)) != hipSuccess) return e;
@@ -467,7 +453,8 @@ hipError_t capture_run(dclust_handle* h, const Dev& d, const RunShape& shape, bo
   if (body == hipSuccess) body = enqueue_core(h, d, shape, f32, true);
   // work still pending after the last pass: the rest of the graph returns at
   // once and the host runs the call eagerly
-  for (int p = 0; body == hipSuccess && p < passes; ++p) {
+  if (body == hipSuccess && !d.chains) body = enqueue_link(h, d, true);
+  for (int p = 0; body == hipSuccess && d.chains && p < passes; ++p) {
     enqueue_pass(d, shape, p, s, p == passes - 1 ? passes : 0);
     if (p == 0) body = mark(h, E_PASS0, true);
   }
@@ -531,7 +518,6 @@ void finish_run(dclust_handle* h, const Dev& d, const RunShape& shape, long long
   for (int c = 0; c < C_NCTL; ++c)
     for (int k = 0; k < kStripes; ++k) ctl_h[c] += stat_h[(size_t)c * kStripes + k];
   h->last_n = d.n;
-  h->prev_nheavy = ctl_h[C_NHEAVY];
   h->last_core = d.core;
   h->last_orig = d.orig;
   h->last_core_out = d.core_out;
@@ -561,7 +547,8 @@ void finish_run(dclust_handle* h, const Dev& d, const RunShape& shape, long long
   stats->n_core = ctl_h[C_NCORE];
   stats->n_noise = ctl_h[C_NNOISE];
   stats->n_clusters = ctl_h[C_NCLUST];
-  stats->n_chains = ctl_h[C_NCHAIN];
+  // without seed lists every near component counts as one chain
+  stats->n_chains = d.chains ? ctl_h[C_NCHAIN] : ctl_h[C_NROOTS];
   stats->n_collisions = ctl_h[C_NPAIR];
   stats->n_overflow = ctl_h[C_OVF];
   stats->n_passes = npass;
@@ -580,7 +567,7 @@ void finish_run(dclust_handle* h, const Dev& d, const RunShape& shape, long long
   stats->diag[4] = (int64_t)(1000.0 * phase_ms(E_ADJ, E_PASS0));
   stats->diag[5] = ctl_h[C_BUSY_SUM];
   stats->diag[6] = ctl_h[C_BUSY_MAX];
-  stats->diag[7] = shape.waves;
+  stats->diag[7] = d.chains ? shape.waves : 0;
   stats->diag[8] = ctl_h[C_ADJ_TESTS];
   stats->diag[9] = ctl_h[C_ADJ_FREE];
   stats->diag[10] = ctl_h[C_FAR_TESTS];
@@ -666,11 +653,7 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
     shape.pair_per = 64;
     shape.pair_cap = (int64_t)shape.pair_per * shape.waves;
   }
-  if (onestep) {  // the expansion buffers stay unused: keep them minimal
-    shape.blocks = 8;
-    shape.waves = 8 * (shape.threads / 64);
-    shape.pair_cap = (int64_t)shape.pair_per * shape.waves;
-  }
+  if (onestep) shape.chains = false;  // (its own loop runs instead)
   const int nchunks = (int)chunks.size();
   const int grid_cells = h->num_cu * 8;
   const hipStream_t s = h->stream;
@@ -681,7 +664,9 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
   d.ninst = ninst;
   d.nchunks = nchunks;
   d.xyz = d_xyz;
-  d.pair_cap = shape.pair_cap;
+  d.chains = shape.chains ? 1 : 0;
+  // (without seed lists the expansion's buffers stay unused and minimal)
+  d.pair_cap = shape.chains ? shape.pair_cap : 0;
   d.pair_per = shape.pair_per;
   d.rstride = ntot;
   // neighbourhood sizes (stats.cand_total / nbr_cells_total) cost an extra
@@ -705,10 +690,16 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
     d.bbox = M.get<unsigned long long>(S_BBOX, (size_t)ninst * kBoxStripes * 8);
     d.ctl = M.get<long long>(S_CTL, C_NCTL);
     d.stat = M.get<long long>(S_STAT, (size_t)C_NCTL * kStripes);
-    d.key[0] = M.get<uint64_t>(S_KEY0, ntot);
-    d.key[1] = M.get<uint64_t>(S_KEY1, ntot);
-    d.val[0] = M.get<int32_t>(S_VAL0, ntot);
-    d.val[1] = M.get<int32_t>(S_VAL1, ntot);
+    // the sort's keys, then (from k_rep on) the cells' representatives
+    d.key[0] = M.get<uint64_t>(S_KEY, 2 * (size_t)ntot);
+    d.key[1] = d.key[0] + ntot;
+    d.rep = (uint4*)d.key[0];
+    // the sort's point ids, then (from k_far on) the listed border pairs
+    d.val[0] = M.get<int32_t>(S_VAL, 2 * (size_t)ntot);
+    d.val[1] = d.val[0] + ntot;
+    d.far_pairs = PairList{(int2*)d.val[0],
+                           (unsigned long long*)(d.stat + (int64_t)C_NFARPAIRS * kStripes),
+                           ntot / kStripes};
     d.hist = M.get<uint32_t>(S_HIST, sort_hist_entries(ntot));
     d.offs = M.get<uint32_t>(S_OFFS, sort_hist_entries(ntot));
     d.dtot = M.get<uint32_t>(S_DTOT, 256);
@@ -720,13 +711,9 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
     d.cell_comp = M.get<int32_t>(S_CCOMP, ntot);
     // striped work lists: sub-list capacity = the most its workgroups append
     const int64_t cap_p = (point_blocks(ntot) + kStripes - 1) / kStripes * 256;
-    const int64_t cap_c = (cell_comp_blocks(ntot) + kStripes - 1) / kStripes * 1024;
-    d.adj_pts = SList{M.get<int32_t>(S_ADJPTS, (size_t)cap_p * kStripes),
-                      (unsigned long long*)(d.stat + (int64_t)C_NADJPTS * kStripes), cap_p};
+    const int64_t cap_c = (cell_blocks(ntot) + kStripes - 1) / kStripes * 1024;
     d.border_pts = SList{M.get<int32_t>(S_BORDERPTS, (size_t)cap_p * kStripes),
                          (unsigned long long*)(d.stat + (int64_t)C_NBORDERPTS * kStripes), cap_p};
-    d.heavy = SList{M.get<int32_t>(S_HEAVY, (size_t)cap_p * kStripes),
-                    (unsigned long long*)(d.stat + (int64_t)C_NHEAVY * kStripes), cap_p};
     d.core_cells = SList{M.get<int32_t>(S_CORECELLS, (size_t)cap_c * kStripes),
                          (unsigned long long*)(d.stat + (int64_t)C_NCORECELLS * kStripes), cap_c};
     const int64_t cap_r = row_list_cap(ntot);
@@ -754,11 +741,16 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
     if (rec_stride > 0) d.rec = M.get<int32_t>(S_REC, (size_t)ntot * rec_stride);
     d.parent = M.get<int32_t>(S_PARENT, ntot);
     d.compmin = M.get<int32_t>(S_COMPMIN, ntot);
-    d.pairs = M.get<int2>(S_PAIRS, shape.pair_cap);
-    d.pair_cnt = M.get<int32_t>(S_PAIRCNT, shape.waves);
-    d.seg_pos = M.get<int64_t>(S_SEGPOS, shape.waves);
-    d.q[0] = M.get<int32_t>(S_Q0, ntot);
-    d.q[1] = M.get<int32_t>(S_Q1, ntot);
+    const int64_t waves = shape.chains ? shape.waves : 0;
+    d.pairs = M.get<int2>(S_PAIRS, d.pair_cap);
+    d.pair_cnt = M.get<int32_t>(S_PAIRCNT, waves);
+    d.seg_pos = M.get<int64_t>(S_SEGPOS, waves);
+    // the first queue, then (from k_comp on) the list of the near roots
+    const int64_t cap_n = list_append_cap(ntot);
+    d.q[0] = M.get<int32_t>(S_Q0, (size_t)std::max(ntot, cap_n * kStripes));
+    d.q[1] = M.get<int32_t>(S_Q1, shape.chains ? ntot : 0);
+    d.near_roots = SList{d.q[0], (unsigned long long*)(d.stat + (int64_t)C_NROOTS * kStripes),
+                         cap_n};
     d.keyv = M.get<int32_t>(S_KEYV, ntot);
     d.flag = M.get<uint8_t>(S_FLAG, ntot);
     d.rank = M.get<int32_t>(S_RANK, ntot + 1);
@@ -899,7 +891,8 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
     // expansion passes until no seed is pending: pass p drains the queue of
     // pass p-1 (overflowed seed lists, lists left when a wave's pop budget
     // ran out) and continues every unfinished seeding segment
-    for (npass = 0; npass < kMaxExpandPasses; ++npass) {
+    if (!d.chains) HIPCHK(enqueue_link(h, d, false));
+    for (npass = 0; d.chains && npass < kMaxExpandPasses; ++npass) {
       enqueue_pass(d, shape, npass, s);
       if (npass == 0) HIPCHK(mark(h, E_PASS0, false));
       HIPCHK(hipMemcpyAsync(ctl_h, d.ctl, sizeof(ctl_h), hipMemcpyDeviceToHost, s));
@@ -1154,19 +1147,12 @@ int dclust_create(dclust_handle** out, int device) {
     (void)hipGetLastError();
     h->scratch = nullptr;
   }
-  if (hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking) != hipSuccess ||
-      hipStreamCreateWithFlags(&h->stream2, hipStreamNonBlocking) != hipSuccess) {
-    if (h->stream) (void)hipStreamDestroy(h->stream);
+  if (hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking) != hipSuccess) {
     delete h;
     return DCLUST_E_HIP;
   }
   for (auto& e : h->ev)
     if (hipEventCreate(&e) != hipSuccess) {
-      dclust_destroy(h);
-      return DCLUST_E_HIP;
-    }
-  for (auto& e : h->fork)
-    if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
       dclust_destroy(h);
       return DCLUST_E_HIP;
     }
@@ -1187,15 +1173,11 @@ void dclust_destroy(dclust_handle* h) {
   if (!h) return;
   (void)hipSetDevice(h->device);
   if (h->stream) (void)hipStreamSynchronize(h->stream);
-  if (h->stream2) (void)hipStreamSynchronize(h->stream2);
   drop_graph(h);
   for (auto& b : h->bufs)
     if (b.p) (void)hipFree(b.p);
   for (auto& e : h->ev)
     if (e) (void)hipEventDestroy(e);
-  for (auto& e : h->fork)
-    if (e) (void)hipEventDestroy(e);
-  if (h->stream2) (void)hipStreamDestroy(h->stream2);
   if (h->stream) (void)hipStreamDestroy(h->stream);
   if (h->pin) (void)hipHostFree(h->pin);
   delete h;

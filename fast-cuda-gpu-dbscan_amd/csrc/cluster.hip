@@ -15,14 +15,15 @@
 //                >= minpts points is all core without a distance test.  A
 //                point that stays below minpts has seen all its neighbours
 //                and records them for the border pass.
-//   k_adj        cell adjacency: bit 5r+k of a core cell's 128-bit mask is
-//                set when stencil slot 5r+k holds a core point within eps of
-//                one of the cell's core points.  Light cells: one lane per
-//                core point.  Heavy cells (> kHeavy points): one wavefront
-//                per cell (k_adj_heavy), which also sets the mirrored bit of
-//                its light neighbours.
-//   k_expand     persistent seed-list expansion (dbscan.cu:254-387) over
-//                cells: each wavefront owns a seed list of cells in LDS and
+//   k_rep, k_adj   the near graph over core cells: two cells in near lines
+//                are linked when their representatives (one core point each)
+//                are certainly joined.
+//   k_link_local, k_link_cross   components of the near graph by union-find,
+//                in LDS over runs of cells, then in global memory.
+//   k_expand     the same components by persistent seed-list expansion
+//                (dbscan.cu:254-387) over cells, for calls that give the
+//                reference's launch values (MAX_SEEDS, THREAD_BLOCKS,
+//                THREAD_COUNT, EXTRA_COLLISION_SIZE): each wavefront owns a seed list of cells in LDS and
 //                pops up to 64 of them at once, one per lane; each lane
 //                claims the adjacent unclaimed cells of its cell with one CAS
 //                each (MarkAsCandidate, dbscan.cu:189-222) and pushes them;
@@ -35,7 +36,9 @@
 //   k_merge_lds / k_union_pairs / k_flatten   GPU atomic union-find over
 //                chain ids (MonitorSeedPoints' CPU BFS over the collision
 //                matrix and thrust::replace relabels, dbscan.cu:60-125).
-//   k_cell_comp / k_flatten_all / k_keys / k_border / rank scan / k_output
+//   k_comp, k_far, k_far_pairs   pairs of stencil cells in two components are
+//                decided exactly and united.
+//   k_flatten_all / k_roots_final / k_keys / k_border / rank scan / k_output
 //                canonical labels:
 //                cluster id = rank of the component's minimum core input
 //                index; border = minimum id over adjacent cores; noise = 0
@@ -51,6 +54,7 @@
 // directions.  Two core points are joined when d^2 <= eps^2 and the box test
 // holds from at least one side (the oracle's union runs from every core
 // point, cpu-dbscan/dbscan_rtree_exp.cpp:379-404).
+#include <algorithm>
 #include <climits>
 
 #include "internal.h"
@@ -58,8 +62,6 @@
 #include "stencil.h"
 
 namespace dclust {
-
-constexpr int kQCache = 256;  // query points a heavy-cell wavefront keeps in LDS
 
 constexpr int kCoreBatch = 4;  // neighbour-count candidates loaded per lane step
 
@@ -137,16 +139,6 @@ __device__ __forceinline__ bool edge_pair(const Dev& d, const Par& P, int32_t a,
   const bool f = box_64<D>(xa, xb, P.eps), r = box_64<D>(xb, xa, P.eps);
   t.asym += (f != r) && a < b;
   return f || r;
-}
-
-__device__ __forceinline__ bool mask_has(unsigned long long m0, unsigned long long m1, int b) {
-  return ((b < 64 ? (m0 >> b) : (m1 >> (b - 64))) & 1ull) != 0;
-}
-__device__ __forceinline__ void mask_set(unsigned long long& m0, unsigned long long& m1, int b) {
-  if (b < 64)
-    m0 |= 1ull << b;
-  else
-    m1 |= 1ull << (b - 64);
 }
 
 // Per-lane dispatch on the instance dimension (a wavefront can straddle two
@@ -302,14 +294,12 @@ __global__ __launch_bounds__(256, F32 ? 6 : 5) void k_core(Dev d) {
   DCLUST_BY_DIM(act, dim, (core_lane<3, F32>(d, P, p, c, qs, qe, R, rk, t, isc)),
                 (core_lane<2, F32>(d, P, p, c, qs, qe, R, rk, t, isc)));
   if (act) d.core[p] = isc;
-  // core points of light cells: the lanes of the near-adjacency pass
-  block_append(isc && qe - qs <= kHeavy, p, d.adj_pts);
   // non-core points: the lanes of the border-label pass
   block_append(act && !isc, p, d.border_pts);
   // per-cell core counts: the lanes of one cell form a contiguous run
   const bool head = act && (p == qs || lane == 0);
   const unsigned long long mh = ballot(head), mc = ballot(isc);
-  long long dense = 0;
+  bool dense = false, heavy = false;
   if (head) {
     const unsigned long long above = lane == 63 ? 0ull : (mh & (~0ull << (lane + 1)));
     const int nxt = above ? __ffsll((long long)above) - 1 : 64;
@@ -317,15 +307,14 @@ __global__ __launch_bounds__(256, F32 ? 6 : 5) void k_core(Dev d) {
     const int k = __popcll(mc & seg);
     if (k) atomicAdd(&d.cell_ncore[c], k);
     if (p == qs) {
-      // first point of its cell: clear the adjacency mask
-      d.amask[c] = 0ull;
       dense = (qe - qs) >= P.minpts;
+      heavy = (qe - qs) > kHeavy;
     }
   }
-  // heavy cells, listed once (by their first point)
-  block_append(act && p == qs && qe - qs > kHeavy, c, d.heavy);
-  stat_add(d, C_NCORE, isc ? 1 : 0);
-  stat_add(d, C_DENSE, dense);
+  stat_count(d, C_NHEAVY, heavy);
+  stat_count(d, C_NADJPTS, isc && qe - qs <= kHeavy);
+  stat_count(d, C_NCORE, isc);
+  stat_count(d, C_DENSE, dense);
   stat_add(d, C_EVAL, t.eval);
   stat_add(d, C_BAND_CORE, t.band);
   stat_add(d, C_BAND, t.band);
@@ -334,7 +323,374 @@ __global__ __launch_bounds__(256, F32 ? 6 : 5) void k_core(Dev d) {
   stat_add(d, C_CORE_LINES, t.lines);
 }
 
-// ------------------------------------------------------------- adjacency --
+// ----------------------------------------------------------- near graph --
+// Stencil lines whose cells can lie above a cell (offsets (a, b) >= (0, 0)
+// in the key order, the own line included), in row order; -1 pads.
+#define DCLUST_UPPER_ROWS3 {0, 2, 4, 7, 8, 10, 12, 15, 16, 18, 20, 23, 24, -1, -1}
+#define DCLUST_UPPER_ROWS2 {0, 2, 4, -1, -1}
+static __constant__ int8_t kUpperRows3[15] = DCLUST_UPPER_ROWS3;
+static __constant__ int8_t kUpperRows2[5] = DCLUST_UPPER_ROWS2;
+
+// Near lines above a cell (offsets of at most one; every cell of them but
+// the own line's lower half has a larger index): (0,0), (1,0), (0,1),
+// (1,-1), (1,1) in 3-D; (0) and (1) in 2-D.  Nibble i of `rows` is the i-th
+// such row, nibble r of `mirror` the line with row r's offsets negated.
+template <int D>
+struct Upper {
+  static constexpr int lines = D == 3 ? 5 : 2;
+  static constexpr unsigned long long rows = D == 3 ? 0x87420ull : 0x20ull;
+  static constexpr unsigned long long mirror = D == 3 ? 0x567834120ull : 0x120ull;
+};
+namespace tables {
+constexpr int8_t up3[15] = DCLUST_UPPER_ROWS3;
+constexpr int8_t up2[5] = DCLUST_UPPER_ROWS2;
+constexpr bool above(int a, int b) { return a > 0 || (a == 0 && b >= 0); }
+constexpr bool upper_ok() {
+  int i = 0;
+  for (int r = 0; r < 25; ++r)
+    if (above(off3[r][0], off3[r][1]) && up3[i++] != r) return false;
+  if (i != 13 || up3[13] != -1 || up3[14] != -1) return false;
+  i = 0;
+  for (int r = 0; r < 5; ++r)
+    if (off2[r] >= 0 && up2[i++] != r) return false;
+  if (i != 3) return false;
+  // near rows of the near graph (nibbles) and their mirrors
+  for (int k = 0; k < 5; ++k) {
+    const int r = (int)((Upper<3>::rows >> (4 * k)) & 15ull);
+    if (r > 8 || !above(off3[r][0], off3[r][1]) || up3[k] != r) return false;
+  }
+  for (int r = 0; r < 9; ++r)
+    if ((int)((Upper<3>::mirror >> (4 * r)) & 15ull) != mir3[r]) return false;
+  for (int k = 0; k < 2; ++k)
+    if ((int)((Upper<2>::rows >> (4 * k)) & 15ull) != up2[k]) return false;
+  for (int r = 0; r < 3; ++r)
+    if ((int)((Upper<2>::mirror >> (4 * r)) & 15ull) != mir2[r]) return false;
+  return true;
+}
+static_assert(upper_ok(), "upper stencil lines");
+}  // namespace tables
+
+// Workgroups of the kernels that walk the list of core cells (grid-stride).
+constexpr int kListGrid = 4096;
+
+// Every core cell is represented by its first core point (the sort is
+// stable, so that is also its smallest core input index).  One lane per cell
+// writes the representative's coordinates and sorted index in one 16-byte
+// record (w = kNoRep for a cell without core points), resets the cell's
+// state of the clustering phases and lists the core cells.
+constexpr uint32_t kNoRep = 0xffffffffu;
+
+__global__ __launch_bounds__(1024) void k_rep(Dev d) {
+  if (abandoned(d)) return;
+  const int64_t C = d.ctl[C_NCELL];
+  const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (c - threadIdx.x >= C) return;  // (block-uniform)
+  const bool in = c < C;
+  const int64_t cc = in ? c : 0;
+  const int32_t ncore = d.cell_ncore[cc], q0 = d.cell_start[cc], q1 = d.cell_start[cc + 1];
+  const bool hc = in && ncore > 0;
+  uint4 r = make_uint4(0u, 0u, 0u, kNoRep);
+  if (hc) {
+    int32_t q = q0;
+    if (ncore != q1 - q0)
+      while (!d.core[q]) ++q;
+    r = make_uint4(d.G[0][q], d.G[1][q], d.G[2][q], (uint32_t)q);
+  }
+  // (the forest covers every cell: the chain merge walks all of it, and the
+  // relabel pass reads entry 0 for points that are not core)
+  if (in) {
+    d.rep[c] = r;
+    d.cell_comp[c] = -1;
+    d.parent[c] = (int32_t)c;
+    d.compmin[c] = kNoKey;
+    d.amask[c] = 0ull;
+    d.cell_label[c] = kUnclaimed;
+  }
+  block_append(hc, (int32_t)c, d.core_cells);
+}
+
+// Near graph: bit 5r+k of a core cell's mask is set when cell k of its near
+// line r (r < 9) holds a representative that is certainly joined to its own
+// (fixed-point distance below the guard band, which implies the FP64
+// predicate in both directions).  Each pair is tested once, by its lower
+// cell.  The graph need not hold every adjacent pair: whatever pair it
+// leaves in two components is decided exactly by the pass over component
+// borders (k_far, k_far_pairs).  Inside a cluster the first pair of points
+// nearly always joins (of 7.3 M near cell pairs of the 4 M point 3-D
+// workload 92 % are joined, with 1.15 point tests per pair), so one 16-byte
+// load and one distance per pair take the place of a scan of both cells'
+// points: 49 + 64 us with k_rep, where testing every near pair to the end
+// took 289 us there, 77 + 90 us on 1 M 2-D points (here 20) and 2.2 ms on
+// 32 M points in dense blobs (cells of more than 32 points wave by wave).
+template <int D>
+__device__ __forceinline__ unsigned long long near_bits(const Dev& d, float d2_in, int32_t A,
+                                                        Tally& t) {
+  constexpr int NN = Upper<D>::lines;
+  const uint4 a4 = d.rep[A];
+  const uint32_t ag[3] = {a4.x, a4.y, a4.z};
+  const RowsOf rows = rows_of(d, A);
+  int32_t pk[NN];
+#pragma unroll
+  for (int i = 0; i < NN; ++i) pk[i] = rows[(int)((Upper<D>::rows >> (4 * i)) & 15ull)];
+  unsigned long long m = 0;
+#pragma unroll
+  for (int i = 0; i < NN; ++i) {
+    const int r = (int)((Upper<D>::rows >> (4 * i)) & 15ull);
+    const int32_t len = pk[i] >> kRowCntShift, st = pk[i] & kRowCellMask;
+    uint4 b4[5];
+#pragma unroll
+    for (int k = 0; k < 5; ++k) {
+      b4[k].w = kNoRep;
+      if (k < len && st + k > A) b4[k] = d.rep[st + k];
+    }
+    t.lines += len > 0;
+    t.cells += len;
+#pragma unroll
+    for (int k = 0; k < 5; ++k) {
+      const uint32_t bg[3] = {b4[k].x, b4[k].y, b4[k].z};
+      if (b4[k].w != kNoRep) {
+        ++t.eval;
+        if (d2fix<D>(ag, bg) < d2_in) m |= 1ull << (5 * r + k);
+      }
+    }
+  }
+  return m;
+}
+
+// Expansion by seed lists: each bit of A is also set in the other cell's
+// mask (A's place in that cell's mirrored line).
+template <int D>
+__device__ void near_mirror(const Dev& d, int32_t A, unsigned long long m) {
+  const RowsOf rows = rows_of(d, A);
+  if (m) atomicOr(&d.amask[A], m);
+  while (m) {
+    const int b = __ffsll((long long)m) - 1;
+    m &= m - 1;
+    const int r = (b * 205) >> 10;  // b / 5 for 0 <= b < 128
+    const int32_t B = (rows[r] & kRowCellMask) + (b - 5 * r);
+    const int rm = (int)((Upper<D>::mirror >> (4 * r)) & 15ull);
+    const int32_t pos = rows_of(d, B)[rm] & kRowCellMask;
+    atomicOr(&d.amask[B], 1ull << (5 * rm + (A - pos)));
+  }
+}
+
+// One lane per core cell.
+__global__ __launch_bounds__(256) void k_adj(Dev d) {
+  if (abandoned(d)) return;
+  __shared__ long long s_pre[kStripes + 1];
+  const long long n = slist_prefix(d.core_cells, s_pre);
+  Tally t;
+  long long edges = 0;
+  for (long long i0 = (long long)blockIdx.x * 256; i0 < n; i0 += (long long)gridDim.x * 256) {
+    const long long i = i0 + threadIdx.x;
+    const bool act = i < n;
+    const int32_t A = act ? slist_at(d.core_cells, s_pre, i) : -1;
+    int dim = 0;
+    float d2_in = 0.f;
+    if (act) {
+      const Inst* I = inst_of_cell(d, A);
+      dim = I->dim;
+      d2_in = I->d2_in;
+    }
+    unsigned long long m = 0;
+    DCLUST_BY_DIM(act, dim, (m = near_bits<3>(d, d2_in, A, t)),
+                  (m = near_bits<2>(d, d2_in, A, t)));
+    if (d.chains) {
+      DCLUST_BY_DIM(act, dim, near_mirror<3>(d, A, m), near_mirror<2>(d, A, m));
+    } else {
+      edges += 2 * __popcll(m);
+      if (act) d.amask[A] = m;
+    }
+  }
+  stat_add(d, C_ADJ_TESTS, t.eval);
+  stat_add(d, C_ADJ_LINES, t.lines);
+  stat_add(d, C_ADJ_CELLS, t.cells);
+  if (!d.chains) stat_add(d, C_EDGES, edges);
+}
+
+// Components of the near graph without seed lists, in two kernels.
+// k_link_local: a workgroup takes a run of consecutive cells and unites the
+// pairs inside it in an LDS copy of the forest, then writes every cell's
+// root; the bits that leave the run stay in the masks.  k_link_cross unites
+// those in global memory, between roots only.  (All pairs in global memory
+// took 1.65-2.1 ms on the 4 M point 3-D workload, against 95 + 87 us: cells
+// of a cluster hook each other link by link into chains that every find then
+// walks with loads past the L2, which is not coherent across XCDs.  Without
+// the runs of the first step k_link_local took 33 us instead of 22 on 10 k
+// 2-D points; without its table of pairs k_link_cross took 150 us, and 114
+// with links by id instead of uf_order.)
+constexpr int kLinkCells = 16384;  // cells of one LDS forest (64 KiB)
+constexpr int kLinkMin = 4096;     // least cells of a run
+constexpr int kLinkGrid = 512;     // workgroups (two per CU)
+
+__device__ __forceinline__ int32_t lds_find(int32_t* par, int32_t x) {
+  for (;;) {
+    int32_t p = par[x];
+    if (p == x) return x;
+    int32_t gp = par[p];
+    if (gp != p) par[x] = gp;
+    x = p;
+  }
+}
+
+// unites the sets of a and b; returns their root
+__device__ __forceinline__ int32_t lds_union(int32_t* par, int32_t a, int32_t b) {
+  a = lds_find(par, a);
+  b = lds_find(par, b);
+  while (a != b) {
+    if (uf_order(a) < uf_order(b)) {
+      const int32_t t = a;
+      a = b;
+      b = t;
+    }
+    const int32_t old = atomicCAS(&par[a], a, b);
+    if (old == a || old == b) return b;
+    a = lds_find(par, old);
+    b = lds_find(par, b);
+  }
+  return a;
+}
+
+__global__ __launch_bounds__(1024) void k_link_local(Dev d) {
+  if (abandoned(d)) return;
+  __shared__ int32_t par[kLinkCells];
+  const int lane = lane_id();
+  const int32_t C = (int32_t)d.ctl[C_NCELL];
+  // cells per run: the workgroups share the cells, in whole wavefronts
+  int32_t K = (C + (int32_t)gridDim.x - 1) / (int32_t)gridDim.x;
+  K = (K + 1023) & ~1023;
+  K = K < kLinkMin ? kLinkMin : (K > kLinkCells ? kLinkCells : K);
+  for (int64_t c0 = (int64_t)blockIdx.x * K; c0 < C; c0 += (int64_t)gridDim.x * K) {
+    const int32_t nc = (int32_t)(C - c0 < K ? C - c0 : K);
+    // the forest starts with the runs of cells joined one to the next along
+    // their line, as far as they lie in one wavefront: united pair by pair
+    // they would form chains as long as the run
+    for (int i = threadIdx.x; i < K; i += 1024) {
+      bool link = false;  // joined to cell i + 1
+      if (i < nc) {
+        const int32_t A = (int32_t)c0 + i;
+        const int q = A + 1 - (rows_of(d, A)[0] & kRowCellMask);
+        link = lane < 63 && i + 1 < nc && q < 5 && ((d.amask[A] >> q) & 1ull);
+      }
+      const unsigned long long heads = ~(ballot(link) << 1);
+      const int head = 63 - __clzll((long long)(heads & (~0ull >> (63 - lane))));
+      if (i < nc) par[i] = i - lane + head;
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < nc; i += 1024) {
+      const int32_t A = (int32_t)c0 + i;
+      unsigned long long m = d.amask[A];
+      if (!m) continue;
+      unsigned long long ext = 0ull;
+      const RowsOf rows = rows_of(d, A);
+      int32_t root = i;
+      while (m) {
+        const int b = __ffsll((long long)m) - 1;
+        const int r = (b * 205) >> 10;  // b / 5 for 0 <= b < 128
+        const int32_t B0 = (rows[r] & kRowCellMask) - (int32_t)c0 - 5 * r;
+        unsigned long long lm = m & (31ull << (5 * r));  // the bits of line r
+        m &= ~lm;
+        while (lm) {
+          const int q = __ffsll((long long)lm) - 1;
+          lm &= lm - 1;
+          if (B0 + q < nc)
+            root = lds_union(par, root, B0 + q);
+          else
+            ext |= 1ull << q;
+        }
+      }
+      d.amask[A] = ext;
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < nc; i += 1024) {
+      int32_t r = i;
+      while (par[r] != r) r = par[r];
+      d.parent[c0 + i] = (int32_t)c0 + r;
+    }
+    __syncthreads();
+  }
+}
+
+constexpr int kLinkSeen = 256;  // root pairs a wavefront remembers
+
+__global__ __launch_bounds__(256) void k_link_cross(Dev d) {
+  if (abandoned(d)) return;
+  __shared__ long long s_pre[kStripes + 1];
+  __shared__ unsigned long long s_seen[4][kLinkSeen];
+  __shared__ uint8_t s_tag[4][kLinkSeen];
+  const int lane = lane_id(), wv = threadIdx.x >> 6;
+  unsigned long long* seen = s_seen[wv];
+  uint8_t* tag = s_tag[wv];
+  for (int i = lane; i < kLinkSeen; i += 64) seen[i] = ~0ull;
+  const long long n = slist_prefix(d.core_cells, s_pre);
+  for (long long i0 = (long long)blockIdx.x * 256; i0 < n; i0 += (long long)gridDim.x * 256) {
+    const long long i = i0 + threadIdx.x;
+    const int32_t A = i < n ? slist_at(d.core_cells, s_pre, i) : -1;
+    unsigned long long m = A >= 0 ? d.amask[A] : 0ull;
+    const int32_t pa = m ? d.parent[A] : 0;
+    const RowsOf rows = rows_of(d, m ? A : 0);
+    while (ballot(m != 0ull)) {
+      int32_t pb = -1;
+      if (m) {
+        const int b = __ffsll((long long)m) - 1;
+        m &= m - 1;
+        const int r = (b * 205) >> 10;
+        pb = d.parent[(rows[r] & kRowCellMask) + (b - 5 * r)];
+      }
+      // neighbouring cells mostly name the same two roots: a pair in the
+      // wave's table is left out, and of the lanes that hold the same pair
+      // now, the one whose id survives in the pair's tag slot unites it
+      const unsigned long long key = ((unsigned long long)(uint32_t)pa << 32) | (uint32_t)pb;
+      const int h = (int)(((uint32_t)pa * 0x9E3779B1u ^ (uint32_t)pb * 0x85EBCA6Bu) >> 24);
+      bool nw = pb >= 0 && seen[h] != key;
+      if (nw) tag[h] = (uint8_t)lane;
+      wave_sync();
+      const int w = nw ? (int)tag[h] : lane;
+      const uint32_t wlo = (uint32_t)__shfl((int)(uint32_t)key, w, 64);
+      const uint32_t whi = (uint32_t)__shfl((int)(uint32_t)(key >> 32), w, 64);
+      if (w != lane && (((unsigned long long)whi << 32) | wlo) == key) nw = false;
+      if (nw) {
+        seen[h] = key;
+        uf_union(d.parent, pa, pb);
+      }
+      wave_sync();
+    }
+  }
+}
+
+// Component of every core cell (the root of its chain, or of the cell
+// itself without seed lists), the component minima of the core input index,
+// and the list of the roots.
+__global__ __launch_bounds__(256) void k_comp(Dev d) {
+  if (abandoned(d)) return;
+  __shared__ long long s_pre[kStripes + 1];
+  const long long n = slist_prefix(d.core_cells, s_pre);
+  for (long long i0 = (long long)blockIdx.x * 256; i0 < n; i0 += (long long)gridDim.x * 256) {
+    const long long i = i0 + threadIdx.x;
+    const bool act = i < n;
+    const int32_t A = act ? slist_at(d.core_cells, s_pre, i) : 0;
+    int32_t comp = -1, cmin = kNoKey;
+    if (act) {
+      cmin = d.orig[d.rep[A].w];
+      comp = uf_find(d.parent, d.chains ? d.cell_label[A] : A);
+      d.cell_comp[A] = comp;
+    }
+    // the wave's leading component: one atomic; the other lanes: one each,
+    // unless the minimum (a plain load is at worst too large) is already
+    // lower
+    const unsigned long long ma = ballot(act);
+    if (ma) {
+      const int32_t lead = rl_i(comp, __ffsll((long long)ma) - 1);
+      const bool mine = act && comp == lead;
+      const int32_t v = wave_min(mine ? cmin : kNoKey);
+      if (lane_id() == 0 && v < d.compmin[lead]) atomicMin(&d.compmin[lead], v);
+      if (act && !mine && cmin < d.compmin[comp]) atomicMin(&d.compmin[comp], cmin);
+    }
+    block_append(act && comp == A, A, d.near_roots);
+  }
+}
+
+// --------------------------------------------------- component borders --
 // Distance (fixed-point units) from a point at fraction f of its cell to
 // the cell o cells away along one axis (0 for o = 0).
 __device__ __forceinline__ float cell_gap(int o, int32_t f) {
@@ -349,19 +705,6 @@ __device__ __forceinline__ float cell_far(int o, int32_t f) {
   const int32_t g = o > 0 ? (o + 1) * W - f : (o < 0 ? f - o * W : (f > W - f ? f : W - f));
   return (float)g;
 }
-
-// Near and far stencil cells.  A stencil cell is "near" when it is at most
-// one cell away on every axis: the cells of lines 0..NN-1 (the lines whose
-// offsets are at most 1) with a last-axis offset of at most 1.  The other
-// stencil cells are "far".  Adjacency over near cells is computed for every
-// core cell and drives the seed-list expansion; a far pair is decided only
-// when its two cells are still in different components after the
-// expansion and merge (k_far), which is rare: in the interior of a cluster
-// the near cells already connect everything.
-template <int D>
-struct Near {
-  static constexpr int lines = D == 3 ? 9 : 3;
-};
 
 // Is some core point of A (points [qs, qe)) joined to some core point of B
 // (points [b0, b1), holding at least one core point)?  off = offset of B's
@@ -425,480 +768,14 @@ __device__ bool cells_joined(const Dev& d, const Par& P, int32_t qs, int32_t qe,
   return false;
 }
 
-// Offset along the last axis of cell B (in stencil line r of cell A).
-// (B lies in a neighbour line of A, so the difference of their last
-// coordinates is the offset.)
-template <int D>
-__device__ __forceinline__ int cell_offset_last(const Dev& d, const Inst& I, int32_t A, int32_t B,
-                                                int r) {
-  (void)I;
-  (void)r;
-  return d.cell_z[B] - d.cell_z[A];
-}
-
-// Near lines above the cell (every cell of them has a larger index): line
-// (0,0) (cells one step up the line only), (1,0), (0,1), (1,-1), (1,1) in
-// 3-D; (0) and (1) in 2-D.  Nibble i of the constant is the i-th such row.
-template <int D>
-struct Upper {
-  static constexpr int lines = D == 3 ? 5 : 2;
-  static constexpr unsigned long long rows = D == 3 ? 0x87420ull : 0x20ull;
-  // nibble r: the mirror of near row r (the line with negated offsets)
-  static constexpr unsigned long long mirror = D == 3 ? 0x567834120ull : 0x120ull;
-};
-
-// Near adjacency of light cells: one lane per core point p of a light cell
-// (compacted list written by k_core).  Adjacency is symmetric (edge_pair
-// is), so a pair of light cells is decided once, by the lower cell: its
-// lanes examine only the near lines above it (Upper) and the bits they find
-// are mirrored into the upper cell's mask at the end.  The lanes of one
-// cell examine those lines in a rotated order (lane rank r0 within the
-// cell's run of lanes starts at line r0) and share what they found through
-// LDS after each step, so a near cell found adjacent by one lane is not
-// tested again by the others.  A near cell is skipped when it is heavy (the
-// heavy-cell pass sets the bits of both cells), is already known adjacent,
-// or its box lies beyond eps of p; it is adjacent without a test when its
-// whole box lies inside the guard band around p and it holds a core point;
-// otherwise its core points are tested until one is joined to p.  The box
-// distances use the same fixed-point arithmetic as the distance, so they
-// bound it.
+// Core cell A, one lane: every stencil cell above A (each unordered pair is
+// taken by its lower cell) with core points in another component is decided;
+// a joined pair unions the two components (lock-free union-find on the chain
+// forest).  A pair whose components have been united meanwhile is skipped.
+// A pair with a heavy cell is listed for k_far_pairs (one wavefront per
+// pair); when its list is full the pair is decided here.
 template <int D, bool F32>
-__device__ void adj_lane(const Dev& d, const Inst& I, const Par& P, int32_t p, int32_t c,
-                         bool act, int head, int rank, int nrun, unsigned long long* xm,
-                         unsigned long long& m0, Tally& t, long long& freeb) {
-  constexpr int NN = Upper<D>::lines;
-  constexpr int B = 4;  // near cells need few tests: a short batch keeps registers low
-  constexpr uint32_t kFrac = (1u << kFixBits) - 1u;
-  uint32_t pg[D];
-  double px[D];
-  int32_t fr[D];
-#pragma unroll
-  for (int k = 0; k < D; ++k) pg[k] = act ? d.G[k][p] : 0u;
-#pragma unroll
-  for (int k = 0; k < D; ++k) px[k] = (!F32 && act) ? d.X[k][p] : 0.0;
-#pragma unroll
-  for (int k = 0; k < D; ++k) fr[k] = (int32_t)(pg[k] & kFrac);
-  const int32_t zA = act ? d.cell_z[c] : 0;
-  const RowsOf rows = rows_of(d, c);
-  // the next line's packed row is loaded while this line is examined
-  auto row_at = [](int i) { return (int)((Upper<D>::rows >> (4 * i)) & 15ull); };
-  int32_t pk_next = act ? rows[row_at(rank % NN)] : 0;
-  for (int step = 0; step < NN; ++step) {
-    const int r = row_at((step + rank) % NN);
-    const int o0 = D == 3 ? kRowOff3[r][0] : kRowOff2[r];
-    const int o1 = D == 3 ? kRowOff3[r][1] : 0;
-    const int32_t pk = pk_next;
-    if (step + 1 < NN) pk_next = act ? rows[row_at((step + 1 + rank) % NN)] : 0;
-    // own line: only the cell one step up; other lines: offsets -1..1
-    const int ol_lo = r == 0 ? 1 : -1;
-    const int32_t len = pk >> kRowCntShift;
-    if (len > 0) {
-      ++t.lines;
-      t.cells += len;
-      const int32_t st = pk & kRowCellMask;
-      int32_t bnd[6], nco[5], zb[5];
-      // unconditional loads at clamped indices (st + len <= C), so that all
-      // sixteen are in flight together; entries past the run are unused
-#pragma unroll
-      for (int k = 0; k < 6; ++k) bnd[k] = d.cell_start[k <= len ? st + k : st];
-#pragma unroll
-      for (int k = 0; k < 5; ++k) {
-        zb[k] = d.cell_z[k < len ? st + k : st];
-        nco[k] = d.cell_ncore[k < len ? st + k : st];
-      }
-      float g2 = 0.f, h2 = 0.f;  // over the line's axes
-      {
-        const float a = cell_gap(o0, fr[0]), fa = cell_far(o0, fr[0]);
-        g2 = a * a;
-        h2 = fa * fa;
-        if (D == 3) {
-          const float b = cell_gap(o1, fr[1]), fb = cell_far(o1, fr[1]);
-          g2 = __builtin_fmaf(b, b, g2);
-          h2 = __builtin_fmaf(fb, fb, h2);
-        }
-      }
-      int32_t aa[5], ll[5];
-      const int base = 5 * r;
-#pragma unroll
-      for (int k = 0; k < 5; ++k) {
-        const int32_t n = k < len ? bnd[k + 1] - bnd[k] : 0;
-        const int ol = zb[k] - zA;  // offset along the last axis
-        const float e = cell_gap(ol, fr[D - 1]), fe = cell_far(ol, fr[D - 1]);
-        const bool reach = !(__builtin_fmaf(e, e, g2) > P.d2_out);
-        const bool inside = __builtin_fmaf(fe, fe, h2) < P.d2_in;
-        bool use = k < len && ol >= ol_lo && ol <= 1 && nco[k] > 0 && n <= kHeavy && reach &&
-                   !((m0 >> (base + k)) & 1ull);
-        if (use && inside) {
-          // every point of the cell is joined to p, and one of them is core
-          m0 |= 1ull << (base + k);
-          ++freeb;
-          use = false;
-        }
-        aa[k] = bnd[k];
-        ll[k] = use ? n : 0;
-      }
-      Stream5 s;
-      s.set(aa, ll);
-      for (int32_t t0 = 0; t0 < s.tot; t0 += B) {
-        int32_t qi[B];
-        int kk[B];
-        bool cf[B], need[B];
-        uint8_t cb[B];
-        uint32_t cg[B][D];
-        double cx[B][D];
-        // flags and coordinates of the batch loaded together, unconditionally
-        // (qi is a point either way)
-#pragma unroll
-        for (int j = 0; j < B; ++j) {
-          int jr = 0;
-          const bool in = t0 + j < s.tot;
-          qi[j] = in ? s.at(t0 + j, jr) : p;
-          kk[j] = jr;
-          need[j] = in && !((m0 >> (base + jr)) & 1ull);
-          cb[j] = d.core[qi[j]];
-#pragma unroll
-          for (int k = 0; k < D; ++k) {
-            if (F32)
-              cg[j][k] = d.G[k][qi[j]];
-            else
-              cx[j][k] = d.X[k][qi[j]];
-          }
-        }
-#pragma unroll
-        for (int j = 0; j < B; ++j) cf[j] = need[j] && cb[j];
-#pragma unroll
-        for (int j = 0; j < B; ++j) {
-          if (cf[j] && !((m0 >> (base + kk[j])) & 1ull)) {
-            ++t.eval;
-            if (edge_pair<D, F32>(d, P, p, qi[j], pg, cg[j], px, cx[j], t))
-              m0 |= 1ull << (base + kk[j]);
-          }
-        }
-      }
-    }
-    // share this step's finds with the other lanes of the cell
-    if (act && m0) atomicOr(&xm[head], m0);
-    wave_sync();
-    if (act) m0 |= xm[head];
-  }
-  // m0 is now the cell's whole find (this wave's run of its lanes).  Each
-  // bit (line r, cell k of its run) names an upper cell B; A's bit in B's
-  // mask is in B's mirrored line rm, at A's place in that line's run.  The
-  // bits are dealt out over the run's lanes, four at a time per lane so
-  // that their loads overlap.
-  if (!act) return;
-  unsigned long long u = m0;
-  int j = 0;
-  while (u) {
-    int32_t tb[4], rm[4], pos[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      while (u && j % nrun != rank) {
-        u &= u - 1;
-        ++j;
-      }
-      const int b = u ? __ffsll((long long)u) - 1 : -1;
-      if (u) {
-        u &= u - 1;
-        ++j;
-      }
-      const int r = b >= 0 ? (b * 205) >> 10 : 0;  // b / 5 for 0 <= b < 128
-      rm[q] = (int)((Upper<D>::mirror >> (4 * r)) & 15ull);
-      tb[q] = b >= 0 ? (rows[r] & kRowCellMask) + (b - 5 * r) : -1;
-    }
-#pragma unroll
-    for (int q = 0; q < 4; ++q) pos[q] = tb[q] >= 0 ? rows_of(d, tb[q])[rm[q]] & kRowCellMask : 0;
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-      if (tb[q] >= 0) atomicOr(&d.amask[tb[q]], 1ull << (5 * rm[q] + (c - pos[q])));
-  }
-}
-
-template <bool F32>
-// 5 waves per SIMD (96 VGPRs, a few bytes of spill): the lanes are latency
-// bound, so residency pays more than the registers
-__global__ __launch_bounds__(256, 5) void k_adj(Dev d) {
-  if (abandoned(d)) return;
-  __shared__ unsigned long long s_m[4][64];
-  __shared__ long long s_pre[kStripes + 1];
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int lane = lane_id(), wv = threadIdx.x >> 6;
-  const bool act = i < slist_prefix(d.adj_pts, s_pre);
-  const int32_t p = act ? slist_at(d.adj_pts, s_pre, i) : 0;
-  const int32_t c = act ? d.cell_of[p] : -1;
-  // the lanes of one cell form a contiguous run; head = its first lane here
-  const int32_t cprev = __shfl_up(c, 1, 64);
-  const unsigned long long mh = ballot(act && (lane == 0 || cprev != c));
-  const unsigned long long below = lane == 63 ? mh : (mh & ((2ull << lane) - 1ull));
-  const int head = below ? 63 - __clzll((long long)below) : 0;
-  const int rank = lane - head;
-  // run length: up to the next head or the end of the active lanes (a prefix)
-  const unsigned long long above = head == 63 ? 0ull : (mh & (~0ull << (head + 1)));
-  const int nact = __popcll(ballot(act));
-  const int nrun = (above ? __ffsll((long long)above) - 1 : nact) - head;
-  s_m[wv][lane] = 0ull;
-  wave_sync();
-  int dim = 0;
-  const Inst* I = d.inst;
-  if (act) {
-    I = inst_of_cell(d, c);
-    dim = I->dim;
-  }
-  Tally t;
-  long long freeb = 0;
-  unsigned long long m0 = 0;
-  const Par P(*I);
-  // every lane runs the line loop (inactive lanes only take part in the
-  // exchange), so the exchange points are uniform over the wave
-  const bool any3 = ballot(act && dim == 3) != 0, any2 = ballot(act && dim == 2) != 0;
-  if (any3)
-    adj_lane<3, F32>(d, *I, P, p, c, act && dim == 3, head, rank, nrun, s_m[wv], m0, t, freeb);
-  if (any2)
-    adj_lane<2, F32>(d, *I, P, p, c, act && dim == 2, head, rank, nrun, s_m[wv], m0, t, freeb);
-  // one atomic per cell run: the exchange slot of its head lane holds the
-  // union of the run's finds
-  if (act && lane == head) {
-    const unsigned long long u = s_m[wv][lane];
-    if (u) atomicOr(&d.amask[c], u);
-  }
-  stat_add(d, C_BAND, t.band);
-  stat_add(d, C_ASYM, t.asym);
-  stat_add(d, C_ADJ_TESTS, t.eval);
-  stat_add(d, C_ADJ_FREE, freeb);
-  stat_add(d, C_ADJ_LINES, t.lines);
-  stat_add(d, C_ADJ_CELLS, t.cells);
-}
-
-// Heavy cell A (more than kHeavy points), one wavefront, near cells only:
-// its core points are the queries (the first kQCache cached in LDS).  Each
-// near cell with core points is decided in turn: its core points within
-// eps of the queries' bounding box are the candidates (one per lane), and
-// the queries near the candidates' bounding box are tried until some lane
-// finds a joined pair.  Light neighbours never test a heavy cell, so A
-// decides every light neighbour; a pair of heavy cells is decided once, by
-// the lower cell.  A joined neighbour also gets the mirrored bit (A lies in
-// its mirrored stencil line), and A's own bits are OR-ed into its mask
-// (lower heavy neighbours set bits there too).
-template <int D, bool F32>
-__device__ void adj_heavy(const Dev& d, const Inst& I, const Par& P, int32_t A, int32_t* s_qi,
-                          uint32_t* s_qg, double* s_qx, Tally& t) {
-  constexpr int NN = Near<D>::lines;
-  const int lane = lane_id();
-  const int32_t qs = d.cell_start[A], qe = d.cell_start[A + 1];
-  const int32_t ncA = d.cell_ncore[A];
-  if (ncA == 0) return;  // no core point: the mask stays clear
-  const bool allc = ncA == qe - qs;
-  uint32_t blo[D], bhi[D];
-#pragma unroll
-  for (int k = 0; k < D; ++k) {
-    blo[k] = 0xffffffffu;
-    bhi[k] = 0u;
-  }
-  int nq = 0;
-  for (int32_t i0 = qs; i0 < qe; i0 += 64) {
-    const int32_t i = i0 + lane;
-    const bool v = i < qe && (allc || d.core[i]);
-    uint32_t g[D];
-#pragma unroll
-    for (int k = 0; k < D; ++k) {
-      g[k] = v ? d.G[k][i] : 0u;
-      blo[k] = v && g[k] < blo[k] ? g[k] : blo[k];
-      bhi[k] = v && g[k] > bhi[k] ? g[k] : bhi[k];
-    }
-    const unsigned long long m = ballot(v);
-    const int pos = nq + mbcnt(m);
-    if (v && pos < kQCache) {
-      s_qi[pos] = i;
-#pragma unroll
-      for (int k = 0; k < D; ++k) {
-        s_qg[pos * 3 + k] = g[k];
-        if (!F32) s_qx[pos * 3 + k] = d.X[k][i];
-      }
-    }
-    nq += __popcll(m);
-  }
-#pragma unroll
-  for (int k = 0; k < D; ++k) {
-    blo[k] = wave_min(blo[k]);
-    bhi[k] = wave_max(bhi[k]);
-  }
-  wave_sync();
-  const bool cached = nq <= kQCache;
-  const int NQ = cached ? nq : (qe - qs);
-  const int32_t pkl = lane < NN ? rows_of(d, A)[lane] : 0;
-  unsigned long long m0 = 0;
-  for (int r = 0; r < NN; ++r) {
-    const int32_t pk = rl_i(pkl, r);
-    const int32_t len = pk >> kRowCntShift, st = pk & kRowCellMask;
-    for (int k = 0; k < len; ++k) {
-      const int32_t Bc = st + k;
-      if (Bc == A) continue;
-      const int ol = cell_offset_last<D>(d, I, A, Bc, r);
-      if (ol < -1 || ol > 1) continue;  // a far cell
-      const int32_t b0 = d.cell_start[Bc], b1 = d.cell_start[Bc + 1];
-      if (d.cell_ncore[Bc] == 0) continue;
-      if (Bc < A && b1 - b0 > kHeavy) continue;  // decided by the lower heavy cell
-      bool edge = false;
-      for (int32_t c0 = b0; c0 < b1 && !edge; c0 += 64) {
-        const int32_t q = c0 + lane;
-        bool cand = q < b1 && d.core[q];
-        uint32_t cg[D];
-        double cx[D];
-#pragma unroll
-        for (int kk = 0; kk < D; ++kk) cg[kk] = cand ? d.G[kk][q] : 0u;
-        cand = cand && !(d2box<D>(cg, blo, bhi) > P.d2_out);
-        if (!ballot(cand)) continue;
-#pragma unroll
-        for (int kk = 0; kk < D; ++kk) cx[kk] = (!F32 && cand) ? d.X[kk][q] : 0.0;
-        uint32_t clo[D], chi[D];
-#pragma unroll
-        for (int kk = 0; kk < D; ++kk) {
-          clo[kk] = wave_min(cand ? cg[kk] : 0xffffffffu);
-          chi[kk] = wave_max(cand ? cg[kk] : 0u);
-        }
-        for (int i = 0; i < NQ && !edge; ++i) {
-          int32_t ui;
-          uint32_t ug[D];
-          double ux[D];
-          if (cached) {
-            ui = s_qi[i];
-#pragma unroll
-            for (int kk = 0; kk < D; ++kk) {
-              ug[kk] = s_qg[i * 3 + kk];
-              ux[kk] = F32 ? 0.0 : s_qx[i * 3 + kk];
-            }
-          } else {
-            ui = qs + i;
-            if (!allc && !d.core[ui]) continue;
-#pragma unroll
-            for (int kk = 0; kk < D; ++kk) {
-              ug[kk] = d.G[kk][ui];
-              ux[kk] = F32 ? 0.0 : d.X[kk][ui];
-            }
-          }
-          if (d2box<D>(ug, clo, chi) > P.d2_out) continue;
-          const bool hit = cand && edge_pair<D, F32>(d, P, ui, q, ug, cg, ux, cx, t);
-          edge = ballot(hit) != 0;
-        }
-      }
-      if (edge) {
-        m0 |= 1ull << (5 * r + k);
-        const int rm = D == 3 ? kRowMirror3[r] : kRowMirror2[r];
-        const int32_t pm = rows_of(d, Bc)[rm];
-        const int bm = 5 * rm + (A - (pm & kRowCellMask));
-        if (lane == 0) atomicOr(&d.amask[Bc], 1ull << bm);
-      }
-    }
-  }
-  if (lane == 0 && m0) atomicOr(&d.amask[A], m0);
-}
-
-template <bool F32>
-__global__ __launch_bounds__(64) void k_adj_heavy(Dev d) {
-  if (abandoned(d)) return;
-  __shared__ int32_t s_qi[kQCache];
-  __shared__ uint32_t s_qg[kQCache * 3];
-  __shared__ double s_qx[F32 ? 1 : kQCache * 3];
-  __shared__ long long s_pre[kStripes + 1];
-  const long long nh = slist_prefix(d.heavy, s_pre);
-  Tally t;
-  for (long long h = blockIdx.x; h < nh; h += gridDim.x) {
-    const int32_t A = slist_at(d.heavy, s_pre, h);
-    const Inst& I = *inst_of_cell(d, A);
-    const Par P(I);
-    if (I.dim == 3)
-      adj_heavy<3, F32>(d, I, P, A, s_qi, s_qg, s_qx, t);
-    else
-      adj_heavy<2, F32>(d, I, P, A, s_qi, s_qg, s_qx, t);
-    wave_sync();  // the query cache is reused
-  }
-  stat_add(d, C_BAND, t.band);
-  stat_add(d, C_ASYM, t.asym);
-}
-
-// ------------------------------------------------------------ far pairs --
-// Component of every core cell after the expansion and merge (the root of
-// its chain), and the compacted list of core cells.
-__global__ __launch_bounds__(1024) void k_cell_comp(Dev d) {
-  if (abandoned(d)) return;
-  const int64_t C = d.ctl[C_NCELL];
-  {
-    const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const bool in = c < C;
-    const int64_t cc = in ? c : 0;
-    // every load before the store (which could alias them as far as the
-    // compiler knows), each level of dependent loads issued together
-    const int32_t ncore = d.cell_ncore[cc], q0 = d.cell_start[cc], q1 = d.cell_start[cc + 1];
-    const int32_t lab = d.cell_label[cc];
-    const bool hc = in && ncore > 0;
-    int32_t chain = -1, cmin = kNoKey, comp = -1;
-    if (hc) {
-      chain = lab;
-      comp = d.parent[chain];
-      // the sort is stable, so input indices increase within a cell: the
-      // cell's smallest core index is that of its first core point
-      int32_t q = q0;
-      if (ncore != q1 - q0)
-        while (!d.core[q]) ++q;
-      cmin = d.orig[q];
-    }
-    if (in) d.cell_comp[c] = comp;
-    // chain minimum: one atomic per distinct chain of the wave
-    bool pend = hc;
-    unsigned long long m = ballot(pend);
-    while (m) {
-      const int32_t lead = rl_i(chain, __ffsll((long long)m) - 1);
-      const bool mine = pend && chain == lead;
-      const int32_t v = wave_min(mine ? cmin : kNoKey);
-      if (lane_id() == 0) atomicMin(&d.compmin[lead], v);
-      pend = pend && !mine;
-      m = ballot(pend);
-    }
-    block_append(hc, (int32_t)c, d.core_cells);
-  }
-}
-
-// Core cell A, one lane: every far stencil cell above A (each unordered pair
-// is taken by its lower cell) with core points in another component is
-// decided; a joined pair unions the two components (lock-free union-find on
-// the chain forest).
-// Stencil lines whose cells can lie above a cell (offsets (a, b) >= (0, 0)
-// in the key order, the own line included), in row order; -1 pads.
-#define DCLUST_UPPER_ROWS3 {0, 2, 4, 7, 8, 10, 12, 15, 16, 18, 20, 23, 24, -1, -1}
-#define DCLUST_UPPER_ROWS2 {0, 2, 4, -1, -1}
-static __constant__ int8_t kUpperRows3[15] = DCLUST_UPPER_ROWS3;
-static __constant__ int8_t kUpperRows2[5] = DCLUST_UPPER_ROWS2;
-namespace tables {
-constexpr int8_t up3[15] = DCLUST_UPPER_ROWS3;
-constexpr int8_t up2[5] = DCLUST_UPPER_ROWS2;
-constexpr bool above(int a, int b) { return a > 0 || (a == 0 && b >= 0); }
-constexpr bool upper_ok() {
-  int i = 0;
-  for (int r = 0; r < 25; ++r)
-    if (above(off3[r][0], off3[r][1]) && up3[i++] != r) return false;
-  if (i != 13 || up3[13] != -1 || up3[14] != -1) return false;
-  i = 0;
-  for (int r = 0; r < 5; ++r)
-    if (off2[r] >= 0 && up2[i++] != r) return false;
-  if (i != 3) return false;
-  // near rows of the adjacency pass (nibbles) and their mirrors
-  for (int k = 0; k < 5; ++k) {
-    const int r = (int)((Upper<3>::rows >> (4 * k)) & 15ull);
-    if (r > 8 || !above(off3[r][0], off3[r][1]) || up3[k] != r) return false;
-  }
-  for (int r = 0; r < 9; ++r)
-    if ((int)((Upper<3>::mirror >> (4 * r)) & 15ull) != mir3[r]) return false;
-  for (int k = 0; k < 2; ++k)
-    if ((int)((Upper<2>::rows >> (4 * k)) & 15ull) != up2[k]) return false;
-  for (int r = 0; r < 3; ++r)
-    if ((int)((Upper<2>::mirror >> (4 * r)) & 15ull) != mir2[r]) return false;
-  return true;
-}
-static_assert(upper_ok(), "upper stencil lines");
-}  // namespace tables
-
-template <int D, bool F32>
-__device__ long long far_cell(const Dev& d, const Inst& I, const Par& P, int32_t A, Tally& t,
+__device__ long long far_cell(const Dev& d, const Par& P, int32_t A, Tally& t,
                               long long& freeb) {
   constexpr int NR = D == 3 ? 13 : 3;  // upper lines
   const int32_t qs = d.cell_start[A], qe = d.cell_start[A + 1];
@@ -942,21 +819,29 @@ __device__ long long far_cell(const Dev& d, const Inst& I, const Par& P, int32_t
         r = j == q ? rr[q] : r;
       }
       const int32_t B = (pkj & kRowCellMask) + k;
+      // B's place along the line, its point range and both roots, together
+      const int32_t zB = d.cell_z[B], b0 = d.cell_start[B], b1 = d.cell_start[B + 1];
+      const int32_t compB = d.cell_comp[B];
+      const int32_t ra = uf_find_cached(d.parent, compA), rb = uf_find_cached(d.parent, compB);
+      if (ra == rb) continue;
+      if (qe - qs > kHeavy || b1 - b0 > kHeavy) {
+        const int s = blockIdx.x & (kStripes - 1);
+        const unsigned long long at = atomicAdd(&d.far_pairs.cnt[s], 1ull);
+        if (at < (unsigned long long)d.far_pairs.cap) {
+          d.far_pairs.data[s * d.far_pairs.cap + (int64_t)at] = make_int2(A, B);
+          continue;
+        }
+      }
       const int o0 = D == 3 ? kRowOff3[r][0] : kRowOff2[r];
       const int o1 = D == 3 ? kRowOff3[r][1] : 0;
-      const bool far_l = o0 == 2 || o0 == -2 || o1 == 2 || o1 == -2;
-      // B's place along the line and its point range, loaded together
-      const int32_t zB = d.cell_z[B], b0 = d.cell_start[B], b1 = d.cell_start[B + 1];
-      const int ol = zB - zA;  // B lies in a neighbour line of A
-      // in a near line only the cells two steps away along the line are far
-      if (!far_l && ol != 2 && ol != -2) continue;
-      if (cells_joined<D, F32>(d, P, qs, qe, allc, b0, b1, o0, o1, ol, t, freeb)) {
-        uf_union(d.parent, compA, d.cell_comp[B]);
+      // (B lies in a neighbour line of A: the difference of their last
+      // coordinates is the offset)
+      if (cells_joined<D, F32>(d, P, qs, qe, allc, b0, b1, o0, o1, zB - zA, t, freeb)) {
+        uf_union(d.parent, ra, rb);
         ++joins;
       }
     }
   }
-  (void)I;
   return joins;
 }
 
@@ -964,49 +849,170 @@ template <bool F32>
 __global__ __launch_bounds__(256, 5) void k_far(Dev d) {
   if (abandoned(d)) return;
   __shared__ long long s_pre[kStripes + 1];
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const bool act = i < slist_prefix(d.core_cells, s_pre);
-  const int32_t A = act ? slist_at(d.core_cells, s_pre, i) : 0;
-  int dim = 0;
-  const Inst* I = d.inst;
-  if (act) {
-    I = inst_of_cell(d, A);
-    dim = I->dim;
-  }
+  const long long n = slist_prefix(d.core_cells, s_pre);
   Tally t;
   long long freeb = 0, joins = 0;
-  const Par P(*I);
-  DCLUST_BY_DIM(act, dim, (joins = far_cell<3, F32>(d, *I, P, A, t, freeb)),
-                (joins = far_cell<2, F32>(d, *I, P, A, t, freeb)));
+  for (long long i0 = (long long)blockIdx.x * 256; i0 < n; i0 += (long long)gridDim.x * 256) {
+    const long long i = i0 + threadIdx.x;
+    const bool act = i < n;
+    const int32_t A = act ? slist_at(d.core_cells, s_pre, i) : 0;
+    int dim = 0;
+    const Inst* I = d.inst;
+    if (act) {
+      I = inst_of_cell(d, A);
+      dim = I->dim;
+    }
+    const Par P(*I);
+    DCLUST_BY_DIM(act, dim, (joins += far_cell<3, F32>(d, P, A, t, freeb)),
+                  (joins += far_cell<2, F32>(d, P, A, t, freeb)));
+  }
+  stat_add(d, C_BAND, t.band);
+  stat_add(d, C_ASYM, t.asym);
+  stat_add(d, C_FAR_TESTS, t.eval);
+  stat_add(d, C_ADJ_FREE, freeb);
+  stat_add(d, C_FAR_JOINS, joins);
+}
+
+// Is some core point of A joined to some core point of B?  The whole
+// wavefront: 64 points of A and 64 of B at a time, one of each per lane.
+// B's points beyond eps of the box of A's are dropped, then A's points
+// beyond eps of the box of those left; the rest are tried in turn (broadcast
+// from their lane) against all lanes, until one joins.
+template <int D, bool F32>
+__device__ bool wave_joined(const Dev& d, const Par& P, int32_t A, int32_t B, Tally& t) {
+  const int lane = lane_id();
+  const int32_t a0 = d.cell_start[A], a1 = d.cell_start[A + 1];
+  const int32_t b0 = d.cell_start[B], b1 = d.cell_start[B + 1];
+  for (int32_t ac = a0; ac < a1; ac += 64) {
+    const int32_t p = ac + lane < a1 ? ac + lane : a0;
+    const bool av = ac + lane < a1 && d.core[p];
+    if (!ballot(av)) continue;
+    uint32_t ag[D], alo[D], ahi[D];
+    double ax[D];
+#pragma unroll
+    for (int k = 0; k < D; ++k) {
+      ag[k] = d.G[k][p];
+      ax[k] = F32 ? 0.0 : d.X[k][p];
+    }
+    // (coordinates of one cell's points do not wrap against each other)
+#pragma unroll
+    for (int k = 0; k < D; ++k) {
+      alo[k] = wave_min(av ? ag[k] : 0xffffffffu);
+      ahi[k] = wave_max(av ? ag[k] : 0u);
+    }
+    for (int32_t bc = b0; bc < b1; bc += 64) {
+      const int32_t q = bc + lane < b1 ? bc + lane : b0;
+      uint32_t bg[D], blo[D], bhi[D];
+      double bx[D];
+#pragma unroll
+      for (int k = 0; k < D; ++k) {
+        bg[k] = d.G[k][q];
+        bx[k] = F32 ? 0.0 : d.X[k][q];
+      }
+      const bool bv = bc + lane < b1 && d.core[q] && !(d2box<D>(bg, alo, ahi) > P.d2_out);
+      if (!ballot(bv)) continue;
+#pragma unroll
+      for (int k = 0; k < D; ++k) {
+        blo[k] = wave_min(bv ? bg[k] : 0xffffffffu);
+        bhi[k] = wave_max(bv ? bg[k] : 0u);
+      }
+      unsigned long long m = ballot(av && !(d2box<D>(ag, blo, bhi) > P.d2_out));
+      while (m) {
+        const int l = __ffsll((long long)m) - 1;
+        m &= m - 1;
+        uint32_t ug[D];
+        double ux[D];
+#pragma unroll
+        for (int k = 0; k < D; ++k) {
+          ug[k] = rl_u(ag[k], l);
+          ux[k] = F32 ? 0.0 : rl_d(ax[k], l);
+        }
+        bool hit = false;
+        if (bv) {
+          ++t.eval;
+          hit = edge_pair<D, F32>(d, P, ac + l, q, ug, bg, ux, bx, t);
+        }
+        if (ballot(hit)) return true;
+      }
+    }
+  }
+  return false;
+}
+
+// The listed pairs with a heavy cell, one wavefront each; a pair whose
+// components have been united meanwhile is skipped.
+template <bool F32>
+__global__ __launch_bounds__(256) void k_far_pairs(Dev d) {
+  if (abandoned(d)) return;
+  __shared__ long long s_pre[kStripes + 1];
+  if (threadIdx.x < kStripes) {
+    const long long v = (long long)d.far_pairs.cnt[threadIdx.x];
+    const long long incl = wave_incl_scan(v < d.far_pairs.cap ? v : (long long)d.far_pairs.cap);
+    s_pre[threadIdx.x + 1] = incl;
+    if (threadIdx.x == 0) s_pre[0] = 0;
+  }
+  __syncthreads();
+  const long long n = s_pre[kStripes];
+  Tally t;
+  long long joins = 0;
+  for (long long i = (long long)blockIdx.x * 4 + (threadIdx.x >> 6); i < n;
+       i += (long long)gridDim.x * 4) {
+    int lo = 0, hi = kStripes - 1;  // last sub-list whose range starts at or before i
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (s_pre[mid] <= i) lo = mid; else hi = mid - 1;
+    }
+    const int2 pr = d.far_pairs.data[(int64_t)lo * d.far_pairs.cap + (i - s_pre[lo])];
+    const int32_t A = rfl_i(pr.x), B = rfl_i(pr.y);
+    // every lane walks the same path: the roots are wave-uniform up to the
+    // moment of each load, so lane 0's are taken
+    const int32_t ra = rfl_i(uf_find_cached(d.parent, d.cell_comp[A]));
+    const int32_t rb = rfl_i(uf_find_cached(d.parent, d.cell_comp[B]));
+    if (ra == rb) continue;
+    const Inst& I = *inst_of_cell(d, A);
+    const Par P(I);
+    const bool j = I.dim == 3 ? wave_joined<3, F32>(d, P, A, B, t)
+                              : wave_joined<2, F32>(d, P, A, B, t);
+    if (j && lane_id() == 0) {
+      uf_union(d.parent, ra, rb);
+      ++joins;
+    }
+  }
   stat_add(d, C_BAND, t.band);
   stat_add(d, C_ASYM, t.asym);
   stat_add(d, C_FAR_TESTS, t.eval);
   stat_add(d, C_FAR_JOINS, joins);
 }
 
-// Roots of every chain after the far-pair unions, in two passes.  The first
-// compresses the forest with path-halving walks; a concurrent walk may
-// leave an entry at an inner ancestor instead of the root, so the second
+// Roots of the near components after the unions across their borders, in two
+// passes over the list of near roots (no other entry is a component id).
+// The first compresses the forest with path-halving walks; a concurrent walk
+// may leave an entry at an inner ancestor instead of the root, so the second
 // pass walks the (now shallow) forest without writing anything but each
-// chain's own root, and moves each chain's minimum core input index to its
+// near root's own entry, and moves its minimum core input index to its final
 // root: every entry is then exactly its root.
 __global__ __launch_bounds__(256) void k_flatten_all(Dev d) {
   if (abandoned(d)) return;
-  const long long nc = chain_ids(d);
-  for (long long c = blockIdx.x * (long long)blockDim.x + threadIdx.x; c < nc;
-       c += (long long)gridDim.x * blockDim.x)
-    d.parent[c] = uf_find(d.parent, (int32_t)c);
+  __shared__ long long s_pre[kStripes + 1];
+  const long long n = slist_prefix(d.near_roots, s_pre);
+  for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n;
+       i += (long long)gridDim.x * 256) {
+    const int32_t c = slist_at(d.near_roots, s_pre, i);
+    d.parent[c] = uf_find(d.parent, c);
+  }
 }
 
 __global__ __launch_bounds__(256) void k_roots_final(Dev d) {
   if (abandoned(d)) return;
-  const long long nc = chain_ids(d);
-  for (long long c = blockIdx.x * (long long)blockDim.x + threadIdx.x; c < nc;
-       c += (long long)gridDim.x * blockDim.x) {
+  __shared__ long long s_pre[kStripes + 1];
+  const long long n = slist_prefix(d.near_roots, s_pre);
+  for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n;
+       i += (long long)gridDim.x * 256) {
+    const int32_t c = slist_at(d.near_roots, s_pre, i);
     const int32_t m = d.compmin[c];
-    const int32_t r = uf_root(d.parent, (int32_t)c);
+    const int32_t r = uf_root(d.parent, c);
     d.parent[c] = r;
-    if (m != kNoKey && r != c) atomicMin(&d.compmin[r], m);
+    if (r != c && m < d.compmin[r]) atomicMin(&d.compmin[r], m);
   }
 }
 
@@ -1362,16 +1368,6 @@ __global__ __launch_bounds__(256) void k_pass_carry(Dev d, int pass, int check) 
 constexpr int kLdsChains = 32768;  // 128 KiB of LDS (gfx950 allows 160 KiB per workgroup)
 constexpr int kMergeChunk = 4096;  // pair buffers scanned at a time (16 KiB of LDS)
 
-__device__ __forceinline__ int32_t lds_find(int32_t* par, int32_t x) {
-  for (;;) {
-    int32_t p = par[x];
-    if (p == x) return x;
-    int32_t gp = par[p];
-    if (gp != p) par[x] = gp;
-    x = p;
-  }
-}
-
 // number of expansion waves whose pair buffers are in use
 __device__ __forceinline__ int64_t pair_waves(const Dev& d) { return d.pair_cap / d.pair_per; }
 
@@ -1432,18 +1428,7 @@ __global__ __launch_bounds__(1024) void k_merge_lds(Dev d) {
       }
 #pragma unroll
       for (int j = 0; j < kBatch; ++j) {
-        int32_t a = lds_find(par, pr[j].x), b = lds_find(par, pr[j].y);
-        while (a != b) {
-          if (a < b) {
-            int32_t tt = a;
-            a = b;
-            b = tt;
-          }
-          int32_t old = atomicCAS(&par[a], a, b);
-          if (old == a) break;
-          a = lds_find(par, old);
-          b = lds_find(par, b);
-        }
+        lds_union(par, pr[j].x, pr[j].y);
       }
     }
     __syncthreads();  // s_pre is rewritten by the next chunk
@@ -1479,11 +1464,6 @@ __global__ __launch_bounds__(256) void k_flatten(Dev d) {
     d.parent[c] = uf_find(d.parent, (int32_t)c);
 }
 
-// chain of a core point: the chain that claimed its cell
-__device__ __forceinline__ int32_t core_chain(const Dev& d, int64_t i) {
-  return d.core[i] ? d.cell_label[d.cell_of[i]] : -1;
-}
-
 // Points per thread step of the per-point relabel passes: each level of
 // their dependent loads is issued for all of them before the next level,
 // and nothing is stored until every load is done, so the latencies overlap.
@@ -1504,9 +1484,9 @@ __global__ __launch_bounds__(256) void k_keys(Dev d) {
       c[u] = d.cell_of[ic[u]];
       o[u] = d.orig[ic[u]];
     }
-    // (a core point's cell is claimed by a chain; other lanes read index 0)
+    // (a core point's cell has a component; the others read entry 0)
 #pragma unroll
-    for (int u = 0; u < kRelU; ++u) li[u] = cr[u] ? d.cell_label[c[u]] : 0;
+    for (int u = 0; u < kRelU; ++u) li[u] = cr[u] ? d.cell_comp[c[u]] : 0;
 #pragma unroll
     for (int u = 0; u < kRelU; ++u) pr[u] = d.parent[li[u]];
 #pragma unroll
@@ -1730,19 +1710,16 @@ __global__ __launch_bounds__(256) void k_output(Dev d) {
 }
 
 // Per-run state of the clustering phases, one launch after the index:
-// chain labels of the cells (unclaimed), the chain forest (every id its own
-// root), component minima, component flags, per-cell core counts (all over
-// the n entries that bound the cells and chain ids), and per expansion
-// wave its pair count and the start of its seeding segment of the cells.
+// component-minimum flags and per-cell core counts (over the n entries that
+// bound the input indices and cells), and per expansion wave (`waves` is 0
+// without seed lists) its pair count and the start of its seeding segment of
+// the cells.  k_rep starts the per-cell state.
 __global__ void k_init_run(Dev d, int64_t waves) {
   const int64_t m = d.n > waves ? d.n : waves;
   const int64_t C = d.ctl[C_NCELL];
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < m;
        i += (int64_t)gridDim.x * blockDim.x) {
     if (i < d.n) {
-      d.cell_label[i] = kUnclaimed;
-      d.parent[i] = (int32_t)i;
-      d.compmin[i] = kNoKey;
       d.flag[i] = 0;
       d.cell_ncore[i] = 0;
     }
@@ -1769,7 +1746,11 @@ static int point_grid(int64_t n) {
 }
 
 int64_t point_blocks(int64_t n) { return point_grid(n); }
-int64_t cell_comp_blocks(int64_t n) { return (n + 1023) / 1024 > 0 ? (n + 1023) / 1024 : 1; }
+int64_t list_append_cap(int64_t n) {
+  const int64_t g = std::min(kListGrid, point_grid(n));
+  return (g + kStripes - 1) / kStripes * 256 * ((n + g * 256 - 1) / (g * 256));
+}
+int64_t cell_blocks(int64_t n) { return (n + 1023) / 1024 > 0 ? (n + 1023) / 1024 : 1; }
 
 void launch_core(const Dev& d, bool f32, hipStream_t s) {
   if (f32)
@@ -1778,23 +1759,23 @@ void launch_core(const Dev& d, bool f32, hipStream_t s) {
     hipLaunchKernelGGL(k_core<false>, dim3(point_grid(d.n)), dim3(256), 0, s, d);
 }
 
-void launch_adj_light(const Dev& d, bool f32, hipStream_t s) {
-  if (f32)
-    hipLaunchKernelGGL(k_adj<true>, dim3(point_grid(d.n)), dim3(256), 0, s, d);
-  else
-    hipLaunchKernelGGL(k_adj<false>, dim3(point_grid(d.n)), dim3(256), 0, s, d);
+// one lane per listed core cell, grid-stride
+static int list_grid(int64_t n) { return std::min(kListGrid, point_grid(n)); }
+
+void launch_near(const Dev& d, hipStream_t s) {
+  hipLaunchKernelGGL(k_rep, dim3((unsigned)cell_blocks(d.n)), dim3(1024), 0, s, d);
+  hipLaunchKernelGGL(k_adj, dim3(list_grid(d.n)), dim3(256), 0, s, d);
 }
 
-void launch_adj_heavy(const Dev& d, bool f32, int heavy_grid, hipStream_t s) {
-  if (f32)
-    hipLaunchKernelGGL(k_adj_heavy<true>, dim3(heavy_grid), dim3(64), 0, s, d);
-  else
-    hipLaunchKernelGGL(k_adj_heavy<false>, dim3(heavy_grid), dim3(64), 0, s, d);
+void launch_link(const Dev& d, hipStream_t s) {
+  const int64_t runs = (d.n + kLinkMin - 1) / kLinkMin;
+  hipLaunchKernelGGL(k_link_local, dim3((unsigned)std::min<int64_t>(kLinkGrid, runs)), dim3(1024),
+                     0, s, d);
+  hipLaunchKernelGGL(k_link_cross, dim3(list_grid(d.n)), dim3(256), 0, s, d);
 }
 
-void launch_adj(const Dev& d, bool f32, int heavy_grid, hipStream_t s) {
-  launch_adj_light(d, f32, s);
-  launch_adj_heavy(d, f32, heavy_grid, s);
+void launch_comp(const Dev& d, hipStream_t s) {
+  hipLaunchKernelGGL(k_comp, dim3(list_grid(d.n)), dim3(256), 0, s, d);
 }
 
 void launch_pass_prep(const Dev& d, int pass, hipStream_t s) {
@@ -1826,13 +1807,16 @@ void launch_merge(const Dev& d, int grid, hipStream_t s) {
 }
 
 void launch_far(const Dev& d, bool f32, int grid, hipStream_t s) {
-  hipLaunchKernelGGL(k_cell_comp, dim3(cell_comp_blocks(d.n)), dim3(1024), 0, s, d);
-  if (f32)
-    hipLaunchKernelGGL(k_far<true>, dim3(point_grid(d.n)), dim3(256), 0, s, d);
-  else
-    hipLaunchKernelGGL(k_far<false>, dim3(point_grid(d.n)), dim3(256), 0, s, d);
-  hipLaunchKernelGGL(k_flatten_all, dim3(grid), dim3(256), 0, s, d);
-  hipLaunchKernelGGL(k_roots_final, dim3(grid), dim3(256), 0, s, d);
+  if (f32) {
+    hipLaunchKernelGGL(k_far<true>, dim3(list_grid(d.n)), dim3(256), 0, s, d);
+    hipLaunchKernelGGL(k_far_pairs<true>, dim3(grid), dim3(256), 0, s, d);
+  } else {
+    hipLaunchKernelGGL(k_far<false>, dim3(list_grid(d.n)), dim3(256), 0, s, d);
+    hipLaunchKernelGGL(k_far_pairs<false>, dim3(grid), dim3(256), 0, s, d);
+  }
+  const int g = std::min(grid, list_grid(d.n));
+  hipLaunchKernelGGL(k_flatten_all, dim3(g), dim3(256), 0, s, d);
+  hipLaunchKernelGGL(k_roots_final, dim3(g), dim3(256), 0, s, d);
 }
 
 void launch_border(const Dev& d, bool f32, hipStream_t s) {

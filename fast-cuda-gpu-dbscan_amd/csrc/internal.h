@@ -6,12 +6,12 @@
 //   sort    key[2]    u64 cell keys (ping-pong), val[2] i32 point ids
 //   CSR     cell_start[C+1], cell_key[C], cell_inst[C], rows[C][25] (packed
 //           runs of the 5^(D-1) neighbour lines, centre line first),
-//           cell_ncore[C], cell_label[C] (chain), amask[C] (near adjacency)
+//           cell_ncore[C], cell_label[C] (chain), amask[C] (near graph), rep[C]
 //   points  (cell-sorted)  X[3][N] FP64 SoA (FP64 form only), G[3][N] u32 fixed-point
 //           coordinates (29 fraction bits per cell, wrapping mod 8 cells),
 //           orig[N], cell_of[N], core[N] u8, rec[N][R] + rec_n[N] (the
 //           neighbours of each non-core point)
-//   merge   parent[] chain union-find, compmin[N], pairs[waves][E] int2
+//   merge   parent[] union-find over cells, compmin[N], pairs[waves][E] int2
 //   output  keyv[N] (component min input index), flag[N] u8, rank[N]
 #pragma once
 #include <hip/hip_runtime.h>
@@ -28,7 +28,7 @@ constexpr int kMaxRows = 25;  // 5^(D-1) neighbour lines for D <= 3
 constexpr int kRowCntShift = 28;  // packed row: first cell | cell count << 28
 constexpr int32_t kRowCellMask = (1 << kRowCntShift) - 1;
 constexpr int64_t kMaxCells = 1LL << kRowCntShift;
-constexpr int kHeavy = 32;    // cells with more points are "heavy" (wavefront paths)
+constexpr int kHeavy = 32;    // cells with more points are "heavy" (a wavefront per border pair)
 constexpr int kRecSlots = 16;  // neighbour records kept per non-core point (at most)
 
 // Stencil lines, nearest first: (offset along axis 0, offset along axis 1)
@@ -132,15 +132,15 @@ enum Ctl : int {
   C_SEGS_LEFT,  // expansion waves whose seeding segment is not finished
   C_NLINES,     // total line-table entries
   C_DENSE,      // cells resolved as all-core without distance tests
-  C_NHEAVY,     // heavy cells (listed in Dev::heavy)
-  C_NADJPTS,    // core points of light cells (listed in Dev::adj_pts)
+  C_NHEAVY,     // heavy cells (more than kHeavy points)
+  C_NADJPTS,    // core points of light cells
   C_NCORECELLS, // cells with core points (listed in Dev::core_cells)
-  C_EDGES,      // adjacency bits of the expanded cells
+  C_EDGES,      // joined pairs of the near graph, from both sides
   C_RECOVF,     // non-core points whose neighbour record overflowed
-  C_ADJ_TESTS,  // pair tests of the adjacency lanes
-  C_ADJ_FREE,   // adjacency bits set without a test (cell inside the eps ball)
-  C_FAR_TESTS,  // pair tests of the far-pair pass
-  C_FAR_JOINS,  // far pairs that joined two components
+  C_ADJ_TESTS,  // representative pairs tested for the near graph
+  C_ADJ_FREE,   // border pairs joined without a test (cell inside the eps ball)
+  C_FAR_TESTS,  // pair tests of the border-pair passes
+  C_FAR_JOINS,  // border pairs that joined two components
   C_LASTPASS,   // 1 + the last expansion pass that popped a cell
   C_POPS_MAX,   // most cells popped by one expansion wave in one pass
   C_SEEDS_MAX,  // most chains started by one expansion wave in one pass
@@ -156,9 +156,11 @@ enum Ctl : int {
   C_ADJ_CELLS,    // k_adj: cells of those lines
   C_NROWSFB,      // row work items left to the global-memory pass (Dev::rows_fb)
   C_NBORDERPTS,   // non-core points (listed in Dev::border_pts)
-  C_NCTL = 49
+  C_NROOTS,       // near components (listed in Dev::near_roots)
+  C_NFARPAIRS,    // border pairs with a heavy cell (listed in Dev::far_pairs)
+  C_NCTL
 };
-static_assert(C_NBORDERPTS < C_NCTL, "control block too small");
+static_assert(C_NFARPAIRS < C_NCTL, "control block too small");
 
 // Cell-key space: the sort key of a cell is its instance's key base plus its
 // linear index, and the radix sort orders keys of up to 63 bits, so the
@@ -187,6 +189,14 @@ constexpr int kStripes = 64;
 // the striped statistics array, so the host reads the total like a counter.
 struct SList {
   int32_t* data;             // [kStripes][cap]
+  unsigned long long* cnt;   // [kStripes]
+  int64_t cap;
+};
+
+// The same for pairs of cells; a counter may exceed cap (the pairs past it
+// were not stored).
+struct PairList {
+  int2* data;                // [kStripes][cap]
   unsigned long long* cnt;   // [kStripes]
   int64_t cap;
 };
@@ -230,12 +240,16 @@ struct Dev {
   int32_t* cell_inst;   // [N]
   int32_t* cell_ncore;  // [N] core points per cell
   int32_t* cell_label;  // [N] chain owning the cell's core points
-  unsigned long long* amask;  // [N] near adjacency: bit 5r+k <-> k-th cell of line r < 9
+  unsigned long long* amask;  // [N] near graph: bit 5r+k <-> k-th cell of line r < 9
   int32_t* cell_comp;   // [N] component (root chain) of each core cell, -1 otherwise
-  SList heavy;          // heavy cells (more than kHeavy points)
-  SList adj_pts;        // core points of light cells (near-adjacency lanes)
+  uint4* rep;           // [N] per cell: its first core point's G and sorted index
+                        // (over the sort keys, which the CSR pass is the last to read)
+  int32_t chains;       // 1: near components by seed-list expansion, 0: by union-find
   SList border_pts;     // non-core points (border-label lanes)
-  SList core_cells;     // cells with core points (far-pair lanes)
+  SList core_cells;     // cells with core points (near-graph and border-pair lanes)
+  SList near_roots;     // roots of the near components
+  PairList far_pairs;   // border pairs with a heavy cell (over the sort's point ids,
+                        // which the gather is the last to read)
   int32_t* rows;        // [kMaxRows][rstride] packed neighbour lines (first cell, count),
                         // line-major so that consecutive cells are adjacent
   int64_t rstride;      // >= number of cells
@@ -354,21 +368,30 @@ __device__ __forceinline__ void wave_add(long long* p, long long v) {
   if (lane_id() == 0 && s != 0) atomicAdd((unsigned long long*)p, (unsigned long long)s);
 }
 
-// Statistics counter update: the wave's sum goes to one of kStripes copies
-// of the counter, picked by the wave's position in the launch, so that a
-// launch of many waves does not serialise on one address.  The host sums
-// the copies.
 // chain ids are seed cell indices: the id space is the cell count
 __device__ __forceinline__ long long chain_ids(const Dev& d) { return d.ctl[C_NCELL]; }
 
 // set when a run with a fixed number of expansion passes left work pending
 __device__ __forceinline__ bool abandoned(const Dev& d) { return d.ctl[C_ABANDON] != 0; }
 
+// Statistics counter update: the wave's sum goes to one of kStripes copies
+// of the counter, picked by the wave's position in the launch, so that a
+// launch of many waves does not serialise on one address.  The host sums
+// the copies.
 __device__ __forceinline__ void stat_add(const Dev& d, int ctr, long long v) {
   const long long s = wave_sum(v);
   if (lane_id() == 0 && s != 0) {
     const unsigned w = (blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) & (kStripes - 1);
     atomicAdd((unsigned long long*)&d.stat[ctr * kStripes + w], (unsigned long long)s);
+  }
+}
+
+// The same for a yes/no count per lane.
+__device__ __forceinline__ void stat_count(const Dev& d, int ctr, bool yes) {
+  const unsigned long long m = ballot(yes);
+  if (lane_id() == 0 && m) {
+    const unsigned w = (blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) & (kStripes - 1);
+    atomicAdd((unsigned long long*)&d.stat[ctr * kStripes + w], (unsigned long long)__popcll(m));
   }
 }
 
@@ -475,14 +498,19 @@ __device__ __forceinline__ double cell_t(double x, double mn, double inv_w) {
   return (x - mn) * inv_w;
 }
 
-// ---- chain union-find (lock-free; roots are the minimum id) ------------
-// Invariant: par[x] <= x, and a link only ever replaces a root's self-pointer
-// (by CAS) with a smaller id, so every value par[x] has held is an ancestor
-// of x.  A plain load may therefore return a stale but still valid ancestor:
-// uf_find_cached walks with plain (L2-cached) loads, which is enough to
-// decide "same set" when two walks meet.  A CAS on a stale "root" fails and
-// the retry walks with coherent (agent-scope) loads, which guarantees
-// progress.
+// ---- lock-free union-find ----------------------------------------------
+// A link only ever replaces a root's self-pointer (by CAS) with a node of
+// smaller uf_order, a bijective scramble of the ids, so links cannot close a
+// cycle and every value par[x] has held is an ancestor of x.  (Linked by the
+// ids themselves, neighbouring sets, whose ids follow the cell order, hook
+// each other into chains as long as the row of sets; in scrambled order the
+// expected depth is logarithmic.)  A plain load may therefore return a stale
+// but still valid ancestor: uf_find_cached walks with plain (L2-cached)
+// loads, which is enough to decide "same set" when two walks meet.  A CAS on
+// a stale "root" fails and the retry walks with coherent (agent-scope)
+// loads, which guarantees progress.
+__device__ __forceinline__ uint32_t uf_order(int32_t x) { return (uint32_t)x * 0x9E3779B1u; }
+
 __device__ __forceinline__ int32_t uf_find(int32_t* par, int32_t x) {
   for (;;) {
     int32_t p = __hip_atomic_load(&par[x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -522,13 +550,14 @@ __device__ __forceinline__ void uf_union(int32_t* par, int32_t a, int32_t b) {
   b = uf_find_cached(par, b);
   for (;;) {
     if (a == b) return;
-    if (a < b) {
+    if (uf_order(a) < uf_order(b)) {
       int32_t t = a;
       a = b;
       b = t;
     }
     int32_t old = atomicCAS(&par[a], a, b);
-    if (old == a) return;
+    // (a concurrent union of the same two sets: the usual reason to fail)
+    if (old == a || old == b) return;
     a = uf_find(par, old);
     b = uf_find(par, b);
   }

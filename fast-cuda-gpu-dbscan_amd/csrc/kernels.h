@@ -29,11 +29,12 @@ int64_t row_list_cap(int64_t n);
 int64_t scan_tmp_entries(int64_t n);
 
 void launch_core(const Dev& d, bool f32, hipStream_t s);
-void launch_adj(const Dev& d, bool f32, int heavy_grid, hipStream_t s);
-// its two kernels apart: light cells (k_adj) and heavy cells (k_adj_heavy)
-// are independent (both only OR bits into the masks)
-void launch_adj_light(const Dev& d, bool f32, hipStream_t s);
-void launch_adj_heavy(const Dev& d, bool f32, int heavy_grid, hipStream_t s);
+// representatives and list of the core cells, then the near graph over them
+void launch_near(const Dev& d, hipStream_t s);
+// components of the near graph by union-find (no seed lists)
+void launch_link(const Dev& d, hipStream_t s);
+// component of every core cell, component minima, list of the near roots
+void launch_comp(const Dev& d, hipStream_t s);
 void launch_pass_prep(const Dev& d, int pass, hipStream_t s);
 void launch_pass_carry(const Dev& d, int pass, int check, hipStream_t s);
 // after `passes` expansion passes: pending work abandons the rest of the run
@@ -42,8 +43,11 @@ void launch_expand(const Dev& d, int pass, int grid, int seeds, int threads, int
 void launch_merge(const Dev& d, int grid, hipStream_t s);
 // workgroups of the producers of the striped work lists (their capacity)
 int64_t point_blocks(int64_t n);
-int64_t cell_comp_blocks(int64_t n);
-// far stencil pairs across components, then final roots
+int64_t cell_blocks(int64_t n);
+// per-stripe capacity of a list that a grid-stride pass over at most n listed
+// cells appends to
+int64_t list_append_cap(int64_t n);
+// stencil pairs across components, then final roots
 void launch_far(const Dev& d, bool f32, int grid, hipStream_t s);
 void launch_border(const Dev& d, bool f32, hipStream_t s);
 void launch_relabel(const Dev& d, int64_t n, hipStream_t s);

@@ -65,7 +65,11 @@ extern "C" {
  *                   workgroup (0 = auto).  Pairs beyond it are merged inline.
  *   precision       DCLUST_PRECISION_*.
  * The launch values never change the labels; the shape a run actually used
- * is reported in dclust_stats.eff_*.
+ * is reported in dclust_stats.eff_*.  A call that leaves seed_list_size,
+ * blocks, block_threads and extra_collision all 0 finds the near components
+ * by a parallel union-find without seed lists (faster than any shape; eff_*
+ * then hold the shape an expansion of that size would take); a call that
+ * gives any of them runs the seed-list expansion with that shape.
  */
 typedef struct dclust_params {
   int32_t dim;
@@ -90,10 +94,10 @@ typedef struct dclust_stats {
   double t_total_ms;   /* first kernel to labels resident on the device   */
   double t_index_ms;   /* bbox + cell keys + radix sort + CSR + rows        */
   double t_core_ms;    /* neighbour-count (core flag) kernel                */
-  double t_adj_ms;     /* near-cell adjacency (core-core pairs within eps)  */
-  double t_expand_ms;  /* seed-list expansion passes                        */
-  double t_merge_ms;   /* union-find merge of collision pairs               */
-  double t_far_ms;     /* far cell pairs across components (+ unions)       */
+  double t_adj_ms;     /* near graph over the core cells                    */
+  double t_expand_ms;  /* near components: seed-list passes or union-find   */
+  double t_merge_ms;   /* merge of collision pairs, component of each cell  */
+  double t_far_ms;     /* cell pairs across components (+ unions)           */
   double t_border_ms;  /* border assignment                                 */
   double t_relabel_ms; /* canonical relabel + output                        */
   int64_t n_points;
@@ -101,7 +105,8 @@ typedef struct dclust_stats {
   int64_t n_core;
   int64_t n_noise;
   int64_t n_clusters;
-  int64_t n_chains;     /* chains started by the expansion kernel           */
+  int64_t n_chains;     /* chains started by the expansion kernel (near
+                         * components of a run without seed lists)          */
   int64_t n_collisions; /* collision pairs recorded                         */
   int64_t n_overflow;   /* points pushed past a full seed list (corrected)  */
   int64_t n_passes;     /* expansion passes                                 */
@@ -119,13 +124,14 @@ typedef struct dclust_stats {
   int32_t hip_error;       /* last hipError_t, 0 if none                    */
   int32_t key_bits;        /* bits of the sort key                          */
   /* diagnostics: [0] cells expanded, [1] cells resolved as all-core without
-   * distance tests, [2] heavy cells (adjacency by one wavefront per cell),
-   * [3] adjacent cell pairs (directed), [4] time of expansion pass 0 (us),
+   * distance tests, [2] heavy cells (their border pairs are decided by one
+   * wavefront each), [3] joined cell pairs of the near graph (directed),
+   * [4] time of expansion pass 0, or of the union-find (us),
    * [5] sum over expansion wavefronts of their lifetime (us), [6] longest
-   * lifetime (us), [7] expansion wavefronts, [8] pair tests of the
-   * near-adjacency kernel, [9] adjacency bits set without a test, [10]
-   * pair tests of the far-pair pass, [11] far pairs that joined two
-   * components, [12] most cells popped by one expansion wave in a pass,
+   * lifetime (us), [7] expansion wavefronts (0 without seed lists), [8]
+   * representative pairs tested for the near graph, [9] border pairs joined
+   * without a test, [10] pair tests of the border-pair passes, [11] border
+   * pairs that joined two components, [12] most cells popped by one expansion wave in a pass,
    * [13] most chains started by one expansion wave in a pass, [14] 1 if
    * the run was a replay of a captured graph, [15] most pop rounds (up to
    * 64 cells each) of one expansion wavefront in a pass */
@@ -138,7 +144,7 @@ typedef struct dclust_stats {
   int32_t eff_extra_collision;
   double t_rows_ms;       /* the neighbour-line kernel alone (inside t_index) */
   int64_t n_core_cells;   /* cells holding core points                       */
-  int64_t n_adj_points;   /* core points of light cells (near-adjacency lanes) */
+  int64_t n_adj_points;   /* core points of light cells                      */
   int64_t n_lines;        /* possible grid lines (line-table entries)        */
   /* work of the neighbour kernels (the units of their algorithmic bytes):
    * [0] k_core line groups streamed (5 lines each), [1] k_core non-empty
