@@ -67,8 +67,8 @@ struct dclust_handle {
   int gpasses = 0;                 // expansion passes it holds
   bool gphases = false;            // it records every phase event
   bool greadback = false;          // it ends with the counters' copies to `pin`
-  // pinned host copy of the control counters ([C_NCTL]) and their stripes
-  // ([C_NCTL][kStripes]), allocated with the handle (null: pageable copies)
+  // pinned host copy of the control counters, their stripes added ([C_NCTL]),
+  // allocated with the handle (null: pageable copies)
   long long* pin = nullptr;
   long long* pin_dev = nullptr;  // its device address
   bool cap_phases = false;         // (set while a capture runs)
@@ -467,25 +467,25 @@ hipError_t capture_run(dclust_handle* h, const Dev& d, const RunShape& shape, bo
   return e;
 }
 
-// Control counters and their striped parts, after the stream drains
-// (`enqueued`: the copies to the pinned buffer are already on the stream).
+// Control counters, their stripes added, after the stream drains
+// (`enqueued`: the copy to the pinned buffer is already on the stream).
 hipError_t read_counters(dclust_handle* h, const Dev& d, hipStream_t s, long long* ctl_h,
-                         std::vector<long long>& stat_h, bool enqueued = false) {
+                         bool enqueued = false) {
   hipError_t e = hipSuccess;
   if (h->pin) {
     if (!enqueued) e = enqueue_readback(h, d, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
-    if (e == hipSuccess) {
-      std::memcpy(ctl_h, h->pin, sizeof(long long) * C_NCTL);
-      std::memcpy(stat_h.data(), h->pin + C_NCTL, sizeof(long long) * C_NCTL * kStripes);
-    }
+    if (e == hipSuccess) std::memcpy(ctl_h, h->pin, sizeof(long long) * C_NCTL);
     return e;
   }
+  std::vector<long long> stat_h((size_t)kStatStride * kStripes);
   e = hipMemcpyAsync(ctl_h, d.ctl, sizeof(long long) * C_NCTL, hipMemcpyDeviceToHost, s);
   if (e == hipSuccess)
     e = hipMemcpyAsync(stat_h.data(), d.stat, sizeof(long long) * stat_h.size(),
                        hipMemcpyDeviceToHost, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
+  for (int c = 0; c < C_NCTL; ++c)
+    for (int k = 0; k < kStripes; ++k) ctl_h[c] += stat_h[(size_t)k * kStatStride + c];
   return e;
 }
 
@@ -511,12 +511,9 @@ void set_shape_stats(const RunShape& shape, dclust_stats* stats) {
 }
 
 // Records the run's device state for dclust_last_core_flags and fills the
-// statistics (counters summed over their stripes, phase times from events).
-void finish_run(dclust_handle* h, const Dev& d, const RunShape& shape, long long* ctl_h,
-                const std::vector<long long>& stat_h, int npass, bool replayed,
-                dclust_stats* stats) {
-  for (int c = 0; c < C_NCTL; ++c)
-    for (int k = 0; k < kStripes; ++k) ctl_h[c] += stat_h[(size_t)c * kStripes + k];
+// statistics (counters, phase times from events).
+void finish_run(dclust_handle* h, const Dev& d, const RunShape& shape, const long long* ctl_h,
+                int npass, bool replayed, dclust_stats* stats) {
   h->last_n = d.n;
   h->last_core = d.core;
   h->last_orig = d.orig;
@@ -689,7 +686,7 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
     d.chunks = M.get<Chunk>(S_CHUNK, nchunks);
     d.bbox = M.get<unsigned long long>(S_BBOX, (size_t)ninst * kBoxStripes * 8);
     d.ctl = M.get<long long>(S_CTL, C_NCTL);
-    d.stat = M.get<long long>(S_STAT, (size_t)C_NCTL * kStripes);
+    d.stat = M.get<long long>(S_STAT, (size_t)kStatStride * kStripes);
     // the sort's keys, then (from k_rep on) the cells' representatives
     d.key[0] = M.get<uint64_t>(S_KEY, 2 * (size_t)ntot);
     d.key[1] = d.key[0] + ntot;
@@ -698,7 +695,7 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
     d.val[0] = M.get<int32_t>(S_VAL, 2 * (size_t)ntot);
     d.val[1] = d.val[0] + ntot;
     d.far_pairs = PairList{(int2*)d.val[0],
-                           (unsigned long long*)(d.stat + (int64_t)C_NFARPAIRS * kStripes),
+                           (unsigned long long*)(d.stat + C_NFARPAIRS),
                            ntot / kStripes};
     d.hist = M.get<uint32_t>(S_HIST, sort_hist_entries(ntot));
     d.offs = M.get<uint32_t>(S_OFFS, sort_hist_entries(ntot));
@@ -713,12 +710,12 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
     const int64_t cap_p = (point_blocks(ntot) + kStripes - 1) / kStripes * 256;
     const int64_t cap_c = (cell_blocks(ntot) + kStripes - 1) / kStripes * 1024;
     d.border_pts = SList{M.get<int32_t>(S_BORDERPTS, (size_t)cap_p * kStripes),
-                         (unsigned long long*)(d.stat + (int64_t)C_NBORDERPTS * kStripes), cap_p};
+                         (unsigned long long*)(d.stat + C_NBORDERPTS), cap_p};
     d.core_cells = SList{M.get<int32_t>(S_CORECELLS, (size_t)cap_c * kStripes),
-                         (unsigned long long*)(d.stat + (int64_t)C_NCORECELLS * kStripes), cap_c};
+                         (unsigned long long*)(d.stat + C_NCORECELLS), cap_c};
     const int64_t cap_r = row_list_cap(ntot);
     d.rows_fb = SList{M.get<int32_t>(S_ROWSFB, (size_t)cap_r * kStripes),
-                      (unsigned long long*)(d.stat + (int64_t)C_NROWSFB * kStripes), cap_r};
+                      (unsigned long long*)(d.stat + C_NROWSFB), cap_r};
     d.cell_inst = M.get<int32_t>(S_CINST, ntot);
     d.cell_ncore = M.get<int32_t>(S_CM, ntot);
     d.rows = M.get<int32_t>(S_ROWS, (size_t)ntot * kMaxRows);
@@ -749,7 +746,7 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
     const int64_t cap_n = list_append_cap(ntot);
     d.q[0] = M.get<int32_t>(S_Q0, (size_t)std::max(ntot, cap_n * kStripes));
     d.q[1] = M.get<int32_t>(S_Q1, shape.chains ? ntot : 0);
-    d.near_roots = SList{d.q[0], (unsigned long long*)(d.stat + (int64_t)C_NROOTS * kStripes),
+    d.near_roots = SList{d.q[0], (unsigned long long*)(d.stat + C_NROOTS),
                          cap_n};
     d.keyv = M.get<int32_t>(S_KEYV, ntot);
     d.flag = M.get<uint8_t>(S_FLAG, ntot);
@@ -801,7 +798,6 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
 
   {
     long long ctl_h[C_NCTL];
-    std::vector<long long> stat_h((size_t)C_NCTL * kStripes);
     // the host-built instance table and chunk list (the kernels rewrite only
     // derived fields of the table, and k_init_head clears its error codes)
     std::vector<uint8_t> up(sizeof(Inst) * ninst + sizeof(Chunk) * nchunks);
@@ -830,7 +826,7 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
       HIPCHK(hipEventRecord(h->ev[E_START], s));
       HIPCHK(hipGraphLaunch(h->gexec, s));
       HIPCHK(hipEventRecord(h->ev[E_END], s));  // (after the counters' readback)
-      HIPCHK(read_counters(h, d, s, ctl_h, stat_h, h->greadback));
+      HIPCHK(read_counters(h, d, s, ctl_h, h->greadback));
       if (!ctl_h[C_ABANDON]) {
         if (ctl_h[C_ERR]) {
           int first = 0;
@@ -838,7 +834,7 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
           if (ninst == 1 || !inst_err) return first ? first : DCLUST_E_PARAM;
           rc = first;
         }
-        finish_run(h, d, shape, ctl_h, stat_h, (int)std::max<long long>(1, ctl_h[C_LASTPASS]),
+        finish_run(h, d, shape, ctl_h, (int)std::max<long long>(1, ctl_h[C_LASTPASS]),
                    true, stats);
         return rc;
       }
@@ -901,8 +897,8 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
     }
     ++npass;
     HIPCHK(enqueue_tail(h, d, f32, grid_cells, false));
-    HIPCHK(read_counters(h, d, s, ctl_h, stat_h));
-    finish_run(h, d, shape, ctl_h, stat_h, npass, false, stats);
+    HIPCHK(read_counters(h, d, s, ctl_h));
+    finish_run(h, d, shape, ctl_h, npass, false, stats);
     if (npass >= kMaxExpandPasses) return DCLUST_E_CAPACITY;
     if (graph_on) {
       h->prev_sig.swap(sig);
@@ -1158,7 +1154,7 @@ int dclust_create(dclust_handle** out, int device) {
     }
   // coherent and mapped: the readback kernel's stores are visible to the
   // host once the stream has drained
-  if (hipHostMalloc((void**)&h->pin, sizeof(long long) * C_NCTL * (1 + kStripes),
+  if (hipHostMalloc((void**)&h->pin, sizeof(long long) * C_NCTL,
                     hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
       hipHostGetDevicePointer((void**)&h->pin_dev, h->pin, 0) != hipSuccess) {
     (void)hipGetLastError();

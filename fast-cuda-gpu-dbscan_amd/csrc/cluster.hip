@@ -296,25 +296,26 @@ __global__ __launch_bounds__(256, F32 ? 6 : 5) void k_core(Dev d) {
   if (act) d.core[p] = isc;
   // non-core points: the lanes of the border-label pass
   block_append(act && !isc, p, d.border_pts);
-  // per-cell core counts: the lanes of one cell form a contiguous run
+  // per-cell core counts: the lanes of one cell form a contiguous run.  A
+  // cell that is core as a whole, or lies inside the wave, is written by its
+  // first point; only the parts of other cells are added up
   const bool head = act && (p == qs || lane == 0);
   const unsigned long long mh = ballot(head), mc = ballot(isc);
-  bool dense = false, heavy = false;
   if (head) {
-    const unsigned long long above = lane == 63 ? 0ull : (mh & (~0ull << (lane + 1)));
-    const int nxt = above ? __ffsll((long long)above) - 1 : 64;
-    const unsigned long long seg = (nxt == 64 ? ~0ull : ((1ull << nxt) - 1ull)) & (~0ull << lane);
-    const int k = __popcll(mc & seg);
-    if (k) atomicAdd(&d.cell_ncore[c], k);
-    if (p == qs) {
-      dense = (qe - qs) >= P.minpts;
-      heavy = (qe - qs) > kHeavy;
+    if (qe - qs >= P.minpts) {
+      if (p == qs) d.cell_ncore[c] = qe - qs;
+    } else {
+      const unsigned long long above = lane == 63 ? 0ull : (mh & (~0ull << (lane + 1)));
+      const int nxt = above ? __ffsll((long long)above) - 1 : 64;
+      const unsigned long long seg =
+          (nxt == 64 ? ~0ull : ((1ull << nxt) - 1ull)) & (~0ull << lane);
+      const int k = __popcll(mc & seg);
+      if (k && p == qs && qe - qs <= 64 - lane)
+        d.cell_ncore[c] = k;
+      else if (k)
+        atomicAdd(&d.cell_ncore[c], k);
     }
   }
-  stat_count(d, C_NHEAVY, heavy);
-  stat_count(d, C_NADJPTS, isc && qe - qs <= kHeavy);
-  stat_count(d, C_NCORE, isc);
-  stat_count(d, C_DENSE, dense);
   stat_add(d, C_EVAL, t.eval);
   stat_add(d, C_BAND_CORE, t.band);
   stat_add(d, C_BAND, t.band);
@@ -388,6 +389,7 @@ __global__ __launch_bounds__(1024) void k_rep(Dev d) {
   const bool in = c < C;
   const int64_t cc = in ? c : 0;
   const int32_t ncore = d.cell_ncore[cc], q0 = d.cell_start[cc], q1 = d.cell_start[cc + 1];
+  const int minpts = inst_of_cell(d, cc)->minpts;
   const bool hc = in && ncore > 0;
   uint4 r = make_uint4(0u, 0u, 0u, kNoRep);
   if (hc) {
@@ -407,6 +409,26 @@ __global__ __launch_bounds__(1024) void k_rep(Dev d) {
     d.cell_label[c] = kUnclaimed;
   }
   block_append(hc, (int32_t)c, d.core_cells);
+  // core points, those of light cells, all-core cells and heavy cells: one
+  // atomic per workgroup and counter (counted by every wave of k_core
+  // instead, these took 1.0 of its 1.6 ms on 32 M points)
+  const int nc = hc ? ncore : 0, m = in ? q1 - q0 : 0;
+  const int sums[4] = {wave_sum(nc), wave_sum(m <= kHeavy ? nc : 0),
+                       (int)__popcll(ballot(in && m >= minpts)),
+                       (int)__popcll(ballot(m > kHeavy))};
+  __shared__ int s_sum[16][4];
+  if (lane_id() == 0)
+    for (int k = 0; k < 4; ++k) s_sum[threadIdx.x >> 6][k] = sums[k];
+  __syncthreads();
+  if (threadIdx.x < 4) {
+    constexpr int ctr[4] = {C_NCORE, C_NADJPTS, C_DENSE, C_NHEAVY};
+    int t = 0;
+    for (int w = 0; w < 16; ++w) t += s_sum[w][threadIdx.x];
+    if (t)
+      atomicAdd((unsigned long long*)&d.stat[(blockIdx.x & (kStripes - 1)) * kStatStride +
+                                             ctr[threadIdx.x]],
+                (unsigned long long)t);
+  }
 }
 
 // Near graph: bit 5r+k of a core cell's mask is set when cell k of its near
@@ -826,7 +848,7 @@ __device__ long long far_cell(const Dev& d, const Par& P, int32_t A, Tally& t,
       if (ra == rb) continue;
       if (qe - qs > kHeavy || b1 - b0 > kHeavy) {
         const int s = blockIdx.x & (kStripes - 1);
-        const unsigned long long at = atomicAdd(&d.far_pairs.cnt[s], 1ull);
+        const unsigned long long at = atomicAdd(&d.far_pairs.cnt[s * kStatStride], 1ull);
         if (at < (unsigned long long)d.far_pairs.cap) {
           d.far_pairs.data[s * d.far_pairs.cap + (int64_t)at] = make_int2(A, B);
           continue;
@@ -946,7 +968,7 @@ __global__ __launch_bounds__(256) void k_far_pairs(Dev d) {
   if (abandoned(d)) return;
   __shared__ long long s_pre[kStripes + 1];
   if (threadIdx.x < kStripes) {
-    const long long v = (long long)d.far_pairs.cnt[threadIdx.x];
+    const long long v = (long long)d.far_pairs.cnt[threadIdx.x * kStatStride];
     const long long incl = wave_incl_scan(v < d.far_pairs.cap ? v : (long long)d.far_pairs.cap);
     s_pre[threadIdx.x + 1] = incl;
     if (threadIdx.x == 0) s_pre[0] = 0;

@@ -39,7 +39,7 @@ static int fill_grid(int64_t n) {
 // non-finite flag, all starting at 0).
 __global__ void k_init_head(Dev d) {
   const int64_t nb = (int64_t)d.ninst * kBoxStripes * 8;
-  const int64_t ns = (int64_t)C_NCTL * kStripes;
+  const int64_t ns = (int64_t)kStatStride * kStripes;
   const int64_t tot = nb + ns + C_NCTL + kMaxPasses + d.ninst;
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < tot;
        i += (int64_t)gridDim.x * blockDim.x) {
@@ -57,19 +57,30 @@ __global__ void k_init_head(Dev d) {
 }
 
 void launch_init_head(const Dev& d, hipStream_t s) {
-  const int64_t tot = (int64_t)d.ninst * kBoxStripes * 8 + (int64_t)C_NCTL * kStripes + C_NCTL +
+  const int64_t tot = (int64_t)d.ninst * kBoxStripes * 8 + (int64_t)kStatStride * kStripes + C_NCTL +
                       kMaxPasses + d.ninst;
   hipLaunchKernelGGL(k_init_head, dim3(fill_grid(tot)), dim3(256), 0, s, d);
 }
 
-// End of a run: the control counters, then their stripes ([C_NCTL], then
-// [C_NCTL][kStripes]) into a host buffer (pinned and mapped), one workgroup.
-// Inside a captured run this follows the last kernel with no gap, where copy
-// nodes would each wait on a separate transfer.
+// End of a run: the control counters, their stripes added, into a host buffer
+// (pinned and mapped): one workgroup, a wavefront per counter, a lane per
+// stripe.  Inside a captured run this follows the last kernel with no gap,
+// where copy nodes would each wait on a separate transfer.
+static_assert((C_NCTL + 15) / 16 * 16 <= kStatStride, "counters of a stripe");
 __global__ __launch_bounds__(1024) void k_readback(Dev d, long long* out) {
-  constexpr int tot = C_NCTL * (1 + kStripes);
-  for (int i = threadIdx.x; i < tot; i += blockDim.x)
-    out[i] = i < C_NCTL ? d.ctl[i] : d.stat[i - C_NCTL];
+  constexpr int R = (C_NCTL + 15) / 16;  // counters per wavefront
+  const int wv = threadIdx.x >> 6;
+  long long v[R], base[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {  // (past the last counter: the stripe's padding)
+    v[r] = d.stat[lane_id() * kStatStride + wv + 16 * r];
+    base[r] = d.ctl[wv + 16 * r < C_NCTL ? wv + 16 * r : 0];
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const long long s = wave_sum(v[r]);
+    if (lane_id() == 0 && wv + 16 * r < C_NCTL) out[wv + 16 * r] = base[r] + s;
+  }
 }
 
 void launch_readback(const Dev& d, long long* out, hipStream_t s) {

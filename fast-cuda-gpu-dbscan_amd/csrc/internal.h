@@ -180,7 +180,12 @@ __host__ __device__ __forceinline__ int key_bits_for(unsigned long long total) {
 }
 
 // Statistics counters are striped: a wave adds to one of kStripes copies.
+// The copies of one counter lie kStatStride counters apart, so that they are
+// on different cache lines (atomics on one line are taken one after the
+// other, about 1 ns each).
 constexpr int kStripes = 64;
+constexpr int kStatStride = 64;
+static_assert(C_NCTL <= kStatStride, "counter stripe too short");
 
 // A work list filled by many workgroups: kStripes sub-lists (workgroup b
 // appends to sub-list b % kStripes, with its own counter), so that the
@@ -189,7 +194,7 @@ constexpr int kStripes = 64;
 // the striped statistics array, so the host reads the total like a counter.
 struct SList {
   int32_t* data;             // [kStripes][cap]
-  unsigned long long* cnt;   // [kStripes]
+  unsigned long long* cnt;   // [kStripes], kStatStride apart
   int64_t cap;
 };
 
@@ -197,7 +202,7 @@ struct SList {
 // were not stored).
 struct PairList {
   int2* data;                // [kStripes][cap]
-  unsigned long long* cnt;   // [kStripes]
+  unsigned long long* cnt;   // [kStripes], kStatStride apart
   int64_t cap;
 };
 
@@ -222,7 +227,7 @@ struct Dev {
   unsigned long long* bbox;  // [ninst][kBoxStripes][8] ordered-u64 min0..2 max0..2,
                              // max |x|, non-finite flag
   long long* ctl;
-  long long* stat;  // [C_NCTL][kStripes] statistics counters (summed by the host)
+  long long* stat;  // [kStripes][kStatStride] statistics counters
 
   // radix sort
   uint64_t* key[2];
@@ -376,22 +381,15 @@ __device__ __forceinline__ bool abandoned(const Dev& d) { return d.ctl[C_ABANDON
 
 // Statistics counter update: the wave's sum goes to one of kStripes copies
 // of the counter, picked by the wave's position in the launch, so that a
-// launch of many waves does not serialise on one address.  The host sums
-// the copies.
+// launch of many waves does not serialise on one address.
+// A wave with nothing to add (most waves of most counters) skips the sum;
+// small counts are summed in 32 bits (half the shuffles).
 __device__ __forceinline__ void stat_add(const Dev& d, int ctr, long long v) {
-  const long long s = wave_sum(v);
-  if (lane_id() == 0 && s != 0) {
+  if (!ballot(v != 0)) return;
+  const long long s = ballot((v >> 24) != 0) ? wave_sum(v) : (long long)wave_sum((int)v);
+  if (lane_id() == 0) {
     const unsigned w = (blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) & (kStripes - 1);
-    atomicAdd((unsigned long long*)&d.stat[ctr * kStripes + w], (unsigned long long)s);
-  }
-}
-
-// The same for a yes/no count per lane.
-__device__ __forceinline__ void stat_count(const Dev& d, int ctr, bool yes) {
-  const unsigned long long m = ballot(yes);
-  if (lane_id() == 0 && m) {
-    const unsigned w = (blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) & (kStripes - 1);
-    atomicAdd((unsigned long long*)&d.stat[ctr * kStripes + w], (unsigned long long)__popcll(m));
+    atomicAdd((unsigned long long*)&d.stat[w * kStatStride + ctr], (unsigned long long)s);
   }
 }
 
@@ -408,7 +406,7 @@ __device__ __forceinline__ void block_append(bool take, int32_t value, const SLi
   if (threadIdx.x == 0) {
     int tot = 0;
     for (int w = 0; w < nw; ++w) tot += s_cnt[w];
-    s_base = tot ? (long long)atomicAdd(&L.cnt[blockIdx.x & (kStripes - 1)],
+    s_base = tot ? (long long)atomicAdd(&L.cnt[(blockIdx.x & (kStripes - 1)) * kStatStride],
                                         (unsigned long long)tot)
                  : 0;
   }
@@ -423,7 +421,7 @@ __device__ __forceinline__ void block_append(bool take, int32_t value, const SLi
 // the list length.  Every thread of the workgroup calls it.
 __device__ __forceinline__ long long slist_prefix(const SList& L, long long* s_pre) {
   if (threadIdx.x < kStripes) {
-    const long long v = (long long)L.cnt[threadIdx.x];
+    const long long v = (long long)L.cnt[threadIdx.x * kStatStride];
     const long long incl = wave_incl_scan(v);
     s_pre[threadIdx.x + 1] = incl;
     if (threadIdx.x == 0) s_pre[0] = 0;
