@@ -112,39 +112,38 @@ def kernel_bytes(st, dim, f32):
     kernel reported for this run (stats.work, pairs_evaluated, diag) times the
     bytes one unit of that work reads or writes, with no credit for caches.
 
-    k_core   per point: cell_of 4, its cell's two starts 8, its coordinates
-             s*D, core flag 1; per line group 5 packed rows (20); per
-             non-empty line its point range (two starts, 8); per candidate
-             its coordinates s*D; per cell the core count 4 and mask clear 8;
-             per listed core point of a light cell the list entry 4.
+    k_core   the three count kernels: per point: cell_of 4, its cell's two
+             starts 8, its coordinates s*D, core flag 1; per row read 8; per
+             non-empty point range of it its two ends 8; per candidate its
+             coordinates s*D; per point left by the first pass its list entry
+             4 and the above again.
     k_adj    per core cell (k_rep's records are written per cell before it:
-             16): list entry 4, its representative 16, the packed rows of the
-             near lines above it (5 in 3-D, 2 in 2-D), its mask 8; per pair
-             tested the other representative 16.
-    k_rows   per cell and group of 5 lines: cell_xyz 8, the cell's sort key
-             staged 8, five packed rows written 20 (the line-table entries
-             of a tile's span and the keys of the extra lines around it are
-             not counted: a lower bound).
-    k_expand with seed lists: per popped cell: chain label 4, near mask 8, 9
-             near rows 36; per bit: the neighbour's label 4 and its claim 4;
-             per cell the seeding scan: core count 4 and label 4.
-    k_link   without: per cell: mask 8, own row 4, root 4; per core cell: mask
-             written 8, list entry 4; per joined pair its line's row 4 and
-             the other cell's entry 4.
+             16): list entry 4, its representative 16, four rows (two in 2-D)
+             32, its mask 4; per pair tested the other representative 16.
+    k_rows   per cell and group of three columns (three groups in 3-D, one in
+             2-D): its column and place 8, the cell's sort key and end staged
+             12, three rows written 24 (the column-table entries of a tile's
+             span and the keys of the extra columns around it are not counted:
+             a lower bound).
+    k_expand with seed lists: per popped cell: chain label 4, near mask 4, 9
+             rows 72; per bit: the neighbour's label 4 and its claim 4; per
+             cell the seeding scan: core count 4 and label 4.
+    k_link   without: per cell: mask 4, root 4; per core cell: mask written 4,
+             list entry 4, place 4; per joined pair its row 8 and the other
+             cell's entry 4.
     s = 4 (fixed point, FP32 form) or 8 (FP64 form)."""
     n, c = st["n_points"], st["n_cells"]
     s = 4 if f32 else 8
     w = st["work"]
-    groups = (25 if dim == 3 else 5) // 5
-    upper = 5 if dim == 3 else 2
-    a, cc = st["n_adj_points"], st["n_core_cells"]
+    groups, near_rows = (3, 4) if dim == 3 else (1, 2)
+    cc = st["n_core_cells"]
     dg = st["diag"]
-    core = (n * (4 + 8 + s * dim + 1) + 20 * w[0] + 8 * w[1] + s * dim * st["pairs_evaluated"] +
-            c * (4 + 8) + 4 * a)
-    near = cc * (4 + 16 + 4 * upper + 8) + 16 * dg[8] + 16 * c
-    rows = c * groups * (8 + 8 + 20)
-    expand = dg[0] * (4 + 8 + 36) + dg[3] * 8 + c * 8
-    link = c * (8 + 4 + 4) + cc * (8 + 4) + (dg[3] // 2) * 8
+    core = ((n + w[2]) * (4 + 8 + s * dim + 1) + 8 * w[0] + 8 * w[1] +
+            s * dim * st["pairs_evaluated"] + 4 * w[2])
+    near = cc * (4 + 16 + 8 * near_rows + 4) + 16 * dg[8] + 16 * c
+    rows = c * groups * (8 + 12 + 24)
+    expand = dg[0] * (4 + 4 + 72) + dg[3] * 8 + c * 8
+    link = c * (4 + 4) + cc * (4 + 4 + 4) + (dg[3] // 2) * 12
     out = {"k_core": core, "k_adj": near, "k_rows": rows}
     out["k_expand" if dg[0] else "k_link"] = expand if dg[0] else link
     return out

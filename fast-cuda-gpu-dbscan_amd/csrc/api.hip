@@ -112,16 +112,16 @@ namespace {
 
 enum Slot {
   S_XYZ, S_INST, S_CHUNK, S_BBOX, S_CTL, S_KEY, S_VAL, S_HIST, S_OFFS,
-  S_DTOT, S_PASS, S_CSTART, S_CKEY, S_CINST, S_CM, S_ROWS, S_CELLOF, S_X0, S_X1, S_X2,
-  S_G0, S_G1, S_G2, S_ORIG, S_CORE, S_LABEL, S_PARENT, S_COMPMIN, S_PAIRS, S_Q0, S_Q1,
+  S_DTOT, S_PASS, S_CSTART, S_CKEY, S_CINST, S_CM, S_ROWS, S_CELLOF, S_X,
+  S_G, S_ORIG, S_CORE, S_LABEL, S_PARENT, S_COMPMIN, S_PAIRS, S_Q0, S_Q1,
   S_KEYV, S_FLAG, S_RANK, S_SCAN, S_LABOUT, S_COREOUT, S_PAIRCNT, S_SEGPOS, S_LINES, S_AMASK,
-  S_REC, S_RECN, S_CXYZ, S_CCOMP, S_BORDERPTS, S_CORECELLS, S_TUNELAB, S_STAT, S_GLINES,
-  S_CZ, S_XOFF, S_OS_LABEL, S_OS_STATE, S_OS_SEEDS, S_OS_LEN, S_OS_CONTACT, S_OS_FIRST, S_ROWSFB
+  S_REC, S_RECN, S_CCOL, S_CCOMP, S_BORDERPTS, S_CORECELLS, S_TUNELAB, S_STAT, S_GLINES,
+  S_CZL, S_XOFF, S_OS_LABEL, S_OS_STATE, S_OS_SEEDS, S_OS_LEN, S_OS_CONTACT, S_OS_FIRST, S_ROWSFB
 };
 
-// line table entries (8 bytes each) above which neighbour lines are found
+// column table entries (8 bytes each) above which neighbour columns are found
 // by binary search instead
-constexpr long long kMaxLineTable = 1LL << 27;  // 1 GiB at most
+constexpr long long kMaxLineTable = 1LL << 26;  // 512 MiB at most
 // expansion passes a captured run may hold; runs that need more stay eager
 constexpr int kGraphMaxPasses = 8;
 
@@ -356,7 +356,7 @@ hipError_t mark(dclust_handle* h, int e, bool graph, hipStream_t s = nullptr) {
                : hipEventRecord(h->ev[e], s);
 }
 
-// Keys, sort, CSR, gather and line table, then the neighbour rows (one
+// Keys, sort, CSR, gather and column table, then the neighbour rows (one
 // stream: the gather fills the device, so running the rows beside it gains
 // nothing).
 hipError_t enqueue_index(dclust_handle* h, const Dev& d, int64_t n, int nchunks, int grid_cells,
@@ -527,10 +527,10 @@ void finish_run(dclust_handle* h, const Dev& d, const RunShape& shape, const lon
   stats->n_core_cells = ctl_h[C_NCORECELLS];
   stats->n_adj_points = ctl_h[C_NADJPTS];
   stats->n_lines = ctl_h[C_NLINES];
-  stats->work[0] = ctl_h[C_CORE_GROUPS];
-  stats->work[1] = ctl_h[C_CORE_LINES];
-  stats->work[2] = ctl_h[C_ADJ_LINES];
-  stats->work[3] = ctl_h[C_ADJ_CELLS];
+  stats->work[0] = ctl_h[C_CORE_ROWS];
+  stats->work[1] = ctl_h[C_CORE_RANGES];
+  stats->work[2] = ctl_h[C_NCOREREST];
+  stats->work[3] = ctl_h[C_NCORECROWD];
   stats->t_core_ms = ev_ms(h, E_CORE0, E_CORE);
   stats->t_adj_ms = phase_ms(E_CORE, E_ADJ);
   stats->t_expand_ms = phase_ms(E_ADJ, E_EXPAND);
@@ -677,7 +677,7 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
   // asymmetric); up to kRecSlots are kept, a longer record is rescanned
   int rec_stride = 0;
   for (int32_t i = 0; i < ninst; ++i) rec_stride = std::max(rec_stride, params[i].minpts);
-  rec_stride = std::min(rec_stride, kRecSlots);
+  rec_stride = std::min(rec_stride, fixed_mem ? kRecSlotsFixed : kRecSlots);
   d.rec_stride = rec_stride;
   RunMem mem{h, region, region_cap};
   {
@@ -691,26 +691,30 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
     d.key[0] = M.get<uint64_t>(S_KEY, 2 * (size_t)ntot);
     d.key[1] = d.key[0] + ntot;
     d.rep = (uint4*)d.key[0];
-    // the sort's point ids, then (from k_far on) the listed border pairs
+    // the sort's point ids, then (from k_far on) the listed pairs of cells
     d.val[0] = M.get<int32_t>(S_VAL, 2 * (size_t)ntot);
     d.val[1] = d.val[0] + ntot;
-    d.far_pairs = PairList{(int2*)d.val[0],
-                           (unsigned long long*)(d.stat + C_NFARPAIRS),
-                           ntot / kStripes};
+    const int64_t cap_f = ntot / 2 / kStripes;
+    d.far_light = PairList{(int2*)d.val[0], (unsigned long long*)(d.stat + C_NFARLIGHT), cap_f};
+    d.far_heavy = PairList{(int2*)d.val[0] + cap_f * kStripes,
+                           (unsigned long long*)(d.stat + C_NFARHEAVY), cap_f};
     d.hist = M.get<uint32_t>(S_HIST, sort_hist_entries(ntot));
     d.offs = M.get<uint32_t>(S_OFFS, sort_hist_entries(ntot));
     d.dtot = M.get<uint32_t>(S_DTOT, 256);
     d.pass_scatter = M.get<int32_t>(S_PASS, kMaxPasses);
     d.cell_start = M.get<int32_t>(S_CSTART, ntot + 1);
     d.cell_key = M.get<uint64_t>(S_CKEY, ntot);
-    d.cell_xyz = M.get<uint64_t>(S_CXYZ, ntot);
-    d.cell_z = M.get<int32_t>(S_CZ, ntot);
-    d.cell_comp = M.get<int32_t>(S_CCOMP, ntot);
+    d.cell_col = M.get<uint32_t>(S_CCOL, ntot);
+    d.cell_zl = M.get<uint32_t>(S_CZL, ntot);
+    d.cell_comp = M.get<int32_t>(S_CCOMP, ntot + 4);  // (read four at a time)
     // striped work lists: sub-list capacity = the most its workgroups append
     const int64_t cap_p = (point_blocks(ntot) + kStripes - 1) / kStripes * 256;
     const int64_t cap_c = (cell_blocks(ntot) + kStripes - 1) / kStripes * 1024;
-    d.border_pts = SList{M.get<int32_t>(S_BORDERPTS, (size_t)cap_p * kStripes),
-                         (unsigned long long*)(d.stat + C_NBORDERPTS), cap_p};
+    const int64_t cap_n = list_append_cap(ntot);
+    // non-core points are appended by three passes, each of at most all points
+    const int64_t cap_b = cap_p + 2 * cap_n;
+    d.border_pts = SList{M.get<int32_t>(S_BORDERPTS, (size_t)cap_b * kStripes),
+                         (unsigned long long*)(d.stat + C_NBORDERPTS), cap_b};
     d.core_cells = SList{M.get<int32_t>(S_CORECELLS, (size_t)cap_c * kStripes),
                          (unsigned long long*)(d.stat + C_NCORECELLS), cap_c};
     const int64_t cap_r = row_list_cap(ntot);
@@ -718,22 +722,18 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
                       (unsigned long long*)(d.stat + C_NROWSFB), cap_r};
     d.cell_inst = M.get<int32_t>(S_CINST, ntot);
     d.cell_ncore = M.get<int32_t>(S_CM, ntot);
-    d.rows = M.get<int32_t>(S_ROWS, (size_t)ntot * kMaxRows);
+    d.rows = M.get<uint2>(S_ROWS, (size_t)ntot * (dims == 1 ? 3 : kMaxRows));
     d.cell_of = M.get<int32_t>(S_CELLOF, ntot);
     if (!f32) {  // the FP32 form reads FP64 coordinates from the caller's rows
-      d.X[0] = M.get<double>(S_X0, ntot);
-      d.X[1] = M.get<double>(S_X1, ntot);
-      d.X[2] = M.get<double>(S_X2, ntot);
+      d.X = M.get<double>(S_X, 3 * (size_t)ntot);
     } else {
       d.xoff = M.get<int64_t>(S_XOFF, ntot);
     }
-    d.G[0] = M.get<uint32_t>(S_G0, ntot);
-    d.G[1] = M.get<uint32_t>(S_G1, ntot);
-    d.G[2] = M.get<uint32_t>(S_G2, ntot);
+    d.G = M.get<uint32_t>(S_G, 3 * (size_t)ntot);
     d.orig = M.get<int32_t>(S_ORIG, ntot);
     d.core = M.get<uint8_t>(S_CORE, ntot);
     d.cell_label = M.get<int32_t>(S_LABEL, ntot);
-    d.amask = M.get<unsigned long long>(S_AMASK, (size_t)ntot);
+    d.amask = M.get<uint32_t>(S_AMASK, (size_t)ntot);
     d.rec_n = M.get<uint8_t>(S_RECN, ntot);
     if (rec_stride > 0) d.rec = M.get<int32_t>(S_REC, (size_t)ntot * rec_stride);
     d.parent = M.get<int32_t>(S_PARENT, ntot);
@@ -743,14 +743,18 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
     d.pair_cnt = M.get<int32_t>(S_PAIRCNT, waves);
     d.seg_pos = M.get<int64_t>(S_SEGPOS, waves);
     // the first queue, then (from k_comp on) the list of the near roots
-    const int64_t cap_n = list_append_cap(ntot);
     d.q[0] = M.get<int32_t>(S_Q0, (size_t)std::max(ntot, cap_n * kStripes));
     d.q[1] = M.get<int32_t>(S_Q1, shape.chains ? ntot : 0);
     d.near_roots = SList{d.q[0], (unsigned long long*)(d.stat + C_NROOTS),
                          cap_n};
-    d.keyv = M.get<int32_t>(S_KEYV, ntot);
+    // the component keys, before them the list of points the first count pass
+    // leaves
+    d.keyv = M.get<int32_t>(S_KEYV, (size_t)std::max(ntot, cap_p * kStripes));
+    d.core_rest = SList{d.keyv, (unsigned long long*)(d.stat + C_NCOREREST), cap_p};
     d.flag = M.get<uint8_t>(S_FLAG, ntot);
-    d.rank = M.get<int32_t>(S_RANK, ntot + 1);
+    // the ranks, before them the list of points with many candidates
+    d.rank = M.get<int32_t>(S_RANK, (size_t)std::max(ntot + 1, cap_n * kStripes));
+    d.core_crowd = SList{d.rank, (unsigned long long*)(d.stat + C_NCORECROWD), cap_n};
     d.scan_tmp = M.get<int64_t>(S_SCAN, scan_tmp_entries(ntot));
     d.core_out = M.get<uint8_t>(S_COREOUT, ntot);
     if (mem.over) return DCLUST_E_CAPACITY;  // the fixed region is too small

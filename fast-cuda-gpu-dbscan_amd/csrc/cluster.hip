@@ -3,20 +3,19 @@
 //
 // Grid: cells of side (eps/2)(1+2^-20), so every cell is a clique (all its
 // points are mutual neighbours) and every neighbour of a point lies in the
-// 5^D stencil of cells around its cell.  The stencil is stored per cell as
-// 5^(D-1) packed runs ("lines") of at most 5 consecutive non-empty cells
-// along the last axis; line r, cell k of a cell's stencil is its stencil
-// slot 5r+k.
+// 5^D stencil of cells around its cell.  The stencil is covered by windows of
+// 3^(D-1) neighbour columns of cells ("rows", internal.h).
 //
-//   k_core       one lane per point: neighbour count with early exit at
-//                minpts -> core flag.  (dbscan.cu:331-369 counts while it
+//   k_core, k_core_rest, k_core_crowd   one lane per point (a wavefront where
+//                the candidates are many): neighbour count with early exit
+//                at minpts -> core flag.  (dbscan.cu:331-369 counts while it
 //                expands; here the count is its own pass, so every later
 //                kernel knows which points are core.)  A cell holding
 //                >= minpts points is all core without a distance test.  A
 //                point that stays below minpts has seen all its neighbours
 //                and records them for the border pass.
-//   k_rep, k_adj   the near graph over core cells: two cells in near lines
-//                are linked when their representatives (one core point each)
+//   k_rep, k_adj   the near graph over core cells: two cells at most one
+//                apart along every axis are linked when their representatives (one core point each)
 //                are certainly joined.
 //   k_link_local, k_link_cross   components of the near graph by union-find,
 //                in LDS over runs of cells, then in global memory.
@@ -64,10 +63,11 @@
 namespace dclust {
 
 constexpr int kCoreBatch = 4;  // neighbour-count candidates loaded per lane step
+                               // (latency bound: residency pays more than longer batches)
 
 struct Tally {  // per-lane event counts (summed per wave by stat_add)
   int band = 0, flip = 0, asym = 0, eval = 0;
-  int groups = 0, lines = 0, cells = 0;  // stencil work (algorithmic bytes)
+  int rows = 0, ranges = 0;  // stencil work (algorithmic bytes)
 };
 
 // FP32 squared distance from fixed-point coordinates (units of w*2^-29).
@@ -155,222 +155,379 @@ __device__ __forceinline__ bool edge_pair(const Dev& d, const Par& P, int32_t a,
 
 
 // ------------------------------------------------------------------ core --
-// Neighbour count of point p with early exit at minpts.  Every candidate
-// pair with d^2 <= eps^2 (either box direction) is recorded while the count
-// is below minpts; a point that ends non-core thereby holds all its
-// neighbours outside its own cell (at most minpts - 1 plus box-asymmetric
-// pairs).
-template <int D, bool F32>
-__device__ void core_lane(const Dev& d, const Par& P, int32_t p, int32_t c, int32_t qs,
-                          int32_t qe, int R, int32_t* rk, Tally& t, bool& isc) {
-  constexpr int NR = D == 3 ? 25 : 5;
-  constexpr int B = kCoreBatch;
-  int cnt = qe - qs;  // the own cell is a clique, p itself included
-  if (cnt >= P.minpts) {
-    isc = true;
-    return;
-  }
-  uint32_t pg[D];
-  double px[D], lo[D], hi[D];
-  if (F32) {
-    load_g<D>(d, p, pg);
-  } else {
-    load_x<D, F32>(d, p, px);
-#pragma unroll
-    for (int k = 0; k < D; ++k) {
-      lo[k] = px[k] - P.eps;
-      hi[k] = px[k] + P.eps;
-    }
-  }
-  // records stay in this lane's LDS slots until the point is known to be
-  // non-core
-  int nrec = 0;
-  int ev = 0;
-  const RowsOf rows = rows_of(d, c);
-  // the next group's packed rows are loaded while this group streams
-  int32_t pkn[5];
-#pragma unroll
-  for (int j = 0; j < 5; ++j) pkn[j] = rows[j];
-  for (int g = 0; g < NR && cnt < P.minpts; g += 5) {
-    int32_t aa[5], ll[5];
-    line_ranges(d, pkn, aa, ll);
-    if (g + 5 < NR) {
-#pragma unroll
-      for (int j = 0; j < 5; ++j) pkn[j] = rows[g + 5 + j];
-    }
-    ++t.groups;
-#pragma unroll
-    for (int j = 0; j < 5; ++j) t.lines += ll[j] > 0;
-    Stream5 s;
-    s.set(aa, ll);
-    for (int32_t t0 = 0; t0 < s.tot && cnt < P.minpts; t0 += B) {
-      int32_t qi[B];
-      uint32_t cg[B][D];
-      double cx[B][D];
-#pragma unroll
-      for (int j = 0; j < B; ++j) {
-        int jr;
-        qi[j] = t0 + j < s.tot ? s.at(t0 + j, jr) : p;
-        if (F32)
-          load_g<D>(d, qi[j], cg[j]);
-        else
-          load_x<D, F32>(d, qi[j], cx[j]);
-      }
-#pragma unroll
-      for (int j = 0; j < B; ++j) {
-        const int32_t q = qi[j];
-        if (t0 + j < s.tot && (q < qs || q >= qe)) {
-          bool fwd, sym;
-          if (F32) {
-            const float sd = d2fix<D>(pg, cg[j]);
-            if (sd < P.d2_in) {
-              fwd = sym = true;
-            } else if (sd > P.d2_out) {
-              fwd = sym = false;
-            } else {
-              double ax[D], bx[D];
-              load_x<D, F32>(d, p, ax);
-              load_x<D, F32>(d, q, bx);
-              const double dd = d2_64<D>(ax, bx);
-              sym = dd <= P.eps2;
-              fwd = sym && box_64<D>(ax, bx, P.eps);
-              t.band++;
-              t.flip += fwd != (sd <= P.d2_mid);
-            }
-          } else {
-            const double dd = d2_64<D>(px, cx[j]);
-            sym = dd <= P.eps2;
-            bool in = true;
-#pragma unroll
-            for (int k = 0; k < D; ++k) in = in && lo[k] <= cx[j][k] && cx[j][k] <= hi[k];
-            fwd = sym && in;
-          }
-          cnt += fwd;
-          if (sym) {
-            if (nrec < kRecSlots) rk[nrec] = q;
-            ++nrec;
-          }
-          ++ev;
-        }
-      }
-    }
-  }
-  isc = cnt >= P.minpts;
-  if (!isc) {
-    int32_t* rec = d.rec + (int64_t)p * R;
-    for (int i = 0; i < nrec && i < R; ++i) rec[i] = rk[i];
-    d.rec_n[p] = (uint8_t)(nrec < 255 ? nrec : 255);
-  }
-  t.eval += ev;
+// Neighbour counts in three kernels.
+//
+//   k_core        one lane per point.  A cell of >= minpts points is all core,
+//                 and a point whose rows hold fewer than minpts points in all
+//                 (the rows carry the counts) is not core.  Else the points of the cells around the point's cell (4 x 4
+//                 x 3 of them in 3-D: the middle steps of its own column's
+//                 window and of those towards the sides of the block that the
+//                 cell lies on) are counted until minpts, kCoreBudget of them
+//                 at most.  That settles most core points; the others are
+//                 listed for k_core_rest.  The count needs no records, and in the FP32 form no
+//                 guard band (a pair inside it is left to the list), so the
+//                 kernel is small enough for full residency.
+//   k_core_rest   one lane per listed point: the exact count over all of its
+//                 rows with early exit at minpts.  Every candidate with d^2 <=
+//                 eps^2 (either box direction) is recorded, so a point that
+//                 ends non-core holds all its neighbours outside its own cell
+//                 (records are kept slot by slot, so that neighbouring lanes
+//                 write neighbouring words).
+//   k_core_crowd  one wavefront per listed point with more than kCoreCrowd
+//                 candidates: one lane would take as long as the rest of the
+//                 launch.
+//
+// 4 M 3-D points, FP32 form: 166 + 172 + 4 us, where one kernel over lines of
+// five cells took 490 (and one kernel with all of this at 80 registers, 31 of
+// them spilled, 636); 32 M points: 240 + 127 + 155 where it took 615 (3.6 ms
+// with whole windows and no wavefront pass: a window's points start two steps
+// below the cell, so crowded windows end late); 1 M 2-D points, FP64: 20 + 17
+// where it took 57.
+//
+// A row's points are consecutive; those of the few cells of a row outside the
+// 5^D stencil fail the distance test.  The non-empty point ranges of a lane
+// wait in a queue of its own in LDS, so that every lane goes on to its next
+// range as soon as it is done with one, whatever the other lanes are at.
+constexpr int kCoreBudget = 64;   // candidates k_core tests per point
+constexpr int kCoreCrowd = 512;   // candidates from which a wavefront takes a point
+
+// Rows from the cell's own column outwards: block offsets in units of the
+// near sides' (ax, ay); the first four (two in 2-D) are the near ones.
+template <int D>
+__device__ __forceinline__ int core_row(int i, int ax, int ay) {
+  constexpr int oa[9] = {0, 1, 0, 1, -1, 0, -1, 1, -1}, ob[9] = {0, 0, 1, 1, 0, -1, 1, -1, -1};
+  if (D == 2) return Win<2>::own + (i == 0 ? 0 : (i == 1 ? ax : -ax));
+  return Win<3>::own + 3 * oa[i] * ax + ob[i] * ay;
+}
+template <int D>
+__device__ __forceinline__ void near_sides(int local, int& ax, int& ay) {
+  ax = D == 3 ? (local & 2 ? 1 : -1) : (local & 1 ? 1 : -1);
+  ay = D == 3 ? (local & 1 ? 1 : -1) : 0;
 }
 
-// 6 waves per SIMD for the FP32 form (80 VGPRs with a batch of four
-// candidates; latency bound, so residency pays more than a longer batch), 5
-// for the FP64 form, whose coordinates need more registers
+// Certain neighbours of p among the points of the near rows' middle steps,
+// its own cell's (`own` = qe - qs) included, until minpts or the budget; -1
+// when all rows together hold fewer than minpts points.
+template <int D, bool F32>
+__device__ int core_near(const Dev& d, const Par& P, int32_t p, int32_t c, int32_t qs,
+                         int32_t own, int2* queue, Tally& t) {
+  constexpr int NN = D == 3 ? 4 : 2;
+  constexpr int nl = Win<D>::nl;
+  constexpr int B = kCoreBatch;
+  constexpr uint32_t kLow = (1u << nl) - 1u, kMid = ((1u << (3 * nl)) - 1u) << nl;
+  int ax, ay;
+  near_sides<D>((int)(d.cell_zl[c] & (nl - 1)), ax, ay);
+  const RowsOf rows = rows_of(d, c);
+  uint2 row[Win<D>::rows];
+#pragma unroll
+  for (int r = 0; r < Win<D>::rows; ++r) row[r] = rows[core_row<D>(r, ax, ay)];
+  uint32_t tot = 0u;
+  bool many = false;
+#pragma unroll
+  for (int r = 0; r < Win<D>::rows; ++r) {
+    tot += row_count(row[r]);
+    many |= row_count(row[r]) == kRowCount;
+  }
+  t.rows += Win<D>::rows;
+  if (!many && (int)tot < P.minpts) return -1;
+  uint32_t pg[D];
+  double px[D];
+  if (F32)
+    load_g<D>(d, p, pg);
+  else
+    load_x<D, F32>(d, p, px);
+  int32_t a[NN], e[NN];
+#pragma unroll
+  for (int r = 0; r < NN; ++r) {
+    const int32_t m0 = (int32_t)row[r].x + __popc(row[r].y & kLow);
+    const int32_t n = __popc(row[r].y & kMid);
+    a[r] = e[r] = 0;
+    if (n) {
+      a[r] = d.cell_start[m0];
+      e[r] = d.cell_start[m0 + n];
+    }
+  }
+  int nq = 0;
+#pragma unroll
+  for (int r = 0; r < NN; ++r)
+    if (e[r] > a[r]) queue[256 * nq++] = make_int2(a[r], e[r]);
+  t.ranges += nq;
+  int cnt = own, j = 0, left = kCoreBudget;
+  int2 cur = make_int2(0, 0);
+  while (cnt < P.minpts && left > 0 && (cur.x < cur.y || j < nq)) {
+    if (cur.x >= cur.y) cur = queue[256 * j++];
+    int32_t qi[B];
+    uint32_t cg[B][D];
+    double cx[B][D];
+#pragma unroll
+    for (int u = 0; u < B; ++u) {
+      // past the end: a point of the own cell, which is not counted
+      qi[u] = cur.x + u < cur.y ? cur.x + u : qs;
+      if (F32)
+        load_g<D>(d, qi[u], cg[u]);
+      else
+        load_x<D, F32>(d, qi[u], cx[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < B; ++u) {
+      bool in;
+      if (F32)
+        in = d2fix<D>(pg, cg[u]) < P.d2_in;
+      else
+        in = d2_64<D>(px, cx[u]) <= P.eps2 && box_64<D>(px, cx[u], P.eps);
+      cnt += in && (uint32_t)(qi[u] - qs) >= (uint32_t)own;
+    }
+    t.eval += cur.y - cur.x < B ? cur.y - cur.x : B;
+    cur.x += B;
+    left -= B;
+  }
+  return cnt;
+}
+
 template <bool F32>
-__global__ __launch_bounds__(256, F32 ? 6 : 5) void k_core(Dev d) {
+__global__ __launch_bounds__(256, F32 ? 8 : 6) void k_core(Dev d) {
   if (abandoned(d)) return;
+  __shared__ int2 s_queue[4 * 256];
   const int64_t pl = (int64_t)xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
   const bool act = pl < d.n;
   const int32_t p = act ? (int32_t)pl : 0;
-  const int lane = lane_id();
-  int32_t c = 0, qs = 0, qe = 0;
+  int32_t c = 0, qs = 0, own = 0;
   int dim = 0;
   const Inst* I = d.inst;
   if (act) {
     c = d.cell_of[p];
     qs = d.cell_start[c];
-    qe = d.cell_start[c + 1];
+    own = d.cell_start[c + 1] - qs;
     I = inst_of_cell(d, c);
     dim = I->dim;
   }
   Tally t;
-  bool isc = false;
-  const int R = d.rec_stride;
   const Par P(*I);
-  // kRecSlots record slots per lane (stride kRecSlots + 1: no bank conflicts)
-  __shared__ int32_t s_rec[256 * (kRecSlots + 1)];
-  int32_t* rk = s_rec + threadIdx.x * (kRecSlots + 1);
-  DCLUST_BY_DIM(act, dim, (core_lane<3, F32>(d, P, p, c, qs, qe, R, rk, t, isc)),
-                (core_lane<2, F32>(d, P, p, c, qs, qe, R, rk, t, isc)));
+  int cnt = own;  // the own cell is a clique, p itself included
+  const bool search = act && own < P.minpts;
+  DCLUST_BY_DIM(search, dim, (cnt = core_near<3, F32>(d, P, p, c, qs, own, s_queue + threadIdx.x, t)),
+                (cnt = core_near<2, F32>(d, P, p, c, qs, own, s_queue + threadIdx.x, t)));
+  const bool isc = cnt >= P.minpts;
   if (act) d.core[p] = isc;
-  // non-core points: the lanes of the border-label pass
-  block_append(act && !isc, p, d.border_pts);
-  // per-cell core counts: the lanes of one cell form a contiguous run.  A
-  // cell that is core as a whole, or lies inside the wave, is written by its
-  // first point; only the parts of other cells are added up
-  const bool head = act && (p == qs || lane == 0);
-  const unsigned long long mh = ballot(head), mc = ballot(isc);
-  if (head) {
-    if (qe - qs >= P.minpts) {
-      if (p == qs) d.cell_ncore[c] = qe - qs;
-    } else {
-      const unsigned long long above = lane == 63 ? 0ull : (mh & (~0ull << (lane + 1)));
-      const int nxt = above ? __ffsll((long long)above) - 1 : 64;
-      const unsigned long long seg =
-          (nxt == 64 ? ~0ull : ((1ull << nxt) - 1ull)) & (~0ull << lane);
-      const int k = __popcll(mc & seg);
-      if (k && p == qs && qe - qs <= 64 - lane)
-        d.cell_ncore[c] = k;
-      else if (k)
-        atomicAdd(&d.cell_ncore[c], k);
+  if (cnt < 0) d.rec_n[p] = kRecFew;
+  block_append(act && !isc && cnt >= 0, p, d.core_rest);
+  block_append(cnt < 0, p, d.border_pts);
+  stat_add(d, C_EVAL, t.eval);
+  stat_add(d, C_CORE_ROWS, t.rows);
+  stat_add(d, C_CORE_RANGES, t.ranges);
+}
+
+// The exact predicate of the pair (p, q): `sym` d^2 <= eps^2, `fwd` the box
+// test from p's side as well.
+template <int D, bool F32>
+__device__ __forceinline__ void core_pred(const Dev& d, const Par& P, int32_t p, int32_t q,
+                                          const uint32_t* pg, const uint32_t* qg,
+                                          const double* px, const double* qx, bool& sym,
+                                          bool& fwd, Tally& t) {
+  if (F32) {
+    const float sd = d2fix<D>(pg, qg);
+    sym = fwd = sd < P.d2_in;
+    if (!(sd < P.d2_in) && !(sd > P.d2_out)) {
+      double ax[D], bx[D];
+      load_x<D, F32>(d, p, ax);
+      load_x<D, F32>(d, q, bx);
+      sym = d2_64<D>(ax, bx) <= P.eps2;
+      fwd = sym && box_64<D>(ax, bx, P.eps);
+      t.band++;
+      t.flip += fwd != (sd <= P.d2_mid);
+    }
+  } else {
+    sym = d2_64<D>(px, qx) <= P.eps2;
+    fwd = sym && box_64<D>(px, qx, P.eps);
+  }
+}
+
+// 0: not core, 1: core, 2: left to a wavefront
+template <int D, bool F32>
+__device__ int core_rest(const Dev& d, const Par& P, int32_t p, int R, int2* queue, int32_t* lrec,
+                         Tally& t) {
+  constexpr int NR = Win<D>::rows;
+  constexpr int B = kCoreBatch;
+  const int32_t c = d.cell_of[p];
+  const int32_t qs = d.cell_start[c], own = d.cell_start[c + 1] - qs;
+  int ax, ay;
+  near_sides<D>((int)(d.cell_zl[c] & (Win<D>::nl - 1)), ax, ay);
+  const RowsOf rows = rows_of(d, c);
+  int32_t a[NR], e[NR];
+  {
+    uint2 row[NR];
+#pragma unroll
+    for (int r = 0; r < NR; ++r) row[r] = rows[core_row<D>(r, ax, ay)];
+#pragma unroll
+    for (int r = 0; r < NR; ++r) row_points(d, row[r], a[r], e[r]);
+  }
+  int nq = 0;
+  int32_t tot = 0;  // (the own cell's points included)
+#pragma unroll
+  for (int r = 0; r < NR; ++r)
+    if (e[r] > a[r]) {
+      queue[256 * nq++] = make_int2(a[r], e[r]);
+      tot += e[r] - a[r];
+    }
+  t.rows += NR;
+  t.ranges += nq;
+  if (tot > kCoreCrowd) return 2;
+  int nrec = 0;
+  uint32_t pg[D];
+  double px[D];
+  if (F32)
+    load_g<D>(d, p, pg);
+  else
+    load_x<D, F32>(d, p, px);
+  int cnt = own, j = 0;
+  int2 cur = make_int2(0, 0);
+  while (cnt < P.minpts && (cur.x < cur.y || j < nq)) {
+    if (cur.x >= cur.y) cur = queue[256 * j++];
+    int32_t qi[B];
+    uint32_t cg[B][D];
+    double cx[B][D];
+#pragma unroll
+    for (int u = 0; u < B; ++u) {
+      qi[u] = cur.x + u < cur.y ? cur.x + u : qs;  // (not counted, as above)
+      if (F32)
+        load_g<D>(d, qi[u], cg[u]);
+      else
+        load_x<D, F32>(d, qi[u], cx[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < B; ++u)
+      if ((uint32_t)(qi[u] - qs) >= (uint32_t)own) {
+        bool sym, fwd;
+        core_pred<D, F32>(d, P, p, qi[u], pg, cg[u], px, cx[u], sym, fwd, t);
+        cnt += fwd;
+        if (sym) {
+          if (nrec < R) lrec[nrec] = qi[u];
+          ++nrec;
+        }
+        ++t.eval;
+      }
+    cur.x += B;
+  }
+  if (cnt >= P.minpts) return 1;
+  for (int i = 0; i < nrec && i < R; ++i) d.rec[(int64_t)i * d.n + p] = lrec[i];
+  d.rec_n[p] = (uint8_t)(nrec <= R ? nrec : kRecNone);
+  return 0;
+}
+
+// LDS of a k_core_rest workgroup: per lane nine ranges, and R record slots
+// (one more: no bank conflicts)
+static size_t core_lds(int R) { return 256 * (kMaxRows * sizeof(int2) + (R + 1) * 4); }
+
+template <bool F32>
+__global__ __launch_bounds__(256, F32 ? 6 : 5) void k_core_rest(Dev d) {
+  if (abandoned(d)) return;
+  extern __shared__ int2 s_core[];
+  __shared__ long long s_pre[kStripes + 1];
+  const long long n = slist_prefix(d.core_rest, s_pre);
+  const int R = d.rec_stride;
+  int2* queue = s_core + threadIdx.x;
+  int32_t* lrec = reinterpret_cast<int32_t*>(s_core + 256 * kMaxRows) + threadIdx.x * (R + 1);
+  Tally t;
+  for (long long i0 = (long long)blockIdx.x * 256; i0 < n; i0 += (long long)gridDim.x * 256) {
+    const long long i = i0 + threadIdx.x;
+    const bool act = i < n;
+    const int32_t p = act ? slist_at(d.core_rest, s_pre, i) : 0;
+    const Inst* I = d.inst;
+    int dim = 0;
+    if (act) {
+      if (d.ninst != 1) I = inst_of_cell(d, d.cell_of[p]);
+      dim = I->dim;
+    }
+    const Par P(*I);
+    int res = 0;
+    DCLUST_BY_DIM(act, dim, (res = core_rest<3, F32>(d, P, p, R, queue, lrec, t)),
+                  (res = core_rest<2, F32>(d, P, p, R, queue, lrec, t)));
+    if (act && res == 1) d.core[p] = 1;
+    block_append(act && res == 0, p, d.border_pts);
+    block_append(act && res == 2, p, d.core_crowd);
+  }
+  stat_add(d, C_EVAL, t.eval);
+  stat_add(d, C_BAND_CORE, t.band);
+  stat_add(d, C_BAND, t.band);
+  stat_add(d, C_FLIP, t.flip);
+  stat_add(d, C_CORE_ROWS, t.rows);
+  stat_add(d, C_CORE_RANGES, t.ranges);
+}
+
+template <int D, bool F32>
+__device__ bool core_wave(const Dev& d, const Par& P, int32_t p, int R, Tally& t) {
+  constexpr int NR = Win<D>::rows;
+  const int lane = lane_id();
+  const int32_t c = d.cell_of[p];
+  const int32_t qs = d.cell_start[c], own = d.cell_start[c + 1] - qs;
+  int ax, ay;
+  near_sides<D>((int)(d.cell_zl[c] & (Win<D>::nl - 1)), ax, ay);
+  const RowsOf rows = rows_of(d, c);
+  uint32_t pg[D];
+  double px[D];
+  if (F32)
+    load_g<D>(d, p, pg);
+  else
+    load_x<D, F32>(d, p, px);
+  int cnt = own, nrec = 0;
+  for (int r = 0; r < NR && cnt < P.minpts; ++r) {
+    int32_t a, e;
+    row_points(d, rows[core_row<D>(r, ax, ay)], a, e);
+    for (; a < e && cnt < P.minpts; a += 64) {
+      const int32_t q = a + lane < e ? a + lane : qs;
+      uint32_t qg[D];
+      double qx[D];
+      if (F32)
+        load_g<D>(d, q, qg);
+      else
+        load_x<D, F32>(d, q, qx);
+      bool sym = false, fwd = false;
+      if ((uint32_t)(q - qs) >= (uint32_t)own) {
+        core_pred<D, F32>(d, P, p, q, pg, qg, px, qx, sym, fwd, t);
+        ++t.eval;
+      }
+      cnt += __popcll(ballot(fwd));
+      const unsigned long long m = ballot(sym);
+      const int slot = nrec + mbcnt(m);
+      if (sym && slot < R) d.rec[(int64_t)slot * d.n + p] = q;
+      nrec += __popcll(m);
+    }
+  }
+  if (lane == 0) d.rec_n[p] = (uint8_t)(nrec <= R ? nrec : kRecNone);
+  return cnt >= P.minpts;
+}
+
+template <bool F32>
+__global__ __launch_bounds__(256) void k_core_crowd(Dev d) {
+  if (abandoned(d)) return;
+  __shared__ long long s_pre[kStripes + 1];
+  const long long n = slist_prefix(d.core_crowd, s_pre);
+  const int R = d.rec_stride;
+  Tally t;
+  for (long long i = (long long)blockIdx.x * 4 + (threadIdx.x >> 6); i < n;
+       i += (long long)gridDim.x * 4) {
+    const int32_t p = rfl_i(slist_at(d.core_crowd, s_pre, i));
+    const Inst& I = *inst_of_cell(d, d.ninst == 1 ? 0 : d.cell_of[p]);
+    const Par P(I);
+    const bool isc = I.dim == 3 ? core_wave<3, F32>(d, P, p, R, t)
+                                : core_wave<2, F32>(d, P, p, R, t);
+    if (lane_id() == 0) {
+      if (isc) {
+        d.core[p] = 1;
+      } else {
+        const SList& L = d.border_pts;
+        const int s = blockIdx.x & (kStripes - 1);
+        L.data[s * L.cap + (int64_t)atomicAdd(&L.cnt[s * kStatStride], 1ull)] = p;
+      }
     }
   }
   stat_add(d, C_EVAL, t.eval);
   stat_add(d, C_BAND_CORE, t.band);
   stat_add(d, C_BAND, t.band);
   stat_add(d, C_FLIP, t.flip);
-  stat_add(d, C_CORE_GROUPS, t.groups);
-  stat_add(d, C_CORE_LINES, t.lines);
 }
 
 // ----------------------------------------------------------- near graph --
-// Stencil lines whose cells can lie above a cell (offsets (a, b) >= (0, 0)
-// in the key order, the own line included), in row order; -1 pads.
-#define DCLUST_UPPER_ROWS3 {0, 2, 4, 7, 8, 10, 12, 15, 16, 18, 20, 23, 24, -1, -1}
-#define DCLUST_UPPER_ROWS2 {0, 2, 4, -1, -1}
-static __constant__ int8_t kUpperRows3[15] = DCLUST_UPPER_ROWS3;
-static __constant__ int8_t kUpperRows2[5] = DCLUST_UPPER_ROWS2;
-
-// Near lines above a cell (offsets of at most one; every cell of them but
-// the own line's lower half has a larger index): (0,0), (1,0), (0,1),
-// (1,-1), (1,1) in 3-D; (0) and (1) in 2-D.  Nibble i of `rows` is the i-th
-// such row, nibble r of `mirror` the line with row r's offsets negated.
-template <int D>
-struct Upper {
-  static constexpr int lines = D == 3 ? 5 : 2;
-  static constexpr unsigned long long rows = D == 3 ? 0x87420ull : 0x20ull;
-  static constexpr unsigned long long mirror = D == 3 ? 0x567834120ull : 0x120ull;
-};
-namespace tables {
-constexpr int8_t up3[15] = DCLUST_UPPER_ROWS3;
-constexpr int8_t up2[5] = DCLUST_UPPER_ROWS2;
-constexpr bool above(int a, int b) { return a > 0 || (a == 0 && b >= 0); }
-constexpr bool upper_ok() {
-  int i = 0;
-  for (int r = 0; r < 25; ++r)
-    if (above(off3[r][0], off3[r][1]) && up3[i++] != r) return false;
-  if (i != 13 || up3[13] != -1 || up3[14] != -1) return false;
-  i = 0;
-  for (int r = 0; r < 5; ++r)
-    if (off2[r] >= 0 && up2[i++] != r) return false;
-  if (i != 3) return false;
-  // near rows of the near graph (nibbles) and their mirrors
-  for (int k = 0; k < 5; ++k) {
-    const int r = (int)((Upper<3>::rows >> (4 * k)) & 15ull);
-    if (r > 8 || !above(off3[r][0], off3[r][1]) || up3[k] != r) return false;
-  }
-  for (int r = 0; r < 9; ++r)
-    if ((int)((Upper<3>::mirror >> (4 * r)) & 15ull) != mir3[r]) return false;
-  for (int k = 0; k < 2; ++k)
-    if ((int)((Upper<2>::rows >> (4 * k)) & 15ull) != up2[k]) return false;
-  for (int r = 0; r < 3; ++r)
-    if ((int)((Upper<2>::mirror >> (4 * r)) & 15ull) != mir2[r]) return false;
-  return true;
-}
-static_assert(upper_ok(), "upper stencil lines");
-}  // namespace tables
-
 // Workgroups of the kernels that walk the list of core cells (grid-stride).
 constexpr int kListGrid = 4096;
 
@@ -388,24 +545,34 @@ __global__ __launch_bounds__(1024) void k_rep(Dev d) {
   if (c - threadIdx.x >= C) return;  // (block-uniform)
   const bool in = c < C;
   const int64_t cc = in ? c : 0;
-  const int32_t ncore = d.cell_ncore[cc], q0 = d.cell_start[cc], q1 = d.cell_start[cc + 1];
+  const int32_t q0 = d.cell_start[cc], q1 = d.cell_start[cc + 1];
   const int minpts = inst_of_cell(d, cc)->minpts;
+  // core points: all of a cell of minpts points, else few flags to count
+  int32_t ncore = q1 - q0, first = q0;
+  if (ncore < minpts) {
+    ncore = 0;
+    for (int32_t q = q1 - 1; q >= q0; --q)
+      if (d.core[q]) {
+        ++ncore;
+        first = q;
+      }
+  }
   const bool hc = in && ncore > 0;
   uint4 r = make_uint4(0u, 0u, 0u, kNoRep);
   if (hc) {
-    int32_t q = q0;
-    if (ncore != q1 - q0)
-      while (!d.core[q]) ++q;
-    r = make_uint4(d.G[0][q], d.G[1][q], d.G[2][q], (uint32_t)q);
+    const int32_t q = first;
+    r = make_uint4(d.G[3 * (int64_t)q], d.G[3 * (int64_t)q + 1], d.G[3 * (int64_t)q + 2],
+                   (uint32_t)q);
   }
   // (the forest covers every cell: the chain merge walks all of it, and the
   // relabel pass reads entry 0 for points that are not core)
   if (in) {
     d.rep[c] = r;
+    d.cell_ncore[c] = ncore;
     d.cell_comp[c] = -1;
     d.parent[c] = (int32_t)c;
     d.compmin[c] = kNoKey;
-    d.amask[c] = 0ull;
+    d.amask[c] = 0u;
     d.cell_label[c] = kUnclaimed;
   }
   block_append(hc, (int32_t)c, d.core_cells);
@@ -431,72 +598,103 @@ __global__ __launch_bounds__(1024) void k_rep(Dev d) {
   }
 }
 
-// Near graph: bit 5r+k of a core cell's mask is set when cell k of its near
-// line r (r < 9) holds a representative that is certainly joined to its own
+// Near graph: near bit b of a core cell's mask is set when the near cell at
+// its offset holds a representative that is certainly joined to its own
 // (fixed-point distance below the guard band, which implies the FP64
-// predicate in both directions).  Each pair is tested once, by its lower
-// cell.  The graph need not hold every adjacent pair: whatever pair it
+// predicate in both directions).  Each pair is tested once, by the cell for
+// which the offset is positive (bits above kNearOwn).
+// The graph need not hold every adjacent pair: whatever pair it
 // leaves in two components is decided exactly by the pass over component
 // borders (k_far, k_far_pairs).  Inside a cluster the first pair of points
 // nearly always joins (of 7.3 M near cell pairs of the 4 M point 3-D
 // workload 92 % are joined, with 1.15 point tests per pair), so one 16-byte
 // load and one distance per pair take the place of a scan of both cells'
-// points: 49 + 64 us with k_rep, where testing every near pair to the end
+// points: 55 + 58 us with k_rep, where testing every near pair to the end
 // took 289 us there, 77 + 90 us on 1 M 2-D points (here 20) and 2.2 ms on
 // 32 M points in dense blobs (cells of more than 32 points wave by wave).
+// Representatives of three consecutive steps (below, at and above the cell)
+// at one place of a row, tested against `ag`: bits b0, b0 + 1, b0 + 2.
 template <int D>
-__device__ __forceinline__ unsigned long long near_bits(const Dev& d, float d2_in, int32_t A,
-                                                        Tally& t) {
-  constexpr int NN = Upper<D>::lines;
+__device__ __forceinline__ void near_line(const Dev& d, float d2_in, const uint32_t* ag,
+                                          uint2 row, int place, int b0, uint32_t& m, Tally& t) {
+  constexpr int nl = Win<D>::nl;
+  uint4 b4[3];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const int s = (k + 1) * nl + place;
+    b4[k].w = kNoRep;
+    if ((row.y >> s) & 1u) b4[k] = d.rep[slot_cell(row, s)];
+  }
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const uint32_t bg[3] = {b4[k].x, b4[k].y, b4[k].z};
+    if (b4[k].w != kNoRep) {
+      ++t.eval;
+      if (d2fix<D>(ag, bg) < d2_in) m |= 1u << (b0 + k);
+    }
+  }
+}
+
+template <int D>
+__device__ __forceinline__ uint32_t near_bits(const Dev& d, float d2_in, int32_t A, Tally& t) {
   const uint4 a4 = d.rep[A];
   const uint32_t ag[3] = {a4.x, a4.y, a4.z};
+  const int local = (int)(d.cell_zl[A] & (Win<D>::nl - 1));
   const RowsOf rows = rows_of(d, A);
-  int32_t pk[NN];
-#pragma unroll
-  for (int i = 0; i < NN; ++i) pk[i] = rows[(int)((Upper<D>::rows >> (4 * i)) & 15ull)];
-  unsigned long long m = 0;
-#pragma unroll
-  for (int i = 0; i < NN; ++i) {
-    const int r = (int)((Upper<D>::rows >> (4 * i)) & 15ull);
-    const int32_t len = pk[i] >> kRowCntShift, st = pk[i] & kRowCellMask;
-    uint4 b4[5];
-#pragma unroll
-    for (int k = 0; k < 5; ++k) {
-      b4[k].w = kNoRep;
-      if (k < len && st + k > A) b4[k] = d.rep[st + k];
-    }
-    t.lines += len > 0;
-    t.cells += len;
-#pragma unroll
-    for (int k = 0; k < 5; ++k) {
-      const uint32_t bg[3] = {b4[k].x, b4[k].y, b4[k].z};
-      if (b4[k].w != kNoRep) {
+  uint32_t m = 0;
+  if (D == 2) {
+    const uint2 own = rows[1], up = rows[1 + local];  // dx = 1 lies in block lx
+    near_line<2>(d, d2_in, ag, up, local ^ 1, 21, m, t);
+    const int s = 3 * 2 + local;  // dx = 0, one step up
+    if ((own.y >> s) & 1u) {
+      const uint4 b4 = d.rep[slot_cell(own, s)];
+      const uint32_t bg[3] = {b4.x, b4.y, b4.z};
+      if (b4.w != kNoRep) {
         ++t.eval;
-        if (d2fix<D>(ag, bg) < d2_in) m |= 1ull << (5 * r + k);
+        if (d2fix<2>(ag, bg) < d2_in) m |= 1u << 14;
+      }
+    }
+  } else {
+    const int lx = local >> 1, ly = local & 1;
+    // dx = 1 lies in block row lx; dy = 0 and the dy towards the cell's own
+    // block in block column 0, the other dy in block column nb; dx = 0,
+    // dy = 1 in block column ly
+    const int nb = ly ? 1 : -1;
+    const uint2 own = rows[4], x0 = rows[4 + 3 * lx], xb = rows[4 + 3 * lx + nb],
+                y1 = rows[4 + ly];
+    const int xo = (lx ^ 1) * 2;
+    near_line<3>(d, d2_in, ag, x0, xo + ly, 21, m, t);
+    near_line<3>(d, d2_in, ag, x0, xo + (ly ^ 1), 21 - 3 * nb, m, t);
+    near_line<3>(d, d2_in, ag, xb, xo + (ly ^ 1), 21 + 3 * nb, m, t);
+    near_line<3>(d, d2_in, ag, y1, lx * 2 + (ly ^ 1), 15, m, t);
+    const int s = 3 * 4 + local;  // dx = dy = 0, one step up
+    if ((own.y >> s) & 1u) {
+      const uint4 b4 = d.rep[slot_cell(own, s)];
+      const uint32_t bg[3] = {b4.x, b4.y, b4.z};
+      if (b4.w != kNoRep) {
+        ++t.eval;
+        if (d2fix<3>(ag, bg) < d2_in) m |= 1u << 14;
       }
     }
   }
   return m;
 }
 
-// Expansion by seed lists: each bit of A is also set in the other cell's
-// mask (A's place in that cell's mirrored line).
-template <int D>
-__device__ void near_mirror(const Dev& d, int32_t A, unsigned long long m) {
-  const RowsOf rows = rows_of(d, A);
-  if (m) atomicOr(&d.amask[A], m);
-  while (m) {
-    const int b = __ffsll((long long)m) - 1;
-    m &= m - 1;
-    const int r = (b * 205) >> 10;  // b / 5 for 0 <= b < 128
-    const int32_t B = (rows[r] & kRowCellMask) + (b - 5 * r);
-    const int rm = (int)((Upper<D>::mirror >> (4 * r)) & 15ull);
-    const int32_t pos = rows_of(d, B)[rm] & kRowCellMask;
-    atomicOr(&d.amask[B], 1ull << (5 * rm + (A - pos)));
-  }
+// Near cell of A at near bit b (one of A's mask bits).
+__device__ __forceinline__ int32_t near_cell(const RowsOf& rows, int dim, int local, int b) {
+  int row, slot;
+  if (dim == 3)
+    near_slot<3>(b, local, row, slot);
+  else
+    near_slot<2>(b, local, row, slot);
+  return slot_cell(rows[row], slot);
+}
+__device__ __forceinline__ int local_of(const Dev& d, int32_t c, int dim) {
+  return (int)(d.cell_zl[c] & (dim == 3 ? 3u : 1u));
 }
 
-// One lane per core cell.
+// One lane per core cell.  For the expansion by seed lists each bit of A is
+// also set in the other cell's mask, at the opposite offset.
 __global__ __launch_bounds__(256) void k_adj(Dev d) {
   if (abandoned(d)) return;
   __shared__ long long s_pre[kStripes + 1];
@@ -506,7 +704,7 @@ __global__ __launch_bounds__(256) void k_adj(Dev d) {
   for (long long i0 = (long long)blockIdx.x * 256; i0 < n; i0 += (long long)gridDim.x * 256) {
     const long long i = i0 + threadIdx.x;
     const bool act = i < n;
-    const int32_t A = act ? slist_at(d.core_cells, s_pre, i) : -1;
+    const int32_t A = act ? slist_at(d.core_cells, s_pre, i) : 0;
     int dim = 0;
     float d2_in = 0.f;
     if (act) {
@@ -514,19 +712,24 @@ __global__ __launch_bounds__(256) void k_adj(Dev d) {
       dim = I->dim;
       d2_in = I->d2_in;
     }
-    unsigned long long m = 0;
+    uint32_t m = 0;
     DCLUST_BY_DIM(act, dim, (m = near_bits<3>(d, d2_in, A, t)),
                   (m = near_bits<2>(d, d2_in, A, t)));
-    if (d.chains) {
-      DCLUST_BY_DIM(act, dim, near_mirror<3>(d, A, m), near_mirror<2>(d, A, m));
-    } else {
-      edges += 2 * __popcll(m);
+    if (!d.chains) {
+      edges += 2 * __popc(m);
       if (act) d.amask[A] = m;
+    } else if (m) {
+      const RowsOf rows = rows_of(d, A);
+      const int local = local_of(d, A, dim);
+      atomicOr(&d.amask[A], m);
+      while (m) {
+        const int b = __ffs(m) - 1;
+        m &= m - 1;
+        atomicOr(&d.amask[near_cell(rows, dim, local, b)], 1u << (2 * kNearOwn - b));
+      }
     }
   }
   stat_add(d, C_ADJ_TESTS, t.eval);
-  stat_add(d, C_ADJ_LINES, t.lines);
-  stat_add(d, C_ADJ_CELLS, t.cells);
   if (!d.chains) stat_add(d, C_EDGES, edges);
 }
 
@@ -576,7 +779,6 @@ __device__ __forceinline__ int32_t lds_union(int32_t* par, int32_t a, int32_t b)
 __global__ __launch_bounds__(1024) void k_link_local(Dev d) {
   if (abandoned(d)) return;
   __shared__ int32_t par[kLinkCells];
-  const int lane = lane_id();
   const int32_t C = (int32_t)d.ctl[C_NCELL];
   // cells per run: the workgroups share the cells, in whole wavefronts
   int32_t K = (C + (int32_t)gridDim.x - 1) / (int32_t)gridDim.x;
@@ -584,42 +786,24 @@ __global__ __launch_bounds__(1024) void k_link_local(Dev d) {
   K = K < kLinkMin ? kLinkMin : (K > kLinkCells ? kLinkCells : K);
   for (int64_t c0 = (int64_t)blockIdx.x * K; c0 < C; c0 += (int64_t)gridDim.x * K) {
     const int32_t nc = (int32_t)(C - c0 < K ? C - c0 : K);
-    // the forest starts with the runs of cells joined one to the next along
-    // their line, as far as they lie in one wavefront: united pair by pair
-    // they would form chains as long as the run
-    for (int i = threadIdx.x; i < K; i += 1024) {
-      bool link = false;  // joined to cell i + 1
-      if (i < nc) {
-        const int32_t A = (int32_t)c0 + i;
-        const int q = A + 1 - (rows_of(d, A)[0] & kRowCellMask);
-        link = lane < 63 && i + 1 < nc && q < 5 && ((d.amask[A] >> q) & 1ull);
-      }
-      const unsigned long long heads = ~(ballot(link) << 1);
-      const int head = 63 - __clzll((long long)(heads & (~0ull >> (63 - lane))));
-      if (i < nc) par[i] = i - lane + head;
-    }
+    for (int i = threadIdx.x; i < nc; i += 1024) par[i] = i;
     __syncthreads();
     for (int i = threadIdx.x; i < nc; i += 1024) {
       const int32_t A = (int32_t)c0 + i;
-      unsigned long long m = d.amask[A];
+      uint32_t m = d.amask[A];
       if (!m) continue;
-      unsigned long long ext = 0ull;
+      const int dim = inst_of_cell(d, A)->dim, local = local_of(d, A, dim);
       const RowsOf rows = rows_of(d, A);
+      uint32_t ext = 0u;
       int32_t root = i;
       while (m) {
-        const int b = __ffsll((long long)m) - 1;
-        const int r = (b * 205) >> 10;  // b / 5 for 0 <= b < 128
-        const int32_t B0 = (rows[r] & kRowCellMask) - (int32_t)c0 - 5 * r;
-        unsigned long long lm = m & (31ull << (5 * r));  // the bits of line r
-        m &= ~lm;
-        while (lm) {
-          const int q = __ffsll((long long)lm) - 1;
-          lm &= lm - 1;
-          if (B0 + q < nc)
-            root = lds_union(par, root, B0 + q);
-          else
-            ext |= 1ull << q;
-        }
+        const int b = __ffs(m) - 1;
+        m &= m - 1;
+        const int32_t B = near_cell(rows, dim, local, b) - (int32_t)c0;
+        if (B >= 0 && B < nc)
+          root = lds_union(par, root, B);
+        else
+          ext |= 1u << b;
       }
       d.amask[A] = ext;
     }
@@ -648,16 +832,16 @@ __global__ __launch_bounds__(256) void k_link_cross(Dev d) {
   for (long long i0 = (long long)blockIdx.x * 256; i0 < n; i0 += (long long)gridDim.x * 256) {
     const long long i = i0 + threadIdx.x;
     const int32_t A = i < n ? slist_at(d.core_cells, s_pre, i) : -1;
-    unsigned long long m = A >= 0 ? d.amask[A] : 0ull;
+    uint32_t m = A >= 0 ? d.amask[A] : 0u;
     const int32_t pa = m ? d.parent[A] : 0;
     const RowsOf rows = rows_of(d, m ? A : 0);
-    while (ballot(m != 0ull)) {
+    const int dim = inst_of_cell(d, m ? A : 0)->dim, local = local_of(d, m ? A : 0, dim);
+    while (ballot(m != 0u)) {
       int32_t pb = -1;
       if (m) {
-        const int b = __ffsll((long long)m) - 1;
+        const int b = __ffs(m) - 1;
         m &= m - 1;
-        const int r = (b * 205) >> 10;
-        pb = d.parent[(rows[r] & kRowCellMask) + (b - 5 * r)];
+        pb = d.parent[near_cell(rows, dim, local, b)];
       }
       // neighbouring cells mostly name the same two roots: a pair in the
       // wave's table is left out, and of the lanes that hold the same pair
@@ -761,7 +945,7 @@ __device__ bool cells_joined(const Dev& d, const Par& P, int32_t qs, int32_t qe,
     }
     double ax[D];
 #pragma unroll
-    for (int x = 0; x < D; ++x) ax[x] = F32 ? 0.0 : d.X[x][a];
+    for (int x = 0; x < D; ++x) ax[x] = F32 ? 0.0 : d.X[3 * (int64_t)a + x];
     for (int32_t q0 = b0; q0 < b1; q0 += 4) {
       bool cf[4];
       uint32_t qg[4][D];
@@ -774,8 +958,8 @@ __device__ bool cells_joined(const Dev& d, const Par& P, int32_t qs, int32_t qe,
         cf[j] = in && d.core[q];
 #pragma unroll
         for (int x = 0; x < D; ++x) {
-          qg[j][x] = F32 ? d.G[x][q] : 0u;
-          qx[j][x] = !F32 ? d.X[x][q] : 0.0;
+          qg[j][x] = F32 ? d.G[3 * (int64_t)q + x] : 0u;
+          qx[j][x] = !F32 ? d.X[3 * (int64_t)q + x] : 0.0;
         }
       }
 #pragma unroll
@@ -790,109 +974,80 @@ __device__ bool cells_joined(const Dev& d, const Par& P, int32_t qs, int32_t qe,
   return false;
 }
 
-// Core cell A, one lane: every stencil cell above A (each unordered pair is
-// taken by its lower cell) with core points in another component is decided;
-// a joined pair unions the two components (lock-free union-find on the chain
-// forest).  A pair whose components have been united meanwhile is skipped.
-// A pair with a heavy cell is listed for k_far_pairs (one wavefront per
-// pair); when its list is full the pair is decided here.
-template <int D, bool F32>
-__device__ long long far_cell(const Dev& d, const Par& P, int32_t A, Tally& t,
-                              long long& freeb) {
-  constexpr int NR = D == 3 ? 13 : 3;  // upper lines
-  const int32_t qs = d.cell_start[A], qe = d.cell_start[A + 1];
-  const bool allc = d.cell_ncore[A] == qe - qs;
-  const int32_t compA = d.cell_comp[A];
-  const int32_t zA = d.cell_z[A];
+// Core cell A, one lane: the stencil cells above A (each unordered pair is
+// taken by its lower cell) with core points in another component are listed,
+// pairs with a heavy cell apart.  (Deciding them here held the lanes of the
+// listing at 5 waves per SIMD with 32 spilled registers: 158 us on the 4 M
+// point 3-D workload, against 65 + 24 with k_far_pairs.)
+template <int D>
+__device__ __forceinline__ void far_cell(const Dev& d, int32_t A, int32_t compA, bool heavyA) {
+  constexpr int NU = Win<D>::rows - Win<D>::own;  // own row and those above
+  constexpr int nl = Win<D>::nl;
+  const int local = (int)(d.cell_zl[A] & (nl - 1));
   const RowsOf rows = rows_of(d, A);
-  long long joins = 0;
-  // five lines at a time: their packed rows in one round of loads, then the
-  // components of all their cells above A in the next; bit 5j+k of `todo`
-  // marks cell k of line j as above A in another component (cell_comp is
-  // -1 for a cell without core points)
-  for (int g = 0; g < NR; g += 5) {
-    int32_t pk[5];
-    int rr[5];
+  uint2 row[NU];
 #pragma unroll
-    for (int j = 0; j < 5; ++j) {
-      rr[j] = D == 3 ? kUpperRows3[g + j] : kUpperRows2[g + j];
-      pk[j] = rr[j] >= 0 ? rows[rr[j]] : 0;
-    }
-    unsigned todo = 0u;
+  for (int j = 0; j < NU; ++j) row[j] = rows[Win<D>::own + j];
+  // cells with core points in another component, by place in each window's
+  // cells (cell_comp is -1 for a cell without core points); the windows'
+  // cells are consecutive, so their components are loaded four at a time (up
+  // to three entries past the last cell may be read: the array has them)
+  uint32_t other[NU];
 #pragma unroll
-    for (int j = 0; j < 5; ++j) {
-      const int32_t len = pk[j] >> kRowCntShift, st = pk[j] & kRowCellMask;
+  for (int j = 0; j < NU; ++j) {
+    const int n = row_cells(row[j]);
+    const int32_t* cp = d.cell_comp + (int64_t)row[j].x;
+    other[j] = 0u;
 #pragma unroll
-      for (int k = 0; k < 5; ++k) {
-        const int32_t comp = (k < len && st + k > A) ? d.cell_comp[st + k] : compA;
-        if (comp >= 0 && comp != compA) todo |= 1u << (5 * j + k);
+    for (int q = 0; q < Win<D>::slots; q += 4)
+      if (q < n) {
+        const int32_t k[4] = {cp[q], cp[q + 1], cp[q + 2], cp[q + 3]};
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          other[j] |= (k[u] >= 0 && k[u] != compA) ? 1u << (q + u) : 0u;
       }
-    }
+    other[j] &= (1u << n) - 1u;
+  }
+#pragma unroll
+  for (int j = 0; j < NU; ++j) {
+    if (!other[j]) continue;
+    const int r = Win<D>::own + j;
+    const int a = D == 3 ? r / 3 - 1 : r - 1, b = D == 3 ? r % 3 - 1 : 0;
+    uint32_t todo = row[j].y & row_valid<D>(a, b, local);
+    if (j == 0) todo &= ~0u << (2 * nl + local + 1);  // above A in its own column
     while (todo) {
-      const int b = __ffs(todo) - 1;
+      const int s = __ffs(todo) - 1;
       todo &= todo - 1;
-      const int j = (b * 205) >> 10;  // b / 5 for b < 25
-      const int k = b - 5 * j;
-      int32_t pkj = pk[0];
-      int r = rr[0];
-#pragma unroll
-      for (int q = 1; q < 5; ++q) {
-        pkj = j == q ? pk[q] : pkj;
-        r = j == q ? rr[q] : r;
-      }
-      const int32_t B = (pkj & kRowCellMask) + k;
-      // B's place along the line, its point range and both roots, together
-      const int32_t zB = d.cell_z[B], b0 = d.cell_start[B], b1 = d.cell_start[B + 1];
-      const int32_t compB = d.cell_comp[B];
-      const int32_t ra = uf_find_cached(d.parent, compA), rb = uf_find_cached(d.parent, compB);
-      if (ra == rb) continue;
-      if (qe - qs > kHeavy || b1 - b0 > kHeavy) {
-        const int s = blockIdx.x & (kStripes - 1);
-        const unsigned long long at = atomicAdd(&d.far_pairs.cnt[s * kStatStride], 1ull);
-        if (at < (unsigned long long)d.far_pairs.cap) {
-          d.far_pairs.data[s * d.far_pairs.cap + (int64_t)at] = make_int2(A, B);
-          continue;
-        }
-      }
-      const int o0 = D == 3 ? kRowOff3[r][0] : kRowOff2[r];
-      const int o1 = D == 3 ? kRowOff3[r][1] : 0;
-      // (B lies in a neighbour line of A: the difference of their last
-      // coordinates is the offset)
-      if (cells_joined<D, F32>(d, P, qs, qe, allc, b0, b1, o0, o1, zB - zA, t, freeb)) {
-        uf_union(d.parent, ra, rb);
-        ++joins;
-      }
+      const int place = __popc(row[j].y & ((1u << s) - 1u));
+      if (!((other[j] >> place) & 1u)) continue;
+      const int32_t B = (int32_t)row[j].x + place;
+      const bool heavy = heavyA || d.cell_start[B + 1] - d.cell_start[B] > kHeavy;
+      const PairList& L = heavy ? d.far_heavy : d.far_light;
+      const int st = blockIdx.x & (kStripes - 1);
+      const unsigned long long at = atomicAdd(&L.cnt[st * kStatStride], 1ull);
+      if (at < (unsigned long long)L.cap) L.data[st * L.cap + (int64_t)at] = make_int2(A, B);
     }
   }
-  return joins;
 }
 
-template <bool F32>
-__global__ __launch_bounds__(256, 5) void k_far(Dev d) {
+__global__ __launch_bounds__(256, 8) void k_far(Dev d) {
   if (abandoned(d)) return;
   __shared__ long long s_pre[kStripes + 1];
   const long long n = slist_prefix(d.core_cells, s_pre);
-  Tally t;
-  long long freeb = 0, joins = 0;
   for (long long i0 = (long long)blockIdx.x * 256; i0 < n; i0 += (long long)gridDim.x * 256) {
     const long long i = i0 + threadIdx.x;
     const bool act = i < n;
-    const int32_t A = act ? slist_at(d.core_cells, s_pre, i) : 0;
+    int32_t A = 0, comp = 0;
     int dim = 0;
-    const Inst* I = d.inst;
+    bool heavy = false;
     if (act) {
-      I = inst_of_cell(d, A);
-      dim = I->dim;
+      A = slist_at(d.core_cells, s_pre, i);
+      dim = inst_of_cell(d, A)->dim;
+      comp = d.cell_comp[A];
+      heavy = d.cell_start[A + 1] - d.cell_start[A] > kHeavy;
     }
-    const Par P(*I);
-    DCLUST_BY_DIM(act, dim, (joins += far_cell<3, F32>(d, P, A, t, freeb)),
-                  (joins += far_cell<2, F32>(d, P, A, t, freeb)));
+    DCLUST_BY_DIM(act, dim, far_cell<3>(d, A, comp, heavy), far_cell<2>(d, A, comp, heavy));
   }
-  stat_add(d, C_BAND, t.band);
-  stat_add(d, C_ASYM, t.asym);
-  stat_add(d, C_FAR_TESTS, t.eval);
-  stat_add(d, C_ADJ_FREE, freeb);
-  stat_add(d, C_FAR_JOINS, joins);
 }
 
 // Is some core point of A joined to some core point of B?  The whole
@@ -913,8 +1068,8 @@ __device__ bool wave_joined(const Dev& d, const Par& P, int32_t A, int32_t B, Ta
     double ax[D];
 #pragma unroll
     for (int k = 0; k < D; ++k) {
-      ag[k] = d.G[k][p];
-      ax[k] = F32 ? 0.0 : d.X[k][p];
+      ag[k] = d.G[3 * (int64_t)p + k];
+      ax[k] = F32 ? 0.0 : d.X[3 * (int64_t)p + k];
     }
     // (coordinates of one cell's points do not wrap against each other)
 #pragma unroll
@@ -928,8 +1083,8 @@ __device__ bool wave_joined(const Dev& d, const Par& P, int32_t A, int32_t B, Ta
       double bx[D];
 #pragma unroll
       for (int k = 0; k < D; ++k) {
-        bg[k] = d.G[k][q];
-        bx[k] = F32 ? 0.0 : d.X[k][q];
+        bg[k] = d.G[3 * (int64_t)q + k];
+        bx[k] = F32 ? 0.0 : d.X[3 * (int64_t)q + k];
       }
       const bool bv = bc + lane < b1 && d.core[q] && !(d2box<D>(bg, alo, ahi) > P.d2_out);
       if (!ballot(bv)) continue;
@@ -961,33 +1116,104 @@ __device__ bool wave_joined(const Dev& d, const Par& P, int32_t A, int32_t B, Ta
   return false;
 }
 
-// The listed pairs with a heavy cell, one wavefront each; a pair whose
-// components have been united meanwhile is skipped.
-template <bool F32>
-__global__ __launch_bounds__(256) void k_far_pairs(Dev d) {
-  if (abandoned(d)) return;
-  __shared__ long long s_pre[kStripes + 1];
+// Prefix of a pair list's sub-list lengths (as stored) in LDS.
+__device__ __forceinline__ long long pairs_prefix(const PairList& L, long long* s_pre) {
   if (threadIdx.x < kStripes) {
-    const long long v = (long long)d.far_pairs.cnt[threadIdx.x * kStatStride];
-    const long long incl = wave_incl_scan(v < d.far_pairs.cap ? v : (long long)d.far_pairs.cap);
+    const long long v = (long long)L.cnt[threadIdx.x * kStatStride];
+    const long long incl = wave_incl_scan(v < L.cap ? v : (long long)L.cap);
     s_pre[threadIdx.x + 1] = incl;
     if (threadIdx.x == 0) s_pre[0] = 0;
   }
   __syncthreads();
-  const long long n = s_pre[kStripes];
-  Tally t;
-  long long joins = 0;
-  for (long long i = (long long)blockIdx.x * 4 + (threadIdx.x >> 6); i < n;
-       i += (long long)gridDim.x * 4) {
-    int lo = 0, hi = kStripes - 1;  // last sub-list whose range starts at or before i
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (s_pre[mid] <= i) lo = mid; else hi = mid - 1;
+  return s_pre[kStripes];
+}
+// this thread's sub-list took more pairs than it holds
+__device__ __forceinline__ bool pairs_over(const PairList& L) {
+  return threadIdx.x < kStripes &&
+         (long long)L.cnt[threadIdx.x * kStatStride] > (long long)L.cap;
+}
+__device__ __forceinline__ int2 pairs_at(const PairList& L, const long long* s_pre, long long i) {
+  int lo = 0, hi = kStripes - 1;  // last sub-list whose range starts at or before i
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (s_pre[mid] <= i) lo = mid; else hi = mid - 1;
+  }
+  return L.data[(int64_t)lo * L.cap + (i - s_pre[lo])];
+}
+
+// Offset of cell B from cell A of its stencil along axis k (the cells'
+// coordinates modulo 8 are the top bits of their points').
+__device__ __forceinline__ int cell_offset(const uint4& a, const uint4& b, int k) {
+  const uint32_t x = k == 0 ? a.x : (k == 1 ? a.y : a.z);
+  const uint32_t y = k == 0 ? b.x : (k == 1 ? b.y : b.z);
+  return (int32_t)(((y >> kFixBits) - (x >> kFixBits)) << kFixBits) >> kFixBits;
+}
+
+// One pair, one lane: decided exactly unless its components have been united
+// meanwhile; joined, they are united (lock-free union-find).
+template <bool F32>
+__device__ __forceinline__ void far_light(const Dev& d, int32_t A, int32_t B, Tally& t,
+                                          long long& freeb, long long& joins) {
+  const Inst& I = *inst_of_cell(d, A);
+  const int32_t qs = d.cell_start[A], qe = d.cell_start[A + 1];
+  const int32_t b0 = d.cell_start[B], b1 = d.cell_start[B + 1];
+  const bool allc = d.cell_ncore[A] == qe - qs;
+  const uint4 ra4 = d.rep[A], rb4 = d.rep[B];
+  const int32_t ra = uf_find_cached(d.parent, d.cell_comp[A]);
+  const int32_t rb = uf_find_cached(d.parent, d.cell_comp[B]);
+  if (ra == rb) return;
+  const Par P(I);
+  const int o0 = cell_offset(ra4, rb4, 0), o1 = cell_offset(ra4, rb4, 1);
+  const bool j =
+      I.dim == 3 ? cells_joined<3, F32>(d, P, qs, qe, allc, b0, b1, o0, o1,
+                                        cell_offset(ra4, rb4, 2), t, freeb)
+                 : cells_joined<2, F32>(d, P, qs, qe, allc, b0, b1, o0, 0, o1, t, freeb);
+  if (j) {
+    uf_union(d.parent, ra, rb);
+    ++joins;
+  }
+}
+
+// Every pair of core cell A's, decided by one lane (when a list of pairs was
+// too short).
+template <int D, bool F32>
+__device__ void far_cell_all(const Dev& d, const Par& P, int32_t A, Tally& t, long long& freeb,
+                             long long& joins) {
+  const int local = (int)(d.cell_zl[A] & (Win<D>::nl - 1));
+  for (int r = Win<D>::own; r < Win<D>::rows; ++r) {
+    const uint2 row = rows_of(d, A)[r];
+    uint32_t todo = row.y & (D == 3 ? row_valid<3>(r / 3 - 1, r % 3 - 1, local)
+                                    : row_valid<2>(r - 1, 0, local));
+    while (todo) {
+      const int32_t B = slot_cell(row, __ffs(todo) - 1);
+      todo &= todo - 1;
+      if (B > A && d.cell_comp[B] >= 0 && d.cell_comp[B] != d.cell_comp[A])
+        far_light<F32>(d, A, B, t, freeb, joins);
     }
-    const int2 pr = d.far_pairs.data[(int64_t)lo * d.far_pairs.cap + (i - s_pre[lo])];
+  }
+}
+
+// The listed pairs: light ones one lane each, those with a heavy cell one
+// wavefront each (wave-uniform: every lane walks the same path, lane 0's
+// roots are taken).
+template <bool F32>
+__global__ __launch_bounds__(256, 4) void k_far_pairs(Dev d) {
+  if (abandoned(d)) return;
+  __shared__ long long s_pre[kStripes + 1];
+  Tally t;
+  long long freeb = 0, joins = 0;
+  const long long nl = pairs_prefix(d.far_light, s_pre);
+  for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < nl;
+       i += (long long)gridDim.x * 256) {
+    const int2 pr = pairs_at(d.far_light, s_pre, i);
+    far_light<F32>(d, pr.x, pr.y, t, freeb, joins);
+  }
+  __syncthreads();  // the prefix is rewritten
+  const long long nh = pairs_prefix(d.far_heavy, s_pre);
+  for (long long i = (long long)blockIdx.x * 4 + (threadIdx.x >> 6); i < nh;
+       i += (long long)gridDim.x * 4) {
+    const int2 pr = pairs_at(d.far_heavy, s_pre, i);
     const int32_t A = rfl_i(pr.x), B = rfl_i(pr.y);
-    // every lane walks the same path: the roots are wave-uniform up to the
-    // moment of each load, so lane 0's are taken
     const int32_t ra = rfl_i(uf_find_cached(d.parent, d.cell_comp[A]));
     const int32_t rb = rfl_i(uf_find_cached(d.parent, d.cell_comp[B]));
     if (ra == rb) continue;
@@ -1000,9 +1226,26 @@ __global__ __launch_bounds__(256) void k_far_pairs(Dev d) {
       ++joins;
     }
   }
+  // pairs that found their list full: all pairs again (those decided above
+  // are skipped or decided the same)
+  const bool over = pairs_over(d.far_light) || pairs_over(d.far_heavy);
+  if (__syncthreads_or(over)) {
+    const long long nc = slist_prefix(d.core_cells, s_pre);
+    for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < nc;
+         i += (long long)gridDim.x * 256) {
+      const int32_t A = slist_at(d.core_cells, s_pre, i);
+      const Inst& I = *inst_of_cell(d, A);
+      const Par P(I);
+      if (I.dim == 3)
+        far_cell_all<3, F32>(d, P, A, t, freeb, joins);
+      else
+        far_cell_all<2, F32>(d, P, A, t, freeb, joins);
+    }
+  }
   stat_add(d, C_BAND, t.band);
   stat_add(d, C_ASYM, t.asym);
   stat_add(d, C_FAR_TESTS, t.eval);
+  stat_add(d, C_ADJ_FREE, freeb);
   stat_add(d, C_FAR_JOINS, joins);
 }
 
@@ -1054,10 +1297,11 @@ constexpr int kSeen = 256;   // per-wave table of recently recorded collision pa
 
 // The cells one wave popped in a round (one per lane).
 struct PopStage {
-  unsigned long long mask[64];  // near adjacency bits
-  int32_t rows[9][64];          // near lines
-  int32_t own[64];              // chain
-  int32_t pre[64];              // exclusive prefix of the mask bit counts
+  uint2 rows[kMaxRows][64];  // windows
+  uint32_t mask[64];         // near bits
+  int32_t own[64];           // chain
+  int32_t pre[64];           // exclusive prefix of the mask bit counts
+  uint8_t kind[64];          // place in the block (bits 0-1), 2-D (bit 2)
 };
 
 __global__ __launch_bounds__(256) void k_expand(Dev d, int pass, int S, int budget) {
@@ -1170,7 +1414,8 @@ __global__ __launch_bounds__(256) void k_expand(Dev d, int pass, int S, int budg
     pops += P;
     ++rounds;
     int32_t own = 0;
-    unsigned long long m0 = 0;
+    uint32_t m0 = 0u;
+    int dim = 3;
     if (act) {
       // A list filled only by this wave's seeding and pushes holds cells of
       // its current chain alone (a new chain is seeded only into an empty
@@ -1181,8 +1426,9 @@ __global__ __launch_bounds__(256) void k_expand(Dev d, int pass, int S, int budg
                                       __HIP_MEMORY_SCOPE_AGENT)
                   : cur;
       m0 = d.amask[A];
+      dim = inst_of_cell(d, A)->dim;
     }
-    // the popped cells' chains, masks and near lines go to LDS (the lines
+    // the popped cells' chains, masks and windows go to LDS (the windows
     // loaded together with the label and mask), and their adjacency bits are
     // dealt out evenly: item t of the round is bit k of the mask of lane
     // src, where src is the last lane whose bit prefix is at most t; a round
@@ -1191,13 +1437,15 @@ __global__ __launch_bounds__(256) void k_expand(Dev d, int pass, int S, int budg
     {
       // all nine loads in flight before the first LDS write
       const RowsOf rows = rows_of(d, A);
-      int32_t rv[9];
+      uint2 rv[kMaxRows];
 #pragma unroll
-      for (int r = 0; r < 9; ++r) rv[r] = act ? rows[r] : 0;
+      for (int r = 0; r < kMaxRows; ++r)
+        rv[r] = act && (dim == 3 || r < 3) ? rows[r] : make_uint2(0u, 0u);
+      pst.kind[lane] = (uint8_t)(local_of(d, A, dim) | (dim == 3 ? 0 : 4));
 #pragma unroll
-      for (int r = 0; r < 9; ++r) pst.rows[r][lane] = rv[r];
+      for (int r = 0; r < kMaxRows; ++r) pst.rows[r][lane] = rv[r];
     }
-    const int nb = __popcll(m0);
+    const int nb = __popc(m0);
     edges += nb;
     const int incl = wave_incl_scan(nb);
     const int total = rfl_i(__shfl(incl, 63, 64));
@@ -1226,19 +1474,26 @@ __global__ __launch_bounds__(256) void k_expand(Dev d, int pass, int S, int budg
           if (pst.pre[src + st] <= t) src += st;
         // bit k of the source mask: its k-th set bit
         int k = t - pst.pre[src];
-        unsigned long long m = pst.mask[src];
+        uint32_t m = pst.mask[src];
         int b = 0;
 #pragma unroll
-        for (int w = 32; w >= 1; w >>= 1) {
-          const int c = __popcll(m & ((1ull << w) - 1ull));
+        for (int w = 16; w >= 1; w >>= 1) {
+          const int c = __popc(m & ((1u << w) - 1u));
           if (k >= c) {
             k -= c;
             m >>= w;
             b += w;
           }
         }
-        const int r = (b * 205) >> 10;  // b / 5 for 0 <= b < 128
-        tg[j] = v[j] ? (pst.rows[r < 9 ? r : 0][src] & kRowCellMask) + (b - 5 * r) : 0;
+        if (v[j]) {
+          const int kind = pst.kind[src];
+          int row, slot;
+          if (kind < 4)
+            near_slot<3>(b, kind, row, slot);
+          else
+            near_slot<2>(b, kind & 3, row, slot);
+          tg[j] = slot_cell(pst.rows[row][src], slot);
+        }
         ow[j] = pst.own[src];
       }
       // a plain load can only be stale as kUnclaimed (a label is written
@@ -1548,60 +1803,104 @@ __device__ __forceinline__ bool pred_to(const Dev& d, const Par& P, int32_t q, i
   return box_64<D>(qx, px, P.eps) && d2_64<D>(qx, px) <= P.eps2;
 }
 
-// Smallest component key over the core points q with P(q -> p): the own
-// cell (a clique), then the recorded neighbours, or the whole stencil when
-// the record overflowed or is absent.
+// Component key of a core cell.
+__device__ __forceinline__ int32_t comp_key(const Dev& d, int32_t comp) {
+  return d.compmin[d.parent[comp]];
+}
+
+// The smallest component key below `best` over the core points q of p's rows
+// with P(q -> p): a cell without core points, or with a key that is no
+// smaller, is passed over as a whole.
 template <int D, bool F32>
-__device__ int32_t border_lane(const Dev& d, const Par& P, int32_t p, int32_t c, int32_t qs,
-                               int32_t qe, int R, Tally& t, long long& ovf) {
-  constexpr int NR = D == 3 ? 25 : 5;
-  int32_t best = kNoKey;
-  for (int32_t q = qs; q < qe; ++q)
-    if (d.core[q]) {
-      const int32_t k = d.keyv[q];
-      best = k < best ? k : best;
+__device__ int32_t border_scan(const Dev& d, const Par& P, int32_t p, int32_t c, int32_t best,
+                               const uint32_t* pg, const double* px, Tally& t) {
+  constexpr int NR = Win<D>::rows;
+  const RowsOf rows = rows_of(d, c);
+  // rows with a core cell among their first four cells, or with more cells:
+  // the loads of all rows in flight together
+  uint32_t todo = 0u;
+  {
+    uint2 row[NR];
+    int32_t k[NR][4];
+#pragma unroll
+    for (int r = 0; r < NR; ++r) row[r] = rows[r];
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      const int n = row_cells(row[r]);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) k[r][u] = -1;
+      if (n) {
+        const int32_t* cp = d.cell_comp + (int64_t)row[r].x;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) k[r][u] = cp[u];
+      }
     }
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      const int n = row_cells(row[r]);
+      bool any = n > 4;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) any |= u < n && k[r][u] >= 0;
+      todo |= any ? 1u << r : 0u;
+    }
+  }
+  while (todo) {
+    const int r = __ffs(todo) - 1;
+    todo &= todo - 1;
+    const uint2 row = rows[r];
+    const int n = row_cells(row);
+    for (int i = 0; i < n; ++i) {
+      const int32_t B = (int32_t)row.x + i;
+      const int32_t comp = d.cell_comp[B];
+      if (comp < 0 || B == c) continue;
+      const int32_t key = comp_key(d, comp);
+      if (key >= best) continue;
+      const int32_t b1 = d.cell_start[B + 1];
+      for (int32_t q = d.cell_start[B]; q < b1; ++q)
+        if (d.core[q] && pred_to<D, F32>(d, P, q, p, pg, px, t)) {
+          best = key;
+          break;
+        }
+    }
+  }
+  return best;
+}
+
+// Smallest component key over the core points q with P(q -> p): the own
+// cell (a clique), then the recorded neighbours, or the rows' core cells
+// when there are no records.
+template <int D, bool F32>
+__device__ int32_t border_lane(const Dev& d, const Par& P, int32_t p, int32_t c, Tally& t,
+                               long long& ovf) {
+  const int32_t comp = d.cell_comp[c];
+  const int n = (int)d.rec_n[p];
+  int32_t best = comp >= 0 ? comp_key(d, comp) : kNoKey;
   uint32_t pg[D];
   double px[D];
   if (F32)
     load_g<D>(d, p, pg);
   else
     load_x<D, F32>(d, p, px);
-  const int n = R > 0 ? (int)d.rec_n[p] : 256;
-  if (n <= R) {
-    const int32_t* rec = d.rec + (int64_t)p * R;
-    // four records at a time: their indices, then their core flags and
-    // keys, each level of loads issued together
-    for (int j0 = 0; j0 < n; j0 += 4) {
-      int32_t q[4], k[4];
-      bool cq[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) q[u] = j0 + u < n ? rec[j0 + u] : p;
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        cq[u] = j0 + u < n && d.core[q[u]];
-        k[u] = d.keyv[q[u]];
-      }
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-        if (cq[u] && k[u] < best && pred_to<D, F32>(d, P, q[u], p, pg, px, t)) best = k[u];
-    }
-    return best;
+  if (n >= kRecFew) {
+    ovf += n == kRecNone;
+    return border_scan<D, F32>(d, P, p, c, best, pg, px, t);
   }
-  if (R > 0) ++ovf;
-  const RowsOf rows = rows_of(d, c);
-  for (int g = 0; g < NR; g += 5) {
-    int32_t aa[5], ll[5];
-    line_group(d, rows, g, aa, ll);
-    Stream5 s;
-    s.set(aa, ll);
-    for (int32_t i = 0; i < s.tot; ++i) {
-      int jr;
-      const int32_t q = s.at(i, jr);
-      if ((q >= qs && q < qe) || !d.core[q]) continue;
-      const int32_t k = d.keyv[q];
-      if (k < best && pred_to<D, F32>(d, P, q, p, pg, px, t)) best = k;
+  // four records at a time: their indices, then their core flags and keys,
+  // each level of loads issued together
+  const int32_t* rec = d.rec + p;
+  for (int j0 = 0; j0 < n; j0 += 4) {
+    int32_t q[4], k[4];
+    bool cq[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) q[u] = j0 + u < n ? rec[(int64_t)(j0 + u) * d.n] : p;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      cq[u] = j0 + u < n && d.core[q[u]];
+      k[u] = d.keyv[q[u]];
     }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (cq[u] && k[u] < best && pred_to<D, F32>(d, P, q[u], p, pg, px, t)) best = k[u];
   }
   return best;
 }
@@ -1612,27 +1911,27 @@ template <bool F32>
 __global__ __launch_bounds__(256) void k_border(Dev d) {
   if (abandoned(d)) return;
   __shared__ long long s_pre[kStripes + 1];
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const bool act = i < slist_prefix(d.border_pts, s_pre);
-  const int32_t p = act ? slist_at(d.border_pts, s_pre, i) : 0;
-  int32_t c = 0, qs = 0, qe = 0;
-  int dim = 0;
-  const Inst* I = d.inst;
-  if (act) {
-    c = d.cell_of[p];
-    qs = d.cell_start[c];
-    qe = d.cell_start[c + 1];
-    I = inst_of_cell(d, c);
-    dim = I->dim;
-  }
+  const long long n = slist_prefix(d.border_pts, s_pre);
   Tally t;
   long long ovf = 0;
-  int32_t best = kNoKey;
-  const int R = d.rec_stride;
-  const Par P(*I);
-  DCLUST_BY_DIM(act, dim, (best = border_lane<3, F32>(d, P, p, c, qs, qe, R, t, ovf)),
-                (best = border_lane<2, F32>(d, P, p, c, qs, qe, R, t, ovf)));
-  if (act) d.keyv[p] = best;
+  for (long long i0 = (long long)blockIdx.x * 256; i0 < n; i0 += (long long)gridDim.x * 256) {
+    const long long i = i0 + threadIdx.x;
+    const bool act = i < n;
+    const int32_t p = act ? slist_at(d.border_pts, s_pre, i) : 0;
+    int32_t c = 0;
+    int dim = 0;
+    const Inst* I = d.inst;
+    if (act) {
+      c = d.cell_of[p];
+      I = inst_of_cell(d, c);
+      dim = I->dim;
+    }
+    int32_t best = kNoKey;
+    const Par P(*I);
+    DCLUST_BY_DIM(act, dim, (best = border_lane<3, F32>(d, P, p, c, t, ovf)),
+                  (best = border_lane<2, F32>(d, P, p, c, t, ovf)));
+    if (act) d.keyv[p] = best;
+  }
   stat_add(d, C_BAND, t.band);
   stat_add(d, C_FLIP, t.flip);
   stat_add(d, C_RECOVF, ovf);
@@ -1732,8 +2031,7 @@ __global__ __launch_bounds__(256) void k_output(Dev d) {
 }
 
 // Per-run state of the clustering phases, one launch after the index:
-// component-minimum flags and per-cell core counts (over the n entries that
-// bound the input indices and cells), and per expansion wave (`waves` is 0
+// component-minimum flags (by input index), and per expansion wave (`waves` is 0
 // without seed lists) its pair count and the start of its seeding segment of
 // the cells.  k_rep starts the per-cell state.
 __global__ void k_init_run(Dev d, int64_t waves) {
@@ -1741,10 +2039,7 @@ __global__ void k_init_run(Dev d, int64_t waves) {
   const int64_t C = d.ctl[C_NCELL];
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < m;
        i += (int64_t)gridDim.x * blockDim.x) {
-    if (i < d.n) {
-      d.flag[i] = 0;
-      d.cell_ncore[i] = 0;
-    }
+    if (i < d.n) d.flag[i] = 0;
     if (i < waves) {
       d.pair_cnt[i] = 0;
       d.seg_pos[i] = C * i / waves;
@@ -1774,15 +2069,22 @@ int64_t list_append_cap(int64_t n) {
 }
 int64_t cell_blocks(int64_t n) { return (n + 1023) / 1024 > 0 ? (n + 1023) / 1024 : 1; }
 
-void launch_core(const Dev& d, bool f32, hipStream_t s) {
-  if (f32)
-    hipLaunchKernelGGL(k_core<true>, dim3(point_grid(d.n)), dim3(256), 0, s, d);
-  else
-    hipLaunchKernelGGL(k_core<false>, dim3(point_grid(d.n)), dim3(256), 0, s, d);
-}
-
 // one lane per listed core cell, grid-stride
 static int list_grid(int64_t n) { return std::min(kListGrid, point_grid(n)); }
+
+void launch_core(const Dev& d, bool f32, hipStream_t s) {
+  const size_t lds = core_lds(d.rec_stride);
+  const int gl = list_grid(d.n);
+  if (f32) {
+    hipLaunchKernelGGL(k_core<true>, dim3(point_grid(d.n)), dim3(256), 0, s, d);
+    hipLaunchKernelGGL(k_core_rest<true>, dim3(gl), dim3(256), lds, s, d);
+    hipLaunchKernelGGL(k_core_crowd<true>, dim3(gl), dim3(256), 0, s, d);
+  } else {
+    hipLaunchKernelGGL(k_core<false>, dim3(point_grid(d.n)), dim3(256), 0, s, d);
+    hipLaunchKernelGGL(k_core_rest<false>, dim3(gl), dim3(256), lds, s, d);
+    hipLaunchKernelGGL(k_core_crowd<false>, dim3(gl), dim3(256), 0, s, d);
+  }
+}
 
 void launch_near(const Dev& d, hipStream_t s) {
   hipLaunchKernelGGL(k_rep, dim3((unsigned)cell_blocks(d.n)), dim3(1024), 0, s, d);
@@ -1829,13 +2131,11 @@ void launch_merge(const Dev& d, int grid, hipStream_t s) {
 }
 
 void launch_far(const Dev& d, bool f32, int grid, hipStream_t s) {
-  if (f32) {
-    hipLaunchKernelGGL(k_far<true>, dim3(list_grid(d.n)), dim3(256), 0, s, d);
+  hipLaunchKernelGGL(k_far, dim3(list_grid(d.n)), dim3(256), 0, s, d);
+  if (f32)
     hipLaunchKernelGGL(k_far_pairs<true>, dim3(grid), dim3(256), 0, s, d);
-  } else {
-    hipLaunchKernelGGL(k_far<false>, dim3(list_grid(d.n)), dim3(256), 0, s, d);
+  else
     hipLaunchKernelGGL(k_far_pairs<false>, dim3(grid), dim3(256), 0, s, d);
-  }
   const int g = std::min(grid, list_grid(d.n));
   hipLaunchKernelGGL(k_flatten_all, dim3(g), dim3(256), 0, s, d);
   hipLaunchKernelGGL(k_roots_final, dim3(g), dim3(256), 0, s, d);
@@ -1847,9 +2147,9 @@ void launch_border(const Dev& d, bool f32, hipStream_t s) {
   if (g2 < 1) g2 = 1;
   hipLaunchKernelGGL(k_keys, dim3(g2), dim3(256), 0, s, d);
   if (f32)
-    hipLaunchKernelGGL(k_border<true>, dim3(point_grid(d.n)), dim3(256), 0, s, d);
+    hipLaunchKernelGGL(k_border<true>, dim3(list_grid(d.n)), dim3(256), 0, s, d);
   else
-    hipLaunchKernelGGL(k_border<false>, dim3(point_grid(d.n)), dim3(256), 0, s, d);
+    hipLaunchKernelGGL(k_border<false>, dim3(list_grid(d.n)), dim3(256), 0, s, d);
 }
 
 // core flags to input order (on request, after a run)

@@ -13,9 +13,9 @@
 //                 ranges (INDEXING_ADJUSTMENT's per-leaf equal_range,
 //                 indexing.cu:23-51)
 //   k_gather      cell-sorted SoA coordinates (FP64 + fixed-point)
-//   k_rows        the 5^(D-1) stencil lines of each cell (cells of side
-//                 eps/2, a 5^D stencil) as runs of point ranges
-//                 (searchPoints' level-by-level descent, dbscan.cu:390-474)
+//   k_rows        the windows of each cell's 3^(D-1) neighbour columns that
+//                 cover its stencil (cells of side eps/2, a 5^D stencil;
+//                 searchPoints' level-by-level descent, dbscan.cu:390-474)
 #include "internal.h"
 #include "kernels.h"
 
@@ -196,17 +196,18 @@ __global__ __launch_bounds__(256) void k_bbox(Dev d) {
 // above (plus the box-test slack from coordinate magnitude) requires more,
 // in which case it is widened to twice the bound.
 //
-// Per instance this also sets the line-table base: a line is the set of
-// cells sharing all coordinates but the last; the dense line table (one
-// entry per possible line) locates a neighbour line in O(1).
+// Per instance this also sets the column-table base: the dense column table
+// (one entry per possible column) locates a neighbour column in O(1).
 __global__ void k_grid_setup(Dev d) {
   __shared__ unsigned long long s_scan[1024];
+  __shared__ unsigned long long s_scanc[1024];
   __shared__ long long s_scanl[1024];
-  __shared__ unsigned long long s_carry;
+  __shared__ unsigned long long s_carry, s_carryc;
   __shared__ long long s_carryl;
   __shared__ int s_err;
   if (threadIdx.x == 0) {
     s_carry = 0;
+    s_carryc = 0;
     s_carryl = 0;
     s_err = 0;
   }
@@ -214,6 +215,7 @@ __global__ void k_grid_setup(Dev d) {
   for (int base = 0; base < d.ninst; base += blockDim.x) {
     const int i = base + threadIdx.x;
     unsigned long long cells = 0;  // at most 2^63 (3 axes of at most 2^21 cells)
+    unsigned long long keys = 0;   // at most 2^63 + 2^43
     long long lines = 0;
     if (i < d.ninst) {
       Inst I = d.inst[i];
@@ -270,7 +272,6 @@ __global__ void k_grid_setup(Dev d) {
       I.w = w;
       I.inv_w = 1.0 / w;
       cells = 1;
-      lines = 1;
       for (int k = 0; k < 3; ++k) {
         I.mn[k] = k < dim ? mn[k] : 0.0;
         I.nk[k] = 1;
@@ -278,10 +279,14 @@ __global__ void k_grid_setup(Dev d) {
           double t = floor(cell_t(mx[k], mn[k], I.inv_w));
           I.nk[k] = (int32_t)t + 1;
           cells *= (unsigned long long)I.nk[k];
-          if (k < dim - 1) lines *= (long long)I.nk[k];
         }
       }
+      const long long bx = ((long long)I.nk[0] + 1) / 2, by = ((long long)I.nk[1] + 1) / 2;
+      I.cstride = dim == 3 ? by + 1 : 1;
+      lines = bx * I.cstride;
       I.nlines = lines;
+      I.nzl = (long long)I.nk[dim - 1] << (dim - 1);
+      keys = (unsigned long long)lines * (unsigned long long)I.nzl;
       // FP32 guard band (units of w * 2^-29)
       const double gs = I.inv_w * 0x1p29;
       const double es = I.eps * gs;
@@ -302,26 +307,30 @@ __global__ void k_grid_setup(Dev d) {
       d.inst[i] = I;
       if (I.err) atomicOr(&s_err, 1);
     }
-    s_scan[threadIdx.x] = cells;
+    s_scan[threadIdx.x] = keys;
+    s_scanc[threadIdx.x] = cells;
     s_scanl[threadIdx.x] = lines;
     __syncthreads();
     // inclusive Hillis-Steele scans over the block
     // (the key-space sums saturate: a total beyond 2^63 fails the call below)
     for (int o = 1; o < (int)blockDim.x; o <<= 1) {
       unsigned long long v = threadIdx.x >= (unsigned)o ? s_scan[threadIdx.x - o] : 0;
+      unsigned long long vc = threadIdx.x >= (unsigned)o ? s_scanc[threadIdx.x - o] : 0;
       long long vl = threadIdx.x >= (unsigned)o ? s_scanl[threadIdx.x - o] : 0;
       __syncthreads();
       s_scan[threadIdx.x] = sat_add(s_scan[threadIdx.x], v);
+      s_scanc[threadIdx.x] = sat_add(s_scanc[threadIdx.x], vc);
       s_scanl[threadIdx.x] += vl;
       __syncthreads();
     }
     if (i < d.ninst) {
-      d.inst[i].key_base = (int64_t)(sat_add(s_carry, s_scan[threadIdx.x]) - cells);
+      d.inst[i].key_base = (int64_t)(sat_add(s_carry, s_scan[threadIdx.x]) - keys);
       d.inst[i].line_base = s_carryl + s_scanl[threadIdx.x] - lines;
     }
     __syncthreads();
     if (threadIdx.x == blockDim.x - 1) {
       s_carry = sat_add(s_carry, s_scan[threadIdx.x]);
+      s_carryc = sat_add(s_carryc, s_scanc[threadIdx.x]);
       s_carryl += s_scanl[threadIdx.x];
     }
     __syncthreads();
@@ -330,7 +339,7 @@ __global__ void k_grid_setup(Dev d) {
     const unsigned long long total = s_carry;
     d.ctl[C_ERR] = s_err;
     d.ctl[C_NLINES] = s_carryl;
-    if (total > kMaxKeySpace) {
+    if (s_carryc > kMaxKeySpace || total == ~0ull) {
       // the keys would not fit the sort: the whole call fails (instances of a
       // batch share one key space), and every later kernel returns at once
       d.ctl[C_KEYOVF] = 1;
@@ -379,9 +388,14 @@ __device__ __forceinline__ void cellkey_points(const Dev& d, const Inst& I, cons
     for (int u = 0; u < kChunkU; ++u) {
       const int64_t i = i0 + u * 256;
       if (i < np) {
-        int64_t lin = cell_index(v[u][0], I, 0);
-#pragma unroll
-        for (int k = 1; k < D; ++k) lin = lin * I.nk[k] + cell_index(v[u][k], I, k);
+        const int32_t cx = cell_index(v[u][0], I, 0), cl = cell_index(v[u][D - 1], I, D - 1);
+        int64_t lin;
+        if (D == 3) {
+          const int32_t cy = cell_index(v[u][1], I, 1);
+          lin = ((cx >> 1) * I.cstride + (cy >> 1)) * I.nzl + cl * 4LL + (cx & 1) * 2 + (cy & 1);
+        } else {
+          lin = (cx >> 1) * I.nzl + cl * 2LL + (cx & 1);
+        }
         key_buf<K32>(d, 0)[ch.begin + i] = (SortKey<K32>)(I.key_base + lin);
         d.val[0][ch.begin + i] = (int32_t)(ch.begin + i);
       }
@@ -713,27 +727,18 @@ __device__ __forceinline__ int32_t inst_of_key(const Dev& d, uint64_t key) {
   return lo;
 }
 
-// Integer cell coordinates of a key, decoded once per cell: 21 bits per
-// axis in 3-D (at most 2^21 cells per axis), 32 bits per axis in 2-D.
-__device__ __forceinline__ uint64_t pack_cell(const Inst& I, uint64_t key) {
-  int64_t lin = (int64_t)(key - (uint64_t)I.key_base);
-  uint64_t kc[3] = {0, 0, 0};
-  for (int k = I.dim - 1; k >= 0; --k) {
-    kc[k] = (uint64_t)(lin % I.nk[k]);
-    lin /= I.nk[k];
-  }
-  return I.dim == 3 ? (kc[0] | (kc[1] << 21) | (kc[2] << 42)) : (kc[0] | (kc[1] << 32));
-}
-
-__device__ __forceinline__ void unpack_cell(int dim, uint64_t pc, int32_t* kc) {
-  if (dim == 3) {
-    kc[0] = (int32_t)(pc & 0x1fffff);
-    kc[1] = (int32_t)((pc >> 21) & 0x1fffff);
-    kc[2] = (int32_t)(pc >> 42);
+// Column (within the instance) and place in the column of a key, decoded once
+// per cell.
+__device__ __forceinline__ void split_key(const Inst& I, uint64_t key, int64_t& col,
+                                          uint32_t& zl) {
+  const uint64_t rel = key - (uint64_t)I.key_base, nzl = (uint64_t)I.nzl;
+  if ((rel >> 32) == 0 && (nzl >> 32) == 0) {
+    const uint32_t q = (uint32_t)rel / (uint32_t)nzl;
+    col = q;
+    zl = (uint32_t)rel - q * (uint32_t)nzl;
   } else {
-    kc[0] = (int32_t)(pc & 0xffffffffu);
-    kc[1] = (int32_t)(pc >> 32);
-    kc[2] = 0;
+    col = (int64_t)(rel / nzl);
+    zl = (uint32_t)(rel - (uint64_t)col * nzl);
   }
 }
 
@@ -747,23 +752,24 @@ __global__ __launch_bounds__(CS_T) void k_csr_write(Dev d) {
   const int wv = threadIdx.x >> 6;
   uint64_t kr[CS_I], kp[CS_I];
   load_key_pairs<CS_I>(d, key, t0, kr, kp);
-  // every round's instance and packed cell coordinates, read from the
+  // every round's instance, column and place, from the
   // instance table before the first store (the stores could alias it as far
   // as the compiler knows, which would hold each round's reads behind the
   // previous round's stores)
-  int32_t ir[CS_I], zr[CS_I];
-  uint64_t pcr[CS_I];
+  int32_t ir[CS_I];
+  uint32_t zr[CS_I], cr[CS_I];
 #pragma unroll
   for (int r = 0; r < CS_I; ++r) {
     ir[r] = 0;
     zr[r] = 0;
-    pcr[r] = 0;
+    cr[r] = 0;
     const int64_t i = t0 + r * CS_T + threadIdx.x;
     if (i < d.n && (i == 0 || kr[r] != kp[r])) {
       ir[r] = inst_of_key(d, kr[r]);
       const Inst& I = d.inst[ir[r]];
-      pcr[r] = pack_cell(I, kr[r]);
-      zr[r] = (int32_t)(I.dim == 3 ? pcr[r] >> 42 : pcr[r] >> 32);
+      int64_t col;
+      split_key(I, kr[r], col, zr[r]);
+      cr[r] = (uint32_t)(I.line_base + col);
     }
   }
   if (threadIdx.x == 0) s_run = d.scan_tmp[blockIdx.x];
@@ -783,12 +789,11 @@ __global__ __launch_bounds__(CS_T) void k_csr_write(Dev d) {
     if (inr) {
       d.cell_of[i] = (int32_t)cid;
       if (f) {
-        const uint64_t pc = pcr[r];
         d.cell_start[cid] = (int32_t)i;
         d.cell_key[cid] = k;
         d.cell_inst[cid] = ir[r];
-        d.cell_xyz[cid] = pc;
-        d.cell_z[cid] = zr[r];
+        d.cell_col[cid] = cr[r];
+        d.cell_zl[cid] = zr[r];
       }
       if (i == d.n - 1) {
         d.cell_start[cid + 1] = (int32_t)d.n;
@@ -816,13 +821,13 @@ __device__ __forceinline__ void gather_point(const Dev& d, const Inst& I, int64_
     mn[k] = I.mn[k];
   }
   const double inv_w = I.inv_w;
-  if (!d.X[0]) d.xoff[i] = off;  // the FP32 form's way back to FP64 rows
+  if (!d.X) d.xoff[i] = off;  // the FP32 form's way back to FP64 rows
 #pragma unroll
   for (int k = 0; k < D; ++k) {
-    if (d.X[0]) d.X[k][i] = x[k];  // the FP64 form's sorted copy
+    if (d.X) d.X[3 * i + k] = x[k];  // the FP64 form's sorted copy
     const double t = cell_t(x[k], mn[k], inv_w);  // same rounding as the key
     const double f = floor(t * 0x1p29);           // exact scaling by 2^29
-    d.G[k][i] = (uint32_t)(unsigned long long)(long long)f;  // wraps mod 8 cells
+    d.G[3 * i + k] = (uint32_t)(unsigned long long)(long long)f;  // wraps mod 8 cells
   }
   d.orig[i] = src;
 }
@@ -842,16 +847,8 @@ __global__ __launch_bounds__(256) void k_gather(Dev d) {
 }
 
 // ------------------------------------------------------------------ rows --
-// line of a cell: all coordinates but the last; global line-table index
-__device__ __forceinline__ int64_t cell_line(const Dev& d, int32_t c) {
-  const Inst& I = *inst_of_cell(d, c);
-  int32_t kc[3];
-  unpack_cell(I.dim, d.cell_xyz[c], kc);
-  return I.line_base + (I.dim == 3 ? (int64_t)kc[0] * I.nk[1] + kc[1] : (int64_t)kc[0]);
-}
-
-// Line table: for every possible line, the range of its non-empty cells in
-// the sorted cell array (-1 when empty).
+// Column table: for every possible column, the range of its non-empty cells
+// in the sorted cell array (-1 when empty).
 __global__ __launch_bounds__(256) void k_line_clear(Dev d) {
   if (abandoned(d)) return;
   const long long P = d.ctl[C_NLINES];
@@ -867,30 +864,32 @@ __global__ __launch_bounds__(256) void k_line_mark(Dev d) {
   if (d.ctl[C_NLINES] > d.line_cap) return;
   for (int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; c < C;
        c += (int64_t)gridDim.x * blockDim.x) {
-    // the three lines are read before either store (which could alias the
+    // the three columns are read before either store (which could alias the
     // cell arrays as far as the compiler knows)
-    const int64_t L = cell_line(d, (int32_t)c);
-    const int64_t Lp = c > 0 ? cell_line(d, (int32_t)c - 1) : -1;
-    const int64_t Ln = c < C - 1 ? cell_line(d, (int32_t)c + 1) : -1;
-    if (Lp != L) d.lines[L].x = (int32_t)c;
-    if (Ln != L) d.lines[L].y = (int32_t)c + 1;
+    const uint32_t L = d.cell_col[c];
+    const bool first = c == 0 || d.cell_col[c > 0 ? c - 1 : 0] != L;
+    const bool last = c == C - 1 || d.cell_col[c < C - 1 ? c + 1 : c] != L;
+    if (first) d.lines[L].x = (int32_t)c;
+    if (last) d.lines[L].y = (int32_t)c + 1;
   }
 }
 
-// Five lower bounds lo[j] = first index in [lo[j], hi[j]) with a[i] >= v[j],
-// in lockstep (the loads of the five searches overlap).
-__device__ __forceinline__ void lower_bound5(const uint64_t* a, int32_t (&lo)[5],
-                                             int32_t (&hi)[5], const uint64_t (&v)[5]) {
+// Three lower bounds lo[j] = first index in [lo[j], hi[j]) with a[i] >= v[j],
+// in lockstep (the loads of the three searches overlap).
+template <typename T>
+__device__ __forceinline__ void lower_bound3(const T* a, int32_t (&lo)[3], int32_t (&hi)[3],
+                                             const T (&v)[3]) {
   for (;;) {
-    uint64_t km[5];
+    T km[3];
     bool any = false;
 #pragma unroll
-    for (int j = 0; j < 5; ++j) {
-      km[j] = lo[j] < hi[j] ? a[(lo[j] + hi[j]) >> 1] : 0;
+    for (int j = 0; j < 3; ++j) {
+      km[j] = lo[j] < hi[j] ? a[(lo[j] + hi[j]) >> 1] : (T)0;
       any |= lo[j] < hi[j];
     }
     if (!any) return;
-    for (int j = 0; j < 5; ++j)
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
       if (lo[j] < hi[j]) {
         const int32_t mid = (lo[j] + hi[j]) >> 1;
         if (km[j] < v[j])
@@ -901,102 +900,30 @@ __device__ __forceinline__ void lower_bound5(const uint64_t* a, int32_t (&lo)[5]
   }
 }
 
-// Per-lane view of one cell and one line group: the cell's coordinates,
-// its window [zlo, zhi] along the last axis, its own line (global
-// line-table index), the shift to the neighbour lines of the group, and
-// which of the five neighbour lines exist.  3-D: the lines with offset
-// g - 2 along axis 0 and -2..2 along axis 1 (consecutive line-table
-// entries); 2-D: the five lines (g = 0).
-struct RowLane {
-  const Inst* I;
-  int32_t iid;
-  int dim;
-  int32_t zlo, zhi;
-  int64_t own, shift;
-  bool ok[5];
-};
-
-__device__ __forceinline__ void row_lane(const Dev& d, int32_t c, bool act, int g, int32_t C,
-                                         RowLane& L) {
-  const int32_t cc = act ? c : C - 1;
-  L.iid = d.ninst == 1 ? 0 : d.cell_inst[cc];
-  L.I = d.inst + L.iid;
-  const Inst& I = *L.I;
-  const int dim = I.dim;
-  L.dim = dim;
-  const int last = dim - 1;
-  int32_t kc[3];
-  unpack_cell(dim, d.cell_xyz[cc], kc);
-  L.zlo = kc[last] >= 2 ? kc[last] - 2 : 0;
-  L.zhi = kc[last] + 2 < I.nk[last] ? kc[last] + 2 : I.nk[last] - 1;
-  const int a = dim == 3 ? g - 2 : 0;
-  L.own = I.line_base + (dim == 3 ? (int64_t)kc[0] * I.nk[1] + kc[1] : (int64_t)kc[0]);
-  L.shift = dim == 3 ? (int64_t)a * I.nk[1] : 0;
-#pragma unroll
-  for (int j = 0; j < 5; ++j) {
-    int o0 = a, o1 = j - 2;
-    if (dim != 3) {
-      o0 = kRowOff2[j];
-      o1 = 0;
-    }
-    const int32_t r0 = kc[0] + o0, r1 = kc[1] + o1;
-    bool ok = act && (dim == 3 || g == 0) && r0 >= 0 && r0 < I.nk[0];
-    if (dim == 3) ok = ok && r1 >= 0 && r1 < I.nk[1];
-    L.ok[j] = ok;
-  }
-}
-
-__device__ __forceinline__ int row_off(int dim, int j) { return dim == 3 ? j - 2 : kRowOff2[j]; }
-
-__device__ __forceinline__ void write_rows(const Dev& d, int32_t c, bool act, int dim, int g,
-                                           const int32_t* packed, long long& cand,
-                                           long long& nbrc) {
-  if (d.nbr_stats) {
-#pragma unroll
-    for (int j = 0; j < 5; ++j)
-      if (packed[j]) {
-        const int32_t a = packed[j] & kRowCellMask, b = a + (packed[j] >> kRowCntShift);
-        nbrc += b - a;
-        cand += (long long)(d.cell_start[c + 1] - d.cell_start[c]) *
-                (d.cell_start[b] - d.cell_start[a]);
-      }
-  }
-  if (act) {
-    // the five row indices are read before the first store
-    int r[5];
-#pragma unroll
-    for (int j = 0; j < 5; ++j) {
-      // (2-D: groups g > 0 write the unused rows 5g .. 5g+4, empty)
-      r[j] = dim == 3 ? kRowOfOff3[g][j] : 5 * g + j;
-    }
-#pragma unroll
-    for (int j = 0; j < 5; ++j) d.rows[(int64_t)r[j] * d.rstride + c] = packed[j];
-  }
-}
-
-// For each (cell, stencil line): the run of non-empty cells of that line
-// whose last coordinate is within +-2 of the cell's, packed as
-// first | count << 28 (count <= 5).  One wavefront per (tile of 64
-// consecutive cells, line group g).  The tile's cells lie in a few
-// consecutive lines (cells are sorted, so the first and last lanes bound
-// them), and so do their neighbour lines: the line table gives the range
-// of cells those lines hold, and the wave copies the cells' sort keys,
-// relative to the span's first line (below 2^29), into LDS with coalesced
-// loads, padded with ~0 to a larger power of two.  A window is then two
-// searches in that sorted array: the first key >= the key of (line, zlo),
-// by a branchless binary search of a depth uniform over the wave, and the
-// last key <= the key of (line, zhi), at most five further.  A tile whose
-// cells do not fit the LDS slots (one that crosses an axis-0 boundary,
-// long or sparse lines, two instances of a batch, no line table, 2-D) is
-// listed for k_rows_global.
-constexpr int RW_LINES = 512;  // line-table entries of a tile's span (at most)
+// Rows of the cells.  One wavefront per (tile of 64 consecutive cells, group
+// g): 3-D group g holds the three columns with block offset g - 1 along axis
+// 0 (consecutive columns); 2-D has one group (g = 0), its three columns
+// being consecutive too.  The tile's cells lie in a few consecutive columns
+// (cells are sorted, so the first and last lanes bound them), and so do
+// their neighbour columns: the column table gives the range of cells those
+// hold, and the wave copies the cells' sort keys, relative to the span's
+// first column, into LDS with coalesced loads, padded with ~0 to a larger
+// power of two and four slots more.  A window then starts at the first key >=
+// its own first key, found by a branchless binary search of a depth uniform
+// over the wave, and its slot bits come from the keys that follow (four per
+// step).  4 M 3-D points: 205 + 57 us with k_rows_global, where 25 lines per
+// cell took 274 + 28 (and 320 MB of rows instead of 240).  A tile whose cells do not fit the LDS slots (one that crosses an
+// axis-0 boundary, long or sparse columns, two instances of a batch, no
+// column table) is listed for k_rows_global.
+constexpr int RW_LINES = 512;  // column-table entries of a tile's span (at most)
 constexpr int RW_CELLS = 512;  // cell keys staged per wavefront (a power of two)
+constexpr int RW_SLOTS = RW_CELLS + 4;
 
-// Rows of one (tile, line group) from LDS; false when the tile does not fit
-// (then nothing is written).  3-D tiles of one instance only, so the
-// instance's fields are wave-uniform (scalar loads).
+// Rows of one (tile, group) from LDS; false when the tile does not fit (then
+// nothing is written).  Tiles of one instance only, so the instance's fields
+// are wave-uniform (scalar loads).
 __device__ __forceinline__ bool rows_staged(const Dev& d, int64_t tile, int g, int32_t C,
-                                            int64_t NL, uint32_t* ck) {
+                                            uint32_t* ck, int32_t* cs) {
   const int lane = lane_id();
   const int32_t c = (int32_t)(tile * 64 + lane);
   const bool act = c < C;
@@ -1009,145 +936,209 @@ __device__ __forceinline__ bool rows_staged(const Dev& d, int64_t tile, int g, i
     if (iid != rl_i(v, nact - 1)) return false;
   }
   const Inst& I = d.inst[iid];
-  if (I.dim != 3) {
-    // 2-D: groups g > 0 hold no lines (their rows are written empty); the
-    // five lines of g = 0 are long and rarely fit the slots
-    if (g == 0) return false;
-    if (act) {
-#pragma unroll
-      for (int j = 0; j < 5; ++j) d.rows[(int64_t)(5 * g + j) * d.rstride + c] = 0;
-    }
-    return true;
-  }
-  const int32_t nk0 = I.nk[0], nk1 = I.nk[1], nk2 = I.nk[2];
-  const uint64_t pc = d.cell_xyz[cc];
-  const int32_t x = (int32_t)(pc & 0x1fffff), y = (int32_t)((pc >> 21) & 0x1fffff);
-  const int32_t z = (int32_t)(pc >> 42);
-  const int a = g - 2;
-  const bool okx = act & (x + a >= 0) & (x + a < nk0);
-  // (the lines of a tile's first and last lanes bound its lines: cells are
-  // sorted)
-  const int64_t own = (int64_t)x * nk1 + y;  // within the instance
-  const int64_t own0 = rl_l(own, 0), own1 = rl_l(own, nact - 1);
-  const int64_t nl = (int64_t)nk0 * nk1;
-  int64_t lmin = own0 + (int64_t)a * nk1 - 2, lmax = own1 + (int64_t)a * nk1 + 2;
+  const bool d3 = I.dim == 3;
+  if (!d3 && g > 0) return true;  // (2-D rows are those of group 0)
+  const int ls = d3 ? 2 : 1;      // log2 of a column's cells per step
+  const int64_t nzl = I.nzl;
+  const int32_t nz = (int32_t)(nzl >> ls);
+  const int64_t shift = d3 ? (g - 1) * I.cstride : 0;
+  // columns of the tile, and of its neighbours in this group, within the
+  // instance
+  const int64_t own = (int64_t)d.cell_col[cc] - I.line_base;
+  const uint32_t z = d.cell_zl[cc] >> ls;
+  int64_t lmin = rl_l(own, 0) + shift - 1, lmax = rl_l(own, nact - 1) + shift + 1;
   lmin = lmin < 0 ? 0 : lmin;
-  lmax = lmax >= nl ? nl - 1 : lmax;
+  lmax = lmax >= I.nlines ? I.nlines - 1 : lmax;
   if (lmax - lmin >= RW_LINES) return false;
-  const int64_t gl = I.line_base + lmin;  // first line-table entry of the span
-  // the cells of the span: [first start, last end) of its non-empty lines
-  // (the lines are in cell order: the first and last non-empty entries)
   const int span = lmax >= lmin ? (int)(lmax - lmin + 1) : 0;
-  int32_t cmin = -1, cmax = -1;
-  // the entries' loads are all issued before the first is used
-  int2 ev[RW_LINES / 64];
-#pragma unroll
-  for (int k = 0; k < RW_LINES / 64; ++k) {
-    const int i = lane + 64 * k;
-    ev[k] = make_int2(-1, -1);
-    if (i < span && gl + i < NL) ev[k] = d.lines[gl + i];
-  }
-#pragma unroll
-  for (int k = 0; k < RW_LINES / 64; ++k) {
-    if (64 * k < span) {
-      const int2 e = ev[k];
-      const unsigned long long m = ballot(e.x >= 0 && e.y > e.x);
-      if (m) {
-        if (cmin < 0) cmin = rl_i(e.x, __ffsll((long long)m) - 1);
-        cmax = rl_i(e.y, 63 - __clzll((long long)m));
+  // relative keys of the span must fit below the ~0 padding
+  if ((unsigned long long)span * (unsigned long long)nzl >= 0xfffffff0ull) return false;
+  const int64_t gl = I.line_base + lmin;  // first column-table entry of the span
+  // Staged cells: [cb[j], cb[j] + sn[j]) one after the other.  A tile within
+  // one column needs only the steps its cells reach of each of the (at most)
+  // three neighbour columns, found by six lanes' binary searches at once
+  // (long columns would not fit whole).  Any other tile takes the cells of
+  // the whole span: [first start, last end) of its non-empty columns (the
+  // columns are in cell order: the first and last non-empty entries).
+  int32_t cb[3] = {0, 0, 0}, sn[3] = {0, 0, 0};
+  int ncz;
+  const bool one = rl_l(own, 0) == rl_l(own, nact - 1);
+  if (one) {
+    const uint32_t z0 = rl_u(z, 0), z1 = rl_u(z, nact - 1);  // (cells are sorted)
+    const uint32_t lo0 = (z0 >= 2 ? z0 - 2 : 0) << ls;
+    // lane 2j: first cell of column j at or above lo0; lane 2j + 1: first cell
+    // above the last place of step z1 + 2
+    int32_t at = 0, hi = 0;
+    if (lane < 2 * span) {
+      const int2 e = d.lines[gl + (lane >> 1)];
+      if (e.x >= 0) {
+        at = e.x;
+        hi = e.y;
       }
     }
+    const unsigned long long key1 = (((unsigned long long)z1 + 3ull) << ls);
+    while (ballot(at < hi)) {
+      if (at < hi) {
+        const int32_t mid = (at + hi) >> 1;
+        const uint32_t v = d.cell_zl[mid];
+        if ((lane & 1) ? (unsigned long long)v < key1 : v < lo0)
+          at = mid + 1;
+        else
+          hi = mid;
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      cb[j] = rl_i(at, 2 * j);
+      sn[j] = rl_i(at, 2 * j + 1) - cb[j];
+    }
+    ncz = sn[0] + sn[1] + sn[2];
+  } else {
+    int32_t cmin = -1, cmax = -1;
+    // the entries' loads are all issued before the first is used
+    int2 ev[RW_LINES / 64];
+#pragma unroll
+    for (int k = 0; k < RW_LINES / 64; ++k) {
+      const int i = lane + 64 * k;
+      ev[k] = make_int2(-1, -1);
+      if (i < span) ev[k] = d.lines[gl + i];
+    }
+#pragma unroll
+    for (int k = 0; k < RW_LINES / 64; ++k) {
+      if (64 * k < span) {
+        const int2 e = ev[k];
+        const unsigned long long m = ballot(e.x >= 0 && e.y > e.x);
+        if (m) {
+          if (cmin < 0) cmin = rl_i(e.x, __ffsll((long long)m) - 1);
+          cmax = rl_i(e.y, 63 - __clzll((long long)m));
+        }
+      }
+    }
+    cb[0] = cmin < 0 ? 0 : cmin;
+    ncz = sn[0] = cmin >= 0 ? cmax - cmin : 0;
   }
-  const int ncz = cmin >= 0 ? cmax - cmin : 0;
   if (ncz >= RW_CELLS) return false;
-  cmin = cmin < 0 ? 0 : cmin;
+  const int n0 = sn[0], n01 = sn[0] + sn[1];
   // a power of two > ncz: the last slot is always a ~0 sentinel, so the
   // search (which reaches index pad - 2 at most) is exact
   const int pad = 1 << (32 - __clz(ncz));
   // keys relative to kbase fit 32 bits, so the low halves of the keys are
   // enough (little-endian), all loaded before the first is stored
-  const uint32_t kbase = (uint32_t)(I.key_base + lmin * nk2);
+  const uint32_t kbase = (uint32_t)(I.key_base + lmin * nzl);
   const uint32_t* key_lo = reinterpret_cast<const uint32_t*>(d.cell_key);
   uint32_t kv[RW_CELLS / 64];
+  int32_t sv[RW_CELLS / 64];  // and the cells' ends, for the windows' point counts
 #pragma unroll
   for (int k = 0; k < RW_CELLS / 64; ++k) {
     const int i = lane + 64 * k;
     kv[k] = 0u;
-    if (i < ncz) kv[k] = key_lo[2 * (int64_t)(cmin + i)];
+    sv[k] = 0;
+    const int32_t ci = i < n0 ? cb[0] + i : (i < n01 ? cb[1] + (i - n0) : cb[2] + (i - n01));
+    if (i < ncz) {
+      kv[k] = key_lo[2 * (int64_t)ci];
+      sv[k] = d.cell_start[ci + 1];
+    }
   }
 #pragma unroll
   for (int k = 0; k < RW_CELLS / 64; ++k) {
     const int i = lane + 64 * k;
-    if (i < pad) ck[i] = i < ncz ? kv[k] - kbase : 0xffffffffu;
+    if (i < pad) {
+      ck[i] = i < ncz ? kv[k] - kbase : 0xffffffffu;
+      cs[i] = sv[k];
+    }
   }
+  if (lane < 4) ck[pad + lane] = 0xffffffffu;
   wave_sync();
-  // keys of (line of j, zlo), relative to the span's first line
-  const int32_t zlo = z >= 2 ? z - 2 : 0, zhi = z + 2 < nk2 ? z + 2 : nk2 - 1;
-  const uint32_t k0 = (uint32_t)((own + (int64_t)a * nk1 - 2 - lmin) * nk2) + (uint32_t)zlo;
-  uint32_t klo[5];
-  int32_t pos[5];
+  // windows: first key, key past the end, and the key of slot 0 (which may
+  // lie below the column: modulo 2^32); a column outside the instance gets an
+  // empty window
+  const uint32_t zlo = z >= 2 ? z - 2 : 0;
+  const uint32_t zhi = z + 2u < (uint32_t)nz ? z + 2u : (uint32_t)nz - 1u;
+  uint32_t klo[3], kend[3], kwin[3];
+  int32_t pos[3];
 #pragma unroll
-  for (int j = 0; j < 5; ++j) {
-    klo[j] = k0 + (uint32_t)(j * nk2);
+  for (int j = 0; j < 3; ++j) {
+    const int64_t col = own + shift + j - 1 - lmin;
+    const bool ok = act && col >= 0 && col < span;
+    const uint32_t base = (uint32_t)(col * nzl);
+    klo[j] = ok ? base + (zlo << ls) : 0u;
+    kend[j] = ok ? base + ((zhi + 1) << ls) : 0u;
+    kwin[j] = base + (z << ls) - (2u << ls);
     pos[j] = -1;  // last index with key < klo
   }
   for (int h = pad >> 1; h > 0; h >>= 1) {
-    uint32_t v[5];
+    uint32_t v[3];
 #pragma unroll
-    for (int j = 0; j < 5; ++j) v[j] = ck[pos[j] + h];
+    for (int j = 0; j < 3; ++j) v[j] = ck[pos[j] + h];
 #pragma unroll
-    for (int j = 0; j < 5; ++j) pos[j] = v[j] < klo[j] ? pos[j] + h : pos[j];
+    for (int j = 0; j < 3; ++j) pos[j] = v[j] < klo[j] ? pos[j] + h : pos[j];
   }
-  const uint32_t dz = (uint32_t)(zhi - zlo);
-  int rrow[5];  // read before the first store
+  uint32_t m[3] = {0u, 0u, 0u};
+  int32_t q[3];
 #pragma unroll
-  for (int j = 0; j < 5; ++j) rrow[j] = kRowOfOff3[g][j];
+  for (int j = 0; j < 3; ++j) q[j] = pos[j] + 1;
+  for (;;) {
+    // (q stays at or below pad: the keys from ncz on end every window)
+    uint32_t v[3][4];
 #pragma unroll
-  for (int j = 0; j < 5; ++j) {
-    // the run: keys up to (line, zhi), at most five after pos
-    int32_t e = pos[j];
+    for (int j = 0; j < 3; ++j)
 #pragma unroll
-    for (int h = 4; h > 0; h >>= 1) {
-      const int32_t q = e + h;
-      e = (q < pad && ck[q < pad ? q : 0] <= klo[j] + dz) ? q : e;
+      for (int i = 0; i < 4; ++i) v[j][i] = ck[q[j] + i];
+    bool more = false;
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (v[j][i] < kend[j]) m[j] |= 1u << (v[j][i] - kwin[j]);
+      if (v[j][3] < kend[j]) {
+        q[j] += 4;
+        more = true;
+      }
     }
-    const int32_t cnt = e - pos[j];
-    const bool ok = okx & (y + j - 2 >= 0) & (y + j - 2 < nk1);
-    const int32_t packed = (ok && cnt > 0) ? ((cmin + pos[j] + 1) | (cnt << kRowCntShift)) : 0;
-    if (act) d.rows[(int64_t)rrow[j] * d.rstride + c] = packed;
+    if (!ballot(more)) break;
+  }
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    const int r = d3 ? 3 * g + j : j;
+    const int f = pos[j] + 1, nc = __popc(m[j]);
+    // (the windows of a one-column tile lie in segment lmin + k, k = the
+    // window's column - lmin)
+    const int k = one ? (int)(own + shift + j - 1 - lmin) : 0;
+    const int32_t first = f + (k <= 0 ? cb[0] : (k == 1 ? cb[1] - n0 : cb[2] - n01));
+    int32_t np = 0;
+    if (act && m[j]) np = cs[f + nc - 1] - d.cell_start[first];
+    if (act) d.rows[(int64_t)r * d.rstride + c] = make_row(first, m[j], np);
   }
   return true;
 }
 
 __global__ __launch_bounds__(256, 8) void k_rows(Dev d) {
   if (abandoned(d)) return;
-  __shared__ uint32_t s_ck[4][RW_CELLS];
+  __shared__ uint32_t s_ck[4][RW_SLOTS];
+  __shared__ int32_t s_cs[4][RW_CELLS];
   const int32_t C = (int32_t)d.ctl[C_NCELL];
-  const int64_t NL = d.ctl[C_NLINES];
-  const bool table = NL <= d.line_cap;
+  const bool table = d.ctl[C_NLINES] <= d.line_cap;
   const int wv = threadIdx.x >> 6;
-  // work item: tile * 5 + line group; the four waves of a workgroup take
-  // four consecutive items per step (the steps are uniform over the
-  // workgroup, as the list append wants)
-  const int64_t items = (((int64_t)C + 63) >> 6) * 5;
+  // work item: tile * 3 + group; the four waves of a workgroup take four
+  // consecutive items per step (the steps are uniform over the workgroup, as
+  // the list append wants)
+  const int64_t items = (((int64_t)C + 63) >> 6) * 3;
   for (int64_t base = (int64_t)blockIdx.x * 4; base < items; base += (int64_t)gridDim.x * 4) {
     const int64_t it = base + wv;
     bool left = false;
     if (it < items) {
-      const int64_t tile = it / 5;
-      // (the neighbourhood statistics run takes the global-memory pass)
-      left = !(table && !d.nbr_stats &&
-               rows_staged(d, tile, (int)(it - tile * 5), C, NL, s_ck[wv]));
+      const int64_t tile = it / 3;
+      left = !(table && rows_staged(d, tile, (int)(it - tile * 3), C, s_ck[wv], s_cs[wv]));
     }
     block_append(lane_id() == 0 && left, (int32_t)it, d.rows_fb);
   }
 }
 
-// The (tile, line group) pairs k_rows left: one lane per cell, the line's
-// cell range from the line table (or by two lower bounds over all cell
-// keys when there is none), then the first cell with z >= zlo by binary
-// search over cell_z in global memory, the five lines' searches in lockstep
-// so that their loads overlap.
+// The (tile, group) pairs k_rows left: one lane per cell, the column's cell
+// range from the column table (or by two lower bounds over all cell keys
+// when there is none), then the first cell of the window by binary search
+// over cell_zl in global memory and its slot bits from the cells that
+// follow, the three columns in lockstep so that their loads overlap.
 __global__ __launch_bounds__(256) void k_rows_global(Dev d) {
   if (abandoned(d)) return;
   __shared__ long long s_pre[kStripes + 1];
@@ -1155,103 +1146,146 @@ __global__ __launch_bounds__(256) void k_rows_global(Dev d) {
   const int32_t C = (int32_t)d.ctl[C_NCELL];
   const bool table = d.ctl[C_NLINES] <= d.line_cap;
   const int wv = threadIdx.x >> 6, lane = lane_id();
-  long long cand = 0, nbrc = 0;
   for (long long w = (long long)blockIdx.x * 4 + wv; w < nit; w += (long long)gridDim.x * 4) {
     const int64_t it = slist_at(d.rows_fb, s_pre, w);
-    const int64_t tile = it / 5;
-    const int g = (int)(it - tile * 5);
+    const int64_t tile = it / 3;
+    const int g = (int)(it - tile * 3);
     const int32_t c = (int32_t)(tile * 64 + lane);
-    const bool act = c < C;
-    RowLane L;
-    row_lane(d, c, act, g, C, L);
-    const Inst& I = *L.I;
-    const int last = L.dim - 1;
-    int32_t ls[5], le[5];
-    uint64_t k0[5];  // first key of each neighbour line (no line table)
-    bool need = false;
+    const int32_t cc = c < C ? c : C - 1;
+    const Inst& I = *inst_of_cell(d, cc);
+    const bool d3 = I.dim == 3;
+    const bool act = c < C && (d3 || g == 0);
+    const int ls = d3 ? 2 : 1;
+    const int64_t nzl = I.nzl;
+    const int32_t nz = (int32_t)(nzl >> ls);
+    const int64_t shift = d3 ? (g - 1) * I.cstride : 0;
+    const uint32_t zl = d.cell_zl[cc], z = zl >> ls;
+    const uint64_t key0 = d.cell_key[cc] - zl;  // first key of the cell's column
+    const int64_t own = table ? (int64_t)d.cell_col[cc] - I.line_base
+                              : (int64_t)((key0 - (uint64_t)I.key_base) / (uint64_t)nzl);
+    int32_t st[3], en[3];
+    bool ok[3];
 #pragma unroll
-    for (int j = 0; j < 5; ++j) {
-      const int64_t line = L.own + L.shift + row_off(L.dim, j) - I.line_base;
-      ls[j] = -1;
-      le[j] = -1;
-      k0[j] = (uint64_t)(I.key_base + line * I.nk[last]);
-      if (L.ok[j] && table) {
-        const int2 lr = d.lines[I.line_base + line];
-        ls[j] = lr.x;
-        le[j] = lr.y;
-      } else if (L.ok[j]) {
-        ls[j] = 0;  // searched below
-        le[j] = C;
-        need = true;
-      }
-    }
-    if (need) {
-      int32_t hi[5];
-#pragma unroll
-      for (int j = 0; j < 5; ++j) hi[j] = le[j];
-      lower_bound5(d.cell_key, ls, hi, k0);
-#pragma unroll
-      for (int j = 0; j < 5; ++j) {
-        hi[j] = le[j];
-        le[j] = ls[j];
-        k0[j] += (uint64_t)I.nk[last];
-      }
-      lower_bound5(d.cell_key, le, hi, k0);
-#pragma unroll
-      for (int j = 0; j < 5; ++j)
-        if (le[j] <= ls[j]) ls[j] = le[j] = -1;  // empty line
-    }
-    // lines of more than 4 cells: first cell with z >= zlo
-    int32_t lo[5], hi[5];
-#pragma unroll
-    for (int j = 0; j < 5; ++j) {
-      const bool srch = ls[j] >= 0 && le[j] - ls[j] > 4;
-      lo[j] = srch ? ls[j] : 0;
-      hi[j] = srch ? le[j] : 0;
-    }
-    for (;;) {
-      int32_t zm[5];
-      bool any = false;
-#pragma unroll
-      for (int j = 0; j < 5; ++j) {
-        zm[j] = lo[j] < hi[j] ? d.cell_z[(lo[j] + hi[j]) >> 1] : 0;
-        any |= lo[j] < hi[j];
-      }
-      if (!any) break;
-#pragma unroll
-      for (int j = 0; j < 5; ++j)
-        if (lo[j] < hi[j]) {
-          const int32_t mid = (lo[j] + hi[j]) >> 1;
-          if (zm[j] < L.zlo)
-            lo[j] = mid + 1;
-          else
-            hi[j] = mid;
+    for (int j = 0; j < 3; ++j) {
+      const int64_t col = own + shift + j - 1;
+      ok[j] = act && col >= 0 && col < I.nlines;
+      st[j] = en[j] = 0;
+      if (ok[j] && table) {
+        const int2 lr = d.lines[I.line_base + col];
+        if (lr.x >= 0) {
+          st[j] = lr.x;
+          en[j] = lr.y;
         }
-    }
-    // from the first candidate (line start of a short line, search result
-    // of a long one) the next up to 5 cells decide the run
-    int32_t packed[5];
-#pragma unroll
-    for (int j = 0; j < 5; ++j) {
-      const bool live = ls[j] >= 0 && le[j] > ls[j];
-      const bool shortl = le[j] - ls[j] <= 4;
-      const int32_t a0 = shortl ? ls[j] : lo[j];
-      int32_t a = a0, b = a0;
-#pragma unroll
-      for (int i = 0; i < 5; ++i) {
-        const int32_t z = (live && a0 + i < le[j] && (i < 4 || !shortl)) ? d.cell_z[a0 + i]
-                                                                         : 0x7fffffff;
-        a += z < L.zlo;
-        b += z <= L.zhi;
       }
-      packed[j] = (ls[j] >= 0 && b > a) ? (a | ((b - a) << kRowCntShift)) : 0;
     }
-    write_rows(d, c, act, L.dim, g, packed, cand, nbrc);
+    if (!table) {
+      int32_t lo[3], hi[3];
+      uint64_t k0[3];
+#pragma unroll
+      for (int j = 0; j < 3; ++j) {
+        k0[j] = key0 + (uint64_t)((shift + j - 1) * nzl);
+        lo[j] = 0;
+        hi[j] = ok[j] ? C : 0;
+      }
+      lower_bound3(d.cell_key, lo, hi, k0);
+#pragma unroll
+      for (int j = 0; j < 3; ++j) {
+        st[j] = lo[j];
+        hi[j] = ok[j] ? C : lo[j];
+        k0[j] += (uint64_t)nzl;
+      }
+      lower_bound3(d.cell_key, lo, hi, k0);
+#pragma unroll
+      for (int j = 0; j < 3; ++j) en[j] = ok[j] ? lo[j] : st[j];
+    }
+    const uint32_t zlo = z >= 2 ? z - 2 : 0;
+    const uint32_t zhi = z + 2u < (uint32_t)nz ? z + 2u : (uint32_t)nz - 1u;
+    int32_t q[3], hi[3];
+    uint32_t lov[3], m[3] = {0u, 0u, 0u};
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      q[j] = st[j];
+      hi[j] = en[j];
+      lov[j] = zlo << ls;
+    }
+    lower_bound3(d.cell_zl, q, hi, lov);
+    // (the last place of a window may be the last 32-bit value: compared
+    // inclusively)
+    const uint32_t last = (zhi << ls) + ((1u << ls) - 1u), win = (z << ls) - (2u << ls);
+    int32_t first[3];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) first[j] = q[j];
+    for (;;) {
+      uint32_t v[3][4];
+      bool in[3][4], more = false;
+#pragma unroll
+      for (int j = 0; j < 3; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          in[j][i] = q[j] + i < en[j];
+          v[j][i] = in[j][i] ? d.cell_zl[q[j] + i] : 0u;
+        }
+#pragma unroll
+      for (int j = 0; j < 3; ++j) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (in[j][i] && v[j][i] <= last) m[j] |= 1u << (v[j][i] - win);
+        if (in[j][3] && v[j][3] <= last) {
+          q[j] += 4;
+          more = true;
+        } else {
+          q[j] = en[j];
+        }
+      }
+      if (!ballot(more)) break;
+    }
+    if (act) {
+#pragma unroll
+      for (int j = 0; j < 3; ++j) {
+        const int r = d3 ? 3 * g + j : j;
+        int32_t np = 0;
+        if (m[j]) np = d.cell_start[first[j] + __popc(m[j])] - d.cell_start[first[j]];
+        d.rows[(int64_t)r * d.rstride + c] = make_row(first[j], m[j], np);
+      }
+    }
+  }
+}
+
+// Neighbourhood sizes (on request): non-empty cells and candidate points of
+// every cell's 5^D stencil.
+template <int D>
+__device__ void nbr_stats_cell(const Dev& d, int32_t c, long long& cand, long long& nbrc) {
+  const int local = (int)(d.cell_zl[c] & (Win<D>::nl - 1));
+  const RowsOf rows = rows_of(d, c);
+  long long pts = 0;
+  for (int r = 0; r < Win<D>::rows; ++r) {
+    const uint2 row = rows[r];
+    uint32_t m = row.y & (D == 3 ? row_valid<3>(r / 3 - 1, r % 3 - 1, local)
+                                 : row_valid<2>(r - 1, 0, local));
+    nbrc += __popc(m);
+    while (m) {
+      const int32_t q = slot_cell(row, __ffs(m) - 1);
+      m &= m - 1;
+      pts += d.cell_start[q + 1] - d.cell_start[q];
+    }
+  }
+  cand += pts * (d.cell_start[c + 1] - d.cell_start[c]);
+}
+
+__global__ __launch_bounds__(256) void k_nbr_stats(Dev d) {
+  if (abandoned(d)) return;
+  const int32_t C = (int32_t)d.ctl[C_NCELL];
+  long long cand = 0, nbrc = 0;
+  for (int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; c < C;
+       c += (int64_t)gridDim.x * blockDim.x) {
+    if (inst_of_cell(d, c)->dim == 3)
+      nbr_stats_cell<3>(d, (int32_t)c, cand, nbrc);
+    else
+      nbr_stats_cell<2>(d, (int32_t)c, cand, nbrc);
   }
   stat_add(d, C_CAND, cand);
   stat_add(d, C_NBRC, nbrc);
 }
-
 
 // ------------------------------------------------------------- launchers --
 void launch_index_head(const Dev& d, int nchunks, hipStream_t s) {
@@ -1311,14 +1345,14 @@ void launch_lines(const Dev& d, int grid_cells, hipStream_t s) {
   hipLaunchKernelGGL(k_line_mark, dim3(grid_cells), dim3(256), 0, s, d);
 }
 
-// Row pass grid: one wavefront per (tile of 64 cells, line group) for up
+// Row pass grid: one wavefront per (tile of 64 cells, group) for up
 // to n cells, at most kRowGrid workgroups (the steps loop beyond).
 constexpr int64_t kRowGrid = 16384;
 int64_t row_blocks(int64_t n) {
-  return std::max<int64_t>(1, std::min<int64_t>(kRowGrid, (((n + 63) / 64) * 5 + 3) / 4));
+  return std::max<int64_t>(1, std::min<int64_t>(kRowGrid, (((n + 63) / 64) * 3 + 3) / 4));
 }
 int64_t row_list_cap(int64_t n) {
-  const int64_t items = ((n + 63) / 64) * 5;
+  const int64_t items = ((n + 63) / 64) * 3;
   const int64_t g = row_blocks(n);
   const int64_t steps = (items + 4 * g - 1) / (4 * g);
   return (g + kStripes - 1) / kStripes * 4 * steps;  // appends per stripe, at most
@@ -1329,6 +1363,7 @@ void launch_rows(const Dev& d, int64_t n, int grid_cells, hipStream_t s) {
   // the tiles left over, one wavefront each: enough waves for the list
   const int64_t gb = std::max<int64_t>(1, std::min<int64_t>(4LL * grid_cells, (n + 255) / 256));
   hipLaunchKernelGGL(k_rows_global, dim3((unsigned)gb), dim3(256), 0, s, d);
+  if (d.nbr_stats) hipLaunchKernelGGL(k_nbr_stats, dim3((unsigned)gb), dim3(256), 0, s, d);
 }
 
 void launch_scan_top(int64_t* v, int nb, hipStream_t s) {

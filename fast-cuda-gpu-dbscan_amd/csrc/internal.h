@@ -4,10 +4,10 @@
 // largest run seen so far and reused):
 //   input   xyz       caller's row-major FP64 rows, instances back to back
 //   sort    key[2]    u64 cell keys (ping-pong), val[2] i32 point ids
-//   CSR     cell_start[C+1], cell_key[C], cell_inst[C], rows[C][25] (packed
-//           runs of the 5^(D-1) neighbour lines, centre line first),
+//   CSR     cell_start[C+1], cell_key[C], cell_inst[C], cell_col[C], cell_zl[C],
+//           rows[3^(D-1)][C] (windows of the neighbour columns),
 //           cell_ncore[C], cell_label[C] (chain), amask[C] (near graph), rep[C]
-//   points  (cell-sorted)  X[3][N] FP64 SoA (FP64 form only), G[3][N] u32 fixed-point
+//   points  (cell-sorted)  X[N][3] FP64 (FP64 form only), G[N][3] u32 fixed-point
 //           coordinates (29 fraction bits per cell, wrapping mod 8 cells),
 //           orig[N], cell_of[N], core[N] u8, rec[N][R] + rec_n[N] (the
 //           neighbours of each non-core point)
@@ -24,52 +24,108 @@ constexpr int kWave = 64;
 constexpr int32_t kUnclaimed = -1;
 constexpr int32_t kNoKey = 0x7fffffff;
 constexpr int kFixBits = 29;  // fixed-point fraction bits per cell width
-constexpr int kMaxRows = 25;  // 5^(D-1) neighbour lines for D <= 3
-constexpr int kRowCntShift = 28;  // packed row: first cell | cell count << 28
-constexpr int32_t kRowCellMask = (1 << kRowCntShift) - 1;
-constexpr int64_t kMaxCells = 1LL << kRowCntShift;
+constexpr int kMaxRows = 9;   // 3^(D-1) neighbour columns for D <= 3
+constexpr int64_t kMaxCells = 1LL << 28;  // points (and so cells) of a call
 constexpr int kHeavy = 32;    // cells with more points are "heavy" (a wavefront per border pair)
-constexpr int kRecSlots = 16;  // neighbour records kept per non-core point (at most)
+constexpr int kRecSlots = 32;  // neighbour records kept per non-core point (at most)
+constexpr int kRecSlotsFixed = 16;  // the same in the fixed region of no-allocation runs
+// rec_n of a point without records, whose rows are scanned instead: fewer
+// than minpts points in all, or more neighbours than slots
+constexpr int kRecFew = 254;
+constexpr int kRecNone = 255;
 
-// Stencil lines, nearest first: (offset along axis 0, offset along axis 1)
-// of line r for D = 3, offset along axis 0 for D = 2.  The mirror of line r
-// is the line with the negated offsets (used to set the adjacency bit of
-// the other cell of a pair).
-#define DCLUST_ROW_OFF3                                                                     \
-  {{0, 0},   {-1, 0}, {1, 0},   {0, -1},  {0, 1},  {-1, -1}, {-1, 1}, {1, -1}, {1, 1},       \
-   {-2, 0},  {2, 0},  {0, -2},  {0, 2},   {-2, -1}, {-2, 1}, {2, -1}, {2, 1},  {-1, -2},     \
-   {1, -2},  {-1, 2}, {1, 2},   {-2, -2}, {-2, 2}, {2, -2}, {2, 2}}
-#define DCLUST_ROW_MIRROR3 \
-  {0, 2, 1, 4, 3, 8, 7, 6, 5, 10, 9, 12, 11, 16, 15, 14, 13, 20, 19, 18, 17, 24, 23, 22, 21}
-// row of the line with offsets (a - 2, b - 2) along axes 0 and 1 (3-D)
-#define DCLUST_ROW_OF_OFF3                                                     \
-  {{21, 13, 9, 14, 22}, {17, 5, 1, 6, 19}, {11, 3, 0, 4, 12}, {18, 7, 2, 8, 20}, \
-   {23, 15, 10, 16, 24}}
-#define DCLUST_ROW_OFF2 {0, -1, 1, -2, 2}
-#define DCLUST_ROW_MIRROR2 {0, 2, 1, 4, 3}
-static __constant__ int8_t kRowOff3[25][2] = DCLUST_ROW_OFF3;
-static __constant__ int8_t kRowOff2[5] = DCLUST_ROW_OFF2;
-static __constant__ int8_t kRowMirror3[25] = DCLUST_ROW_MIRROR3;
-static __constant__ int8_t kRowMirror2[5] = DCLUST_ROW_MIRROR2;
-static __constant__ int8_t kRowOfOff3[5][5] = DCLUST_ROW_OF_OFF3;
+// Cell order.  A column is the cells of a 2 x 2 block of the first two axes
+// (3-D; of two cells of the first axis in 2-D) along the whole last axis.
+// Cells are sorted by column, then by position along the last axis, then by
+// place in the block (`local`, 2 bits in 3-D, 1 in 2-D: x & 1, then y & 1).
+// So the 5^D stencil of a cell is covered by the same window of five steps
+// along the last axis in 3^(D-1) neighbouring columns, and each window is a
+// run of consecutive cells.  Row r of a cell is the window of the column with
+// block offsets (a, b): r = 3(a+1) + b+1 in 3-D, r = a+1 in 2-D.  It holds the
+// window's first cell, one bit per window slot: slot = step * nl + local, step
+// 0..4 from two below the cell, nl = 2^(D-1) cells of a column per step, and
+// above the 20 slot bits the number of the window's points (at most
+// kRowCount).  The cell in slot s is first + (number of bits below s).  (One line per
+// pair of offsets along the first two axes, as before, took 25 searches per
+// cell instead of 9 and 100 bytes per cell instead of 72.)
+template <int D>
+struct Win {
+  static constexpr int nl = 1 << (D - 1);
+  static constexpr int rows = D == 3 ? 9 : 3;
+  static constexpr int own = D == 3 ? 4 : 1;  // row of the cell's own column
+  static constexpr int slots = 5 * nl;
+  // local bits of all five steps from those of one
+  static constexpr uint32_t steps = D == 3 ? 0x11111u : 0x155u;
+};
+
+constexpr uint32_t kRowBits = (1u << 20) - 1u;
+constexpr uint32_t kRowCount = (1u << 12) - 1u;  // this many points or more
+
+// Cells of block offset a that lie within two cells of a cell at place l of
+// its block, along one axis (bit 0: place 0, bit 1: place 1).
+__host__ __device__ __forceinline__ constexpr uint32_t axis_valid(int a, int l) {
+  return a == 0 ? 3u : (a > 0 ? (l ? 3u : 1u) : (l ? 2u : 3u));
+}
+
+// Slots of row (a, b) inside the 5^D stencil of a cell at `local`.
+template <int D>
+__host__ __device__ __forceinline__ constexpr uint32_t row_valid(int a, int b, int local) {
+  if (D == 2) return axis_valid(a, local & 1) * Win<2>::steps;
+  const uint32_t vx = axis_valid(a, local >> 1), vy = axis_valid(b, local & 1);
+  return ((vx & 1u ? vy : 0u) | (vx & 2u ? vy << 2 : 0u)) * Win<3>::steps;
+}
+
+// Near cells: at most one cell away along every axis.  Offset (dx, dy, dz)
+// has the bit (dx+1)*9 + (dy+1)*3 + dz+1 of a cell's near mask (2-D: dy = 0);
+// the opposite offset has bit 26 - b.
+constexpr int kNearOwn = 13;
+
+// Row and slot of near bit b for a cell at `local`.
+template <int D>
+__host__ __device__ __forceinline__ constexpr void near_slot(int b, int local, int& row,
+                                                             int& slot) {
+  const int dx = (b * 57) >> 9;           // b / 9 for b < 27
+  const int r9 = b - 9 * dx;
+  const int dy = (r9 * 11) >> 5;          // r9 / 3 for r9 < 9
+  const int dz = r9 - 3 * dy;
+  if (D == 2) {
+    const int tx = (local & 1) + dx - 1;  // -1..2
+    row = 1 + (tx >> 1);
+    slot = (dz + 1) * 2 + (tx & 1);
+  } else {
+    const int tx = (local >> 1) + dx - 1, ty = (local & 1) + dy - 1;
+    row = 4 + 3 * (tx >> 1) + (ty >> 1);
+    slot = (dz + 1) * 4 + (tx & 1) * 2 + (ty & 1);
+  }
+}
 
 namespace tables {
-constexpr int8_t off3[25][2] = DCLUST_ROW_OFF3;
-constexpr int8_t mir3[25] = DCLUST_ROW_MIRROR3;
-constexpr int8_t off2[5] = DCLUST_ROW_OFF2;
-constexpr int8_t mir2[5] = DCLUST_ROW_MIRROR2;
-constexpr int8_t rof3[5][5] = DCLUST_ROW_OF_OFF3;
-constexpr bool mirrors_ok() {
-  for (int r = 0; r < 25; ++r)
-    if (off3[mir3[r]][0] != -off3[r][0] || off3[mir3[r]][1] != -off3[r][1]) return false;
-  for (int a = 0; a < 5; ++a)
-    for (int b = 0; b < 5; ++b)
-      if (off3[rof3[a][b]][0] != a - 2 || off3[rof3[a][b]][1] != b - 2) return false;
-  for (int r = 0; r < 5; ++r)
-    if (off2[mir2[r]] != -off2[r]) return false;
+// every offset of the 5^D stencil lies in exactly one valid slot, and the
+// near bits name the slots of their offsets
+template <int D>
+constexpr bool windows_ok() {
+  for (int local = 0; local < Win<D>::nl; ++local) {
+    const int lx = D == 3 ? local >> 1 : local, ly = D == 3 ? local & 1 : 0;
+    int count = 0;
+    for (int a = -1; a <= 1; ++a)
+      for (int b = D == 3 ? -1 : 0; b <= (D == 3 ? 1 : 0); ++b)
+        for (int s = 0; s < Win<D>::slots; ++s) {
+          const int l = s % Win<D>::nl, dz = s / Win<D>::nl - 2;
+          const int dx = 2 * a + (D == 3 ? l >> 1 : l) - lx;
+          const int dy = D == 3 ? 2 * b + (l & 1) - ly : 0;
+          const bool in = dx >= -2 && dx <= 2 && dy >= -2 && dy <= 2;
+          if (in != (((row_valid<D>(a, b, local) >> s) & 1u) != 0)) return false;
+          count += in;
+          if (dx < -1 || dx > 1 || dy < -1 || dy > 1 || dz < -1 || dz > 1) continue;
+          int row = 0, slot = 0;
+          near_slot<D>((dx + 1) * 9 + (dy + 1) * 3 + dz + 1, local, row, slot);
+          if (row != (D == 3 ? 3 * (a + 1) + b + 1 : a + 1) || slot != s) return false;
+        }
+    if (count != (D == 3 ? 125 : 25)) return false;
+  }
   return true;
 }
-static_assert(mirrors_ok(), "stencil line mirror table");
+static_assert(windows_ok<2>() && windows_ok<3>(), "stencil windows");
 }  // namespace tables
 
 // Per-instance parameters and derived grid (device table, one per instance).
@@ -89,8 +145,12 @@ struct Inst {
   int32_t nk[3];   // cells per axis
   int32_t err;     // per-instance error code (DCLUST_E_*)
   int64_t key_base;            // first key of this instance's cell space
-  int64_t line_base;           // first entry of this instance's line table
-  int64_t nlines;              // possible lines (product of all but the last axis)
+  int64_t line_base;           // first entry of this instance's column table
+  int64_t nlines;              // its columns
+  int64_t nzl;                 // keys of a column: cells along the last axis * nl
+  int64_t cstride;             // columns per step of the first axis' blocks (3-D: one
+                               // more than there are, so that the column before the
+                               // first and after the last of a step is always empty)
   int64_t pt_begin, pt_end;    // global point-index range
   int64_t xyz_off;             // element offset of the first coordinate
 };
@@ -130,7 +190,7 @@ enum Ctl : int {
   C_BUSY_SUM,  // expansion: sum over waves of their lifetime (us)
   C_BUSY_MAX,
   C_SEGS_LEFT,  // expansion waves whose seeding segment is not finished
-  C_NLINES,     // total line-table entries
+  C_NLINES,     // total column-table entries
   C_DENSE,      // cells resolved as all-core without distance tests
   C_NHEAVY,     // heavy cells (more than kHeavy points)
   C_NADJPTS,    // core points of light cells
@@ -150,32 +210,35 @@ enum Ctl : int {
   C_ROUNDS_MAX, // most pop rounds of one expansion wave in one pass
   C_KEYOVF,     // the cell-key space of the whole call exceeds 2^63 keys
   // work counts of the neighbour kernels (their algorithmic bytes)
-  C_CORE_GROUPS,  // k_core: groups of 5 stencil lines streamed
-  C_CORE_LINES,   // k_core: non-empty stencil lines streamed
-  C_ADJ_LINES,    // k_adj: non-empty near lines examined
-  C_ADJ_CELLS,    // k_adj: cells of those lines
+  C_CORE_ROWS,    // neighbour counts: rows read
+  C_CORE_RANGES,  // neighbour counts: non-empty point ranges of them
   C_NROWSFB,      // row work items left to the global-memory pass (Dev::rows_fb)
   C_NBORDERPTS,   // non-core points (listed in Dev::border_pts)
+  C_NCOREREST,    // points left by the first count pass (Dev::core_rest)
+  C_NCORECROWD,   // those taken by a wavefront each (Dev::core_crowd)
   C_NROOTS,       // near components (listed in Dev::near_roots)
-  C_NFARPAIRS,    // border pairs with a heavy cell (listed in Dev::far_pairs)
+  C_NFARLIGHT,    // pairs across components (listed in Dev::far_light)
+  C_NFARHEAVY,    // those with a heavy cell (listed in Dev::far_heavy)
   C_NCTL
 };
-static_assert(C_NFARPAIRS < C_NCTL, "control block too small");
+static_assert(C_NFARHEAVY < C_NCTL, "control block too small");
 
 // Cell-key space: the sort key of a cell is its instance's key base plus its
-// linear index, and the radix sort orders keys of up to 63 bits, so the
+// place in the cell order, and the
 // cells of all instances of a call must number at most 2^63.  Sums are
-// saturating, so an overflowing total stays above the limit.
+// saturating, so an overflowing total stays above the limit.  (The keys
+// themselves number a little more: odd axes are rounded up to whole blocks,
+// and every step of blocks has one empty column.)
 constexpr unsigned long long kMaxKeySpace = 1ull << 63;
 __host__ __device__ __forceinline__ unsigned long long sat_add(unsigned long long a,
                                                                 unsigned long long b) {
   const unsigned long long s = a + b;
   return s < a ? ~0ull : s;
 }
-// Radix-sort key width for a key space of `total` keys (total <= 2^63).
+// Radix-sort key width for a key space of `total` keys.
 __host__ __device__ __forceinline__ int key_bits_for(unsigned long long total) {
   int bits = 1;
-  while (bits < 63 && (1ull << bits) < total) ++bits;
+  while (bits < 64 && (1ull << bits) < total) ++bits;
   return bits;
 }
 
@@ -240,37 +303,40 @@ struct Dev {
   // CSR
   int32_t* cell_start;  // [N+1]
   uint64_t* cell_key;   // [N]
-  uint64_t* cell_xyz;   // [N] packed integer cell coordinates
-  int32_t* cell_z;      // [N] last integer cell coordinate (position in its line)
+  uint32_t* cell_col;   // [N] column-table index (when there is a column table)
+  uint32_t* cell_zl;    // [N] place in the column: last coordinate * nl + local
   int32_t* cell_inst;   // [N]
   int32_t* cell_ncore;  // [N] core points per cell
   int32_t* cell_label;  // [N] chain owning the cell's core points
-  unsigned long long* amask;  // [N] near graph: bit 5r+k <-> k-th cell of line r < 9
-  int32_t* cell_comp;   // [N] component (root chain) of each core cell, -1 otherwise
+  uint32_t* amask;      // [N] near graph: joined near cells, by near bit
+  int32_t* cell_comp;   // [N+4] component (root chain) of each core cell, -1 otherwise
   uint4* rep;           // [N] per cell: its first core point's G and sorted index
                         // (over the sort keys, which the CSR pass is the last to read)
   int32_t chains;       // 1: near components by seed-list expansion, 0: by union-find
+  SList core_rest;      // points the first count pass leaves (over keyv)
+  SList core_crowd;     // those of them with many candidates (over rank)
   SList border_pts;     // non-core points (border-label lanes)
   SList core_cells;     // cells with core points (near-graph and border-pair lanes)
   SList near_roots;     // roots of the near components
-  PairList far_pairs;   // border pairs with a heavy cell (over the sort's point ids,
-                        // which the gather is the last to read)
-  int32_t* rows;        // [kMaxRows][rstride] packed neighbour lines (first cell, count),
-                        // line-major so that consecutive cells are adjacent
+  PairList far_light;   // pairs of cells across components without a heavy cell and
+  PairList far_heavy;   // with one (over the sort's point ids, which the gather is the
+                        // last to read)
+  uint2* rows;          // [kMaxRows][rstride] neighbour windows (first cell, slot bits and
+                        // point count), row-major so that consecutive cells are adjacent
   int64_t rstride;      // >= number of cells
   int32_t* cell_of;     // [N] per sorted point
-  int2* lines;          // [line_cap] first / end cell of every possible line
-  int64_t line_cap;     // 0: no line table, rows found by binary search
-  int32_t nbr_stats;    // 1: k_rows also sums the neighbourhood sizes
+  int2* lines;          // [line_cap] first / end cell of every column
+  int64_t line_cap;     // 0: no column table, windows found by binary search
+  int32_t nbr_stats;    // 1: the neighbourhood sizes are summed
 
   // sorted point data
-  double* X[3];         // FP64 form only (null in the FP32 form)
+  double* X;            // [N][3] FP64 form only (null in the FP32 form)
   int64_t* xoff;        // FP32 form: offset of each point's row in xyz
-  uint32_t* G[3];
+  uint32_t* G;          // [N][3]
   int32_t* orig;
   uint8_t* core;
-  int32_t* rec;         // [N][rec_stride] neighbours of non-core points
-  uint8_t* rec_n;       // [N] records written (saturates at 255)
+  int32_t* rec;         // [rec_stride][N] neighbours of non-core points
+  uint8_t* rec_n;       // [N] records written, kRecFew or kRecNone
   int32_t rec_stride;   // record slots per point: min(minpts, kRecSlots)
   int32_t* parent;
   int32_t* compmin;
@@ -281,7 +347,7 @@ struct Dev {
   int32_t* q[2];
   int64_t* seg_pos;     // [waves] seeding cursor of each expansion wave
   int32_t* keyv;
-  SList rows_fb;         // row work items (tile * 5 + line group) left to k_rows_global
+  SList rows_fb;         // row work items (tile * 3 + group) left to k_rows_global
   uint8_t* flag;
   int32_t* rank;
   int64_t* scan_tmp;  // block sums for scans
@@ -473,14 +539,25 @@ struct OneStep {
   int32_t blocks, S, cap, pad;
 };
 
-// The stencil lines of one cell: rows_of(d, c)[r] is line r (packed).
+// The rows of one cell.
 struct RowsOf {
-  const int32_t* base;
+  const uint2* base;
   int64_t stride;
-  __device__ __forceinline__ int32_t operator[](int r) const { return base[(int64_t)r * stride]; }
+  __device__ __forceinline__ uint2 operator[](int r) const { return base[(int64_t)r * stride]; }
 };
 __device__ __forceinline__ RowsOf rows_of(const Dev& d, int64_t c) {
   return RowsOf{d.rows + c, d.rstride};
+}
+// cells and points of a row's window
+__device__ __forceinline__ int row_cells(uint2 row) { return __popc(row.y & kRowBits); }
+__device__ __forceinline__ uint32_t row_count(uint2 row) { return row.y >> 20; }
+__device__ __forceinline__ uint2 make_row(int32_t first, uint32_t bits, int32_t points) {
+  const uint32_t n = (uint32_t)points < kRowCount ? (uint32_t)points : kRowCount;
+  return make_uint2(bits ? (uint32_t)first : 0u, bits | (n << 20));
+}
+// cell in slot s of a row
+__device__ __forceinline__ int32_t slot_cell(uint2 row, int s) {
+  return (int32_t)row.x + __popc(row.y & ((1u << s) - 1u));
 }
 
 // Instance of a cell (a run of one instance reads the table entry directly,

@@ -108,21 +108,17 @@ __device__ void os_step(const Dev& d, const OneStep& o, int32_t chain) {
   }
   const Inst& I = *d.inst;
   const double eps = I.eps, eps2 = I.eps2;
-  constexpr int NR = D == 3 ? 25 : 5;
+  constexpr int NR = Win<D>::rows;
   double px[D];
   load_x<D, false>(d, p, px);
   const RowsOf rows = rows_of(d, d.cell_of[p]);
 
   // neighbour count of p, self included (dbscan_indexing.cu:581-617)
   int cnt = 0;
-  for (int g = 0; g < NR; g += 5) {
-    int32_t aa[5], ll[5];
-    line_group(d, rows, g, aa, ll);
-    Stream5 st;
-    st.set(aa, ll);
-    for (int32_t i = tid; i < st.tot; i += T) {
-      int jr;
-      const int32_t q = st.at(i, jr);
+  for (int r = 0; r < NR; ++r) {
+    int32_t a, e;
+    row_points(d, rows[r], a, e);
+    for (int32_t q = a + tid; q < e; q += T) {
       double qx[D];
       load_x<D, false>(d, q, qx);
       cnt += box_64<D>(px, qx, eps) && d2_64<D>(px, qx) <= eps2;
@@ -147,14 +143,10 @@ __device__ void os_step(const Dev& d, const OneStep& o, int32_t chain) {
   // claim and push the unclassified neighbours, take the noise ones as
   // border points, record contacts with expanded core points of other
   // chains (MarkAsCandidate, dbscan_indexing.cu:783-807)
-  for (int g = 0; g < NR; g += 5) {
-    int32_t aa[5], ll[5];
-    line_group(d, rows, g, aa, ll);
-    Stream5 st;
-    st.set(aa, ll);
-    for (int32_t i = tid; i < st.tot; i += T) {
-      int jr;
-      const int32_t q = st.at(i, jr);
+  for (int r = 0; r < NR; ++r) {
+    int32_t a, e;
+    row_points(d, rows[r], a, e);
+    for (int32_t q = a + tid; q < e; q += T) {
       if (q == p) continue;
       double qx[D];
       load_x<D, false>(d, q, qx);
@@ -198,18 +190,14 @@ __global__ __launch_bounds__(1024) void k_os_step(Dev d, OneStep o, int32_t chai
 template <int D>
 __device__ void os_border(const Dev& d, const OneStep& o, int32_t p) {
   const Inst& I = *d.inst;
-  constexpr int NR = D == 3 ? 25 : 5;
+  constexpr int NR = Win<D>::rows;
   double px[D];
   load_x<D, false>(d, p, px);
   const RowsOf rows = rows_of(d, d.cell_of[p]);
-  for (int g = 0; g < NR; g += 5) {
-    int32_t aa[5], ll[5];
-    line_group(d, rows, g, aa, ll);
-    Stream5 st;
-    st.set(aa, ll);
-    for (int32_t i = 0; i < st.tot; ++i) {
-      int jr;
-      const int32_t q = st.at(i, jr);
+  for (int r = 0; r < NR; ++r) {
+    int32_t a, e;
+    row_points(d, rows[r], a, e);
+    for (int32_t q = a; q < e; ++q) {
       if (o.state[q] != 2) continue;
       double qx[D];
       load_x<D, false>(d, q, qx);

@@ -145,10 +145,10 @@ typedef struct dclust_stats {
   double t_rows_ms;       /* the neighbour-line kernel alone (inside t_index) */
   int64_t n_core_cells;   /* cells holding core points                       */
   int64_t n_adj_points;   /* core points of light cells                      */
-  int64_t n_lines;        /* possible grid lines (line-table entries)        */
-  /* work of the neighbour kernels (the units of their algorithmic bytes):
-   * [0] k_core line groups streamed (5 lines each), [1] k_core non-empty
-   * lines, [2] k_adj non-empty near lines, [3] k_adj cells on them */
+  int64_t n_lines;        /* possible grid columns (column-table entries)    */
+  /* work of the neighbour counts (the units of their algorithmic bytes):
+   * [0] rows (column windows) read, [1] non-empty point ranges of them, [2]
+   * points left by the first pass, [3] those taken by a wavefront each */
   int64_t work[4];
 } dclust_stats;
 
