@@ -75,6 +75,12 @@ struct dclust_handle {
   bool graph_broken = false;       // capture failed on this device: eager only
   bool graph_off = false;          // eager only (while autotuning)
   uint8_t* scratch = nullptr;      // this device's scratch array (no-allocation runs)
+  // two pinned halves of kStageBytes each through which small host arrays go
+  // (allocated by the first call that can use them; null: copies straight from
+  // and to the caller's pageable memory), and the events of their last copies
+  uint8_t* stage = nullptr;
+  bool stage_failed = false;
+  hipEvent_t stage_ev[2] = {};
   // the instance table and chunk list last copied to the device, and where
   // (a replay with the same bytes at the same place skips the copies)
   std::vector<uint8_t> up_bytes;
@@ -154,6 +160,124 @@ hipError_t scratch_address(int device, uint8_t** out) {
   }
   *out = g_scratch[device];
   return hipSuccess;
+}
+
+// Host arrays of the entry points that take them.  A copy from or to pageable
+// memory costs about 10 us however small it is (a batch of 400 instances of a
+// few kilobytes took 9.1 ms, 8 ms of it 800 such copies), so consecutive
+// pieces are packed into a pinned half and copied at once, one half in flight
+// while the other is packed.  A piece of kStageDirect bytes or more goes
+// straight from or to the caller's memory (the runtime's own staging then
+// keeps up).
+constexpr size_t kStageBytes = 4ull << 20;
+constexpr size_t kStageDirect = 1ull << 20;
+
+bool stage_ready(dclust_handle* h) {
+  if (h->stage) return true;
+  if (h->stage_failed) return false;
+  bool ok = hipHostMalloc((void**)&h->stage, 2 * kStageBytes, 0) == hipSuccess;
+  for (auto& e : h->stage_ev)
+    ok = ok && (e || hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess);
+  if (!ok) {
+    (void)hipGetLastError();
+    if (h->stage) (void)hipHostFree(h->stage);
+    h->stage = nullptr;
+    h->stage_failed = true;
+  }
+  return ok;
+}
+
+// One piece of host memory; the pieces of a list are back to back on the
+// device.
+struct HostPiece {
+  void* p;
+  size_t bytes;
+};
+
+// Host pieces -> dst.  On return every piece has been read, or its copy is
+// on the stream (pageable copies are complete).
+hipError_t pieces_to_device(dclust_handle* h, const std::vector<HostPiece>& v, uint8_t* dst) {
+  const hipStream_t s = h->stream;
+  const bool staged = stage_ready(h);
+  hipError_t e = hipSuccess;
+  int half = 0;
+  size_t fill = 0;
+  bool busy[2] = {false, false};
+  auto flush = [&]() {
+    if (!fill || e != hipSuccess) return;
+    e = hipMemcpyAsync(dst, h->stage + half * kStageBytes, fill, hipMemcpyHostToDevice, s);
+    if (e == hipSuccess) e = hipEventRecord(h->stage_ev[half], s);
+    busy[half] = true;
+    dst += fill;
+    fill = 0;
+    half ^= 1;
+    if (e == hipSuccess && busy[half]) e = hipEventSynchronize(h->stage_ev[half]);
+  };
+  for (const HostPiece& x : v) {
+    if (x.bytes == 0) continue;
+    if (!staged || x.bytes >= kStageDirect) {
+      flush();
+      if (e == hipSuccess) e = hipMemcpyAsync(dst, x.p, x.bytes, hipMemcpyHostToDevice, s);
+      dst += x.bytes;
+    } else {
+      if (fill + x.bytes > kStageBytes) flush();
+      if (e == hipSuccess) std::memcpy(h->stage + half * kStageBytes + fill, x.p, x.bytes);
+      fill += x.bytes;
+    }
+    if (e != hipSuccess) return e;
+  }
+  flush();
+  return e;
+}
+
+// src -> host pieces, complete on return.  `first` bytes at the head of the
+// first half are there already (their copy was enqueued with the run and the
+// stream has drained since).
+hipError_t pieces_from_device(dclust_handle* h, const std::vector<HostPiece>& v,
+                              const uint8_t* src, size_t first = 0) {
+  const hipStream_t s = h->stream;
+  const bool staged = stage_ready(h);
+  hipError_t e = hipSuccess;
+  // groups of pieces that share a half, one in flight while the previous one
+  // is unpacked
+  size_t i = 0, out = 0;  // next piece to fetch, next piece to unpack
+  size_t end[2] = {0, 0};  // pieces fetched into each half end here
+  int half = 0;
+  bool pending = false;
+  auto unpack = [&](int hf) {
+    if (e == hipSuccess) e = hipEventSynchronize(h->stage_ev[hf]);
+    const uint8_t* q = h->stage + hf * kStageBytes;
+    for (; out < end[hf]; ++out) {
+      if (e == hipSuccess) std::memcpy(v[out].p, q, v[out].bytes);
+      q += v[out].bytes;
+    }
+  };
+  while (i < v.size() && e == hipSuccess) {
+    if (!staged || v[i].bytes >= kStageDirect) {
+      if (pending) unpack(half ^ 1);
+      pending = false;
+      if (v[i].bytes && e == hipSuccess)
+        e = hipMemcpyAsync(v[i].p, src, v[i].bytes, hipMemcpyDeviceToHost, s);
+      src += v[i].bytes;
+      out = ++i;
+      continue;
+    }
+    size_t fill = 0;
+    while (i < v.size() && v[i].bytes < kStageDirect && fill + v[i].bytes <= kStageBytes)
+      fill += v[i++].bytes;
+    end[half] = i;
+    if (fill > first)
+      e = hipMemcpyAsync(h->stage + half * kStageBytes, src, fill, hipMemcpyDeviceToHost, s);
+    first = 0;
+    if (e == hipSuccess) e = hipEventRecord(h->stage_ev[half], s);
+    src += fill;
+    if (pending) unpack(half ^ 1);
+    pending = true;
+    half ^= 1;
+  }
+  if (pending) unpack(half ^ 1);
+  if (e == hipSuccess) e = hipStreamSynchronize(s);
+  return e;
 }
 
 // Where a run's device buffers come from: the handle's arena (grown with
@@ -576,6 +700,13 @@ void finish_run(dclust_handle* h, const Dev& d, const RunShape& shape, const lon
   set_shape_stats(shape, stats);
 }
 
+int host_copy_failed(dclust_handle* h, dclust_stats* stats) {
+  const hipError_t e = hipGetLastError();
+  h->last_err = (int)e;
+  if (stats) stats->hip_error = (int32_t)e;
+  return DCLUST_E_HIP;
+}
+
 #define HIPCHK(x)                          \
   do {                                     \
     hipError_t e_ = (x);                   \
@@ -594,10 +725,12 @@ int onestep_loop(dclust_handle* h, const Dev& d, const dclust_params& prm, int t
 // runs after the index instead of the clustering phases
 // region != null: every device buffer of the run comes from that region
 // (cap bytes), nothing is allocated and the run is eager (no graph capture).
+// host_labels != null: the labels are also copied to that pinned buffer, the
+// copy enqueued behind the run so that one wait serves both.
 int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64_t* n,
                const dclust_params* params, int32_t* d_labels, int32_t* inst_err,
                dclust_stats* stats, int onestep_threads = 0, uint8_t* region = nullptr,
-               size_t region_cap = 0) {
+               size_t region_cap = 0, void* host_labels = nullptr) {
   const bool onestep = onestep_threads > 0;
   const bool fixed_mem = region != nullptr;
   hipError_t herr = hipSuccess;
@@ -825,11 +958,17 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
       }
       return ue;
     };
+    auto copy_labels = [&]() -> hipError_t {
+      if (!host_labels) return hipSuccess;
+      return hipMemcpyAsync(host_labels, d_labels, sizeof(int32_t) * ntot, hipMemcpyDeviceToHost,
+                            s);
+    };
     if (h->gexec && !fixed_mem) {
       HIPCHK(upload());
       HIPCHK(hipEventRecord(h->ev[E_START], s));
       HIPCHK(hipGraphLaunch(h->gexec, s));
       HIPCHK(hipEventRecord(h->ev[E_END], s));  // (after the counters' readback)
+      HIPCHK(copy_labels());
       HIPCHK(read_counters(h, d, s, ctl_h, h->greadback));
       if (!ctl_h[C_ABANDON]) {
         if (ctl_h[C_ERR]) {
@@ -901,6 +1040,7 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
     }
     ++npass;
     HIPCHK(enqueue_tail(h, d, f32, grid_cells, false));
+    HIPCHK(copy_labels());
     HIPCHK(read_counters(h, d, s, ctl_h));
     finish_run(h, d, shape, ctl_h, npass, false, stats);
     if (npass >= kMaxExpandPasses) return DCLUST_E_CAPACITY;
@@ -1180,6 +1320,9 @@ void dclust_destroy(dclust_handle* h) {
     if (e) (void)hipEventDestroy(e);
   if (h->stream) (void)hipStreamDestroy(h->stream);
   if (h->pin) (void)hipHostFree(h->pin);
+  for (auto& e : h->stage_ev)
+    if (e) (void)hipEventDestroy(e);
+  if (h->stage) (void)hipHostFree(h->stage);
   delete h;
 }
 
@@ -1231,15 +1374,20 @@ int dclust_run(dclust_handle* h, const double* xyz, int64_t n, const dclust_para
   double* dx = h->get<double>(S_XYZ, (size_t)n * p->dim, &herr);
   int32_t* dl = h->get<int32_t>(S_LABOUT, n, &herr);
   if (!dx || !dl) return DCLUST_E_OOM;
-  if (hipMemcpyAsync(dx, xyz, sizeof(double) * n * p->dim, hipMemcpyHostToDevice, h->stream) !=
-      hipSuccess)
-    return DCLUST_E_HIP;
-  int rc = run_device(h, 1, dx, &n, p, dl, nullptr, stats);
-  if (rc != DCLUST_OK) return rc;
-  if (hipMemcpyAsync(labels_out, dl, sizeof(int32_t) * n, hipMemcpyDeviceToHost, h->stream) !=
-          hipSuccess ||
-      hipStreamSynchronize(h->stream) != hipSuccess)
-    return DCLUST_E_HIP;
+  const std::vector<HostPiece> in = {{(void*)xyz, sizeof(double) * (size_t)n * p->dim}};
+  const std::vector<HostPiece> out = {{labels_out, sizeof(int32_t) * (size_t)n}};
+  if (pieces_to_device(h, in, (uint8_t*)dx) != hipSuccess) return host_copy_failed(h, stats);
+  // labels of a staged size come with the run (the first half: the points, at
+  // most as many bytes as one piece, have been copied before its labels are)
+  const size_t with_run = h->stage && out[0].bytes < kStageDirect ? out[0].bytes : 0;
+  int rc = run_device(h, 1, dx, &n, p, dl, nullptr, stats, 0, nullptr, 0,
+                      with_run ? h->stage : nullptr);
+  if (rc != DCLUST_OK) {
+    (void)hipStreamSynchronize(h->stream);  // (the staged points may be in flight yet)
+    return rc;
+  }
+  if (pieces_from_device(h, out, (const uint8_t*)dl, with_run) != hipSuccess)
+    return host_copy_failed(h, stats);
   return DCLUST_OK;
 }
 
@@ -1274,24 +1422,17 @@ int dclust_run_batched(dclust_handle* h, int32_t count, const double* const* xyz
   double* dx = h->get<double>(S_XYZ, el, &herr);
   int32_t* dl = h->get<int32_t>(S_LABOUT, tot, &herr);
   if (!dx || !dl) return DCLUST_E_OOM;
-  int64_t e = 0;
-  for (int32_t i = 0; i < count; ++i) {
-    if (n[i] > 0 && hipMemcpyAsync(dx + e, xyz[i], sizeof(double) * n[i] * params[i].dim,
-                                   hipMemcpyHostToDevice, h->stream) != hipSuccess)
-      return DCLUST_E_HIP;
-    e += n[i] * params[i].dim;
-  }
+  std::vector<HostPiece> v(count);
+  for (int32_t i = 0; i < count; ++i)
+    v[i] = {(void*)xyz[i], sizeof(double) * (size_t)(n[i] * params[i].dim)};
+  if (pieces_to_device(h, v, (uint8_t*)dx) != hipSuccess) return host_copy_failed(h, stats);
   int rc = run_device(h, count, dx, n, params, dl, inst_err, stats);
-  if (rc != DCLUST_OK && !(inst_err && rc < 0 && rc != DCLUST_E_HIP && rc != DCLUST_E_OOM))
+  if (rc != DCLUST_OK && !(inst_err && rc < 0 && rc != DCLUST_E_HIP && rc != DCLUST_E_OOM)) {
+    (void)hipStreamSynchronize(h->stream);
     return rc;
-  int64_t o = 0;
-  for (int32_t i = 0; i < count; ++i) {
-    if (n[i] > 0 && hipMemcpyAsync(labels[i], dl + o, sizeof(int32_t) * n[i],
-                                   hipMemcpyDeviceToHost, h->stream) != hipSuccess)
-      return DCLUST_E_HIP;
-    o += n[i];
   }
-  if (hipStreamSynchronize(h->stream) != hipSuccess) return DCLUST_E_HIP;
+  for (int32_t i = 0; i < count; ++i) v[i] = {labels[i], sizeof(int32_t) * (size_t)n[i]};
+  if (pieces_from_device(h, v, (const uint8_t*)dl) != hipSuccess) return host_copy_failed(h, stats);
   return rc;
 }
 

@@ -280,13 +280,17 @@ class Handle:
         k = len(arrays)
         xs = [np.ascontiguousarray(a, dtype=np.float64) for a in arrays]
         ns = np.array([a.shape[0] for a in xs], dtype=np.int64)
-        ptrs = (C.c_void_p * k)(*[a.ctypes.data for a in xs])
-        labs = [np.empty(a.shape[0], dtype=np.int32) for a in xs]
-        lptr = (C.c_void_p * k)(*[a.ctypes.data for a in labs])
+        # the labels of all instances in one array, returned as its parts
+        ends = np.cumsum(ns)
+        lab = np.empty(int(ends[-1]) if k else 0, dtype=np.int32)
+        labs = [lab[e - n:e] for e, n in zip(ends.tolist(), ns.tolist())]
+        ptrs = np.array([a.__array_interface__["data"][0] for a in xs], dtype=np.uint64)
+        lptr = (lab.__array_interface__["data"][0] + 4 * (ends - ns)).astype(np.uint64)
         parr = (Params * k)(*params_list)
         errs = np.zeros(k, dtype=np.int32)
         st = Stats()
-        rc = _lib().dclust_run_batched(self._h, k, ptrs, ns.ctypes.data, parr, lptr,
+        rc = _lib().dclust_run_batched(self._h, k, ptrs.ctypes.data, ns.ctypes.data, parr,
+                                       lptr.ctypes.data,
                                        errs.ctypes.data, C.byref(st))
         if rc not in (OK,) and not (rc < 0 and np.any(errs != 0)):
             raise DclustError(rc, "dclust_run_batched")
