@@ -68,11 +68,13 @@ struct dclust_handle {
   bool gphases = false;            // it records every phase event
   bool greadback = false;          // it ends with the counters' copies to `pin`
   // pinned host copy of the control counters, their stripes added ([C_NCTL]),
-  // allocated with the handle (null: pageable copies)
+  // then the Io a replay reads; allocated with the handle (null: pageable
+  // copies, and a captured run serves one input and output only)
   long long* pin = nullptr;
   long long* pin_dev = nullptr;  // its device address
   bool cap_phases = false;         // (set while a capture runs)
   bool graph_broken = false;       // capture failed on this device: eager only
+  bool phases_broken = false;      // capture with phase events failed: such runs are eager
   bool graph_off = false;          // eager only (while autotuning)
   uint8_t* scratch = nullptr;      // this device's scratch array (no-allocation runs)
   // two pinned halves of kStageBytes each through which small host arrays go
@@ -122,7 +124,7 @@ enum Slot {
   S_G, S_ORIG, S_CORE, S_LABEL, S_PARENT, S_COMPMIN, S_PAIRS, S_Q0, S_Q1,
   S_KEYV, S_FLAG, S_RANK, S_SCAN, S_LABOUT, S_COREOUT, S_PAIRCNT, S_SEGPOS, S_LINES, S_AMASK,
   S_REC, S_RECN, S_CCOL, S_CCOMP, S_BORDERPTS, S_CORECELLS, S_TUNELAB, S_STAT, S_GLINES,
-  S_CZL, S_XOFF, S_OS_LABEL, S_OS_STATE, S_OS_SEEDS, S_OS_LEN, S_OS_CONTACT, S_OS_FIRST, S_ROWSFB
+  S_CZL, S_XROW, S_OS_LABEL, S_OS_STATE, S_OS_SEEDS, S_OS_LEN, S_OS_CONTACT, S_OS_FIRST, S_ROWSFB
 };
 
 // column table entries (8 bytes each) above which neighbour columns are found
@@ -423,8 +425,11 @@ RunShape pick_shape(dclust_handle* h, const dclust_params& p, int64_t n, bool f3
   return r;
 }
 
+bool phase_times_requested();
+
 bool graph_enabled(const dclust_handle* h) {
   if (h->graph_off || h->graph_broken) return false;
+  if (h->phases_broken && phase_times_requested()) return false;
   const char* e = std::getenv("DCLUST_GRAPH");
   return !(e && e[0] == '0');
 }
@@ -440,21 +445,22 @@ void drop_graph(dclust_handle* h) {
 }
 
 // Phase times of a replay: each event recorded inside a graph is a node that
-// leaves the device idle for about 5.5 us.  The run's start and end events
-// are recorded on the stream around the graph launch, outside the graph; a
-// captured run holds only the two events of the neighbour-count kernel,
-// unless the environment variable DCLUST_PHASE_TIMES=1 asks for every phase.
+// leaves the device idle for about 5.5 us (and not every runtime can capture
+// one).  The run's start and end events are recorded on the stream around
+// the graph launch, outside the graph; the index and neighbour-count times
+// come from the device clock (C_T_*); the graph records events only when the
+// environment variable DCLUST_PHASE_TIMES=1 asks for every phase.
 bool phase_times_requested() {
   const char* e = std::getenv("DCLUST_PHASE_TIMES");
   return e && e[0] == '1';
 }
 bool outside_graph(int e) { return e == E_START || e == E_END; }
-bool always_in_graph(int e) { return e == E_CORE0 || e == E_CORE; }
 
-// Everything a launch sequence depends on besides the coordinates: the
-// device state (sizes, buffer and input/output pointers, switches), the
-// launch shape, the precision form and the instance and chunk tables.
-std::vector<uint8_t> launch_signature(const Dev& d, const RunShape& r, bool f32,
+// Everything a launch sequence depends on besides the input and output: the
+// device state (sizes, buffer pointers, switches), the launch shape, the
+// precision form and the instance and chunk tables.
+std::vector<uint8_t> launch_signature(const dclust_handle* h, const Dev& d, const Io& io,
+                                      const RunShape& r, bool f32,
                                       const std::vector<Inst>& inst,
                                       const std::vector<Chunk>& chunks) {
   std::vector<uint8_t> v;
@@ -463,6 +469,7 @@ std::vector<uint8_t> launch_signature(const Dev& d, const RunShape& r, bool f32,
     v.insert(v.end(), b, b + nb);
   };
   put(&d, sizeof(d));
+  if (!h->pin) put(&io, sizeof(io));  // (captured by value)
   const int64_t sh[9] = {r.seeds,    r.threads, r.blocks,  r.waves,
                          r.pair_per, r.budget,  r.pair_cap, f32 ? 1 : 0,
                          phase_times_requested() ? 1 : 0};
@@ -474,7 +481,7 @@ std::vector<uint8_t> launch_signature(const Dev& d, const RunShape& r, bool f32,
 
 // Phase event; inside a stream capture it becomes a node of the graph.
 hipError_t mark(dclust_handle* h, int e, bool graph, hipStream_t s = nullptr) {
-  if (graph && (outside_graph(e) || (!h->cap_phases && !always_in_graph(e)))) return hipSuccess;
+  if (graph && (outside_graph(e) || !h->cap_phases)) return hipSuccess;
   if (!s) s = h->stream;
   return graph ? hipEventRecordWithFlags(h->ev[e], s, hipEventRecordExternal)
                : hipEventRecord(h->ev[e], s);
@@ -496,8 +503,8 @@ hipError_t enqueue_index(dclust_handle* h, const Dev& d, int64_t n, int nchunks,
 }
 
 // counters, bounding boxes, grid set-up
-void enqueue_head(const Dev& d, int nchunks, hipStream_t s) {
-  launch_init_head(d, s);
+void enqueue_head(const Dev& d, const Io* src, const Io& io, int nchunks, hipStream_t s) {
+  launch_init_head(d, src, io, s);
   launch_index_head(d, nchunks, s);
 }
 
@@ -561,7 +568,7 @@ hipError_t enqueue_readback(dclust_handle* h, const Dev& d, hipStream_t s) {
 // `sort_passes` radix passes (the key width of the previous run; a wider key
 // abandons the run on the device) and `passes` expansion passes (a pass with
 // nothing pending exits at once).
-hipError_t capture_run(dclust_handle* h, const Dev& d, const RunShape& shape, bool f32,
+hipError_t capture_run(dclust_handle* h, const Dev& d, const Io& io, const RunShape& shape, bool f32,
                        int nchunks, int grid_cells, int sort_passes, int passes,
                        hipGraphExec_t* out) {
   const hipStream_t s = h->stream;
@@ -572,7 +579,7 @@ hipError_t capture_run(dclust_handle* h, const Dev& d, const RunShape& shape, bo
   // (the start and end events are recorded on the stream around each
   // launch, outside the graph: the start event is processed while the host
   // is still submitting the graph)
-  enqueue_head(d, nchunks, s);
+  enqueue_head(d, h->pin ? (const Io*)(h->pin_dev + C_NCTL) : nullptr, io, nchunks, s);
   hipError_t body = enqueue_index(h, d, d.n, nchunks, grid_cells, sort_passes, true);
   if (body == hipSuccess) body = enqueue_core(h, d, shape, f32, true);
   // work still pending after the last pass: the rest of the graph returns at
@@ -646,7 +653,9 @@ void finish_run(dclust_handle* h, const Dev& d, const RunShape& shape, const lon
   // a replay of a graph without the phase events reports those phases as 0
   const bool all_ev = !replayed || h->gphases;
   auto phase_ms = [&](int a, int b) { return all_ev ? (double)ev_ms(h, a, b) : 0.0; };
-  stats->t_index_ms = ev_ms(h, E_START, E_CORE0);
+  // (a replay's from the device clock)
+  auto clock_ms = [&](int a, int b) { return (double)(ctl_h[b] - ctl_h[a]) * 1e-3 / kClockMHz; };
+  stats->t_index_ms = replayed ? clock_ms(C_T_START, C_T_CORE0) : ev_ms(h, E_START, E_CORE0);
   stats->t_rows_ms = phase_ms(E_ROWS0, E_INDEX);
   stats->n_core_cells = ctl_h[C_NCORECELLS];
   stats->n_adj_points = ctl_h[C_NADJPTS];
@@ -655,7 +664,7 @@ void finish_run(dclust_handle* h, const Dev& d, const RunShape& shape, const lon
   stats->work[1] = ctl_h[C_CORE_RANGES];
   stats->work[2] = ctl_h[C_NCOREREST];
   stats->work[3] = ctl_h[C_NCORECROWD];
-  stats->t_core_ms = ev_ms(h, E_CORE0, E_CORE);
+  stats->t_core_ms = replayed ? clock_ms(C_T_CORE0, C_T_CORE1) : ev_ms(h, E_CORE0, E_CORE);
   stats->t_adj_ms = phase_ms(E_CORE, E_ADJ);
   stats->t_expand_ms = phase_ms(E_ADJ, E_EXPAND);
   stats->t_merge_ms = phase_ms(E_EXPAND, E_MERGE);
@@ -793,7 +802,7 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
   d.n = ntot;
   d.ninst = ninst;
   d.nchunks = nchunks;
-  d.xyz = d_xyz;
+  const Io io{d_xyz, d_labels};
   d.chains = shape.chains ? 1 : 0;
   // (without seed lists the expansion's buffers stay unused and minimal)
   d.pair_cap = shape.chains ? shape.pair_cap : 0;
@@ -860,7 +869,7 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
     if (!f32) {  // the FP32 form reads FP64 coordinates from the caller's rows
       d.X = M.get<double>(S_X, 3 * (size_t)ntot);
     } else {
-      d.xoff = M.get<int64_t>(S_XOFF, ntot);
+      d.xrow = M.get<const double*>(S_XROW, ntot);
     }
     d.G = M.get<uint32_t>(S_G, 3 * (size_t)ntot);
     d.orig = M.get<int32_t>(S_ORIG, ntot);
@@ -896,13 +905,11 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
       return DCLUST_E_OOM;
     }
   }
-  d.labels_out = d_labels;
-
   // A call whose launch state equals the previous call's (sizes, parameters,
   // pointers) is captured once into a graph and replayed from then on.
   std::vector<uint8_t> sig;
   const bool graph_on = !onestep && !fixed_mem && graph_enabled(h);
-  if (graph_on) sig = launch_signature(d, shape, f32, inst, chunks);
+  if (graph_on) sig = launch_signature(h, d, io, shape, f32, inst, chunks);
   // (a run in a fixed region leaves the handle's graph alone: destroying it
   // would free memory)
   if (!fixed_mem && h->gexec && (!graph_on || sig != h->gsig)) drop_graph(h);
@@ -920,7 +927,7 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
       const int gp = std::max(2, h->prev_npass + 1);
       hipGraphExec_t ge = nullptr;
       const int sp = std::max(1, std::min(kMaxPasses, h->prev_sort_passes));
-      if (capture_run(h, dg, shape, f32, nchunks, grid_cells, sp, gp, &ge) == hipSuccess) {
+      if (capture_run(h, dg, io, shape, f32, nchunks, grid_cells, sp, gp, &ge) == hipSuccess) {
         h->gexec = ge;
         h->gsig = sig;
         h->gpasses = gp;
@@ -928,7 +935,11 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
         h->greadback = h->pin != nullptr;
       } else {
         (void)hipGetLastError();
-        h->graph_broken = true;  // capture unsupported here: stay eager
+        // capture (of events) unsupported here: stay eager
+        if (h->cap_phases)
+          h->phases_broken = true;
+        else
+          h->graph_broken = true;
       }
     }
   }
@@ -965,6 +976,7 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
     };
     if (h->gexec && !fixed_mem) {
       HIPCHK(upload());
+      if (h->pin) std::memcpy(h->pin + C_NCTL, &io, sizeof(io));
       HIPCHK(hipEventRecord(h->ev[E_START], s));
       HIPCHK(hipGraphLaunch(h->gexec, s));
       HIPCHK(hipEventRecord(h->ev[E_END], s));  // (after the counters' readback)
@@ -989,7 +1001,7 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
     int npass = 0;
     HIPCHK(upload());
     HIPCHK(mark(h, E_START, false));
-    enqueue_head(d, nchunks, s);
+    enqueue_head(d, nullptr, io, nchunks, s);
     HIPCHK(hipMemcpyAsync(ctl_h, d.ctl, sizeof(ctl_h), hipMemcpyDeviceToHost, s));
     HIPCHK(hipStreamSynchronize(s));
     // more cells than the 63-bit sort key holds, over all instances
@@ -1297,8 +1309,8 @@ int dclust_create(dclust_handle** out, int device) {
       return DCLUST_E_HIP;
     }
   // coherent and mapped: the readback kernel's stores are visible to the
-  // host once the stream has drained
-  if (hipHostMalloc((void**)&h->pin, sizeof(long long) * C_NCTL,
+  // host once the stream has drained, the host's Io to the run's first kernel
+  if (hipHostMalloc((void**)&h->pin, sizeof(long long) * C_NCTL + sizeof(Io),
                     hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
       hipHostGetDevicePointer((void**)&h->pin_dev, h->pin, 0) != hipSuccess) {
     (void)hipGetLastError();

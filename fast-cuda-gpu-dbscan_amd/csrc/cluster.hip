@@ -287,6 +287,7 @@ __device__ int core_near(const Dev& d, const Par& P, int32_t p, int32_t c, int32
 template <bool F32>
 __global__ __launch_bounds__(256, F32 ? 8 : 6) void k_core(Dev d) {
   if (abandoned(d)) return;
+  stamp(d, C_T_CORE0);
   __shared__ int2 s_queue[4 * 256];
   const int64_t pl = (int64_t)xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
   const bool act = pl < d.n;
@@ -540,6 +541,7 @@ constexpr uint32_t kNoRep = 0xffffffffu;
 
 __global__ __launch_bounds__(1024) void k_rep(Dev d) {
   if (abandoned(d)) return;
+  stamp(d, C_T_CORE1);
   const int64_t C = d.ctl[C_NCELL];
   const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (c - threadIdx.x >= C) return;  // (block-uniform)
@@ -1571,8 +1573,8 @@ __global__ __launch_bounds__(256) void k_expand(Dev d, int pass, int S, int budg
     wave_sync();
   }
   if (lane == 0) {
-    // 100 MHz constant clock -> microseconds of this wave's life
-    const unsigned long long us = (__builtin_amdgcn_s_memrealtime() - t_begin) / 100ull;
+    // device clock -> microseconds of this wave's life
+    const unsigned long long us = (__builtin_amdgcn_s_memrealtime() - t_begin) / kClockMHz;
     d.pair_cnt[gw] = pc;
     d.seg_pos[gw] = seg;
     if (seg < seg_end) atomicAdd((unsigned long long*)&d.ctl[C_SEGS_LEFT], 1ull);
@@ -1999,6 +2001,7 @@ __global__ __launch_bounds__(RK_T) void k_rank_write(Dev d) {
 
 __global__ __launch_bounds__(256) void k_output(Dev d) {
   if (abandoned(d)) return;
+  int32_t* labels = out_labels(d);
   long long noise = 0;
   for (int64_t i0 = blockIdx.x * (int64_t)(kRelU * 256); i0 < d.n;
        i0 += (int64_t)gridDim.x * (kRelU * 256)) {
@@ -2022,7 +2025,7 @@ __global__ __launch_bounds__(256) void k_output(Dev d) {
       const int64_t i = i0 + u * 256 + threadIdx.x;
       if (i < d.n) {
         const int32_t lab = k[u] == kNoKey ? 0 : rk[u] - rb[u] + 1;
-        d.labels_out[o[u]] = lab;
+        labels[o[u]] = lab;
         noise += lab == 0;
       }
     }

@@ -37,7 +37,10 @@ static int fill_grid(int64_t n) {
 // pass flags and the bounding-box stripes (per instance and stripe: 0..2 min
 // as ordered keys starting at the largest key, 3..5 max, 6 max |x|, 7
 // non-finite flag, all starting at 0).
-__global__ void k_init_head(Dev d) {
+// The call's input and output go into the control block: from `src` (pinned
+// host memory) in a captured run, whose replays read what the host left there,
+// else from `v`.
+__global__ void k_init_head(Dev d, const Io* src, Io v) {
   const int64_t nb = (int64_t)d.ninst * kBoxStripes * 8;
   const int64_t ns = (int64_t)kStatStride * kStripes;
   const int64_t tot = nb + ns + C_NCTL + kMaxPasses + d.ninst;
@@ -48,7 +51,14 @@ __global__ void k_init_head(Dev d) {
     else if (i < nb + ns)
       d.stat[i - nb] = 0;
     else if (i < nb + ns + C_NCTL)
-      d.ctl[i - nb - ns] = 0;
+      {
+        const int c = (int)(i - nb - ns);
+        long long w = 0;
+        if (c == C_XYZ) w = reinterpret_cast<long long>(src ? src->xyz : v.xyz);
+        if (c == C_LABELS) w = reinterpret_cast<long long>(src ? src->labels : v.labels);
+        if (c == C_T_START) w = (long long)__builtin_amdgcn_s_memrealtime();
+        d.ctl[c] = w;
+      }
     else if (i < nb + ns + C_NCTL + kMaxPasses)
       d.pass_scatter[i - nb - ns - C_NCTL] = 0;
     else
@@ -56,10 +66,10 @@ __global__ void k_init_head(Dev d) {
   }
 }
 
-void launch_init_head(const Dev& d, hipStream_t s) {
+void launch_init_head(const Dev& d, const Io* src, const Io& v, hipStream_t s) {
   const int64_t tot = (int64_t)d.ninst * kBoxStripes * 8 + (int64_t)kStatStride * kStripes + C_NCTL +
                       kMaxPasses + d.ninst;
-  hipLaunchKernelGGL(k_init_head, dim3(fill_grid(tot)), dim3(256), 0, s, d);
+  hipLaunchKernelGGL(k_init_head, dim3(fill_grid(tot)), dim3(256), 0, s, d, src, v);
 }
 
 // End of a run: the control counters, their stripes added, into a host buffer
@@ -128,7 +138,7 @@ __global__ __launch_bounds__(256) void k_bbox(Dev d) {
   double mx[3] = {-INFINITY, -INFINITY, -INFINITY};
   double ma = 0.0;
   bool bad = false;
-  const double* p0 = d.xyz + I.xyz_off + (ch.begin - I.pt_begin) * dim;
+  const double* p0 = in_xyz(d) + I.xyz_off + (ch.begin - I.pt_begin) * dim;
   if (dim == 3)
     bbox_points<3>(p0, ch.end - ch.begin, mn, mx, ma, bad);
   else
@@ -374,7 +384,7 @@ __device__ __forceinline__ int32_t cell_index(double x, const Inst& I, int k) {
 
 template <int D, bool K32>
 __device__ __forceinline__ void cellkey_points(const Dev& d, const Inst& I, const Chunk& ch) {
-  const double* p0 = d.xyz + I.xyz_off + (ch.begin - I.pt_begin) * D;
+  const double* p0 = in_xyz(d) + I.xyz_off + (ch.begin - I.pt_begin) * D;
   const int64_t np = ch.end - ch.begin;
   for (int64_t i0 = threadIdx.x; i0 < np; i0 += kChunkU * 256) {
     double v[kChunkU][D];
@@ -811,9 +821,10 @@ __global__ __launch_bounds__(CS_T) void k_csr_write(Dev d) {
 // could alias the row as far as the compiler knows, which would otherwise
 // hold each coordinate's random-access load until the previous store).
 template <int D>
-__device__ __forceinline__ void gather_point(const Dev& d, const Inst& I, int64_t i, int32_t src) {
+__device__ __forceinline__ void gather_point(const Dev& d, const Inst& I, const double* xyz,
+                                             int64_t i, int32_t src) {
   const int64_t off = I.xyz_off + ((int64_t)src - I.pt_begin) * D;
-  const double* p = d.xyz + off;
+  const double* p = xyz + off;
   double x[D], mn[D];
 #pragma unroll
   for (int k = 0; k < D; ++k) {
@@ -821,7 +832,7 @@ __device__ __forceinline__ void gather_point(const Dev& d, const Inst& I, int64_
     mn[k] = I.mn[k];
   }
   const double inv_w = I.inv_w;
-  if (!d.X) d.xoff[i] = off;  // the FP32 form's way back to FP64 rows
+  if (!d.X) d.xrow[i] = p;  // the FP32 form's way back to FP64 rows
 #pragma unroll
   for (int k = 0; k < D; ++k) {
     if (d.X) d.X[3 * i + k] = x[k];  // the FP64 form's sorted copy
@@ -835,14 +846,15 @@ __device__ __forceinline__ void gather_point(const Dev& d, const Inst& I, int64_
 __global__ __launch_bounds__(256) void k_gather(Dev d) {
   if (abandoned(d)) return;
   const int32_t* vsrc = d.val[sort_parity(d, kMaxPasses)];
+  const double* xyz = in_xyz(d);
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < d.n;
        i += (int64_t)gridDim.x * blockDim.x) {
     const int32_t src = vsrc[i];
     const Inst& I = *inst_of_cell(d, d.ninst == 1 ? 0 : d.cell_of[i]);
     if (I.dim == 3)
-      gather_point<3>(d, I, i, src);
+      gather_point<3>(d, I, xyz, i, src);
     else
-      gather_point<2>(d, I, i, src);
+      gather_point<2>(d, I, xyz, i, src);
   }
 }
 

@@ -219,9 +219,17 @@ enum Ctl : int {
   C_NROOTS,       // near components (listed in Dev::near_roots)
   C_NFARLIGHT,    // pairs across components (listed in Dev::far_light)
   C_NFARHEAVY,    // those with a heavy cell (listed in Dev::far_heavy)
+  // this call's input and output (addresses), written by the run's first kernel
+  C_XYZ,
+  C_LABELS,
+  // device clock (kClockMHz) at the start of the run, of the neighbour counts
+  // and of what follows them
+  C_T_START,
+  C_T_CORE0,
+  C_T_CORE1,
   C_NCTL
 };
-static_assert(C_NFARHEAVY < C_NCTL, "control block too small");
+static_assert(C_T_CORE1 < C_NCTL, "control block too small");
 
 // Cell-key space: the sort key of a cell is its instance's key base plus its
 // place in the cell order, and the
@@ -279,12 +287,21 @@ constexpr int kMaxPasses = 8;
 // the grid set-up reduces the stripes.
 constexpr int kBoxStripes = 32;
 
+// Input and output of a call.  They reach the kernels through the control
+// block, not through Dev: a captured run is replayed for calls with other
+// buffers.
+struct Io {
+  const double* xyz;
+  int32_t* labels;
+};
+
+constexpr int kClockMHz = 100;  // of the constant device clock
+
 // All device pointers of one run, passed to kernels by value.
 struct Dev {
   int64_t n;
   int32_t ninst;
   int32_t nchunks;
-  const double* xyz;
   Inst* inst;
   const Chunk* chunks;
   unsigned long long* bbox;  // [ninst][kBoxStripes][8] ordered-u64 min0..2 max0..2,
@@ -331,7 +348,7 @@ struct Dev {
 
   // sorted point data
   double* X;            // [N][3] FP64 form only (null in the FP32 form)
-  int64_t* xoff;        // FP32 form: offset of each point's row in xyz
+  const double** xrow;  // FP32 form: each point's row of the input
   uint32_t* G;          // [N][3]
   int32_t* orig;
   uint8_t* core;
@@ -352,9 +369,7 @@ struct Dev {
   int32_t* rank;
   int64_t* scan_tmp;  // block sums for scans
 
-  // outputs (input order)
-  int32_t* labels_out;
-  uint8_t* core_out;
+  uint8_t* core_out;    // core flags in input order
 };
 
 // ------------------------------------------------------------ helpers ----
@@ -441,6 +456,17 @@ __device__ __forceinline__ void wave_add(long long* p, long long v) {
 
 // chain ids are seed cell indices: the id space is the cell count
 __device__ __forceinline__ long long chain_ids(const Dev& d) { return d.ctl[C_NCELL]; }
+
+__device__ __forceinline__ const double* in_xyz(const Dev& d) {
+  return reinterpret_cast<const double*>(d.ctl[C_XYZ]);
+}
+__device__ __forceinline__ int32_t* out_labels(const Dev& d) {
+  return reinterpret_cast<int32_t*>(d.ctl[C_LABELS]);
+}
+// the device clock, stamped by one thread of the launch
+__device__ __forceinline__ void stamp(const Dev& d, int ctr) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) d.ctl[ctr] = (long long)__builtin_amdgcn_s_memrealtime();
+}
 
 // set when a run with a fixed number of expansion passes left work pending
 __device__ __forceinline__ bool abandoned(const Dev& d) { return d.ctl[C_ABANDON] != 0; }

@@ -5,7 +5,8 @@
 namespace dclust {
 
 // start of a run: control counters, statistics, radix pass flags, bbox
-void launch_init_head(const Dev& d, hipStream_t s);
+// (the call's input and output: read from `src` on the device, or `v` if null)
+void launch_init_head(const Dev& d, const Io* src, const Io& v, hipStream_t s);
 void launch_readback(const Dev& d, long long* out, hipStream_t s);
 // per-run state of the clustering phases (labels, forest, minima, flags,
 // per-cell core counts, per-wave pair counts)

@@ -9,11 +9,11 @@ namespace dclust {
 // ------------------------------------------------------------ predicates --
 // FP64 coordinates of cell-sorted point i.  The FP32 form keeps no sorted
 // FP64 copy (only its guard-band rechecks need FP64): they are read from
-// the caller's rows at the point's row offset.
+// the caller's rows.
 template <int D, bool F32>
 __device__ __forceinline__ void load_x(const Dev& d, int32_t i, double* x) {
   if constexpr (F32) {
-    const double* p = d.xyz + d.xoff[i];
+    const double* p = d.xrow[i];
 #pragma unroll
     for (int k = 0; k < D; ++k) x[k] = p[k];
   } else {
