@@ -28,7 +28,6 @@ using namespace dclust;
 
 namespace {
 
-constexpr int64_t kChunk = 4096;  // points per chunk of bbox / cell-key blocks
 constexpr int kMaxExpandPasses = 100000;
 
 struct Buf {
@@ -68,8 +67,8 @@ struct dclust_handle {
   bool gphases = false;            // it records every phase event
   bool greadback = false;          // it ends with the counters' copies to `pin`
   // pinned host copy of the control counters, their stripes added ([C_NCTL]),
-  // then the Io a replay reads; allocated with the handle (null: pageable
-  // copies, and a captured run serves one input and output only)
+  // then the Call a replay reads; allocated with the handle (null: pageable
+  // copies, and a captured run serves one input, output and parameters only)
   long long* pin = nullptr;
   long long* pin_dev = nullptr;  // its device address
   bool cap_phases = false;         // (set while a capture runs)
@@ -127,9 +126,6 @@ enum Slot {
   S_CZL, S_XROW, S_OS_LABEL, S_OS_STATE, S_OS_SEEDS, S_OS_LEN, S_OS_CONTACT, S_OS_FIRST, S_ROWSFB
 };
 
-// column table entries (8 bytes each) above which neighbour columns are found
-// by binary search instead
-constexpr long long kMaxLineTable = 1LL << 26;  // 512 MiB at most
 // expansion passes a captured run may hold; runs that need more stay eager
 constexpr int kGraphMaxPasses = 8;
 
@@ -456,26 +452,29 @@ bool phase_times_requested() {
 }
 bool outside_graph(int e) { return e == E_START || e == E_END; }
 
-// Everything a launch sequence depends on besides the input and output: the
-// device state (sizes, buffer pointers, switches), the launch shape, the
-// precision form and the instance and chunk tables.
-std::vector<uint8_t> launch_signature(const dclust_handle* h, const Dev& d, const Io& io,
+// Everything a launch sequence depends on: the device state (sizes, buffer
+// pointers, switches), the launch shape, the precision form and the instances'
+// dimensions and sizes.  Not the input and output, nor eps, minpts (beyond the
+// record slots in the device state) and r: the kernels read those from memory
+// that each call fills.
+std::vector<uint8_t> launch_signature(const dclust_handle* h, const Dev& d, const Call& call,
                                       const RunShape& r, bool f32,
-                                      const std::vector<Inst>& inst,
-                                      const std::vector<Chunk>& chunks) {
+                                      const std::vector<Inst>& inst) {
   std::vector<uint8_t> v;
   auto put = [&v](const void* p, size_t nb) {
     const uint8_t* b = (const uint8_t*)p;
     v.insert(v.end(), b, b + nb);
   };
   put(&d, sizeof(d));
-  if (!h->pin) put(&io, sizeof(io));  // (captured by value)
+  if (!h->pin) put(&call, sizeof(call));  // (captured by value)
   const int64_t sh[9] = {r.seeds,    r.threads, r.blocks,  r.waves,
                          r.pair_per, r.budget,  r.pair_cap, f32 ? 1 : 0,
                          phase_times_requested() ? 1 : 0};
   put(sh, sizeof(sh));
-  put(inst.data(), sizeof(Inst) * inst.size());
-  put(chunks.data(), sizeof(Chunk) * chunks.size());
+  for (const Inst& I : inst) {
+    const int64_t w[2] = {I.dim, I.pt_end - I.pt_begin};
+    put(w, sizeof(w));
+  }
   return v;
 }
 
@@ -491,30 +490,27 @@ hipError_t mark(dclust_handle* h, int e, bool graph, hipStream_t s = nullptr) {
 // stream: the gather fills the device, so running the rows beside it gains
 // nothing).
 hipError_t enqueue_index(dclust_handle* h, const Dev& d, int64_t n, int nchunks, int grid_cells,
-                         int passes, bool graph) {
+                         int passes, int64_t waves, bool graph) {
   const hipStream_t s = h->stream;
   hipError_t e;
   launch_index_sort(d, n, nchunks, passes, h->num_cu, s);
-  launch_gather(d, n, s);
-  launch_lines(d, grid_cells, s);
+  launch_gather(d, n, waves, s);
   if ((e = mark(h, E_ROWS0, graph)) != hipSuccess) return e;
   launch_rows(d, n, grid_cells, s);
   return hipSuccess;
 }
 
 // counters, bounding boxes, grid set-up
-void enqueue_head(const Dev& d, const Io* src, const Io& io, int nchunks, hipStream_t s) {
-  launch_init_head(d, src, io, s);
+void enqueue_head(const Dev& d, const Call* src, const Call& call, int nchunks, hipStream_t s) {
+  launch_init_head(d, src, call, s);
   launch_index_head(d, nchunks, s);
 }
 
-// per-cell state, core flags, near graph, seeding segments
-hipError_t enqueue_core(dclust_handle* h, const Dev& d, const RunShape& shape, bool f32,
-                        bool graph) {
+// core flags, near graph
+hipError_t enqueue_core(dclust_handle* h, const Dev& d, bool f32, bool graph) {
   const hipStream_t s = h->stream;
   hipError_t e;
   if ((e = mark(h, E_INDEX, graph)) != hipSuccess) return e;
-  launch_init_run(d, shape.chains ? shape.waves : 0, s);
   // the core (neighbour-count) kernel is bracketed by its own events
   if ((e = mark(h, E_CORE0, graph)) != hipSuccess) return e;
   launch_core(d, f32, s);
@@ -568,7 +564,8 @@ hipError_t enqueue_readback(dclust_handle* h, const Dev& d, hipStream_t s) {
 // `sort_passes` radix passes (the key width of the previous run; a wider key
 // abandons the run on the device) and `passes` expansion passes (a pass with
 // nothing pending exits at once).
-hipError_t capture_run(dclust_handle* h, const Dev& d, const Io& io, const RunShape& shape, bool f32,
+hipError_t capture_run(dclust_handle* h, const Dev& d, const Call& call, const RunShape& shape,
+                       bool f32,
                        int nchunks, int grid_cells, int sort_passes, int passes,
                        hipGraphExec_t* out) {
   const hipStream_t s = h->stream;
@@ -579,9 +576,10 @@ hipError_t capture_run(dclust_handle* h, const Dev& d, const Io& io, const RunSh
   // (the start and end events are recorded on the stream around each
   // launch, outside the graph: the start event is processed while the host
   // is still submitting the graph)
-  enqueue_head(d, h->pin ? (const Io*)(h->pin_dev + C_NCTL) : nullptr, io, nchunks, s);
-  hipError_t body = enqueue_index(h, d, d.n, nchunks, grid_cells, sort_passes, true);
-  if (body == hipSuccess) body = enqueue_core(h, d, shape, f32, true);
+  enqueue_head(d, h->pin ? (const Call*)(h->pin_dev + C_NCTL) : nullptr, call, nchunks, s);
+  hipError_t body = enqueue_index(h, d, d.n, nchunks, grid_cells, sort_passes,
+                                  shape.chains ? shape.waves : 0, true);
+  if (body == hipSuccess) body = enqueue_core(h, d, f32, true);
   // work still pending after the last pass: the rest of the graph returns at
   // once and the host runs the call eagerly
   if (body == hipSuccess && !d.chains) body = enqueue_link(h, d, true);
@@ -765,7 +763,7 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
     I.pt_begin = ntot;
     I.pt_end = ntot + n[i];
     I.xyz_off = off;
-    for (int64_t b = 0; b < n[i]; b += kChunk) {
+    for (int64_t b = 0; ninst > 1 && b < n[i]; b += kChunk) {
       Chunk ch;
       ch.inst = i;
       ch.pad = 0;
@@ -793,7 +791,8 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
     shape.pair_cap = (int64_t)shape.pair_per * shape.waves;
   }
   if (onestep) shape.chains = false;  // (its own loop runs instead)
-  const int nchunks = (int)chunks.size();
+  // (one instance's chunks are computed on the device)
+  const int nchunks = ninst > 1 ? (int)chunks.size() : (int)((ntot + kChunk - 1) / kChunk);
   const int grid_cells = h->num_cu * 8;
   const hipStream_t s = h->stream;
 
@@ -802,7 +801,7 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
   d.n = ntot;
   d.ninst = ninst;
   d.nchunks = nchunks;
-  const Io io{d_xyz, d_labels};
+  const Call call{d_xyz, d_labels, inst[0]};
   d.chains = shape.chains ? 1 : 0;
   // (without seed lists the expansion's buffers stay unused and minimal)
   d.pair_cap = shape.chains ? shape.pair_cap : 0;
@@ -819,13 +818,15 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
   // asymmetric); up to kRecSlots are kept, a longer record is rescanned
   int rec_stride = 0;
   for (int32_t i = 0; i < ninst; ++i) rec_stride = std::max(rec_stride, params[i].minpts);
-  rec_stride = std::min(rec_stride, fixed_mem ? kRecSlotsFixed : kRecSlots);
+  // (in eights in the arena: calls of similar minpts share a captured run)
+  rec_stride = fixed_mem ? std::min(rec_stride, kRecSlotsFixed)
+                         : (std::min(rec_stride, kRecSlots) + 7) & ~7;
   d.rec_stride = rec_stride;
   RunMem mem{h, region, region_cap};
   {
     RunMem& M = mem;
     d.inst = M.get<Inst>(S_INST, ninst);
-    d.chunks = M.get<Chunk>(S_CHUNK, nchunks);
+    d.chunks = M.get<Chunk>(S_CHUNK, ninst > 1 ? nchunks : 0);
     d.bbox = M.get<unsigned long long>(S_BBOX, (size_t)ninst * kBoxStripes * 8);
     d.ctl = M.get<long long>(S_CTL, C_NCTL);
     d.stat = M.get<long long>(S_STAT, (size_t)kStatStride * kStripes);
@@ -879,7 +880,9 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
     d.rec_n = M.get<uint8_t>(S_RECN, ntot);
     if (rec_stride > 0) d.rec = M.get<int32_t>(S_REC, (size_t)ntot * rec_stride);
     d.parent = M.get<int32_t>(S_PARENT, ntot);
-    d.compmin = M.get<int32_t>(S_COMPMIN, ntot);
+    // the component minima, before them the list of points with many candidates
+    d.compmin = M.get<int32_t>(S_COMPMIN, (size_t)std::max(ntot, cap_n * kStripes));
+    d.core_crowd = SList{d.compmin, (unsigned long long*)(d.stat + C_NCORECROWD), cap_n};
     const int64_t waves = shape.chains ? shape.waves : 0;
     d.pairs = M.get<int2>(S_PAIRS, d.pair_cap);
     d.pair_cnt = M.get<int32_t>(S_PAIRCNT, waves);
@@ -893,10 +896,8 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
     // leaves
     d.keyv = M.get<int32_t>(S_KEYV, (size_t)std::max(ntot, cap_p * kStripes));
     d.core_rest = SList{d.keyv, (unsigned long long*)(d.stat + C_NCOREREST), cap_p};
-    d.flag = M.get<uint8_t>(S_FLAG, ntot);
-    // the ranks, before them the list of points with many candidates
-    d.rank = M.get<int32_t>(S_RANK, (size_t)std::max(ntot + 1, cap_n * kStripes));
-    d.core_crowd = SList{d.rank, (unsigned long long*)(d.stat + C_NCORECROWD), cap_n};
+    d.flag = M.get<unsigned long long>(S_FLAG, ntot / 64 + 1);
+    d.rank = M.get<int32_t>(S_RANK, ntot / 64 + 1);
     d.scan_tmp = M.get<int64_t>(S_SCAN, scan_tmp_entries(ntot));
     d.core_out = M.get<uint8_t>(S_COREOUT, ntot);
     if (mem.over) return DCLUST_E_CAPACITY;  // the fixed region is too small
@@ -905,21 +906,22 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
       return DCLUST_E_OOM;
     }
   }
-  // A call whose launch state equals the previous call's (sizes, parameters,
-  // pointers) is captured once into a graph and replayed from then on.
+  // A call whose launch state equals the previous call's (dimensions, sizes,
+  // launch shape) is captured once into a graph and replayed from then on.
   std::vector<uint8_t> sig;
   const bool graph_on = !onestep && !fixed_mem && graph_enabled(h);
-  if (graph_on) sig = launch_signature(h, d, io, shape, f32, inst, chunks);
+  if (graph_on) sig = launch_signature(h, d, call, shape, f32, inst);
   // (a run in a fixed region leaves the handle's graph alone: destroying it
   // would free memory)
   if (!fixed_mem && h->gexec && (!graph_on || sig != h->gsig)) drop_graph(h);
   if (graph_on && !h->gexec && !h->prev_sig.empty() && sig == h->prev_sig &&
       h->prev_npass < kGraphMaxPasses) {
     Dev dg = d;
-    // line table sized from the previous run; a larger line count falls back
-    // to the binary search on the device
-    const long long cap = std::min<long long>(
-        kMaxLineTable, std::max<long long>(h->prev_nlines + h->prev_nlines / 4, 1024));
+    // column table and radix passes sized from the runs of this launch state
+    // so far; a call that needs more (a smaller eps) abandons the replay on
+    // the device, runs eagerly and is captured with the larger sizes
+    const long long cap =
+        std::min<long long>(kMaxLineTable, std::max<long long>(2 * h->prev_nlines, 1 << 16));
     hipError_t ae = hipSuccess;
     dg.lines = h->get<int2>(S_GLINES, (size_t)cap, &ae);
     if (dg.lines) {
@@ -927,7 +929,7 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
       const int gp = std::max(2, h->prev_npass + 1);
       hipGraphExec_t ge = nullptr;
       const int sp = std::max(1, std::min(kMaxPasses, h->prev_sort_passes));
-      if (capture_run(h, dg, io, shape, f32, nchunks, grid_cells, sp, gp, &ge) == hipSuccess) {
+      if (capture_run(h, dg, call, shape, f32, nchunks, grid_cells, sp, gp, &ge) == hipSuccess) {
         h->gexec = ge;
         h->gsig = sig;
         h->gpasses = gp;
@@ -946,12 +948,17 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
 
   {
     long long ctl_h[C_NCTL];
-    // the host-built instance table and chunk list (the kernels rewrite only
-    // derived fields of the table, and k_init_head clears its error codes)
-    std::vector<uint8_t> up(sizeof(Inst) * ninst + sizeof(Chunk) * nchunks);
-    std::memcpy(up.data(), inst.data(), sizeof(Inst) * ninst);
-    std::memcpy(up.data() + sizeof(Inst) * ninst, chunks.data(), sizeof(Chunk) * nchunks);
+    // the host-built instance table and chunk list of a batch (the kernels
+    // rewrite only derived fields of the table, and k_init_head clears its
+    // error codes; a single instance comes with the first kernel)
     auto upload = [&]() -> hipError_t {
+      if (ninst == 1) {
+        h->up_bytes.clear();  // (the arena's table is overwritten)
+        return hipSuccess;
+      }
+      std::vector<uint8_t> up(sizeof(Inst) * ninst + sizeof(Chunk) * nchunks);
+      std::memcpy(up.data(), inst.data(), sizeof(Inst) * ninst);
+      std::memcpy(up.data() + sizeof(Inst) * ninst, chunks.data(), sizeof(Chunk) * nchunks);
       if (!fixed_mem && up == h->up_bytes && h->up_inst == d.inst && h->up_chunks == d.chunks)
         return hipSuccess;
       hipError_t ue =
@@ -963,7 +970,7 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
         h->up_bytes.clear();  // (a fixed region is not the arena)
         h->up_inst = h->up_chunks = nullptr;
       } else {
-        h->up_bytes = up;
+        h->up_bytes.swap(up);
         h->up_inst = d.inst;
         h->up_chunks = d.chunks;
       }
@@ -976,7 +983,7 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
     };
     if (h->gexec && !fixed_mem) {
       HIPCHK(upload());
-      if (h->pin) std::memcpy(h->pin + C_NCTL, &io, sizeof(io));
+      if (h->pin) std::memcpy(h->pin + C_NCTL, &call, sizeof(call));
       HIPCHK(hipEventRecord(h->ev[E_START], s));
       HIPCHK(hipGraphLaunch(h->gexec, s));
       HIPCHK(hipEventRecord(h->ev[E_END], s));  // (after the counters' readback)
@@ -993,15 +1000,15 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
                    true, stats);
         return rc;
       }
-      // the expansion needed more passes than the graph holds: run eagerly
-      // (the next identical call captures a graph with more passes)
+      // more expansion or radix passes or columns than the graph holds: run
+      // eagerly (the next call of this launch state captures a larger one)
       drop_graph(h);
     }
 
     int npass = 0;
     HIPCHK(upload());
     HIPCHK(mark(h, E_START, false));
-    enqueue_head(d, nullptr, io, nchunks, s);
+    enqueue_head(d, nullptr, call, nchunks, s);
     HIPCHK(hipMemcpyAsync(ctl_h, d.ctl, sizeof(ctl_h), hipMemcpyDeviceToHost, s));
     HIPCHK(hipStreamSynchronize(s));
     // more cells than the 63-bit sort key holds, over all instances
@@ -1032,12 +1039,13 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
       // (a fixed region without room for the table: the rows are found by
       // binary search over the cell keys instead)
     }
-    HIPCHK(enqueue_index(h, d, ntot, nchunks, grid_cells, passes, false));
+    HIPCHK(enqueue_index(h, d, ntot, nchunks, grid_cells, passes, shape.chains ? shape.waves : 0,
+                         false));
     if (onestep) {
       HIPCHK(mark(h, E_INDEX, false));
       return onestep_loop(h, d, params[0], onestep_threads, d_labels, stats);
     }
-    HIPCHK(enqueue_core(h, d, shape, f32, false));
+    HIPCHK(enqueue_core(h, d, f32, false));
 
     // expansion passes until no seed is pending: pass p drains the queue of
     // pass p-1 (overflowed seed lists, lists left when a wave's pop budget
@@ -1057,10 +1065,13 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
     finish_run(h, d, shape, ctl_h, npass, false, stats);
     if (npass >= kMaxExpandPasses) return DCLUST_E_CAPACITY;
     if (graph_on) {
+      // (the largest of the calls that share a launch state, so that calls of
+      // alternating parameters settle on one graph)
+      const bool same = sig == h->prev_sig;
       h->prev_sig.swap(sig);
-      h->prev_npass = npass;
-      h->prev_nlines = nlines;
-      h->prev_sort_passes = passes;
+      h->prev_npass = same ? std::max(npass, h->prev_npass) : npass;
+      h->prev_nlines = same ? std::max(nlines, h->prev_nlines) : nlines;
+      h->prev_sort_passes = same ? std::max(passes, h->prev_sort_passes) : passes;
     }
     return rc;
   }
@@ -1309,8 +1320,8 @@ int dclust_create(dclust_handle** out, int device) {
       return DCLUST_E_HIP;
     }
   // coherent and mapped: the readback kernel's stores are visible to the
-  // host once the stream has drained, the host's Io to the run's first kernel
-  if (hipHostMalloc((void**)&h->pin, sizeof(long long) * C_NCTL + sizeof(Io),
+  // host once the stream has drained, the host's Call to the run's first kernel
+  if (hipHostMalloc((void**)&h->pin, sizeof(long long) * C_NCTL + sizeof(Call),
                     hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
       hipHostGetDevicePointer((void**)&h->pin_dev, h->pin, 0) != hipSuccess) {
     (void)hipGetLastError();

@@ -37,7 +37,7 @@
 //                matrix and thrust::replace relabels, dbscan.cu:60-125).
 //   k_comp, k_far, k_far_pairs   pairs of stencil cells in two components are
 //                decided exactly and united.
-//   k_flatten_all / k_roots_final / k_keys / k_border / rank scan / k_output
+//   k_roots_final / k_keys / k_border / rank scan / k_output
 //                canonical labels:
 //                cluster id = rank of the component's minimum core input
 //                index; border = minimum id over adjacent cores; noise = 0
@@ -1251,24 +1251,12 @@ __global__ __launch_bounds__(256, 4) void k_far_pairs(Dev d) {
   stat_add(d, C_FAR_JOINS, joins);
 }
 
-// Roots of the near components after the unions across their borders, in two
-// passes over the list of near roots (no other entry is a component id).
-// The first compresses the forest with path-halving walks; a concurrent walk
-// may leave an entry at an inner ancestor instead of the root, so the second
-// pass walks the (now shallow) forest without writing anything but each
-// near root's own entry, and moves its minimum core input index to its final
-// root: every entry is then exactly its root.
-__global__ __launch_bounds__(256) void k_flatten_all(Dev d) {
-  if (abandoned(d)) return;
-  __shared__ long long s_pre[kStripes + 1];
-  const long long n = slist_prefix(d.near_roots, s_pre);
-  for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n;
-       i += (long long)gridDim.x * 256) {
-    const int32_t c = slist_at(d.near_roots, s_pre, i);
-    d.parent[c] = uf_find(d.parent, c);
-  }
-}
-
+// Final roots of the near components (the only component ids) after the
+// unions across their borders, and their minima moved to them.  The walk
+// writes nothing but each near root's own entry: a path-halving write of
+// another thread's walk could otherwise replace a root that its owner has just
+// stored with an inner ancestor, and a later read of "the root" would get
+// that.  (uf_order keeps the walks short, so no compressing pass precedes.)
 __global__ __launch_bounds__(256) void k_roots_final(Dev d) {
   if (abandoned(d)) return;
   __shared__ long long s_pre[kStripes + 1];
@@ -1775,7 +1763,7 @@ __global__ __launch_bounds__(256) void k_keys(Dev d) {
       const int64_t i = i0 + u * 256 + threadIdx.x;
       if (i < d.n) {
         d.keyv[i] = cr[u] ? k[u] : kNoKey;
-        if (cr[u] && o[u] == k[u]) d.flag[k[u]] = 1;
+        if (cr[u] && o[u] == k[u]) atomicOr(&d.flag[k[u] >> 6], 1ull << (k[u] & 63));
       }
     }
   }
@@ -1940,28 +1928,24 @@ __global__ __launch_bounds__(256) void k_border(Dev d) {
 }
 
 // ------------------------------------------------------------ rank + out --
-// exclusive scan of the component-minimum flags (indexed by input index):
-// rank[k] = number of clusters whose minimum core index is below k.
+// Ranks of the clusters: the flags of their smallest core input indices are
+// bits, so rank(k) = the flags before k's word (a scan over N/64 words: small
+// enough to stay in L2 for the random reads of k_output, where one entry per
+// point was not) + the bits below k in its word.
 constexpr int RK_T = 256;
-constexpr int RK_I = 16;
-constexpr int RK_TILE = RK_T * RK_I;
-
-// component-minimum flag of input index i (false past the end); the load is
-// unconditional so that a thread's loads for all of its rounds overlap
-__device__ __forceinline__ bool rank_flag(const Dev& d, int64_t i) {
-  const uint8_t f = d.flag[i < d.n ? i : 0];
-  return i < d.n && f;
-}
+constexpr int RK_I = 4;
+constexpr int RK_TILE = RK_T * RK_I;  // words per workgroup
 
 __global__ __launch_bounds__(RK_T) void k_rank_count(Dev d) {
   if (abandoned(d)) return;
-  const int64_t t0 = (int64_t)blockIdx.x * RK_TILE;
-  bool f[RK_I];
-#pragma unroll
-  for (int r = 0; r < RK_I; ++r) f[r] = rank_flag(d, t0 + r * RK_T + threadIdx.x);
+  const int64_t nf = (d.n + 63) / 64, t0 = (int64_t)blockIdx.x * RK_TILE;
   int c = 0;
 #pragma unroll
-  for (int r = 0; r < RK_I; ++r) c += __popcll(ballot(f[r]));
+  for (int r = 0; r < RK_I; ++r) {
+    const int64_t i = t0 + r * RK_T + threadIdx.x;
+    if (i < nf) c += __popcll(d.flag[i]);
+  }
+  c = wave_sum(c);
   __shared__ int s[4];
   if (lane_id() == 0) s[threadIdx.x >> 6] = c;
   __syncthreads();
@@ -1970,33 +1954,41 @@ __global__ __launch_bounds__(RK_T) void k_rank_count(Dev d) {
 
 __global__ __launch_bounds__(RK_T) void k_rank_write(Dev d) {
   if (abandoned(d)) return;
-  const int64_t t0 = (int64_t)blockIdx.x * RK_TILE;
+  const int64_t nf = (d.n + 63) / 64, t0 = (int64_t)blockIdx.x * RK_TILE;
   __shared__ int s_w[4];
-  __shared__ int64_t s_run;
-  const int wv = threadIdx.x >> 6;
-  bool fr[RK_I];
-#pragma unroll
-  for (int r = 0; r < RK_I; ++r) fr[r] = rank_flag(d, t0 + r * RK_T + threadIdx.x);
-  if (threadIdx.x == 0) s_run = d.scan_tmp[blockIdx.x];
-  __syncthreads();
+  __shared__ int64_t s_p[4];
+  // flags of the workgroups before (at most 2^28 / 64 / 1024 = 4096 counts)
+  int64_t pre = 0;
+  for (int i = threadIdx.x; i < (int)blockIdx.x; i += RK_T) pre += d.scan_tmp[i];
+  pre = wave_sum(pre);
+  // RK_I consecutive words per thread
+  int c[RK_I], sum = 0;
 #pragma unroll
   for (int r = 0; r < RK_I; ++r) {
-    int64_t i = t0 + r * RK_T + threadIdx.x;
-    bool f = fr[r];
-    unsigned long long m = ballot(f);
-    if (lane_id() == 0) s_w[wv] = __popcll(m);
-    __syncthreads();
-    int64_t pre = s_run;
-    for (int w = 0; w < wv; ++w) pre += s_w[w];
-    if (i < d.n) d.rank[i] = (int32_t)(pre + mbcnt(m));
-    if (i == d.n - 1) {
-      d.rank[d.n] = (int32_t)(pre + mbcnt(m) + (f ? 1 : 0));
-      d.ctl[C_NCLUST] = pre + mbcnt(m) + (f ? 1 : 0);
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) s_run += s_w[0] + s_w[1] + s_w[2] + s_w[3];
-    __syncthreads();
+    const int64_t i = t0 + (int64_t)threadIdx.x * RK_I + r;
+    c[r] = i < nf ? __popcll(d.flag[i]) : 0;
+    sum += c[r];
   }
+  const int incl = wave_incl_scan(sum), wv = threadIdx.x >> 6;
+  if (lane_id() == 63) {
+    s_w[wv] = incl;
+    s_p[wv] = pre;
+  }
+  __syncthreads();
+  int run = (int)(s_p[0] + s_p[1] + s_p[2] + s_p[3]) + incl - sum;
+  for (int w = 0; w < wv; ++w) run += s_w[w];
+#pragma unroll
+  for (int r = 0; r < RK_I; ++r) {
+    const int64_t i = t0 + (int64_t)threadIdx.x * RK_I + r;
+    if (i < nf) d.rank[i] = run;
+    run += c[r];
+    if (i == nf - 1) d.ctl[C_NCLUST] = run;
+  }
+}
+
+// flags before input index k
+__device__ __forceinline__ int32_t rank_of(const Dev& d, int64_t k) {
+  return d.rank[k >> 6] + __popcll(d.flag[k >> 6] & ((1ull << (k & 63)) - 1ull));
 }
 
 __global__ __launch_bounds__(256) void k_output(Dev d) {
@@ -2017,8 +2009,8 @@ __global__ __launch_bounds__(256) void k_output(Dev d) {
     }
 #pragma unroll
     for (int u = 0; u < kRelU; ++u) {
-      rk[u] = d.rank[k[u] == kNoKey ? 0 : k[u]];
-      rb[u] = d.rank[pb[u]];
+      rk[u] = rank_of(d, k[u] == kNoKey ? 0 : k[u]);
+      rb[u] = d.ninst == 1 ? 0 : rank_of(d, pb[u]);
     }
 #pragma unroll
     for (int u = 0; u < kRelU; ++u) {
@@ -2033,31 +2025,7 @@ __global__ __launch_bounds__(256) void k_output(Dev d) {
   stat_add(d, C_NNOISE, noise);
 }
 
-// Per-run state of the clustering phases, one launch after the index:
-// component-minimum flags (by input index), and per expansion wave (`waves` is 0
-// without seed lists) its pair count and the start of its seeding segment of
-// the cells.  k_rep starts the per-cell state.
-__global__ void k_init_run(Dev d, int64_t waves) {
-  const int64_t m = d.n > waves ? d.n : waves;
-  const int64_t C = d.ctl[C_NCELL];
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < m;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    if (i < d.n) d.flag[i] = 0;
-    if (i < waves) {
-      d.pair_cnt[i] = 0;
-      d.seg_pos[i] = C * i / waves;
-    }
-  }
-}
-
 // ------------------------------------------------------------- launchers --
-void launch_init_run(const Dev& d, int64_t waves, hipStream_t s) {
-  const int64_t m = d.n > waves ? d.n : waves;
-  int64_t b = (m + 255) / 256;
-  b = b > 4096 ? 4096 : (b < 1 ? 1 : b);
-  hipLaunchKernelGGL(k_init_run, dim3((int)b), dim3(256), 0, s, d, waves);
-}
-
 // one lane per point, grid a multiple of 8 (XCD remap)
 static int point_grid(int64_t n) {
   int64_t b = (n + 255) / 256;
@@ -2139,9 +2107,7 @@ void launch_far(const Dev& d, bool f32, int grid, hipStream_t s) {
     hipLaunchKernelGGL(k_far_pairs<true>, dim3(grid), dim3(256), 0, s, d);
   else
     hipLaunchKernelGGL(k_far_pairs<false>, dim3(grid), dim3(256), 0, s, d);
-  const int g = std::min(grid, list_grid(d.n));
-  hipLaunchKernelGGL(k_flatten_all, dim3(g), dim3(256), 0, s, d);
-  hipLaunchKernelGGL(k_roots_final, dim3(g), dim3(256), 0, s, d);
+  hipLaunchKernelGGL(k_roots_final, dim3(std::min(grid, list_grid(d.n))), dim3(256), 0, s, d);
 }
 
 void launch_border(const Dev& d, bool f32, hipStream_t s) {
@@ -2172,9 +2138,8 @@ void launch_core_out(const uint8_t* core, const int32_t* orig, int64_t n, uint8_
 }
 
 void launch_relabel(const Dev& d, int64_t n, hipStream_t s) {
-  const int nb = (int)((n + RK_TILE - 1) / RK_TILE);
+  const int nb = (int)(((n + 63) / 64 + RK_TILE - 1) / RK_TILE);
   hipLaunchKernelGGL(k_rank_count, dim3(nb), dim3(RK_T), 0, s, d);
-  launch_scan_top(d.scan_tmp, nb, s);
   hipLaunchKernelGGL(k_rank_write, dim3(nb), dim3(RK_T), 0, s, d);
   int g2 = (int)((n + 255) / 256);
   if (g2 > 4096) g2 = 4096;

@@ -36,39 +36,49 @@ static int fill_grid(int64_t n) {
 // Start of a run, one launch: control counters, statistics stripes, radix
 // pass flags and the bounding-box stripes (per instance and stripe: 0..2 min
 // as ordered keys starting at the largest key, 3..5 max, 6 max |x|, 7
-// non-finite flag, all starting at 0).
-// The call's input and output go into the control block: from `src` (pinned
-// host memory) in a captured run, whose replays read what the host left there,
+// non-finite flag, all starting at 0).  What the call brings (input, output,
+// the parameters of a single instance) is taken from `src` (pinned host
+// memory) in a captured run, whose replays read what the host left there,
 // else from `v`.
-__global__ void k_init_head(Dev d, const Io* src, Io v) {
+__global__ __launch_bounds__(256) void k_init_head(Dev d, const Call* src, Call v) {
+  constexpr int kInstWords = sizeof(Inst) / 8;
   const int64_t nb = (int64_t)d.ninst * kBoxStripes * 8;
   const int64_t ns = (int64_t)kStatStride * kStripes;
-  const int64_t tot = nb + ns + C_NCTL + kMaxPasses + d.ninst;
+  const int64_t ni = d.ninst == 1 ? kInstWords : d.ninst;
+  const int64_t tot = nb + ns + C_NCTL + kMaxPasses + ni;
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < tot;
        i += (int64_t)gridDim.x * blockDim.x) {
-    if (i < nb)
+    if (i < nb) {
       d.bbox[i] = (i & 7) < 3 ? ~0ull : 0ull;
-    else if (i < nb + ns)
+    } else if (i < nb + ns) {
       d.stat[i - nb] = 0;
-    else if (i < nb + ns + C_NCTL)
-      {
-        const int c = (int)(i - nb - ns);
-        long long w = 0;
-        if (c == C_XYZ) w = reinterpret_cast<long long>(src ? src->xyz : v.xyz);
-        if (c == C_LABELS) w = reinterpret_cast<long long>(src ? src->labels : v.labels);
-        if (c == C_T_START) w = (long long)__builtin_amdgcn_s_memrealtime();
-        d.ctl[c] = w;
-      }
-    else if (i < nb + ns + C_NCTL + kMaxPasses)
+    } else if (i < nb + ns + C_NCTL) {
+      const int c = (int)(i - nb - ns);
+      long long w = 0;
+      if (c == C_XYZ) w = reinterpret_cast<long long>(src ? src->xyz : v.xyz);
+      if (c == C_LABELS) w = reinterpret_cast<long long>(src ? src->labels : v.labels);
+      if (c == C_T_START) w = (long long)__builtin_amdgcn_s_memrealtime();
+      d.ctl[c] = w;
+    } else if (i < nb + ns + C_NCTL + kMaxPasses) {
       d.pass_scatter[i - nb - ns - C_NCTL] = 0;
-    else
-      d.inst[i - nb - ns - C_NCTL - kMaxPasses].err = 0;  // (the table may be last run's)
+    } else {
+      const int64_t k = i - nb - ns - C_NCTL - kMaxPasses;
+      if (d.ninst == 1) {
+        // (src is null or not for the whole launch; v stays in the kernel's
+        // argument memory)
+        const unsigned long long* from =
+            reinterpret_cast<const unsigned long long*>(src ? &src->inst : &v.inst);
+        reinterpret_cast<unsigned long long*>(d.inst)[k] = from[k];
+      } else {
+        d.inst[k].err = 0;  // (the table may be last run's)
+      }
+    }
   }
 }
 
-void launch_init_head(const Dev& d, const Io* src, const Io& v, hipStream_t s) {
+void launch_init_head(const Dev& d, const Call* src, const Call& v, hipStream_t s) {
   const int64_t tot = (int64_t)d.ninst * kBoxStripes * 8 + (int64_t)kStatStride * kStripes + C_NCTL +
-                      kMaxPasses + d.ninst;
+                      kMaxPasses + std::max<int64_t>(d.ninst, sizeof(Inst) / 8);
   hipLaunchKernelGGL(k_init_head, dim3(fill_grid(tot)), dim3(256), 0, s, d, src, v);
 }
 
@@ -130,8 +140,17 @@ __device__ __forceinline__ void bbox_points(const double* p0, int64_t np, double
   }
 }
 
+__device__ void setup_instance(Inst& I, const unsigned long long (&bb)[8],
+                               unsigned long long& cells, unsigned long long& keys,
+                               long long& lines);
+__device__ void setup_totals(const Dev& d, unsigned long long cells, unsigned long long keys,
+                             long long lines, int err);
+
+// (a call of one instance has no separate grid set-up: the workgroup that
+// finishes last does it, from coherent loads of the stripes, which saves a
+// launch of one workgroup that took 11 to 19 us)
 __global__ __launch_bounds__(256) void k_bbox(Dev d) {
-  const Chunk ch = d.chunks[blockIdx.x];
+  const Chunk ch = chunk_at(d, blockIdx.x);
   const Inst& I = d.inst[ch.inst];
   const int dim = I.dim;
   double mn[3] = {INFINITY, INFINITY, INFINITY};
@@ -179,6 +198,39 @@ __global__ __launch_bounds__(256) void k_bbox(Dev d) {
     atomicMax(&bb[6], ord_d(s_red[0][6]));
     if (s_bad) atomicOr((unsigned long long*)&bb[7], 1ULL);
   }
+  if (d.ninst != 1) return;
+  __shared__ int s_last;
+  if (threadIdx.x == 0) {
+    // the stripes' atomics before the count: both are done at device scope,
+    // so it is enough that they have completed (a device-wide fence per
+    // workgroup writes L2 back: 4 M points 65 us with it, 22 without)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    s_last = atomicAdd((unsigned long long*)&d.ctl[C_BOXES], 1ull) + 1 == gridDim.x;
+  }
+  __syncthreads();
+  if (!s_last || threadIdx.x >= 64) return;
+  unsigned long long bx[8];
+  static_assert(kBoxStripes <= 64, "one lane per stripe");
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const unsigned long long none = k < 3 ? ~0ull : 0ull;
+    bx[k] = threadIdx.x < kBoxStripes
+                ? __hip_atomic_load(&d.bbox[threadIdx.x * 8 + k], __ATOMIC_RELAXED,
+                                    __HIP_MEMORY_SCOPE_AGENT)
+                : none;
+  }
+#pragma unroll
+  for (int k = 0; k < 8; ++k) bx[k] = k < 3 ? wave_min(bx[k]) : wave_max(bx[k]);
+  if (threadIdx.x == 0) {
+    Inst J = d.inst[0];
+    unsigned long long cells, keys;
+    long long lines;
+    setup_instance(J, bx, cells, keys, lines);
+    J.key_base = 0;
+    J.line_base = 0;
+    d.inst[0] = J;
+    setup_totals(d, cells, keys, lines, J.err);
+  }
 }
 
 // ------------------------------------------------------------ grid setup --
@@ -208,7 +260,103 @@ __global__ __launch_bounds__(256) void k_bbox(Dev d) {
 //
 // Per instance this also sets the column-table base: the dense column table
 // (one entry per possible column) locates a neighbour column in O(1).
-__global__ void k_grid_setup(Dev d) {
+__device__ void setup_instance(Inst& I, const unsigned long long (&bb)[8],
+                               unsigned long long& cells, unsigned long long& keys,
+                               long long& lines) {
+  const int dim = I.dim;
+  double mn[3] = {0, 0, 0}, mx[3] = {0, 0, 0};
+  double emin = INFINITY;
+  bool empty = I.pt_end <= I.pt_begin;
+  for (int k = 0; k < dim; ++k) {
+    mn[k] = empty ? 0.0 : unord_d(bb[k]);
+    mx[k] = empty ? 0.0 : unord_d(bb[3 + k]);
+    emin = fmin(emin, mx[k] - mn[k]);
+  }
+  I.maxabs = empty ? 0.0 : unord_d(bb[6]);
+  if (bb[7]) {
+    // DCLUST_E_PARAM: non-finite input.  The instance keeps a one-cell
+    // grid (every point in cell 0) so that every kernel stays in bounds;
+    // its result is discarded.
+    I.err = -1;
+    for (int k = 0; k < dim; ++k) mn[k] = mx[k] = 0.0;
+    I.maxabs = 0.0;
+  }
+  if (I.r > 0) {
+    double wr = emin / (double)I.r;
+    if (!(wr >= I.eps) && I.err == 0 && !empty) I.err = -2;  // DCLUST_E_BINWIDTH
+  }
+  // coordinates so large that FP64 cannot resolve eps
+  if (I.maxabs > I.eps * 0x1p40 && I.err == 0) I.err = -1;
+  double w = 0.5 * I.eps * (1.0 + 0x1p-20);
+  const double cap = dim == 3 ? 2097152.0 : 2147483647.0;
+  for (;;) {
+    // an oversized input keeps a valid (coarser) grid so that every
+    // kernel stays in bounds; its result is discarded (error set)
+    double inv = 1.0 / w;
+    bool ok = true;
+    for (int k = 0; k < dim; ++k)
+      if (floor((mx[k] - mn[k]) * inv) + 1.0 > cap) ok = false;
+    if (ok) break;
+    if (I.err == 0) I.err = -6;  // DCLUST_E_CAPACITY
+    w *= 2.0;
+  }
+  I.w = w;
+  I.inv_w = 1.0 / w;
+  cells = 1;
+  for (int k = 0; k < 3; ++k) {
+    I.mn[k] = k < dim ? mn[k] : 0.0;
+    I.nk[k] = 1;
+    if (k < dim) {
+      double t = floor(cell_t(mx[k], mn[k], I.inv_w));
+      I.nk[k] = (int32_t)t + 1;
+      cells *= (unsigned long long)I.nk[k];
+    }
+  }
+  const long long bx = ((long long)I.nk[0] + 1) / 2, by = ((long long)I.nk[1] + 1) / 2;
+  I.cstride = dim == 3 ? by + 1 : 1;
+  lines = bx * I.cstride;
+  I.nlines = lines;
+  I.nzl = (long long)I.nk[dim - 1] << (dim - 1);
+  keys = (unsigned long long)lines * (unsigned long long)I.nzl;
+  // FP32 guard band (units of w * 2^-29)
+  const double gs = I.inv_w * 0x1p29;
+  const double es = I.eps * gs;
+  const double e2 = es * es;
+  const double u = 0x1p-24;
+  double bound = 5.0 * u * (1.0 + 4.0 * u);
+  bound += 2.0 * 1.7320508075688772 * 2.5 / es + 6.25 * 3.0 / e2;  // quantisation
+  bound += 8.0 * 0x1p-52 * (I.maxabs / I.eps + 1.0);             // box slack
+  double band = 0x1p-20;
+  if (bound > 0.5 * band) band = 2.0 * bound;
+  float fin = (float)(e2 * (1.0 - band));
+  if ((double)fin > e2 * (1.0 - band)) fin = __int_as_float(__float_as_int(fin) - 1);
+  float fout = (float)(e2 * (1.0 + band));
+  if ((double)fout < e2 * (1.0 + band)) fout = __int_as_float(__float_as_int(fout) + 1);
+  I.d2_in = fin;
+  I.d2_out = fout;
+  I.d2_mid = (float)e2;
+}
+
+// The call's totals: key width, columns, errors.
+__device__ void setup_totals(const Dev& d, unsigned long long cells, unsigned long long keys,
+                             long long lines, int err) {
+  d.ctl[C_ERR] = err != 0;
+  d.ctl[C_NLINES] = lines;
+  if (cells > kMaxKeySpace || keys == ~0ull) {
+    // the keys would not fit the sort: the whole call fails (instances of a
+    // batch share one key space), and every later kernel returns at once
+    d.ctl[C_KEYOVF] = 1;
+    d.ctl[C_ERR] = 1;
+    d.ctl[C_ABANDON] = 1;
+    d.ctl[C_KEYBITS] = 8;
+  } else {
+    d.ctl[C_KEYBITS] = key_bits_for(keys);
+  }
+}
+
+// Grid set-up of a batch, one workgroup: per instance, then the scans of key
+// and column bases over the instances.
+__global__ __launch_bounds__(1024) void k_grid_setup(Dev d) {
   __shared__ unsigned long long s_scan[1024];
   __shared__ unsigned long long s_scanc[1024];
   __shared__ long long s_scanl[1024];
@@ -242,78 +390,7 @@ __global__ void k_grid_setup(Dev d) {
             bb[k] = k < 3 ? (v < bb[k] ? v : bb[k]) : (v > bb[k] ? v : bb[k]);
           }
       }
-      const int dim = I.dim;
-      double mn[3] = {0, 0, 0}, mx[3] = {0, 0, 0};
-      double emin = INFINITY;
-      bool empty = I.pt_end <= I.pt_begin;
-      for (int k = 0; k < dim; ++k) {
-        mn[k] = empty ? 0.0 : unord_d(bb[k]);
-        mx[k] = empty ? 0.0 : unord_d(bb[3 + k]);
-        emin = fmin(emin, mx[k] - mn[k]);
-      }
-      I.maxabs = empty ? 0.0 : unord_d(bb[6]);
-      if (bb[7]) {
-        // DCLUST_E_PARAM: non-finite input.  The instance keeps a one-cell
-        // grid (every point in cell 0) so that every kernel stays in bounds;
-        // its result is discarded.
-        I.err = -1;
-        for (int k = 0; k < dim; ++k) mn[k] = mx[k] = 0.0;
-        I.maxabs = 0.0;
-      }
-      if (I.r > 0) {
-        double wr = emin / (double)I.r;
-        if (!(wr >= I.eps) && I.err == 0 && !empty) I.err = -2;  // DCLUST_E_BINWIDTH
-      }
-      // coordinates so large that FP64 cannot resolve eps
-      if (I.maxabs > I.eps * 0x1p40 && I.err == 0) I.err = -1;
-      double w = 0.5 * I.eps * (1.0 + 0x1p-20);
-      const double cap = dim == 3 ? 2097152.0 : 2147483647.0;
-      for (;;) {
-        // an oversized input keeps a valid (coarser) grid so that every
-        // kernel stays in bounds; its result is discarded (error set)
-        double inv = 1.0 / w;
-        bool ok = true;
-        for (int k = 0; k < dim; ++k)
-          if (floor((mx[k] - mn[k]) * inv) + 1.0 > cap) ok = false;
-        if (ok) break;
-        if (I.err == 0) I.err = -6;  // DCLUST_E_CAPACITY
-        w *= 2.0;
-      }
-      I.w = w;
-      I.inv_w = 1.0 / w;
-      cells = 1;
-      for (int k = 0; k < 3; ++k) {
-        I.mn[k] = k < dim ? mn[k] : 0.0;
-        I.nk[k] = 1;
-        if (k < dim) {
-          double t = floor(cell_t(mx[k], mn[k], I.inv_w));
-          I.nk[k] = (int32_t)t + 1;
-          cells *= (unsigned long long)I.nk[k];
-        }
-      }
-      const long long bx = ((long long)I.nk[0] + 1) / 2, by = ((long long)I.nk[1] + 1) / 2;
-      I.cstride = dim == 3 ? by + 1 : 1;
-      lines = bx * I.cstride;
-      I.nlines = lines;
-      I.nzl = (long long)I.nk[dim - 1] << (dim - 1);
-      keys = (unsigned long long)lines * (unsigned long long)I.nzl;
-      // FP32 guard band (units of w * 2^-29)
-      const double gs = I.inv_w * 0x1p29;
-      const double es = I.eps * gs;
-      const double e2 = es * es;
-      const double u = 0x1p-24;
-      double bound = 5.0 * u * (1.0 + 4.0 * u);
-      bound += 2.0 * 1.7320508075688772 * 2.5 / es + 6.25 * 3.0 / e2;  // quantisation
-      bound += 8.0 * 0x1p-52 * (I.maxabs / I.eps + 1.0);             // box slack
-      double band = 0x1p-20;
-      if (bound > 0.5 * band) band = 2.0 * bound;
-      float fin = (float)(e2 * (1.0 - band));
-      if ((double)fin > e2 * (1.0 - band)) fin = __int_as_float(__float_as_int(fin) - 1);
-      float fout = (float)(e2 * (1.0 + band));
-      if ((double)fout < e2 * (1.0 + band)) fout = __int_as_float(__float_as_int(fout) + 1);
-      I.d2_in = fin;
-      I.d2_out = fout;
-      I.d2_mid = (float)e2;
+      setup_instance(I, bb, cells, keys, lines);
       d.inst[i] = I;
       if (I.err) atomicOr(&s_err, 1);
     }
@@ -345,21 +422,7 @@ __global__ void k_grid_setup(Dev d) {
     }
     __syncthreads();
   }
-  if (threadIdx.x == 0) {
-    const unsigned long long total = s_carry;
-    d.ctl[C_ERR] = s_err;
-    d.ctl[C_NLINES] = s_carryl;
-    if (s_carryc > kMaxKeySpace || total == ~0ull) {
-      // the keys would not fit the sort: the whole call fails (instances of a
-      // batch share one key space), and every later kernel returns at once
-      d.ctl[C_KEYOVF] = 1;
-      d.ctl[C_ERR] = 1;
-      d.ctl[C_ABANDON] = 1;
-      d.ctl[C_KEYBITS] = 8;
-    } else {
-      d.ctl[C_KEYBITS] = key_bits_for(total);
-    }
-  }
+  if (threadIdx.x == 0) setup_totals(d, s_carryc, s_carry, s_carryl, s_err);
 }
 
 // --------------------------------------------------------------- cellkey --
@@ -415,7 +478,7 @@ __device__ __forceinline__ void cellkey_points(const Dev& d, const Inst& I, cons
 
 template <bool K32>
 __global__ __launch_bounds__(256) void k_cellkey(Dev d) {
-  const Chunk ch = d.chunks[blockIdx.x];
+  const Chunk ch = chunk_at(d, blockIdx.x);
   // a copy: the key stores could alias the instance table as far as the
   // compiler knows, which would reload its fields after every store
   const Inst I = d.inst[ch.inst];
@@ -674,18 +737,28 @@ __device__ __forceinline__ void load_key_pairs(const Dev& d, const KT* key, int6
   }
 }
 
-// (also, after a fixed number of radix passes: a key wider than they cover
-// leaves the keys unsorted, so the run is abandoned: every later kernel
-// returns at once and the host runs the call again; counting unsorted keys
-// here is harmless)
+// (also, in a captured run, whose radix passes and column table are fixed: a
+// key wider than the passes cover leaves the keys unsorted, and more columns
+// than the table has would be searched for slowly, so the run is abandoned:
+// every later kernel returns at once and the host runs the call again;
+// counting unsorted keys here is harmless)
 template <bool K32>
 __global__ __launch_bounds__(CS_T) void k_csr_count(Dev d, int passes) {
-  if (blockIdx.x == 0 && threadIdx.x == 0 && passes < kMaxPasses &&
-      d.ctl[C_KEYBITS] > 8 * passes)
+  if (blockIdx.x == 0 && threadIdx.x == 0 &&
+      (d.ctl[C_KEYBITS] > 8 * passes ||
+       (d.line_cap > 0 && d.line_cap < kMaxLineTable && d.ctl[C_NLINES] > d.line_cap)))
     d.ctl[C_ABANDON] = 1;
   if (abandoned(d)) return;
+  // the column table, cleared by the whole grid (which is larger than the
+  // tiles need when there are few)
+  const long long P = d.ctl[C_NLINES];
+  if (P <= d.line_cap)
+    for (int64_t i = (int64_t)blockIdx.x * CS_T + threadIdx.x; i < P;
+         i += (int64_t)gridDim.x * CS_T)
+      d.lines[i] = make_int2(-1, -1);
   const auto* key = sorted_keys<K32>(d);
   const int64_t t0 = (int64_t)blockIdx.x * CS_TILE;
+  if (t0 >= d.n) return;
   uint64_t kr[CS_I], kp[CS_I];
   load_key_pairs<CS_I>(d, key, t0, kr, kp);
   int c = 0;
@@ -752,9 +825,39 @@ __device__ __forceinline__ void split_key(const Inst& I, uint64_t key, int64_t& 
   }
 }
 
+// Column-table index of a key.
+__device__ __forceinline__ int64_t column_of(const Dev& d, uint64_t key) {
+  const Inst& I = d.inst[inst_of_key(d, key)];
+  int64_t col;
+  uint32_t zl;
+  split_key(I, key, col, zl);
+  return I.line_base + col;
+}
+
+// Sum of the block counts v[0..b) (`scanned` false: they are counts; true:
+// already their exclusive prefix), by the whole workgroup of 256.  Where
+// there are at most kScanInline blocks every block sums its own prefix, which
+// takes fewer microseconds than a launch that scans them all.
+constexpr int kScanInline = 2048;
+__device__ __forceinline__ int64_t block_prefix(const int64_t* v, int b, bool scanned) {
+  __shared__ int64_t s_part[4];
+  if (scanned) return v[b];
+  int64_t sum = 0;
+  for (int i = threadIdx.x; i < b; i += 256) sum += v[i];
+  sum = wave_sum(sum);
+  if (lane_id() == 0) s_part[threadIdx.x >> 6] = sum;
+  __syncthreads();
+  sum = s_part[0] + s_part[1] + s_part[2] + s_part[3];
+  __syncthreads();
+  return sum;
+}
+
+// Also fills the column table: a cell whose predecessor's key lies below its
+// column's first key starts the column and ends the one before.
 template <bool K32>
-__global__ __launch_bounds__(CS_T) void k_csr_write(Dev d) {
+__global__ __launch_bounds__(CS_T) void k_csr_write(Dev d, bool scanned) {
   if (abandoned(d)) return;
+  const bool table = d.ctl[C_NLINES] <= d.line_cap;
   const auto* key = sorted_keys<K32>(d);
   const int64_t t0 = (int64_t)blockIdx.x * CS_TILE;
   __shared__ int s_w[4];
@@ -782,7 +885,10 @@ __global__ __launch_bounds__(CS_T) void k_csr_write(Dev d) {
       cr[r] = (uint32_t)(I.line_base + col);
     }
   }
-  if (threadIdx.x == 0) s_run = d.scan_tmp[blockIdx.x];
+  {
+    const int64_t pre = block_prefix(d.scan_tmp, blockIdx.x, scanned);
+    if (threadIdx.x == 0) s_run = pre;
+  }
   __syncthreads();
 #pragma unroll
   for (int r = 0; r < CS_I; ++r) {
@@ -804,8 +910,13 @@ __global__ __launch_bounds__(CS_T) void k_csr_write(Dev d) {
         d.cell_inst[cid] = ir[r];
         d.cell_col[cid] = cr[r];
         d.cell_zl[cid] = zr[r];
+        if (table && (i == 0 || kp[r] < k - zr[r])) {
+          d.lines[cr[r]].x = (int32_t)cid;
+          if (i > 0) d.lines[column_of(d, kp[r])].y = (int32_t)cid;
+        }
       }
       if (i == d.n - 1) {
+        if (table) d.lines[column_of(d, k)].y = (int32_t)cid + 1;
         d.cell_start[cid + 1] = (int32_t)d.n;
         d.ctl[C_NCELL] = cid + 1;
       }
@@ -843,8 +954,20 @@ __device__ __forceinline__ void gather_point(const Dev& d, const Inst& I, const 
   d.orig[i] = src;
 }
 
-__global__ __launch_bounds__(256) void k_gather(Dev d) {
+// Also the run's state: cluster flags (none), and per expansion wave (`waves`
+// is 0 without seed lists) its pair count and the start of its seeding
+// segment of the cells.
+__global__ __launch_bounds__(256) void k_gather(Dev d, int64_t waves) {
   if (abandoned(d)) return;
+  const int64_t nf = (d.n + 63) / 64, C = d.ctl[C_NCELL];
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < nf || i < waves;
+       i += (int64_t)gridDim.x * blockDim.x) {
+    if (i < nf) d.flag[i] = 0ull;
+    if (i < waves) {
+      d.pair_cnt[i] = 0;
+      d.seg_pos[i] = C * i / waves;
+    }
+  }
   const int32_t* vsrc = d.val[sort_parity(d, kMaxPasses)];
   const double* xyz = in_xyz(d);
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < d.n;
@@ -859,33 +982,6 @@ __global__ __launch_bounds__(256) void k_gather(Dev d) {
 }
 
 // ------------------------------------------------------------------ rows --
-// Column table: for every possible column, the range of its non-empty cells
-// in the sorted cell array (-1 when empty).
-__global__ __launch_bounds__(256) void k_line_clear(Dev d) {
-  if (abandoned(d)) return;
-  const long long P = d.ctl[C_NLINES];
-  if (P > d.line_cap) return;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < P;
-       i += (int64_t)gridDim.x * blockDim.x)
-    d.lines[i] = make_int2(-1, -1);
-}
-
-__global__ __launch_bounds__(256) void k_line_mark(Dev d) {
-  if (abandoned(d)) return;
-  const int32_t C = (int32_t)d.ctl[C_NCELL];
-  if (d.ctl[C_NLINES] > d.line_cap) return;
-  for (int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; c < C;
-       c += (int64_t)gridDim.x * blockDim.x) {
-    // the three columns are read before either store (which could alias the
-    // cell arrays as far as the compiler knows)
-    const uint32_t L = d.cell_col[c];
-    const bool first = c == 0 || d.cell_col[c > 0 ? c - 1 : 0] != L;
-    const bool last = c == C - 1 || d.cell_col[c < C - 1 ? c + 1 : c] != L;
-    if (first) d.lines[L].x = (int32_t)c;
-    if (last) d.lines[L].y = (int32_t)c + 1;
-  }
-}
-
 // Three lower bounds lo[j] = first index in [lo[j], hi[j]) with a[i] >= v[j],
 // in lockstep (the loads of the three searches overlap).
 template <typename T>
@@ -1302,7 +1398,7 @@ __global__ __launch_bounds__(256) void k_nbr_stats(Dev d) {
 // ------------------------------------------------------------- launchers --
 void launch_index_head(const Dev& d, int nchunks, hipStream_t s) {
   hipLaunchKernelGGL(k_bbox, dim3(nchunks), dim3(256), 0, s, d);
-  hipLaunchKernelGGL(k_grid_setup, dim3(1), dim3(1024), 0, s, d);
+  if (d.ninst != 1) hipLaunchKernelGGL(k_grid_setup, dim3(1), dim3(1024), 0, s, d);
 }
 
 // Keys per thread of the radix passes over n keys.  A scatter workgroup of
@@ -1319,6 +1415,8 @@ int sort_items(bool k32, int64_t n, int cus) {
   return 16 * r4 < 10 * r2 ? 16 : RS_I;
 }
 
+constexpr int kClearGrid = 1024;
+
 template <bool K32, int NI>
 static void index_sort(const Dev& d, int64_t n, int nchunks, int passes, hipStream_t s) {
   hipLaunchKernelGGL(k_cellkey<K32>, dim3(nchunks), dim3(256), 0, s, d);
@@ -1329,9 +1427,14 @@ static void index_sort(const Dev& d, int64_t n, int nchunks, int passes, hipStre
     hipLaunchKernelGGL((k_rs_scatter<K32, NI>), dim3(nblk), dim3(RS_T), 0, s, d, p, nblk);
   }
   const int ncs = (int)((n + CS_TILE - 1) / CS_TILE);
-  hipLaunchKernelGGL(k_csr_count<K32>, dim3(ncs), dim3(CS_T), 0, s, d, passes);
-  hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(1024), 0, s, d.scan_tmp, ncs, (long long*)nullptr);
-  hipLaunchKernelGGL(k_csr_write<K32>, dim3(ncs), dim3(CS_T), 0, s, d);
+  // (the grid also clears the column table: not too small for a large one)
+  const int ncc = std::max(ncs, d.line_cap > (1 << 16) ? kClearGrid : 1);
+  hipLaunchKernelGGL(k_csr_count<K32>, dim3(ncc), dim3(CS_T), 0, s, d, passes);
+  const bool scan = ncs > kScanInline;
+  if (scan)
+    hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(1024), 0, s, d.scan_tmp, ncs,
+                       (long long*)nullptr);
+  hipLaunchKernelGGL(k_csr_write<K32>, dim3(ncs), dim3(CS_T), 0, s, d, scan);
 }
 
 // `passes` radix passes: keys of at most 32 bits (four passes) are sorted as
@@ -1345,16 +1448,11 @@ void launch_index_sort(const Dev& d, int64_t n, int nchunks, int passes, int cus
     index_sort<true, RS_I>(d, n, nchunks, passes, s);
 }
 
-void launch_gather(const Dev& d, int64_t n, hipStream_t s) {
+void launch_gather(const Dev& d, int64_t n, int64_t waves, hipStream_t s) {
   // random-access gather: more blocks in flight than a fill needs
   const int64_t gb = (n + 255) / 256;
   hipLaunchKernelGGL(k_gather, dim3((int)std::max<int64_t>(1, std::min<int64_t>(16384, gb))),
-                     dim3(256), 0, s, d);
-}
-
-void launch_lines(const Dev& d, int grid_cells, hipStream_t s) {
-  hipLaunchKernelGGL(k_line_clear, dim3(grid_cells), dim3(256), 0, s, d);
-  hipLaunchKernelGGL(k_line_mark, dim3(grid_cells), dim3(256), 0, s, d);
+                     dim3(256), 0, s, d, waves);
 }
 
 // Row pass grid: one wavefront per (tile of 64 cells, group) for up
@@ -1376,10 +1474,6 @@ void launch_rows(const Dev& d, int64_t n, int grid_cells, hipStream_t s) {
   const int64_t gb = std::max<int64_t>(1, std::min<int64_t>(4LL * grid_cells, (n + 255) / 256));
   hipLaunchKernelGGL(k_rows_global, dim3((unsigned)gb), dim3(256), 0, s, d);
   if (d.nbr_stats) hipLaunchKernelGGL(k_nbr_stats, dim3((unsigned)gb), dim3(256), 0, s, d);
-}
-
-void launch_scan_top(int64_t* v, int nb, hipStream_t s) {
-  hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(1024), 0, s, v, nb, (long long*)nullptr);
 }
 
 int64_t sort_hist_entries(int64_t n) { return 256 * ((n + RS_TILE - 1) / RS_TILE); }

@@ -155,8 +155,14 @@ struct Inst {
   int64_t xyz_off;             // element offset of the first coordinate
 };
 
-// Chunk of points of one instance (host-built work list for per-point
-// kernels that need the instance, so no point->instance search is needed).
+// column table entries (8 bytes each) above which neighbour columns are found
+// by binary search instead
+constexpr long long kMaxLineTable = 1LL << 26;  // 512 MiB at most
+
+// Chunk of at most kChunk points of one instance (work list of the per-point
+// kernels that need the instance, so no point->instance search is needed;
+// host-built for a batch, computed from the chunk's number for one instance).
+constexpr int64_t kChunk = 4096;
 struct Chunk {
   int32_t inst;
   int32_t pad;
@@ -219,6 +225,7 @@ enum Ctl : int {
   C_NROOTS,       // near components (listed in Dev::near_roots)
   C_NFARLIGHT,    // pairs across components (listed in Dev::far_light)
   C_NFARHEAVY,    // those with a heavy cell (listed in Dev::far_heavy)
+  C_BOXES,        // chunks whose bounding box is done (one instance)
   // this call's input and output (addresses), written by the run's first kernel
   C_XYZ,
   C_LABELS,
@@ -287,13 +294,16 @@ constexpr int kMaxPasses = 8;
 // the grid set-up reduces the stripes.
 constexpr int kBoxStripes = 32;
 
-// Input and output of a call.  They reach the kernels through the control
-// block, not through Dev: a captured run is replayed for calls with other
-// buffers.
-struct Io {
+// What a call brings besides its sizes: input and output, and its parameters
+// if it has one instance.  They reach the kernels through the control block
+// and the instance table, not through Dev: a captured run is replayed for
+// calls with other buffers and other parameters.
+struct Call {
   const double* xyz;
   int32_t* labels;
+  Inst inst;
 };
+static_assert(sizeof(Inst) % 8 == 0, "the instance table is copied in words");
 
 constexpr int kClockMHz = 100;  // of the constant device clock
 
@@ -331,7 +341,7 @@ struct Dev {
                         // (over the sort keys, which the CSR pass is the last to read)
   int32_t chains;       // 1: near components by seed-list expansion, 0: by union-find
   SList core_rest;      // points the first count pass leaves (over keyv)
-  SList core_crowd;     // those of them with many candidates (over rank)
+  SList core_crowd;     // those of them with many candidates (over compmin)
   SList border_pts;     // non-core points (border-label lanes)
   SList core_cells;     // cells with core points (near-graph and border-pair lanes)
   SList near_roots;     // roots of the near components
@@ -354,7 +364,7 @@ struct Dev {
   uint8_t* core;
   int32_t* rec;         // [rec_stride][N] neighbours of non-core points
   uint8_t* rec_n;       // [N] records written, kRecFew or kRecNone
-  int32_t rec_stride;   // record slots per point: min(minpts, kRecSlots)
+  int32_t rec_stride;   // record slots per point: minpts or more, at most kRecSlots
   int32_t* parent;
   int32_t* compmin;
   int2* pairs;          // [waves][pair_per] collision pairs per expansion wave
@@ -365,8 +375,8 @@ struct Dev {
   int64_t* seg_pos;     // [waves] seeding cursor of each expansion wave
   int32_t* keyv;
   SList rows_fb;         // row work items (tile * 3 + group) left to k_rows_global
-  uint8_t* flag;
-  int32_t* rank;
+  unsigned long long* flag;  // [N/64] bit per input index: smallest core point of a cluster
+  int32_t* rank;             // [N/64] flags before each word
   int64_t* scan_tmp;  // block sums for scans
 
   uint8_t* core_out;    // core flags in input order
@@ -586,6 +596,17 @@ __device__ __forceinline__ int32_t slot_cell(uint2 row, int s) {
   return (int32_t)row.x + __popc(row.y & ((1u << s) - 1u));
 }
 
+// Chunk b of the call's points.
+__device__ __forceinline__ Chunk chunk_at(const Dev& d, int b) {
+  if (d.ninst != 1) return d.chunks[b];
+  Chunk ch;
+  ch.inst = 0;
+  ch.pad = 0;
+  ch.begin = b * kChunk;
+  ch.end = ch.begin + kChunk < d.n ? ch.begin + kChunk : d.n;
+  return ch;
+}
+
 // Instance of a cell (a run of one instance reads the table entry directly,
 // with no per-cell load).
 __device__ __forceinline__ const Inst* inst_of_cell(const Dev& d, int64_t c) {
@@ -623,11 +644,8 @@ __device__ __forceinline__ int32_t uf_find(int32_t* par, int32_t x) {
   }
 }
 
-// Root of x by a walk that writes nothing.  The final flatten uses it (no
-// unions running): a path-halving write from another thread's walk could
-// otherwise replace a root that its owner has just stored with an inner
-// ancestor, and a later read of "the root" would then get an inner node.
-// The walk does not compress, so it is run on an already compressed forest.
+// Root of x by a walk that writes nothing (for a pass in which every thread
+// stores a root of its own and no unions run).
 __device__ __forceinline__ int32_t uf_root(const int32_t* par, int32_t x) {
   for (;;) {
     const int32_t p = par[x];

@@ -5,25 +5,19 @@
 namespace dclust {
 
 // start of a run: control counters, statistics, radix pass flags, bbox
-// (the call's input and output: read from `src` on the device, or `v` if null)
-void launch_init_head(const Dev& d, const Io* src, const Io& v, hipStream_t s);
+// (what the call brings: read from `src` on the device, or `v` if null)
+void launch_init_head(const Dev& d, const Call* src, const Call& v, hipStream_t s);
 void launch_readback(const Dev& d, long long* out, hipStream_t s);
-// per-run state of the clustering phases (labels, forest, minima, flags,
-// per-cell core counts, per-wave pair counts)
-void launch_init_run(const Dev& d, int64_t waves, hipStream_t s);
 // bbox + grid set-up (per-instance cell width, cells per axis, key space)
 void launch_index_head(const Dev& d, int nchunks, hipStream_t s);
-// the index after the grid set-up, in three parts: cell keys, `passes`
-// radix passes and CSR compaction (tile size from the CU count `cus`); the
-// gather of the coordinates; the column table (the last two are independent)
+// the index after the grid set-up, in two parts: cell keys, `passes` radix
+// passes, CSR compaction and column table (tile size from the CU count
+// `cus`); the gather of the coordinates, and the start of the run's state for
+// `waves` expansion waves
 void launch_index_sort(const Dev& d, int64_t n, int nchunks, int passes, int cus, hipStream_t s);
-void launch_gather(const Dev& d, int64_t n, hipStream_t s);
-void launch_lines(const Dev& d, int grid_cells, hipStream_t s);
+void launch_gather(const Dev& d, int64_t n, int64_t waves, hipStream_t s);
 // neighbour rows of every cell (k_rows)
 void launch_rows(const Dev& d, int64_t n, int grid_cells, hipStream_t s);
-// exclusive in-place scan of nb int64 values by one block
-void launch_scan_top(int64_t* v, int nb, hipStream_t s);
-
 int64_t sort_hist_entries(int64_t n);
 // per-stripe capacity of the row pass's work list for up to n cells
 int64_t row_list_cap(int64_t n);
