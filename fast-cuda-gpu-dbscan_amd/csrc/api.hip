@@ -60,7 +60,7 @@ struct dclust_handle {
   std::vector<uint8_t> prev_sig;   // launch state of the last eager run
   int prev_npass = 0;              // its expansion passes
   long long prev_nlines = 0;       // its neighbour-line count
-  int prev_sort_passes = 0;        // its radix passes
+  int prev_key_bits = 0;           // its sort key width
   hipGraphExec_t gexec = nullptr;  // captured run
   std::vector<uint8_t> gsig;       // launch state it was captured for
   int gpasses = 0;                 // expansion passes it holds
@@ -119,7 +119,7 @@ namespace {
 
 enum Slot {
   S_XYZ, S_INST, S_CHUNK, S_BBOX, S_CTL, S_KEY, S_VAL, S_HIST, S_OFFS,
-  S_DTOT, S_PASS, S_CSTART, S_CKEY, S_CINST, S_CM, S_ROWS, S_CELLOF, S_X,
+  S_DTOT, S_CSTART, S_CKEY, S_CINST, S_CM, S_ROWS, S_CELLOF, S_X,
   S_G, S_ORIG, S_CORE, S_LABEL, S_PARENT, S_COMPMIN, S_PAIRS, S_Q0, S_Q1,
   S_KEYV, S_FLAG, S_RANK, S_SCAN, S_LABOUT, S_COREOUT, S_PAIRCNT, S_SEGPOS, S_LINES, S_AMASK,
   S_REC, S_RECN, S_CCOL, S_CCOMP, S_BORDERPTS, S_CORECELLS, S_TUNELAB, S_STAT, S_GLINES,
@@ -490,11 +490,11 @@ hipError_t mark(dclust_handle* h, int e, bool graph, hipStream_t s = nullptr) {
 // stream: the gather fills the device, so running the rows beside it gains
 // nothing).
 hipError_t enqueue_index(dclust_handle* h, const Dev& d, int64_t n, int nchunks, int grid_cells,
-                         int passes, int64_t waves, bool graph) {
+                         int bits, int64_t waves, bool graph) {
   const hipStream_t s = h->stream;
   hipError_t e;
-  launch_index_sort(d, n, nchunks, passes, h->num_cu, s);
-  launch_gather(d, n, waves, s);
+  launch_index_sort(d, n, nchunks, bits, s);
+  launch_gather(d, n, waves, bits, s);
   if ((e = mark(h, E_ROWS0, graph)) != hipSuccess) return e;
   launch_rows(d, n, grid_cells, s);
   return hipSuccess;
@@ -561,12 +561,12 @@ hipError_t enqueue_readback(dclust_handle* h, const Dev& d, hipStream_t s) {
 }
 
 // A whole run with no host read in between, captured into a graph:
-// `sort_passes` radix passes (the key width of the previous run; a wider key
-// abandons the run on the device) and `passes` expansion passes (a pass with
+// a sort of `key_bits` bits (the largest of this launch state's runs; a wider
+// key abandons the run on the device) and `passes` expansion passes (a pass with
 // nothing pending exits at once).
 hipError_t capture_run(dclust_handle* h, const Dev& d, const Call& call, const RunShape& shape,
                        bool f32,
-                       int nchunks, int grid_cells, int sort_passes, int passes,
+                       int nchunks, int grid_cells, int key_bits, int passes,
                        hipGraphExec_t* out) {
   const hipStream_t s = h->stream;
   hipGraph_t g = nullptr;
@@ -577,7 +577,7 @@ hipError_t capture_run(dclust_handle* h, const Dev& d, const Call& call, const R
   // launch, outside the graph: the start event is processed while the host
   // is still submitting the graph)
   enqueue_head(d, h->pin ? (const Call*)(h->pin_dev + C_NCTL) : nullptr, call, nchunks, s);
-  hipError_t body = enqueue_index(h, d, d.n, nchunks, grid_cells, sort_passes,
+  hipError_t body = enqueue_index(h, d, d.n, nchunks, grid_cells, key_bits,
                                   shape.chains ? shape.waves : 0, true);
   if (body == hipSuccess) body = enqueue_core(h, d, f32, true);
   // work still pending after the last pass: the rest of the graph returns at
@@ -843,8 +843,7 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
                            (unsigned long long*)(d.stat + C_NFARHEAVY), cap_f};
     d.hist = M.get<uint32_t>(S_HIST, sort_hist_entries(ntot));
     d.offs = M.get<uint32_t>(S_OFFS, sort_hist_entries(ntot));
-    d.dtot = M.get<uint32_t>(S_DTOT, 256);
-    d.pass_scatter = M.get<int32_t>(S_PASS, kMaxPasses);
+    d.dtot = M.get<uint32_t>(S_DTOT, 1 << kDigitBits);
     d.cell_start = M.get<int32_t>(S_CSTART, ntot + 1);
     d.cell_key = M.get<uint64_t>(S_CKEY, ntot);
     d.cell_col = M.get<uint32_t>(S_CCOL, ntot);
@@ -928,8 +927,8 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
       dg.line_cap = cap;
       const int gp = std::max(2, h->prev_npass + 1);
       hipGraphExec_t ge = nullptr;
-      const int sp = std::max(1, std::min(kMaxPasses, h->prev_sort_passes));
-      if (capture_run(h, dg, call, shape, f32, nchunks, grid_cells, sp, gp, &ge) == hipSuccess) {
+      if (capture_run(h, dg, call, shape, f32, nchunks, grid_cells, h->prev_key_bits, gp,
+                      &ge) == hipSuccess) {
         h->gexec = ge;
         h->gsig = sig;
         h->gpasses = gp;
@@ -1023,7 +1022,7 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
       if (ninst == 1 || !inst_err) return first ? first : DCLUST_E_PARAM;
       rc = first;  // batched with per-instance errors: keep going
     }
-    const int passes = (int)((ctl_h[C_KEYBITS] + 7) / 8);
+    const int bits = (int)ctl_h[C_KEYBITS];
     const long long nlines = ctl_h[C_NLINES];
     if (stats) stats->key_bits = (int32_t)ctl_h[C_KEYBITS];
     // dense line table when it is small enough, else binary search
@@ -1039,7 +1038,7 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
       // (a fixed region without room for the table: the rows are found by
       // binary search over the cell keys instead)
     }
-    HIPCHK(enqueue_index(h, d, ntot, nchunks, grid_cells, passes, shape.chains ? shape.waves : 0,
+    HIPCHK(enqueue_index(h, d, ntot, nchunks, grid_cells, bits, shape.chains ? shape.waves : 0,
                          false));
     if (onestep) {
       HIPCHK(mark(h, E_INDEX, false));
@@ -1071,7 +1070,7 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
       h->prev_sig.swap(sig);
       h->prev_npass = same ? std::max(npass, h->prev_npass) : npass;
       h->prev_nlines = same ? std::max(nlines, h->prev_nlines) : nlines;
-      h->prev_sort_passes = same ? std::max(passes, h->prev_sort_passes) : passes;
+      h->prev_key_bits = same ? std::max(bits, h->prev_key_bits) : bits;
     }
     return rc;
   }

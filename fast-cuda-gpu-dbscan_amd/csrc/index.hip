@@ -33,8 +33,8 @@ static int fill_grid(int64_t n) {
   return (int)b;
 }
 
-// Start of a run, one launch: control counters, statistics stripes, radix
-// pass flags and the bounding-box stripes (per instance and stripe: 0..2 min
+// Start of a run, one launch: control counters, statistics stripes and the
+// bounding-box stripes (per instance and stripe: 0..2 min
 // as ordered keys starting at the largest key, 3..5 max, 6 max |x|, 7
 // non-finite flag, all starting at 0).  What the call brings (input, output,
 // the parameters of a single instance) is taken from `src` (pinned host
@@ -45,7 +45,7 @@ __global__ __launch_bounds__(256) void k_init_head(Dev d, const Call* src, Call 
   const int64_t nb = (int64_t)d.ninst * kBoxStripes * 8;
   const int64_t ns = (int64_t)kStatStride * kStripes;
   const int64_t ni = d.ninst == 1 ? kInstWords : d.ninst;
-  const int64_t tot = nb + ns + C_NCTL + kMaxPasses + ni;
+  const int64_t tot = nb + ns + C_NCTL + ni;
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < tot;
        i += (int64_t)gridDim.x * blockDim.x) {
     if (i < nb) {
@@ -59,10 +59,8 @@ __global__ __launch_bounds__(256) void k_init_head(Dev d, const Call* src, Call 
       if (c == C_LABELS) w = reinterpret_cast<long long>(src ? src->labels : v.labels);
       if (c == C_T_START) w = (long long)__builtin_amdgcn_s_memrealtime();
       d.ctl[c] = w;
-    } else if (i < nb + ns + C_NCTL + kMaxPasses) {
-      d.pass_scatter[i - nb - ns - C_NCTL] = 0;
     } else {
-      const int64_t k = i - nb - ns - C_NCTL - kMaxPasses;
+      const int64_t k = i - nb - ns - C_NCTL;
       if (d.ninst == 1) {
         // (src is null or not for the whole launch; v stays in the kernel's
         // argument memory)
@@ -78,7 +76,7 @@ __global__ __launch_bounds__(256) void k_init_head(Dev d, const Call* src, Call 
 
 void launch_init_head(const Dev& d, const Call* src, const Call& v, hipStream_t s) {
   const int64_t tot = (int64_t)d.ninst * kBoxStripes * 8 + (int64_t)kStatStride * kStripes + C_NCTL +
-                      kMaxPasses + std::max<int64_t>(d.ninst, sizeof(Inst) / 8);
+                      std::max<int64_t>(d.ninst, sizeof(Inst) / 8);
   hipLaunchKernelGGL(k_init_head, dim3(fill_grid(tot)), dim3(256), 0, s, d, src, v);
 }
 
@@ -426,17 +424,31 @@ __global__ __launch_bounds__(1024) void k_grid_setup(Dev d) {
 }
 
 // --------------------------------------------------------------- cellkey --
-// Sort keys are 32-bit when the key space of the call fits (at most four
-// 8-bit passes), else 64-bit; the key buffers are viewed as either.  The
-// host picks the width from the key bits it knows (the grid set-up's, or
-// the previous run's for a captured graph: a replay whose keys are wider
-// than its passes cover is abandoned by k_csr_count, so a truncated key is
-// never used).
-template <bool K32>
-using SortKey = typename std::conditional<K32, uint32_t, uint64_t>::type;
-template <bool K32>
-__device__ __forceinline__ SortKey<K32>* key_buf(const Dev& d, int b) {
-  return reinterpret_cast<SortKey<K32>*>(d.key[b]);
+// Forms of the sort keys.  Up to 32 bits: 32-bit keys beside 32-bit ids.  Up
+// to 36 bits, ids of 28 bits: the key's lower four bits ride in the id's
+// upper four (only the first pass looks at them, so the later passes count
+// from the keys alone), and a pass still moves 8 bytes a point where a 64-bit
+// key moves 12.
+// Above that 64-bit keys; the buffers are viewed as any of them.  The host
+// picks the form from the key bits it knows (the grid set-up's, or the largest
+// so far for a captured graph: a replay whose keys are wider is abandoned by
+// k_csr_count, so a truncated key is never used).
+template <int KF>
+using SortKey = typename std::conditional<KF == 64, uint64_t, uint32_t>::type;
+template <int KF>
+__device__ __forceinline__ SortKey<KF>* key_buf(const Dev& d, int b) {
+  return reinterpret_cast<SortKey<KF>*>(d.key[b]);
+}
+constexpr uint32_t kIdMask = (1u << 28) - 1;  // of the 36-bit form
+// the whole key of a sort entry
+template <int KF>
+__device__ __forceinline__ uint64_t entry_key(SortKey<KF> k, int32_t v) {
+  return KF == 36 ? (uint64_t)k << 4 | (uint32_t)v >> 28 : (uint64_t)k;
+}
+template <int KF>
+__device__ __forceinline__ uint32_t entry_digit(SortKey<KF> k, int32_t v, int shift,
+                                                uint32_t mask) {
+  return (uint32_t)(entry_key<KF>(k, v) >> shift) & mask;
 }
 
 __device__ __forceinline__ int32_t cell_index(double x, const Inst& I, int k) {
@@ -445,21 +457,102 @@ __device__ __forceinline__ int32_t cell_index(double x, const Inst& I, int k) {
   return c;
 }
 
-template <int D, bool K32>
-__device__ __forceinline__ void cellkey_points(const Dev& d, const Inst& I, const Chunk& ch) {
-  const double* p0 = in_xyz(d) + I.xyz_off + (ch.begin - I.pt_begin) * D;
-  const int64_t np = ch.end - ch.begin;
-  for (int64_t i0 = threadIdx.x; i0 < np; i0 += kChunkU * 256) {
+// ------------------------------------------------------------ radix sort --
+// LSD radix sort by digits of at most 9 bits, three launches a pass.  Every
+// workgroup owns one contiguous range of the entries, so the digit counts are
+// few ([workgroups][512], a scan of a few microseconds), and its tiles write
+// one after the other to neighbouring places, whose partial lines its L2
+// joins.  Buffer parity: the number of passes.
+//
+// Bound by the bytes it moves, in runs of a few dozen bytes, at the larger sizes
+// and by launches and each workgroup's chain of barriers at the smaller.  Per
+// pass, 32 M points of 33 bits: count 29 us, scan 6, scatter 147 to 177 (four
+// passes); 4 M of 32 bits 6 + 6 + 24 (four).  Before (8-bit digits, one tile of
+// 2048 keys a workgroup, counts [256][n / 2048]) 88 + 43 + 233 (five passes of
+// 64-bit keys) and 15 + 6 + 22.  Interleaving the tiles of neighbouring
+// workgroups instead (one tile each) took longer, 225 us a scatter.
+constexpr int RS_T = 512;
+constexpr int RS_D = 1 << kDigitBits;  // a thread per digit
+static_assert(RS_T == RS_D, "one digit per thread");
+
+// The fewest passes of at most 9 bits, of widths as equal as they can be; the
+// wider digits come last, where the entries already have long runs.
+__device__ __forceinline__ int sort_passes(const Dev& d) {
+  return ((int)d.ctl[C_KEYBITS] + kDigitBits - 1) / kDigitBits;
+}
+struct SortDigit {
+  int shift, width;
+};
+__device__ __forceinline__ SortDigit sort_digit(const Dev& d, int pass, int passes) {
+  const int bits = (int)d.ctl[C_KEYBITS], w = bits / passes, first_wide = passes - bits % passes;
+  SortDigit g;
+  g.shift = pass * w + (pass > first_wide ? pass - first_wide : 0);
+  g.width = w + (pass >= first_wide);
+  return g;
+}
+
+// Entries of workgroup b of nblk.
+__device__ __forceinline__ void sort_range(int64_t n, int b, int nblk, int64_t& lo, int64_t& hi) {
+  const int64_t per = ((n + nblk - 1) / nblk + 63) & ~63LL;
+  lo = b * per < n ? b * per : n;
+  hi = lo + per < n ? lo + per : n;
+}
+
+// Workgroups of one XCD own neighbouring ranges.
+__device__ __forceinline__ int sort_block(int nblk) {
+  const int b = blockIdx.x;
+  return nblk % 8 == 0 ? (b & 7) * (nblk / 8) + (b >> 3) : b;
+}
+
+// lanes of the wave with the same digit among the `valid` ones
+__device__ __forceinline__ unsigned long long match_digit(uint32_t dg, int width, bool valid) {
+  unsigned long long peers = ballot(valid);
+#pragma unroll
+  for (int b = 0; b < kDigitBits; ++b) {
+    if (b < width) {
+      const bool bit = (dg >> b) & 1;
+      const unsigned long long m = ballot(bit);
+      peers &= bit ? m : ~m;
+    }
+  }
+  return peers;
+}
+
+// Digit counts of each workgroup's range.  The lanes of a wave count in
+// kHistCopies copies in turn: the upper digits of clustered points are few, and
+// their atomics on one address would queue (32 M points, one copy: 28 us for
+// the lower digits and 130 for the upper).
+constexpr int kHistCopies = 8;
+__device__ __forceinline__ void hist_clear(uint32_t (&h)[RS_D * kHistCopies]) {
+#pragma unroll
+  for (int c = 0; c < kHistCopies; ++c) h[c * RS_T + threadIdx.x] = 0;
+  __syncthreads();
+}
+__device__ __forceinline__ void hist_store(const Dev& d, uint32_t (&h)[RS_D * kHistCopies],
+                                           int b) {
+  __syncthreads();
+  uint32_t sum = 0;
+#pragma unroll
+  for (int c = 0; c < kHistCopies; ++c) sum += h[threadIdx.x * kHistCopies + c];
+  d.hist[(int64_t)b * RS_D + threadIdx.x] = sum;
+}
+
+template <int D, int KF, int T, typename F>
+__device__ __forceinline__ void cellkey_points(const Dev& d, const Inst& I, int64_t begin,
+                                               int64_t end, const F& count) {
+  const double* p0 = in_xyz(d) + I.xyz_off + (begin - I.pt_begin) * D;
+  const int64_t np = end - begin;
+  for (int64_t i0 = threadIdx.x; i0 < np; i0 += kChunkU * T) {
     double v[kChunkU][D];
 #pragma unroll
     for (int u = 0; u < kChunkU; ++u) {
-      const int64_t i = i0 + u * 256 < np ? i0 + u * 256 : np - 1;
+      const int64_t i = i0 + u * T < np ? i0 + u * T : np - 1;
 #pragma unroll
       for (int k = 0; k < D; ++k) v[u][k] = p0[i * D + k];
     }
 #pragma unroll
     for (int u = 0; u < kChunkU; ++u) {
-      const int64_t i = i0 + u * 256;
+      const int64_t i = i0 + u * T;
       if (i < np) {
         const int32_t cx = cell_index(v[u][0], I, 0), cl = cell_index(v[u][D - 1], I, D - 1);
         int64_t lin;
@@ -469,242 +562,243 @@ __device__ __forceinline__ void cellkey_points(const Dev& d, const Inst& I, cons
         } else {
           lin = (cx >> 1) * I.nzl + cl * 2LL + (cx & 1);
         }
-        key_buf<K32>(d, 0)[ch.begin + i] = (SortKey<K32>)(I.key_base + lin);
-        d.val[0][ch.begin + i] = (int32_t)(ch.begin + i);
+        const uint64_t key = I.key_base + lin;
+        key_buf<KF>(d, 0)[begin + i] = (SortKey<KF>)(KF == 36 ? key >> 4 : key);
+        // (the first pass knows the ids, which are the positions)
+        if (KF == 36)
+          d.val[0][begin + i] = (int32_t)((uint32_t)(begin + i) | (uint32_t)key << 28);
+        count((uint32_t)key);
       }
     }
   }
 }
 
-template <bool K32>
-__global__ __launch_bounds__(256) void k_cellkey(Dev d) {
-  const Chunk ch = chunk_at(d, blockIdx.x);
+template <int KF, int T, typename F>
+__device__ __forceinline__ void cellkeys(const Dev& d, int inst, int64_t begin, int64_t end,
+                                         const F& count) {
   // a copy: the key stores could alias the instance table as far as the
   // compiler knows, which would reload its fields after every store
-  const Inst I = d.inst[ch.inst];
+  const Inst I = d.inst[inst];
   if (I.dim == 3)
-    cellkey_points<3, K32>(d, I, ch);
+    cellkey_points<3, KF, T>(d, I, begin, end, count);
   else
-    cellkey_points<2, K32>(d, I, ch);
+    cellkey_points<2, KF, T>(d, I, begin, end, count);
 }
 
-// ------------------------------------------------------------ radix sort --
-// LSD radix sort, 8-bit digits, 2048-key tiles (256 threads x 8 keys; with
-// 64-bit keys the scatter's 31 KiB of LDS lets five workgroups share a CU,
-// and 4096-key tiles were slower, 1024-key tiles too), or 4096-key tiles for
-// 32-bit keys where they need fewer rounds of workgroups (sort_items).
-// Buffer parity: the number of scatters executed so far.
-constexpr int RS_T = 256;
-constexpr int RS_I = 8;
-constexpr int RS_TILE = RS_T * RS_I;
-// Keys per thread: 8 (2048-key tiles), or 16 (4096-key tiles) for 32-bit
-// keys when that takes fewer rounds of resident workgroups (the histogram
-// buffers are sized for the smaller tiles; see sort_items).
-
-__device__ __forceinline__ int sort_parity(const Dev& d, int pass) {
-  int p = 0;
-  for (int q = 0; q < pass; ++q) p += d.pass_scatter[q];
-  return p & 1;
+// Keys of a batch, a chunk of one instance per workgroup.
+template <int KF>
+__global__ __launch_bounds__(256) void k_cellkey(Dev d) {
+  const Chunk ch = d.chunks[blockIdx.x];
+  cellkeys<KF, 256>(d, ch.inst, ch.begin, ch.end, [](uint32_t) {});
 }
 
-// peers of this lane with the same 8-bit digit among `valid` lanes
-__device__ __forceinline__ unsigned long long match8(uint32_t dg, bool valid) {
-  unsigned long long peers = ballot(valid);
-#pragma unroll
-  for (int b = 0; b < 8; ++b) {
-    bool bit = (dg >> b) & 1;
-    unsigned long long m = ballot(bit);
-    peers &= bit ? m : ~m;
-  }
-  return peers;
+// Keys of a single instance, and the first pass's digit counts: a workgroup
+// takes its range of the sort.
+template <int KF>
+__global__ __launch_bounds__(RS_T) void k_cellkey_hist(Dev d, int nblk) {
+  const uint32_t mask = (1u << sort_digit(d, 0, sort_passes(d)).width) - 1;
+  __shared__ uint32_t h[RS_D * kHistCopies];
+  hist_clear(h);
+  const int b = sort_block(nblk);
+  int64_t lo, hi;
+  sort_range(d.n, b, nblk, lo, hi);
+  const int copy = threadIdx.x & (kHistCopies - 1);
+  cellkeys<KF, RS_T>(d, 0, lo, hi,
+                     [&](uint32_t k) { atomicAdd(&h[(k & mask) * kHistCopies + copy], 1u); });
+  hist_store(d, h, b);
 }
 
-__device__ __forceinline__ bool pass_active(const Dev& d, int pass) {
-  return pass * 8 < (int)d.ctl[C_KEYBITS];
-}
-
-template <bool K32, int NI>
+template <int KF>
 __global__ __launch_bounds__(RS_T) void k_rs_hist(Dev d, int pass, int nblk) {
-  if (!pass_active(d, pass)) return;
-  const SortKey<K32>* keys = key_buf<K32>(d, sort_parity(d, pass));
-  const int shift = pass * 8;
-  const int64_t t0 = (int64_t)blockIdx.x * (RS_T * NI);
-  // all of the thread's keys are loaded at once (an index past the end reads
-  // key 0 and is not counted), so their latencies overlap
-  uint32_t dg[NI];
+  const int np = sort_passes(d);
+  if (pass >= np) return;
+  const SortDigit P = sort_digit(d, pass, np);
+  const SortKey<KF>* kin = key_buf<KF>(d, pass & 1);
+  const int32_t* vin = d.val[pass & 1];
+  const int shift = P.shift;
+  const uint32_t mask = (1u << P.width) - 1;
+  const bool ids = KF == 36 && shift < 4;
+  __shared__ uint32_t h[RS_D * kHistCopies];
+  hist_clear(h);
+  const int copy = threadIdx.x & (kHistCopies - 1);
+  const int b = sort_block(nblk);
+  int64_t lo, hi;
+  sort_range(d.n, b, nblk, lo, hi);
+  constexpr int U = 8;
+  for (int64_t i0 = lo + threadIdx.x; i0 < hi; i0 += U * RS_T) {
+    SortKey<KF> k[U];
+    int32_t v[U];
 #pragma unroll
-  for (int r = 0; r < NI; ++r) {
-    const int64_t i = t0 + r * RS_T + threadIdx.x;
-    dg[r] = (uint32_t)(keys[i < d.n ? i : 0] >> shift) & 255u;
-  }
-  __shared__ uint32_t h[256];
-  h[threadIdx.x] = 0;
-  __syncthreads();
-#pragma unroll
-  for (int r = 0; r < NI; ++r) {
-    const bool v = t0 + r * RS_T + threadIdx.x < d.n;
-    const unsigned long long peers = match8(dg[r], v);
-    if (v && mbcnt(peers) == 0) atomicAdd(&h[dg[r]], (uint32_t)__popcll(peers));
-  }
-  __syncthreads();
-  d.hist[(int64_t)threadIdx.x * nblk + blockIdx.x] = h[threadIdx.x];
-  // the pass runs unless the row scan finds one digit holding every key
-  // (no other block of this launch reads the flag of this pass)
-  if (blockIdx.x == 0 && threadIdx.x == 0) d.pass_scatter[pass] = 1;
-}
-
-// Per-digit row scans, one block per digit: offs[d][b] = keys of digit d in
-// the blocks before b; the block also publishes its digit's total (the
-// scatter derives the digit bases from the 256 totals).  A pass in which one
-// digit holds every key leaves the data in order: that digit's block unmarks
-// the pass, so its scatter is skipped and the buffers are not swapped.
-__global__ __launch_bounds__(256) void k_rs_rowscan(Dev d, int pass, int nblk) {
-  if (!pass_active(d, pass)) return;
-  __shared__ uint32_t s_w[4];
-  __shared__ uint32_t s_carry;
-  if (threadIdx.x == 0) s_carry = 0;
-  const uint32_t* row = d.hist + (int64_t)blockIdx.x * nblk;
-  uint32_t* out = d.offs + (int64_t)blockIdx.x * nblk;
-  // eight chunks' loads in flight per thread, then the chunks scanned in turn
-  constexpr int RU = 8;
-  uint32_t xv[RU];
-  for (int b0 = 0; b0 < nblk; b0 += blockDim.x) {
-    const int u = (b0 / 256) % RU;
-    if (u == 0) {
-#pragma unroll
-      for (int q = 0; q < RU; ++q) {
-        const int bq = b0 + q * 256 + threadIdx.x;
-        xv[q] = row[bq < nblk ? bq : nblk - 1];
-      }
+    for (int u = 0; u < U; ++u) {
+      const int64_t i = i0 + u * RS_T < hi ? i0 + u * RS_T : lo;
+      k[u] = kin[i];
+      v[u] = ids ? vin[i] : 0;
     }
-    int b = b0 + threadIdx.x;
-    uint32_t x = 0;
 #pragma unroll
-    for (int q = 0; q < RU; ++q) x = q == u ? xv[q] : x;
-    x = b < nblk ? x : 0u;
-    uint32_t inc = wave_incl_scan(x);
-    if (lane_id() == 63) s_w[threadIdx.x >> 6] = inc;
-    __syncthreads();
-    uint32_t pre = s_carry;
-    for (int w = 0; w < (int)(threadIdx.x >> 6); ++w) pre += s_w[w];
-    if (b < nblk) out[b] = pre + inc - x;
-    __syncthreads();
-    if (threadIdx.x == 0) s_carry += s_w[0] + s_w[1] + s_w[2] + s_w[3];
-    __syncthreads();
+    for (int u = 0; u < U; ++u)
+      if (i0 + u * RS_T < hi) 
+        atomicAdd(&h[entry_digit<KF>(k[u], v[u], shift, mask) * kHistCopies + copy], 1u);
   }
-  if (threadIdx.x == 0) {
-    d.dtot[blockIdx.x] = s_carry;
-    if ((int64_t)s_carry == d.n) d.pass_scatter[pass] = 0;  // every key has this digit
+  hist_store(d, h, b);
+}
+
+// Counts of the workgroups before each, and the digit totals: a workgroup
+// takes eight digits, 32 segments of the rows each.
+__global__ __launch_bounds__(256) void k_rs_rowscan(Dev d, int pass, int nblk) {
+  if (pass >= sort_passes(d)) return;
+  __shared__ uint32_t s_seg[32][8];
+  const int dg = blockIdx.x * 8 + (threadIdx.x & 7), sg = threadIdx.x >> 3;
+  const int per = (nblk + 31) / 32;
+  const int r0 = sg * per < nblk ? sg * per : nblk, r1 = r0 + per < nblk ? r0 + per : nblk;
+  uint32_t sum = 0;
+#pragma unroll 8
+  for (int r = r0; r < r1; ++r) sum += d.hist[(int64_t)r * RS_D + dg];
+  s_seg[sg][threadIdx.x & 7] = sum;
+  __syncthreads();
+  uint32_t pre = 0;
+  for (int s = 0; s < sg; ++s) pre += s_seg[s][threadIdx.x & 7];
+  if (sg == 31) d.dtot[dg] = pre + sum;
+#pragma unroll 8
+  for (int r = r0; r < r1; ++r) {
+    const uint32_t c = d.hist[(int64_t)r * RS_D + dg];
+    d.offs[(int64_t)r * RS_D + dg] = pre;
+    pre += c;
   }
 }
 
-// Stable scatter.  Each wave owns a contiguous run of 64 * NI keys of the
-// tile and ranks them round by round (64 consecutive keys per round, lanes in
-// order) against counters of its own in LDS, with no barrier between rounds
-// (a wave's LDS accesses complete in order); one barrier later, each digit's
-// counts of the waves before it and the tile's local starts turn the ranks
-// into positions, so equal digits keep their input order.  The tile is
-// staged in LDS in local digit order and written out coalesced per digit run.
-template <bool K32, int NI>
-__global__ __launch_bounds__(RS_T) void k_rs_scatter(Dev d, int pass, int nblk) {
-  using KT = SortKey<K32>;
-  constexpr int TILE = RS_T * NI;
-  if (!pass_active(d, pass) || !d.pass_scatter[pass]) return;
-  const int par = sort_parity(d, pass);
-  const KT* kin = key_buf<K32>(d, par);
-  const int32_t* vin = d.val[par];
-  KT* kout = key_buf<K32>(d, par ^ 1);
-  int32_t* vout = d.val[par ^ 1];
-  const int shift = pass * 8;
+// Exclusive scan over the workgroup's RS_T threads (a barrier inside; s_w is
+// free again after the caller's next barrier).
+__device__ __forceinline__ uint32_t sort_scan(uint32_t v, uint32_t (&s_w)[RS_T / 64]) {
+  const uint32_t inc = wave_incl_scan(v);
+  const int wv = threadIdx.x >> 6;
+  if (lane_id() == 63) s_w[wv] = inc;
+  __syncthreads();
+  uint32_t e = inc - v;
+#pragma unroll
+  for (int w = 0; w < RS_T / 64; ++w) e += w < wv ? s_w[w] : 0u;
+  return e;
+}
+
+// Stable scatter, tile by tile of RS_T * NI entries.  Each wave owns a
+// contiguous run of 64 * NI entries of the tile and ranks them round by round
+// (64 consecutive entries per round, lanes in order) against counters of its
+// own in LDS, with no barrier between rounds (a wave's LDS accesses complete
+// in order); one barrier later each digit's counts of the waves before it and
+// the tile's local starts turn the ranks into positions, so equal digits keep
+// their order.  The tile is staged in LDS in local digit order and written
+// out in runs per digit.  `inline_scan`: few workgroups, which add up the
+// counts before them here instead of in a launch of their own.
+constexpr int kSortInline = 32;
+template <int KF, int NI>
+__global__ __launch_bounds__(RS_T, 4) void k_rs_scatter(Dev d, int pass, int nblk,
+                                                        bool inline_scan) {
+  using KT = SortKey<KF>;
+  constexpr int TILE = RS_T * NI, NW = RS_T / 64;
+  const int np = sort_passes(d);
+  if (pass >= np) return;
+  const SortDigit P = sort_digit(d, pass, np);
+  const KT* kin = key_buf<KF>(d, pass & 1);
+  const int32_t* vin = d.val[pass & 1];
+  KT* kout = key_buf<KF>(d, (pass & 1) ^ 1);
+  int32_t* vout = d.val[(pass & 1) ^ 1];
+  const bool ids = KF != 36 && pass == 0;  // the ids are the positions
+  const int shift = P.shift;
+  const uint32_t mask = (1u << P.width) - 1;
   __shared__ KT s_k[TILE];
   __shared__ int32_t s_v[TILE];
-  __shared__ uint32_t s_lstart[256], s_goff[256];
-  __shared__ uint32_t s_wc[4][256];
-  __shared__ uint32_t s_ws[4], s_wt[4];
+  __shared__ uint32_t s_gd[RS_D];
+  __shared__ uint16_t s_wc[NW][RS_D];
+  __shared__ uint32_t s_w0[NW], s_w1[NW];
   const int tid = threadIdx.x, wv = tid >> 6;
-  const int64_t t0 = (int64_t)blockIdx.x * TILE;
-  const int64_t w0 = t0 + (int64_t)wv * (64 * NI) + lane_id();
-  // the wave's keys and values are loaded at once, before the digit
-  // offsets, so that their latencies overlap (an index past the end reads
-  // element 0, which is not ranked)
+  const int b = sort_block(nblk);
+  int64_t lo, hi;
+  sort_range(d.n, b, nblk, lo, hi);
+  // where this workgroup's next entry of digit tid goes
+  uint32_t pre = 0, tot = 0;
+  if (inline_scan) {
+#pragma unroll 8
+    for (int q = 0; q < nblk; ++q) {
+      const uint32_t c = d.hist[(int64_t)q * RS_D + tid];
+      tot += c;
+      pre += q < b ? c : 0u;
+    }
+  } else {
+    pre = d.offs[(int64_t)b * RS_D + tid];
+    tot = d.dtot[tid];
+  }
+  uint32_t goff = sort_scan(tot, s_w1) + pre;
+  // (32-bit places from here on: ids are 32-bit too)
+  kin += lo;
+  vin += lo;
+  const uint32_t len = (uint32_t)(hi - lo);
   KT kr[NI];
   int32_t vr[NI];
+  auto load = [&](uint32_t t0) {
+    const uint32_t w0 = t0 + wv * (64 * NI) + lane_id();
 #pragma unroll
-  for (int r = 0; r < NI; ++r) {
-    const int64_t i = w0 + r * 64;
-    const int64_t ic = i < d.n ? i : 0;
-    kr[r] = kin[ic];
-    vr[r] = vin[ic];
-  }
-  const uint32_t c = d.hist[(int64_t)tid * nblk + blockIdx.x];
-  const uint32_t off = d.offs[(int64_t)tid * nblk + blockIdx.x];
-  const uint32_t tot = d.dtot[tid];
-#pragma unroll
-  for (int w = 0; w < 4; ++w) s_wc[w][tid] = 0;
-  // the tile's local digit starts (an exclusive scan of its digit counts)
-  // and the digit bases (an exclusive scan of the pass's digit totals)
-  const uint32_t inc = wave_incl_scan(c);
-  const uint32_t inct = wave_incl_scan(tot);
-  if (lane_id() == 63) {
-    s_ws[wv] = inc;
-    s_wt[wv] = inct;
-  }
-  __syncthreads();
-  uint32_t lst = inc - c, base = inct - tot;
-  for (int w = 0; w < wv; ++w) {
-    lst += s_ws[w];
-    base += s_wt[w];
-  }
-  s_lstart[tid] = lst;
-  s_goff[tid] = base + off;
-  uint32_t lr[NI];
-#pragma unroll
-  for (int r = 0; r < NI; ++r) {
-    const bool v = w0 + r * 64 < d.n;
-    const uint32_t dg = (uint32_t)(kr[r] >> shift) & 255u;
-    const unsigned long long peers = match8(dg, v);
-    const uint32_t rank = mbcnt(peers);
-    const uint32_t base = s_wc[wv][dg];
-    if (v && rank == 0) s_wc[wv][dg] = base + (uint32_t)__popcll(peers);
-    lr[r] = base + rank;
-  }
-  __syncthreads();
-  {
-    // position of wave w's first key with digit tid
-    const uint32_t a0 = s_wc[0][tid], a1 = s_wc[1][tid], a2 = s_wc[2][tid];
-    s_wc[0][tid] = lst;
-    s_wc[1][tid] = lst + a0;
-    s_wc[2][tid] = lst + a0 + a1;
-    s_wc[3][tid] = lst + a0 + a1 + a2;
-  }
-  __syncthreads();
-#pragma unroll
-  for (int r = 0; r < NI; ++r) {
-    if (w0 + r * 64 < d.n) {
-      const uint32_t dg = (uint32_t)(kr[r] >> shift) & 255u;
-      const uint32_t lp = s_wc[wv][dg] + lr[r];
-      s_k[lp] = kr[r];
-      s_v[lp] = vr[r];
+    for (int r = 0; r < NI; ++r) {
+      const uint32_t i = w0 + r * 64 < len ? w0 + r * 64 : 0u;
+      kr[r] = kin[i];
+      vr[r] = ids ? (int32_t)(lo + i) : vin[i];
     }
-  }
-  __syncthreads();
-  // write-out: every slot is read (past the tile's end the reads are
-  // unused), the stores are guarded
-  const int64_t tn = (d.n - t0) < TILE ? (d.n - t0) : TILE;
+  };
+  if (len > 0) load(0);
+  for (uint32_t t0 = 0; t0 < len; t0 += TILE) {
+    const uint32_t w0 = t0 + wv * (64 * NI) + lane_id();
 #pragma unroll
-  for (int r = 0; r < NI; ++r) {
-    const int l = r * RS_T + tid;
-    kr[r] = s_k[l];
-    vr[r] = s_v[l];
-  }
+    for (int q = 0; q < RS_D / 64; ++q) s_wc[wv][q * 64 + lane_id()] = 0;
+    uint32_t lr[NI / 2];  // (two 16-bit ranks a register)
 #pragma unroll
-  for (int r = 0; r < NI; ++r) {
-    const int l = r * RS_T + tid;
-    const uint32_t dg = (uint32_t)(kr[r] >> shift) & 255u;
-    const int64_t g = (int64_t)s_goff[dg] + (l - (int)s_lstart[dg]);
-    if (l < tn) {
-      kout[g] = kr[r];
-      vout[g] = vr[r];
+    for (int r = 0; r < NI; ++r) {
+      const bool v = w0 + r * 64 < len;
+      const uint32_t dg = entry_digit<KF>(kr[r], vr[r], shift, mask);
+      const unsigned long long peers = match_digit(dg, P.width, v);
+      const uint32_t rank = mbcnt(peers);
+      const uint32_t base = s_wc[wv][dg];
+      if (v && rank == 0) s_wc[wv][dg] = (uint16_t)(base + (uint32_t)__popcll(peers));
+      lr[r / 2] = r & 1 ? lr[r / 2] | (base + rank) << 16 : base + rank;
+    }
+    __syncthreads();
+    uint32_t cw[NW], c = 0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      cw[w] = s_wc[w][tid];
+      c += cw[w];
+    }
+    uint32_t lst = sort_scan(c, s_w0);
+    s_gd[tid] = goff - lst;
+    goff += c;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      s_wc[w][tid] = (uint16_t)lst;
+      lst += cw[w];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < NI; ++r) {
+      if (w0 + r * 64 < len) {
+        const uint32_t lp = s_wc[wv][entry_digit<KF>(kr[r], vr[r], shift, mask)] +
+                            (r & 1 ? lr[r / 2] >> 16 : lr[r / 2] & 0xffffu);
+        s_k[lp] = kr[r];
+        s_v[lp] = vr[r];
+      }
+    }
+    __syncthreads();
+    // the next tile's entries travel while this one is written out
+    if (t0 + TILE < len) load(t0 + TILE);
+    // every slot is read (past the tile's end the reads are unused), the
+    // stores are guarded
+    const uint32_t tn = len - t0 < TILE ? len - t0 : TILE;
+#pragma unroll 4
+    for (int r = 0; r < NI; ++r) {
+      const uint32_t l = r * RS_T + tid;
+      const KT k = s_k[l];
+      const int32_t v = s_v[l];
+      const uint32_t g = s_gd[entry_digit<KF>(k, v, shift, mask)] + l;
+      if (l < tn) {
+        kout[g] = k;
+        vout[g] = v;
+      }
     }
   }
 }
@@ -717,23 +811,21 @@ constexpr int CS_T = 256;
 constexpr int CS_I = 8;
 constexpr int CS_TILE = CS_T * CS_I;
 
-template <bool K32>
-__device__ __forceinline__ const SortKey<K32>* sorted_keys(const Dev& d) {
-  return key_buf<K32>(d, sort_parity(d, kMaxPasses));
-}
-
 // Sorted keys i and i - 1 of each of a thread's rounds, loaded before any
 // is used (indices clamped into the array) so that the loads are in flight
 // together; key i starts a cell when i < n and it differs from key i - 1.
-template <int NI, typename KT>
-__device__ __forceinline__ void load_key_pairs(const Dev& d, const KT* key, int64_t t0,
-                                               uint64_t (&k)[NI], uint64_t (&kp)[NI]) {
+template <int KF, int NI>
+__device__ __forceinline__ void load_key_pairs(const Dev& d, int64_t t0, uint64_t (&k)[NI],
+                                               uint64_t (&kp)[NI]) {
+  const int par = sort_passes(d) & 1;
+  const SortKey<KF>* key = key_buf<KF>(d, par);
+  const int32_t* val = d.val[par];
 #pragma unroll
   for (int r = 0; r < NI; ++r) {
     const int64_t i = t0 + r * CS_T + threadIdx.x;
-    const int64_t ic = i < d.n ? i : 0;
-    k[r] = key[ic];
-    kp[r] = key[ic > 0 ? ic - 1 : 0];
+    const int64_t ic = i < d.n ? i : 0, ip = ic > 0 ? ic - 1 : 0;
+    k[r] = entry_key<KF>(key[ic], KF == 36 ? val[ic] : 0);
+    kp[r] = entry_key<KF>(key[ip], KF == 36 ? val[ip] : 0);
   }
 }
 
@@ -742,10 +834,10 @@ __device__ __forceinline__ void load_key_pairs(const Dev& d, const KT* key, int6
 // than the table has would be searched for slowly, so the run is abandoned:
 // every later kernel returns at once and the host runs the call again;
 // counting unsorted keys here is harmless)
-template <bool K32>
-__global__ __launch_bounds__(CS_T) void k_csr_count(Dev d, int passes) {
+template <int KF>
+__global__ __launch_bounds__(CS_T) void k_csr_count(Dev d, int bits) {
   if (blockIdx.x == 0 && threadIdx.x == 0 &&
-      (d.ctl[C_KEYBITS] > 8 * passes ||
+      (d.ctl[C_KEYBITS] > bits ||
        (d.line_cap > 0 && d.line_cap < kMaxLineTable && d.ctl[C_NLINES] > d.line_cap)))
     d.ctl[C_ABANDON] = 1;
   if (abandoned(d)) return;
@@ -756,11 +848,10 @@ __global__ __launch_bounds__(CS_T) void k_csr_count(Dev d, int passes) {
     for (int64_t i = (int64_t)blockIdx.x * CS_T + threadIdx.x; i < P;
          i += (int64_t)gridDim.x * CS_T)
       d.lines[i] = make_int2(-1, -1);
-  const auto* key = sorted_keys<K32>(d);
   const int64_t t0 = (int64_t)blockIdx.x * CS_TILE;
   if (t0 >= d.n) return;
   uint64_t kr[CS_I], kp[CS_I];
-  load_key_pairs<CS_I>(d, key, t0, kr, kp);
+  load_key_pairs<KF, CS_I>(d, t0, kr, kp);
   int c = 0;
 #pragma unroll
   for (int r = 0; r < CS_I; ++r) {
@@ -854,17 +945,16 @@ __device__ __forceinline__ int64_t block_prefix(const int64_t* v, int b, bool sc
 
 // Also fills the column table: a cell whose predecessor's key lies below its
 // column's first key starts the column and ends the one before.
-template <bool K32>
+template <int KF>
 __global__ __launch_bounds__(CS_T) void k_csr_write(Dev d, bool scanned) {
   if (abandoned(d)) return;
   const bool table = d.ctl[C_NLINES] <= d.line_cap;
-  const auto* key = sorted_keys<K32>(d);
   const int64_t t0 = (int64_t)blockIdx.x * CS_TILE;
   __shared__ int s_w[4];
   __shared__ int64_t s_run;
   const int wv = threadIdx.x >> 6;
   uint64_t kr[CS_I], kp[CS_I];
-  load_key_pairs<CS_I>(d, key, t0, kr, kp);
+  load_key_pairs<KF, CS_I>(d, t0, kr, kp);
   // every round's instance, column and place, from the
   // instance table before the first store (the stores could alias it as far
   // as the compiler knows, which would hold each round's reads behind the
@@ -957,7 +1047,7 @@ __device__ __forceinline__ void gather_point(const Dev& d, const Inst& I, const 
 // Also the run's state: cluster flags (none), and per expansion wave (`waves`
 // is 0 without seed lists) its pair count and the start of its seeding
 // segment of the cells.
-__global__ __launch_bounds__(256) void k_gather(Dev d, int64_t waves) {
+__global__ __launch_bounds__(256) void k_gather(Dev d, int64_t waves, uint32_t id_mask) {
   if (abandoned(d)) return;
   const int64_t nf = (d.n + 63) / 64, C = d.ctl[C_NCELL];
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < nf || i < waves;
@@ -968,11 +1058,11 @@ __global__ __launch_bounds__(256) void k_gather(Dev d, int64_t waves) {
       d.seg_pos[i] = C * i / waves;
     }
   }
-  const int32_t* vsrc = d.val[sort_parity(d, kMaxPasses)];
+  const int32_t* vsrc = d.val[sort_passes(d) & 1];
   const double* xyz = in_xyz(d);
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < d.n;
        i += (int64_t)gridDim.x * blockDim.x) {
-    const int32_t src = vsrc[i];
+    const int32_t src = (int32_t)((uint32_t)vsrc[i] & id_mask);
     const Inst& I = *inst_of_cell(d, d.ninst == 1 ? 0 : d.cell_of[i]);
     if (I.dim == 3)
       gather_point<3>(d, I, xyz, i, src);
@@ -1401,58 +1491,90 @@ void launch_index_head(const Dev& d, int nchunks, hipStream_t s) {
   if (d.ninst != 1) hipLaunchKernelGGL(k_grid_setup, dim3(1), dim3(1024), 0, s, d);
 }
 
-// Keys per thread of the radix passes over n keys.  A scatter workgroup of
-// 2048 32-bit keys (23 KiB of LDS) shares a CU with five others, one of
-// 4096 keys (39 KiB) with three; a 4096-key tile takes about 1.6x as long.
-// The larger tiles are taken when their rounds of resident workgroups cost
-// less: config 3's 4 M keys run as 977 tiles in one round instead of 1954
-// tiles in two; 1 M keys (one partial round either way) and 32 M keys stay
-// with the smaller tiles.
-int sort_items(bool k32, int64_t n, int cus) {
-  if (!k32 || cus <= 0) return RS_I;
-  const int64_t r2 = (n + 2048 * 6LL * cus - 1) / (2048 * 6LL * cus);
-  const int64_t r4 = (n + 4096 * 4LL * cus - 1) / (4096 * 4LL * cus);
-  return 16 * r4 < 10 * r2 ? 16 : RS_I;
+// Workgroups and entries per thread of the radix passes over n entries: at most
+// kSortGrid workgroups (two per CU; more of them only lengthen the scan), and
+// the largest tile of which each still gets one and a half or more, so that one
+// tile's loads run beside another's write-out.  Scatter of all passes, us, at
+// 2 / 4 / 8 / 16 entries per thread: 10 k points 12 / 15 / 17 / -, 262 k
+// 26 / 30 / 41 / 45, 614 k 37 / 43 / 54 / 84, 1 M 32 / 38 / 45 / 69, 1.5 M
+// 44 / 45 / 60 / 55, 4 M 152 / 112 / 96 / 126, 8 M (batch) 233 / 178 / 171 / 156,
+// 32 M - / 833 / 692 / 622.  (64-bit keys stop at 8: the tile has 12 bytes an
+// entry.)
+constexpr int kSortGrid = 512;
+struct SortShape {
+  int blocks, items;
+};
+SortShape sort_shape(int form, int64_t n) {
+  SortShape s;
+  s.items = form == 64 ? 8 : 16;
+  while (s.items > 2 && 2 * n < 3LL * kSortGrid * RS_T * s.items) s.items /= 2;
+  const int64_t tile = (int64_t)RS_T * s.items;
+  s.blocks = (int)std::max<int64_t>(1, std::min<int64_t>(kSortGrid, (n + tile - 1) / tile));
+  if (s.blocks >= 64) s.blocks &= ~7;  // (XCD-wise ranges)
+  return s;
 }
 
 constexpr int kClearGrid = 1024;
 
-template <bool K32, int NI>
-static void index_sort(const Dev& d, int64_t n, int nchunks, int passes, hipStream_t s) {
-  hipLaunchKernelGGL(k_cellkey<K32>, dim3(nchunks), dim3(256), 0, s, d);
-  const int nblk = (int)((n + RS_T * NI - 1) / (RS_T * NI));
+template <int KF, int NI>
+static void radix_passes(const Dev& d, int passes, int nblk, hipStream_t s) {
+  const bool inl = nblk <= kSortInline;
   for (int p = 0; p < passes; ++p) {
-    hipLaunchKernelGGL((k_rs_hist<K32, NI>), dim3(nblk), dim3(RS_T), 0, s, d, p, nblk);
-    hipLaunchKernelGGL(k_rs_rowscan, dim3(256), dim3(256), 0, s, d, p, nblk);
-    hipLaunchKernelGGL((k_rs_scatter<K32, NI>), dim3(nblk), dim3(RS_T), 0, s, d, p, nblk);
+    if (p > 0 || d.ninst != 1)
+      hipLaunchKernelGGL(k_rs_hist<KF>, dim3(nblk), dim3(RS_T), 0, s, d, p, nblk);
+    if (!inl) hipLaunchKernelGGL(k_rs_rowscan, dim3(RS_D / 8), dim3(256), 0, s, d, p, nblk);
+    hipLaunchKernelGGL((k_rs_scatter<KF, NI>), dim3(nblk), dim3(RS_T), 0, s, d, p, nblk, inl);
   }
+}
+
+template <int KF>
+static void index_sort(const Dev& d, int64_t n, int nchunks, int bits, hipStream_t s) {
+  const int passes = (bits + kDigitBits - 1) / kDigitBits;
+  const SortShape sh = sort_shape(KF, n);
+  if (d.ninst == 1)
+    hipLaunchKernelGGL(k_cellkey_hist<KF>, dim3(sh.blocks), dim3(RS_T), 0, s, d, sh.blocks);
+  else
+    hipLaunchKernelGGL(k_cellkey<KF>, dim3(nchunks), dim3(256), 0, s, d);
+  if (sh.items == 2)
+    radix_passes<KF, 2>(d, passes, sh.blocks, s);
+  else if (sh.items == 4)
+    radix_passes<KF, 4>(d, passes, sh.blocks, s);
+  else if (KF == 64 || sh.items == 8)
+    radix_passes<KF, 8>(d, passes, sh.blocks, s);
+  else
+    radix_passes<KF, KF == 64 ? 8 : 16>(d, passes, sh.blocks, s);
   const int ncs = (int)((n + CS_TILE - 1) / CS_TILE);
   // (the grid also clears the column table: not too small for a large one)
   const int ncc = std::max(ncs, d.line_cap > (1 << 16) ? kClearGrid : 1);
-  hipLaunchKernelGGL(k_csr_count<K32>, dim3(ncc), dim3(CS_T), 0, s, d, passes);
+  hipLaunchKernelGGL(k_csr_count<KF>, dim3(ncc), dim3(CS_T), 0, s, d,
+                     std::min(KF, kDigitBits * passes));
   const bool scan = ncs > kScanInline;
   if (scan)
     hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(1024), 0, s, d.scan_tmp, ncs,
                        (long long*)nullptr);
-  hipLaunchKernelGGL(k_csr_write<K32>, dim3(ncs), dim3(CS_T), 0, s, d, scan);
+  hipLaunchKernelGGL(k_csr_write<KF>, dim3(ncs), dim3(CS_T), 0, s, d, scan);
 }
 
-// `passes` radix passes: keys of at most 32 bits (four passes) are sorted as
-// 32-bit keys
-void launch_index_sort(const Dev& d, int64_t n, int nchunks, int passes, int cus, hipStream_t s) {
-  if (passes > 4)
-    index_sort<false, RS_I>(d, n, nchunks, passes, s);
-  else if (sort_items(true, n, cus) == 16)
-    index_sort<true, 16>(d, n, nchunks, passes, s);
+// the sort's form for keys of `bits` bits over n points
+static int sort_form(int64_t n, int bits) {
+  return bits <= 32 ? 32 : bits <= 36 && n <= (int64_t)kIdMask + 1 ? 36 : 64;
+}
+
+void launch_index_sort(const Dev& d, int64_t n, int nchunks, int bits, hipStream_t s) {
+  const int form = sort_form(n, bits);
+  if (form == 32)
+    index_sort<32>(d, n, nchunks, bits, s);
+  else if (form == 36)
+    index_sort<36>(d, n, nchunks, bits, s);
   else
-    index_sort<true, RS_I>(d, n, nchunks, passes, s);
+    index_sort<64>(d, n, nchunks, bits, s);
 }
 
-void launch_gather(const Dev& d, int64_t n, int64_t waves, hipStream_t s) {
+void launch_gather(const Dev& d, int64_t n, int64_t waves, int bits, hipStream_t s) {
   // random-access gather: more blocks in flight than a fill needs
   const int64_t gb = (n + 255) / 256;
   hipLaunchKernelGGL(k_gather, dim3((int)std::max<int64_t>(1, std::min<int64_t>(16384, gb))),
-                     dim3(256), 0, s, d, waves);
+                     dim3(256), 0, s, d, waves, sort_form(n, bits) == 36 ? kIdMask : ~0u);
 }
 
 // Row pass grid: one wavefront per (tile of 64 cells, group) for up
@@ -1476,7 +1598,11 @@ void launch_rows(const Dev& d, int64_t n, int grid_cells, hipStream_t s) {
   if (d.nbr_stats) hipLaunchKernelGGL(k_nbr_stats, dim3((unsigned)gb), dim3(256), 0, s, d);
 }
 
-int64_t sort_hist_entries(int64_t n) { return 256 * ((n + RS_TILE - 1) / RS_TILE); }
+// digit counts of the workgroups: room for any form of the keys
+int64_t sort_hist_entries(int64_t n) {
+  return (int64_t)RS_D * std::max(sort_shape(32, n).blocks,
+                                  std::max(sort_shape(36, n).blocks, sort_shape(64, n).blocks));
+}
 int64_t scan_tmp_entries(int64_t n) { return (n + CS_TILE - 1) / CS_TILE + 16; }
 
 }  // namespace dclust

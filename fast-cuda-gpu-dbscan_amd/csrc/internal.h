@@ -287,7 +287,7 @@ struct PairList {
 // Sort-pass bookkeeping: pass p is active when p*8 < key bits; its scatter
 // runs unless every key has the same digit (then the data is already in
 // order and the buffers are not swapped).
-constexpr int kMaxPasses = 8;
+constexpr int kDigitBits = 9;  // of a radix pass, at most
 
 // Bounding-box partials: chunk b reduces into stripe b % kBoxStripes of its
 // instance (so that the atomics of many chunks do not meet on one address);
@@ -322,10 +322,9 @@ struct Dev {
   // radix sort
   uint64_t* key[2];
   int32_t* val[2];
-  uint32_t* hist;   // [256][nblk] digit-major block histograms
-  uint32_t* offs;   // [256][nblk] scanned offsets
-  uint32_t* dtot;   // [256] digit totals of the current pass
-  int32_t* pass_scatter;  // [kMaxPasses] 1 if the scatter of pass p ran
+  uint32_t* hist;   // [nblk][512] digit counts of the sort's workgroups
+  uint32_t* offs;   // [nblk][512] digit counts of the workgroups before
+  uint32_t* dtot;   // [512] digit totals of the current pass
 
   // CSR
   int32_t* cell_start;  // [N+1]

@@ -10,12 +10,11 @@ void launch_init_head(const Dev& d, const Call* src, const Call& v, hipStream_t 
 void launch_readback(const Dev& d, long long* out, hipStream_t s);
 // bbox + grid set-up (per-instance cell width, cells per axis, key space)
 void launch_index_head(const Dev& d, int nchunks, hipStream_t s);
-// the index after the grid set-up, in two parts: cell keys, `passes` radix
-// passes, CSR compaction and column table (tile size from the CU count
-// `cus`); the gather of the coordinates, and the start of the run's state for
-// `waves` expansion waves
-void launch_index_sort(const Dev& d, int64_t n, int nchunks, int passes, int cus, hipStream_t s);
-void launch_gather(const Dev& d, int64_t n, int64_t waves, hipStream_t s);
+// the index after the grid set-up, in two parts: cell keys, the sort for keys
+// of at most `bits` bits, CSR compaction and column table; the gather of the
+// coordinates, and the start of the run's state for `waves` expansion waves
+void launch_index_sort(const Dev& d, int64_t n, int nchunks, int bits, hipStream_t s);
+void launch_gather(const Dev& d, int64_t n, int64_t waves, int bits, hipStream_t s);
 // neighbour rows of every cell (k_rows)
 void launch_rows(const Dev& d, int64_t n, int grid_cells, hipStream_t s);
 int64_t sort_hist_entries(int64_t n);
