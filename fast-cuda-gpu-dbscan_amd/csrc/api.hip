@@ -852,11 +852,8 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
     // striped work lists: sub-list capacity = the most its workgroups append
     const int64_t cap_p = (point_blocks(ntot) + kStripes - 1) / kStripes * 256;
     const int64_t cap_c = (cell_blocks(ntot) + kStripes - 1) / kStripes * 1024;
-    const int64_t cap_n = list_append_cap(ntot);
-    // non-core points are appended by three passes, each of at most all points
-    const int64_t cap_b = cap_p + 2 * cap_n;
-    d.border_pts = SList{M.get<int32_t>(S_BORDERPTS, (size_t)cap_b * kStripes),
-                         (unsigned long long*)(d.stat + C_NBORDERPTS), cap_b};
+    d.border_pts = SList{M.get<int32_t>(S_BORDERPTS, (size_t)cap_p * kStripes),
+                         (unsigned long long*)(d.stat + C_NBORDERPTS), cap_p};
     d.core_cells = SList{M.get<int32_t>(S_CORECELLS, (size_t)cap_c * kStripes),
                          (unsigned long long*)(d.stat + C_NCORECELLS), cap_c};
     const int64_t cap_r = row_list_cap(ntot);
@@ -880,17 +877,17 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
     if (rec_stride > 0) d.rec = M.get<int32_t>(S_REC, (size_t)ntot * rec_stride);
     d.parent = M.get<int32_t>(S_PARENT, ntot);
     // the component minima, before them the list of points with many candidates
-    d.compmin = M.get<int32_t>(S_COMPMIN, (size_t)std::max(ntot, cap_n * kStripes));
-    d.core_crowd = SList{d.compmin, (unsigned long long*)(d.stat + C_NCORECROWD), cap_n};
+    d.compmin = M.get<int32_t>(S_COMPMIN, (size_t)std::max(ntot, cap_p * kStripes));
+    d.core_crowd = SList{d.compmin, (unsigned long long*)(d.stat + C_NCORECROWD), cap_p};
     const int64_t waves = shape.chains ? shape.waves : 0;
     d.pairs = M.get<int2>(S_PAIRS, d.pair_cap);
     d.pair_cnt = M.get<int32_t>(S_PAIRCNT, waves);
     d.seg_pos = M.get<int64_t>(S_SEGPOS, waves);
     // the first queue, then (from k_comp on) the list of the near roots
-    d.q[0] = M.get<int32_t>(S_Q0, (size_t)std::max(ntot, cap_n * kStripes));
+    d.q[0] = M.get<int32_t>(S_Q0, (size_t)std::max(ntot, cap_c * kStripes));
     d.q[1] = M.get<int32_t>(S_Q1, shape.chains ? ntot : 0);
     d.near_roots = SList{d.q[0], (unsigned long long*)(d.stat + C_NROOTS),
-                         cap_n};
+                         cap_c};
     // the component keys, before them the list of points the first count pass
     // leaves
     d.keyv = M.get<int32_t>(S_KEYV, (size_t)std::max(ntot, cap_p * kStripes));

@@ -167,27 +167,37 @@ __device__ __forceinline__ bool edge_pair(const Dev& d, const Par& P, int32_t a,
 //                 listed for k_core_rest.  The count needs no records, and in the FP32 form no
 //                 guard band (a pair inside it is left to the list), so the
 //                 kernel is small enough for full residency.
-//   k_core_rest   one lane per listed point: the exact count over all of its
-//                 rows with early exit at minpts.  Every candidate with d^2 <=
-//                 eps^2 (either box direction) is recorded, so a point that
-//                 ends non-core holds all its neighbours outside its own cell
-//                 (records are kept slot by slot, so that neighbouring lanes
-//                 write neighbouring words).
+//   k_core_rest   two or four lanes per listed point: the exact count over all
+//                 of its rows with early exit at minpts.  Every candidate with
+//                 d^2 <= eps^2 (either box direction) is recorded, so a point
+//                 that ends non-core holds all its neighbours outside its own
+//                 cell (records are kept slot by slot, so that neighbouring
+//                 points write neighbouring words).
 //   k_core_crowd  one wavefront per listed point with more than kCoreCrowd
-//                 candidates: one lane would take as long as the rest of the
-//                 launch.
+//                 candidates (a few lanes would take as long as the rest of the
+//                 launch), and in the FP32 form per point that a pair inside the
+//                 guard band decides.
 //
-// 4 M 3-D points, FP32 form: 166 + 172 + 4 us, where one kernel over lines of
-// five cells took 490 (and one kernel with all of this at 80 registers, 31 of
-// them spilled, 636); 32 M points: 240 + 127 + 155 where it took 615 (3.6 ms
-// with whole windows and no wavefront pass: a window's points start two steps
-// below the cell, so crowded windows end late); 1 M 2-D points, FP64: 20 + 17
-// where it took 57.
+// Both passes over points are bound by the rows and coordinates they fetch at
+// random: neighbouring points name the same ones, so each XCD takes runs of
+// kXcdRun workgroups of points, and the lists of k_core are walked on the XCD
+// that filled them.  k_core / k_core_rest / k_core_crowd, us: 4 M 3-D points,
+// FP32 form, 147 / 145 / 18 (with whole eighths of the points per XCD, lists
+// walked in order and a lane per listed point 162 / 204 / 5); the batch of 7 M
+// points 198 / 179 / 18 (233 / 270 / 33); 262 k dense 3-D points, FP64 form,
+// 29 / 47 / 10 (31 / 110 / 18); 100 k 3-D points, FP32 form, 14 / 15 / 4 (13 /
+// 47 / 4).  Lists walked with whole eighths per XCD suit the batch but not one
+// clustered instance, whose work then sits on few XCDs (4 M: 214 us).
 //
 // A row's points are consecutive; those of the few cells of a row outside the
-// 5^D stencil fail the distance test.  The non-empty point ranges of a lane
-// wait in a queue of its own in LDS, so that every lane goes on to its next
-// range as soon as it is done with one, whatever the other lanes are at.
+// 5^D stencil fail the distance test.  The non-empty point ranges of a point
+// wait in a queue of its own in LDS, so that its lanes go on to the next range
+// as soon as they are done with one, whatever the others are at.
+constexpr int kXcdRun = 64;
+// points from which two lanes share a listed point instead of four: with fewer,
+// the chain of loads of one point sets the time (262 k points 47 us against
+// 67), with more the work does (4 M 166 against 145; 614 k 27 against 26)
+constexpr int64_t kRestQuad = 1 << 19;
 constexpr int kCoreBudget = 64;   // candidates k_core tests per point
 constexpr int kCoreCrowd = 512;   // candidates from which a wavefront takes a point
 
@@ -289,7 +299,7 @@ __global__ __launch_bounds__(256, F32 ? 8 : 6) void k_core(Dev d) {
   if (abandoned(d)) return;
   stamp(d, C_T_CORE0);
   __shared__ int2 s_queue[4 * 256];
-  const int64_t pl = (int64_t)xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+  const int64_t pl = (int64_t)xcd_runs<kXcdRun>(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
   const bool act = pl < d.n;
   const int32_t p = act ? (int32_t)pl : 0;
   int32_t c = 0, qs = 0, own = 0;
@@ -343,96 +353,207 @@ __device__ __forceinline__ void core_pred(const Dev& d, const Par& P, int32_t p,
   }
 }
 
-// 0: not core, 1: core, 2: left to a wavefront
-template <int D, bool F32>
-__device__ int core_rest(const Dev& d, const Par& P, int32_t p, int R, int2* queue, int32_t* lrec,
-                         Tally& t) {
-  constexpr int NR = Win<D>::rows;
-  constexpr int B = kCoreBatch;
+// Block offsets of row i in units of the near sides (core_row for an i that is
+// not a constant; 1 + offset in two bits).
+template <int D>
+__device__ __forceinline__ void row_sides(int i, int& oa, int& ob) {
+  constexpr uint32_t a3 = 0x08499u, b3 = 0x021A5u, a2 = 0x09u;
+  oa = (int)(((D == 3 ? a3 : a2) >> (2 * i)) & 3u) - 1;
+  ob = D == 3 ? (int)((b3 >> (2 * i)) & 3u) - 1 : 0;
+}
+
+// Squared distances (fixed-point units) from a point to what its rows hold, by
+// axis: to the blocks on the near and the far side, and to the cells one and
+// two steps below and above.  The cells of a row beyond eps of the point are
+// those of its first and last steps, so what is left is again one range of
+// points: 132 of the 180 cells of a 3-D stencil's rows on average.  The
+// distances use the arithmetic of d2fix, so d2_out bounds them.
+template <int D>
+struct Reach {
+  float xn, xf, yn, yf, below1, below2, above1, above2;
+  __device__ __forceinline__ Reach(const uint32_t* g, int local) {
+    constexpr uint32_t W = 1u << kFixBits, F = W - 1u;
+    const uint32_t fx = g[0] & F, fl = g[D - 1] & F;
+    const bool lx = D == 3 ? (local & 2) : (local & 1);
+    xn = sq(lx ? W - fx : fx);
+    xf = sq(lx ? W + fx : 2u * W - fx);
+    yn = yf = 0.f;
+    if (D == 3) {
+      const uint32_t fy = g[1] & F;
+      yn = sq(local & 1 ? W - fy : fy);
+      yf = sq(local & 1 ? W + fy : 2u * W - fy);
+    }
+    below1 = sq(fl);
+    below2 = sq(fl + W);
+    above1 = sq(W - fl);
+    above2 = sq(2u * W - fl);
+  }
+  static __device__ __forceinline__ float sq(uint32_t v) {
+    const float f = (float)(int32_t)v;
+    return f * f;
+  }
+  // slots of the row on sides (oa, ob) that the point may reach
+  __device__ __forceinline__ uint32_t slots(int oa, int ob, float d2_out) const {
+    constexpr int nl = Win<D>::nl;
+    const float s = (oa == 0 ? 0.f : oa > 0 ? xn : xf) + (ob == 0 ? 0.f : ob > 0 ? yn : yf);
+    const int lo = s + below2 <= d2_out ? 0 : s + below1 <= d2_out ? 1 : 2;
+    const int hi = s + above2 <= d2_out ? 5 : s + above1 <= d2_out ? 4 : 3;
+    return s > d2_out ? 0u : ((1u << (hi * nl)) - 1u) & ~((1u << (lo * nl)) - 1u);
+  }
+};
+
+// points of the row's cells in a run of slots: [a, e)
+__device__ __forceinline__ void row_points_in(const Dev& d, uint2 row, uint32_t slots, int32_t& a,
+                                              int32_t& e) {
+  a = e = 0;
+  const uint32_t in = row.y & slots;
+  if (in) {
+    const int32_t m0 = (int32_t)row.x + __popc(row.y & ((slots & (0u - slots)) - 1u));
+    a = d.cell_start[m0];
+    e = d.cell_start[m0 + __popc(in)];
+  }
+}
+
+// Count of p over all of its rows by the Q lanes that share it.  0:
+// not core, 1: core, 2: left to a wavefront (many candidates, or in the FP32
+// form a pair inside the guard band that the others do not make up for: the
+// exact test costs 20 registers).
+template <int D, bool F32, int Q>
+__device__ int core_rest(const Dev& d, const Par& P, int32_t p, int R,
+                         int2* ranges, int32_t* lrec, Tally& t) {
+  constexpr int NR = Win<D>::rows, NK = (NR + Q - 1) / Q;
+  constexpr int B = 8 / Q;
+  const int sub = lane_id() & (Q - 1), q0 = lane_id() & ~(Q - 1);
+  // the group's bits of a ballot
+  const auto mine = [&](unsigned long long m) {
+    return ((q0 & 32 ? (uint32_t)(m >> 32) : (uint32_t)m) >> (q0 & 31)) & ((1u << Q) - 1u);
+  };
+  const uint32_t below = (1u << sub) - 1u;
   const int32_t c = d.cell_of[p];
   const int32_t qs = d.cell_start[c], own = d.cell_start[c + 1] - qs;
   int ax, ay;
-  near_sides<D>((int)(d.cell_zl[c] & (Win<D>::nl - 1)), ax, ay);
+  const int local = (int)(d.cell_zl[c] & (Win<D>::nl - 1));
+  near_sides<D>(local, ax, ay);
+  uint32_t pg[D];
+  load_g<D>(d, p, pg);
   const RowsOf rows = rows_of(d, c);
-  int32_t a[NR], e[NR];
+  int32_t a[NK], e[NK];
   {
-    uint2 row[NR];
+    uint2 row[NK];
 #pragma unroll
-    for (int r = 0; r < NR; ++r) row[r] = rows[core_row<D>(r, ax, ay)];
+    for (int k = 0; k < NK; ++k) {
+      const int r = k * Q + sub;
+      row[k] = make_uint2(0u, 0u);
+      if (r < NR) {
+        int oa, ob;
+        row_sides<D>(r, oa, ob);
+        row[k] = rows[Win<D>::own + (D == 3 ? 3 * oa * ax + ob * ay : oa * ax)];
+      }
+    }
+    const Reach<D> reach(pg, local);
 #pragma unroll
-    for (int r = 0; r < NR; ++r) row_points(d, row[r], a[r], e[r]);
+    for (int k = 0; k < NK; ++k) {
+      int oa, ob;
+      row_sides<D>(k * Q + sub, oa, ob);
+      row_points_in(d, row[k], reach.slots(oa, ob, P.d2_out), a[k], e[k]);
+    }
   }
   int nq = 0;
   int32_t tot = 0;  // (the own cell's points included)
 #pragma unroll
-  for (int r = 0; r < NR; ++r)
-    if (e[r] > a[r]) {
-      queue[256 * nq++] = make_int2(a[r], e[r]);
-      tot += e[r] - a[r];
-    }
-  t.rows += NR;
-  t.ranges += nq;
+  for (int k = 0; k < NK; ++k) {
+    const uint32_t m = mine(ballot(e[k] > a[k]));
+    if (e[k] > a[k]) ranges[nq + __popc(m & below)] = make_int2(a[k], e[k]);
+    nq += __popc(m);
+    tot += e[k] - a[k];
+  }
+#pragma unroll
+  for (int o = 1; o < Q; o <<= 1) tot += __shfl_xor(tot, o, 64);
+  if (sub == 0) {
+    t.rows += NR;
+    t.ranges += nq;
+  }
   if (tot > kCoreCrowd) return 2;
+  wave_sync();  // the ranges, before the lanes read each other's
   int nrec = 0;
-  uint32_t pg[D];
   double px[D];
-  if (F32)
-    load_g<D>(d, p, pg);
-  else
-    load_x<D, F32>(d, p, px);
-  int cnt = own, j = 0;
-  int2 cur = make_int2(0, 0);
-  while (cnt < P.minpts && (cur.x < cur.y || j < nq)) {
-    if (cur.x >= cur.y) cur = queue[256 * j++];
+  if (!F32) load_x<D, F32>(d, p, px);
+  // the ranges one after the other, the lanes side by side
+  bool band = false;
+  int cnt = own, j = 0;  // cnt: own + nrec, less what only one box test finds
+  int2 cur = ranges[0];
+  int32_t at = cur.x + sub;
+  for (int32_t i0 = sub; i0 - sub < tot && cnt < P.minpts; i0 += Q * B) {
     int32_t qi[B];
     uint32_t cg[B][D];
     double cx[B][D];
 #pragma unroll
     for (int u = 0; u < B; ++u) {
-      qi[u] = cur.x + u < cur.y ? cur.x + u : qs;  // (not counted, as above)
+      while (at >= cur.y && j + 1 < nq) {
+        at -= cur.y;
+        cur = ranges[++j];
+        at += cur.x;
+      }
+      // past the end: a point of the own cell, which is not counted
+      qi[u] = i0 + u * Q < tot ? at : qs;
+      at += Q;
       if (F32)
         load_g<D>(d, qi[u], cg[u]);
       else
         load_x<D, F32>(d, qi[u], cx[u]);
     }
 #pragma unroll
-    for (int u = 0; u < B; ++u)
+    for (int u = 0; u < B; ++u) {
+      bool sym = false, fwd = false;
       if ((uint32_t)(qi[u] - qs) >= (uint32_t)own) {
-        bool sym, fwd;
-        core_pred<D, F32>(d, P, p, qi[u], pg, cg[u], px, cx[u], sym, fwd, t);
-        cnt += fwd;
-        if (sym) {
-          if (nrec < R) lrec[nrec] = qi[u];
-          ++nrec;
+        if (F32) {
+          const float sd = d2fix<D>(pg, cg[u]);
+          sym = fwd = sd < P.d2_in;
+          band |= !(sd < P.d2_in) && !(sd > P.d2_out);
+        } else {
+          core_pred<D, F32>(d, P, p, qi[u], pg, cg[u], px, cx[u], sym, fwd, t);
         }
         ++t.eval;
       }
-    cur.x += B;
+      const uint32_t m = mine(ballot(sym));
+      const int slot = nrec + __popc(m & below);
+      if (sym && slot < R) lrec[slot] = qi[u];
+      nrec += __popc(m);
+      cnt += __popc(m);
+      if (!F32)
+        if (const unsigned long long one = ballot(sym && !fwd)) cnt -= __popc(mine(one));
+    }
   }
   if (cnt >= P.minpts) return 1;
-  for (int i = 0; i < nrec && i < R; ++i) d.rec[(int64_t)i * d.n + p] = lrec[i];
-  d.rec_n[p] = (uint8_t)(nrec <= R ? nrec : kRecNone);
+  if (F32 && mine(ballot(band))) return 2;
+  wave_sync();
+  for (int i = sub; i < nrec && i < R; i += Q) d.rec[(int64_t)i * d.n + p] = lrec[i];
+  if (sub == 0) d.rec_n[p] = (uint8_t)(nrec <= R ? nrec : kRecNone);
   return 0;
 }
 
-// LDS of a k_core_rest workgroup: per lane nine ranges, and R record slots
-// (one more: no bank conflicts)
-static size_t core_lds(int R) { return 256 * (kMaxRows * sizeof(int2) + (R + 1) * 4); }
+// LDS of a k_core_rest workgroup: per point nine ranges, and R record slots
+// (one more: fewer bank conflicts)
+static size_t core_lds(int R, int Q) {
+  return 256 / Q * (kMaxRows * sizeof(int2) + (R + 1) * 4);
+}
 
-template <bool F32>
-__global__ __launch_bounds__(256, F32 ? 6 : 5) void k_core_rest(Dev d) {
+template <bool F32, int Q>
+__global__ __launch_bounds__(256, (F32 ? 7 : 5) + (Q == 4)) void k_core_rest(Dev d) {
   if (abandoned(d)) return;
   extern __shared__ int2 s_core[];
-  __shared__ long long s_pre[kStripes + 1];
-  const long long n = slist_prefix(d.core_rest, s_pre);
+  constexpr int PB = 256 / Q;  // points of a workgroup
+  const Stripe L(d.core_rest);
   const int R = d.rec_stride;
-  int2* queue = s_core + threadIdx.x;
-  int32_t* lrec = reinterpret_cast<int32_t*>(s_core + 256 * kMaxRows) + threadIdx.x * (R + 1);
+  const int pt = threadIdx.x / Q;
+  const bool lead = threadIdx.x % Q == 0;
+  int2* ranges = s_core + pt * kMaxRows;
+  int32_t* lrec = reinterpret_cast<int32_t*>(s_core + PB * kMaxRows) + pt * (R + 1);
   Tally t;
-  for (long long i0 = (long long)blockIdx.x * 256; i0 < n; i0 += (long long)gridDim.x * 256) {
-    const long long i = i0 + threadIdx.x;
-    const bool act = i < n;
-    const int32_t p = act ? slist_at(d.core_rest, s_pre, i) : 0;
+  for (int64_t i0 = L.first(PB); i0 < L.n; i0 += L.step(PB)) {
+    const int64_t i = i0 + pt;
+    const bool act = i < L.n;
+    const int32_t p = act ? L.data[i] : 0;
     const Inst* I = d.inst;
     int dim = 0;
     if (act) {
@@ -441,16 +562,13 @@ __global__ __launch_bounds__(256, F32 ? 6 : 5) void k_core_rest(Dev d) {
     }
     const Par P(*I);
     int res = 0;
-    DCLUST_BY_DIM(act, dim, (res = core_rest<3, F32>(d, P, p, R, queue, lrec, t)),
-                  (res = core_rest<2, F32>(d, P, p, R, queue, lrec, t)));
-    if (act && res == 1) d.core[p] = 1;
-    block_append(act && res == 0, p, d.border_pts);
-    block_append(act && res == 2, p, d.core_crowd);
+    DCLUST_BY_DIM(act, dim, (res = core_rest<3, F32, Q>(d, P, p, R, ranges, lrec, t)),
+                  (res = core_rest<2, F32, Q>(d, P, p, R, ranges, lrec, t)));
+    if (act && lead && res == 1) d.core[p] = 1;
+    block_append(act && lead && res == 0, p, d.border_pts);
+    block_append(act && lead && res == 2, p, d.core_crowd);
   }
   stat_add(d, C_EVAL, t.eval);
-  stat_add(d, C_BAND_CORE, t.band);
-  stat_add(d, C_BAND, t.band);
-  stat_add(d, C_FLIP, t.flip);
   stat_add(d, C_CORE_ROWS, t.rows);
   stat_add(d, C_CORE_RANGES, t.ranges);
 }
@@ -462,18 +580,21 @@ __device__ bool core_wave(const Dev& d, const Par& P, int32_t p, int R, Tally& t
   const int32_t c = d.cell_of[p];
   const int32_t qs = d.cell_start[c], own = d.cell_start[c + 1] - qs;
   int ax, ay;
-  near_sides<D>((int)(d.cell_zl[c] & (Win<D>::nl - 1)), ax, ay);
+  const int local = (int)(d.cell_zl[c] & (Win<D>::nl - 1));
+  near_sides<D>(local, ax, ay);
   const RowsOf rows = rows_of(d, c);
   uint32_t pg[D];
   double px[D];
-  if (F32)
-    load_g<D>(d, p, pg);
-  else
-    load_x<D, F32>(d, p, px);
+  load_g<D>(d, p, pg);
+  if (!F32) load_x<D, F32>(d, p, px);
+  const Reach<D> reach(pg, local);
   int cnt = own, nrec = 0;
   for (int r = 0; r < NR && cnt < P.minpts; ++r) {
     int32_t a, e;
-    row_points(d, rows[core_row<D>(r, ax, ay)], a, e);
+    int oa, ob;
+    row_sides<D>(r, oa, ob);
+    row_points_in(d, rows[Win<D>::own + (D == 3 ? 3 * oa * ax + ob * ay : oa * ax)],
+                  reach.slots(oa, ob, P.d2_out), a, e);
     for (; a < e && cnt < P.minpts; a += 64) {
       const int32_t q = a + lane < e ? a + lane : qs;
       uint32_t qg[D];
@@ -501,13 +622,11 @@ __device__ bool core_wave(const Dev& d, const Par& P, int32_t p, int R, Tally& t
 template <bool F32>
 __global__ __launch_bounds__(256) void k_core_crowd(Dev d) {
   if (abandoned(d)) return;
-  __shared__ long long s_pre[kStripes + 1];
-  const long long n = slist_prefix(d.core_crowd, s_pre);
+  const Stripe L(d.core_crowd);
   const int R = d.rec_stride;
   Tally t;
-  for (long long i = (long long)blockIdx.x * 4 + (threadIdx.x >> 6); i < n;
-       i += (long long)gridDim.x * 4) {
-    const int32_t p = rfl_i(slist_at(d.core_crowd, s_pre, i));
+  for (int64_t i = L.first(4) + (threadIdx.x >> 6); i < L.n; i += L.step(4)) {
+    const int32_t p = rfl_i(L.data[i]);
     const Inst& I = *inst_of_cell(d, d.ninst == 1 ? 0 : d.cell_of[p]);
     const Par P(I);
     const bool isc = I.dim == 3 ? core_wave<3, F32>(d, P, p, R, t)
@@ -516,9 +635,9 @@ __global__ __launch_bounds__(256) void k_core_crowd(Dev d) {
       if (isc) {
         d.core[p] = 1;
       } else {
-        const SList& L = d.border_pts;
+        const SList& B = d.border_pts;
         const int s = blockIdx.x & (kStripes - 1);
-        L.data[s * L.cap + (int64_t)atomicAdd(&L.cnt[s * kStatStride], 1ull)] = p;
+        B.data[s * B.cap + (int64_t)atomicAdd(&B.cnt[s * kStatStride], 1ull)] = p;
       }
     }
   }
@@ -695,18 +814,50 @@ __device__ __forceinline__ int local_of(const Dev& d, int32_t c, int dim) {
   return (int)(d.cell_zl[c] & (dim == 3 ? 3u : 1u));
 }
 
+// The rows that hold a cell's forward near cells (bits above kNearOwn), loaded
+// once: the loops over mask bits then wait for no row.
+struct NearRows {
+  uint32_t ox, oy, x0x, x0y, xbx, xby, y1x, y1y;
+  int dim, local, gb;  // gb: the group of three bits whose row is xb
+};
+__device__ __forceinline__ NearRows near_rows(const Dev& d, int32_t A, int dim) {
+  const RowsOf rows = rows_of(d, A);
+  const int local = local_of(d, A, dim);
+  const int lx = local >> 1, nb = local & 1 ? 1 : -1;
+  const bool d3 = dim == 3;
+  const uint2 own = rows[d3 ? 4 : 1], x0 = rows[d3 ? 4 + 3 * lx : 1 + local],
+              xb = rows[d3 ? 4 + 3 * lx + nb : 1 + local], y1 = rows[d3 ? 4 + (local & 1) : 1];
+  return NearRows{own.x, own.y, x0.x, x0.y, xb.x, xb.y, y1.x, y1.y, dim, local, d3 ? 7 + nb : -1};
+}
+__device__ __forceinline__ uint32_t pick(bool c, uint32_t a, uint32_t b) {
+  const uint32_t m = 0u - (uint32_t)c;  // (a ?: of two fields goes through scratch)
+  return (a & m) | (b & ~m);
+}
+// forward near cell at bit b
+__device__ __forceinline__ int32_t near_cell(const NearRows& n, int b) {
+  const int g = (b * 11) >> 5;  // b / 3 for b < 27
+  int row, slot;
+  if (n.dim == 3)
+    near_slot<3>(b, n.local, row, slot);
+  else
+    near_slot<2>(b, n.local, row, slot);
+  uint2 r;
+  r.x = pick(g == 4, n.ox, pick(g == 5, n.y1x, pick(g == n.gb, n.xbx, n.x0x)));
+  r.y = pick(g == 4, n.oy, pick(g == 5, n.y1y, pick(g == n.gb, n.xby, n.x0y)));
+  return slot_cell(r, slot);
+}
+
 // One lane per core cell.  For the expansion by seed lists each bit of A is
 // also set in the other cell's mask, at the opposite offset.
 __global__ __launch_bounds__(256) void k_adj(Dev d) {
   if (abandoned(d)) return;
-  __shared__ long long s_pre[kStripes + 1];
-  const long long n = slist_prefix(d.core_cells, s_pre);
+  const Stripe L(d.core_cells);
   Tally t;
   long long edges = 0;
-  for (long long i0 = (long long)blockIdx.x * 256; i0 < n; i0 += (long long)gridDim.x * 256) {
-    const long long i = i0 + threadIdx.x;
-    const bool act = i < n;
-    const int32_t A = act ? slist_at(d.core_cells, s_pre, i) : 0;
+  for (int64_t i0 = L.first(256); i0 < L.n; i0 += L.step(256)) {
+    const int64_t i = i0 + threadIdx.x;
+    const bool act = i < L.n;
+    const int32_t A = act ? L.data[i] : 0;
     int dim = 0;
     float d2_in = 0.f;
     if (act) {
@@ -740,15 +891,24 @@ __global__ __launch_bounds__(256) void k_adj(Dev d) {
 // pairs inside it in an LDS copy of the forest, then writes every cell's
 // root; the bits that leave the run stay in the masks.  k_link_cross unites
 // those in global memory, between roots only.  (All pairs in global memory
-// took 1.65-2.1 ms on the 4 M point 3-D workload, against 95 + 87 us: cells
+// took 1.65-2.1 ms on the 4 M point 3-D workload, against 61 + 64 us: cells
 // of a cluster hook each other link by link into chains that every find then
 // walks with loads past the L2, which is not coherent across XCDs.  Without
-// the runs of the first step k_link_local took 33 us instead of 22 on 10 k
-// 2-D points; without its table of pairs k_link_cross took 150 us, and 114
-// with links by id instead of uf_order.)
+// its table of pairs k_link_cross took 150 us, and 114 with links by id
+// instead of uf_order.)
+//
+// A thread unites the pairs of its cells one after the other, so short runs
+// and many workgroups pay until the pairs between runs weigh more: runs of at
+// least 4096 cells on 512 workgroups took 104 + 61 us on the 4 M points, 57 +
+// 10 on 100 k (15 + 17 now), 30 + 13 on 1 M 2-D points (10 + 15); 8192
+// workgroups 65 + 78 on the 4 M.
+//
+// k_link_cross walks the whole list, neighbouring workgroups on neighbouring
+// entries: with the entries of a stripe on one XCD its plain loads find parents
+// that are stale in that L2, and it took 121 us.
 constexpr int kLinkCells = 16384;  // cells of one LDS forest (64 KiB)
-constexpr int kLinkMin = 4096;     // least cells of a run
-constexpr int kLinkGrid = 512;     // workgroups (two per CU)
+constexpr int kLinkMin = 1024;     // least cells of a run
+constexpr int kLinkGrid = 2048;    // workgroups
 
 __device__ __forceinline__ int32_t lds_find(int32_t* par, int32_t x) {
   for (;;) {
@@ -794,14 +954,13 @@ __global__ __launch_bounds__(1024) void k_link_local(Dev d) {
       const int32_t A = (int32_t)c0 + i;
       uint32_t m = d.amask[A];
       if (!m) continue;
-      const int dim = inst_of_cell(d, A)->dim, local = local_of(d, A, dim);
-      const RowsOf rows = rows_of(d, A);
+      const NearRows near = near_rows(d, A, inst_of_cell(d, A)->dim);
       uint32_t ext = 0u;
       int32_t root = i;
       while (m) {
         const int b = __ffs(m) - 1;
         m &= m - 1;
-        const int32_t B = near_cell(rows, dim, local, b) - (int32_t)c0;
+        const int32_t B = near_cell(near, b) - (int32_t)c0;
         if (B >= 0 && B < nc)
           root = lds_union(par, root, B);
         else
@@ -836,14 +995,13 @@ __global__ __launch_bounds__(256) void k_link_cross(Dev d) {
     const int32_t A = i < n ? slist_at(d.core_cells, s_pre, i) : -1;
     uint32_t m = A >= 0 ? d.amask[A] : 0u;
     const int32_t pa = m ? d.parent[A] : 0;
-    const RowsOf rows = rows_of(d, m ? A : 0);
-    const int dim = inst_of_cell(d, m ? A : 0)->dim, local = local_of(d, m ? A : 0, dim);
+    const NearRows near = near_rows(d, m ? A : 0, inst_of_cell(d, m ? A : 0)->dim);
     while (ballot(m != 0u)) {
       int32_t pb = -1;
       if (m) {
         const int b = __ffs(m) - 1;
         m &= m - 1;
-        pb = d.parent[near_cell(rows, dim, local, b)];
+        pb = d.parent[near_cell(near, b)];
       }
       // neighbouring cells mostly name the same two roots: a pair in the
       // wave's table is left out, and of the lanes that hold the same pair
@@ -871,12 +1029,11 @@ __global__ __launch_bounds__(256) void k_link_cross(Dev d) {
 // and the list of the roots.
 __global__ __launch_bounds__(256) void k_comp(Dev d) {
   if (abandoned(d)) return;
-  __shared__ long long s_pre[kStripes + 1];
-  const long long n = slist_prefix(d.core_cells, s_pre);
-  for (long long i0 = (long long)blockIdx.x * 256; i0 < n; i0 += (long long)gridDim.x * 256) {
-    const long long i = i0 + threadIdx.x;
-    const bool act = i < n;
-    const int32_t A = act ? slist_at(d.core_cells, s_pre, i) : 0;
+  const Stripe L(d.core_cells);
+  for (int64_t i0 = L.first(256); i0 < L.n; i0 += L.step(256)) {
+    const int64_t i = i0 + threadIdx.x;
+    const bool act = i < L.n;
+    const int32_t A = act ? L.data[i] : 0;
     int32_t comp = -1, cmin = kNoKey;
     if (act) {
       cmin = d.orig[d.rep[A].w];
@@ -1259,11 +1416,9 @@ __global__ __launch_bounds__(256, 4) void k_far_pairs(Dev d) {
 // that.  (uf_order keeps the walks short, so no compressing pass precedes.)
 __global__ __launch_bounds__(256) void k_roots_final(Dev d) {
   if (abandoned(d)) return;
-  __shared__ long long s_pre[kStripes + 1];
-  const long long n = slist_prefix(d.near_roots, s_pre);
-  for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n;
-       i += (long long)gridDim.x * 256) {
-    const int32_t c = slist_at(d.near_roots, s_pre, i);
+  const Stripe L(d.near_roots);
+  for (int64_t i = L.first(256) + threadIdx.x; i < L.n; i += L.step(256)) {
+    const int32_t c = L.data[i];
     const int32_t m = d.compmin[c];
     const int32_t r = uf_root(d.parent, c);
     d.parent[c] = r;
@@ -1900,14 +2055,13 @@ __device__ int32_t border_lane(const Dev& d, const Par& P, int32_t p, int32_t c,
 template <bool F32>
 __global__ __launch_bounds__(256) void k_border(Dev d) {
   if (abandoned(d)) return;
-  __shared__ long long s_pre[kStripes + 1];
-  const long long n = slist_prefix(d.border_pts, s_pre);
+  const Stripe L(d.border_pts);
   Tally t;
   long long ovf = 0;
-  for (long long i0 = (long long)blockIdx.x * 256; i0 < n; i0 += (long long)gridDim.x * 256) {
-    const long long i = i0 + threadIdx.x;
-    const bool act = i < n;
-    const int32_t p = act ? slist_at(d.border_pts, s_pre, i) : 0;
+  for (int64_t i0 = L.first(256); i0 < L.n; i0 += L.step(256)) {
+    const int64_t i = i0 + threadIdx.x;
+    const bool act = i < L.n;
+    const int32_t p = act ? L.data[i] : 0;
     int32_t c = 0;
     int dim = 0;
     const Inst* I = d.inst;
@@ -2034,27 +2188,26 @@ static int point_grid(int64_t n) {
 }
 
 int64_t point_blocks(int64_t n) { return point_grid(n); }
-int64_t list_append_cap(int64_t n) {
-  const int64_t g = std::min(kListGrid, point_grid(n));
-  return (g + kStripes - 1) / kStripes * 256 * ((n + g * 256 - 1) / (g * 256));
-}
-int64_t cell_blocks(int64_t n) { return (n + 1023) / 1024 > 0 ? (n + 1023) / 1024 : 1; }
+int64_t cell_blocks(int64_t n) { return (n + 1023) / 1024; }
 
-// one lane per listed core cell, grid-stride
-static int list_grid(int64_t n) { return std::min(kListGrid, point_grid(n)); }
+// walkers of a list of up to n items, a lane each; k_core_rest takes several
+static int list_grid(int64_t n) {
+  return std::min(kListGrid, (point_grid(n) + kStripes - 1) / kStripes * kStripes);
+}
+
+template <bool F32, int Q>
+static void core_kernels(const Dev& d, hipStream_t s) {
+  hipLaunchKernelGGL(k_core<F32>, dim3(point_grid(d.n)), dim3(256), 0, s, d);
+  hipLaunchKernelGGL((k_core_rest<F32, Q>), dim3(list_grid(d.n * Q)), dim3(256),
+                     core_lds(d.rec_stride, Q), s, d);
+  hipLaunchKernelGGL(k_core_crowd<F32>, dim3(list_grid(d.n)), dim3(256), 0, s, d);
+}
 
 void launch_core(const Dev& d, bool f32, hipStream_t s) {
-  const size_t lds = core_lds(d.rec_stride);
-  const int gl = list_grid(d.n);
-  if (f32) {
-    hipLaunchKernelGGL(k_core<true>, dim3(point_grid(d.n)), dim3(256), 0, s, d);
-    hipLaunchKernelGGL(k_core_rest<true>, dim3(gl), dim3(256), lds, s, d);
-    hipLaunchKernelGGL(k_core_crowd<true>, dim3(gl), dim3(256), 0, s, d);
-  } else {
-    hipLaunchKernelGGL(k_core<false>, dim3(point_grid(d.n)), dim3(256), 0, s, d);
-    hipLaunchKernelGGL(k_core_rest<false>, dim3(gl), dim3(256), lds, s, d);
-    hipLaunchKernelGGL(k_core_crowd<false>, dim3(gl), dim3(256), 0, s, d);
-  }
+  if (d.n < kRestQuad)
+    f32 ? core_kernels<true, 4>(d, s) : core_kernels<false, 4>(d, s);
+  else
+    f32 ? core_kernels<true, 2>(d, s) : core_kernels<false, 2>(d, s);
 }
 
 void launch_near(const Dev& d, hipStream_t s) {
@@ -2107,7 +2260,7 @@ void launch_far(const Dev& d, bool f32, int grid, hipStream_t s) {
     hipLaunchKernelGGL(k_far_pairs<true>, dim3(grid), dim3(256), 0, s, d);
   else
     hipLaunchKernelGGL(k_far_pairs<false>, dim3(grid), dim3(256), 0, s, d);
-  hipLaunchKernelGGL(k_roots_final, dim3(std::min(grid, list_grid(d.n))), dim3(256), 0, s, d);
+  hipLaunchKernelGGL(k_roots_final, dim3(list_grid(d.n)), dim3(256), 0, s, d);
 }
 
 void launch_border(const Dev& d, bool f32, hipStream_t s) {

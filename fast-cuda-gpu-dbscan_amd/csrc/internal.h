@@ -518,6 +518,30 @@ __device__ __forceinline__ void block_append(bool take, int32_t value, const SLi
   __syncthreads();  // s_cnt / s_base are reused by the next call
 }
 
+// The part of a list that a workgroup walks: the sub-list that the workgroups
+// with its stripe filled, shared by the grid's workgroups of that stripe (the
+// grid is a multiple of kStripes).  A stripe is on one XCD, and the kernels
+// that fill lists give each XCD one range of points or cells, so a walker
+// finds the lists' neighbourhoods in its own L2.  A walker that appends to
+// another list appends to the same stripe, so that list needs no more room a
+// stripe than this one.
+struct Stripe {
+  const int32_t* data;
+  int64_t n;
+  __device__ __forceinline__ explicit Stripe(const SList& L) {
+    const int s = blockIdx.x & (kStripes - 1);
+    data = L.data + s * L.cap;
+    n = (int64_t)L.cnt[s * kStatStride];
+  }
+  // first item of this workgroup and its stride, `per` items at a time
+  __device__ __forceinline__ int64_t first(int per) const {
+    return (int64_t)(blockIdx.x / kStripes) * per;
+  }
+  __device__ __forceinline__ int64_t step(int per) const {
+    return (int64_t)(gridDim.x / kStripes) * per;
+  }
+};
+
 // Prefix of the sub-list counts of L in LDS (s_pre[kStripes + 1]); returns
 // the list length.  Every thread of the workgroup calls it.
 __device__ __forceinline__ long long slist_prefix(const SList& L, long long* s_pre) {
@@ -560,6 +584,15 @@ __host__ __device__ inline double unord_d(unsigned long long u) {
 __device__ __forceinline__ int xcd_block(int b, int G) {
   int per = G >> 3;
   return (b & 7) * per + (b >> 3);
+}
+
+// The same in runs: the XCDs take runs of CH consecutive workgroups in turn,
+// so that a clustered input's work spreads over all of them (the last, partial
+// round of runs is not remapped).
+template <int CH>
+__device__ __forceinline__ int xcd_runs(int b, int G) {
+  const int q = b >> 3, round = q / CH;
+  return (round + 1) * 8 * CH <= G ? round * 8 * CH + (b & 7) * CH + q % CH : b;
 }
 
 // State of the one-step (CUDA-DClust) baseline, cell-sorted order.

@@ -38,9 +38,6 @@ void launch_merge(const Dev& d, int grid, hipStream_t s);
 // workgroups of the producers of the striped work lists (their capacity)
 int64_t point_blocks(int64_t n);
 int64_t cell_blocks(int64_t n);
-// per-stripe capacity of a list that a grid-stride pass over at most n listed
-// cells appends to
-int64_t list_append_cap(int64_t n);
 // stencil pairs across components, then final roots
 void launch_far(const Dev& d, bool f32, int grid, hipStream_t s);
 void launch_border(const Dev& d, bool f32, hipStream_t s);
