@@ -37,7 +37,7 @@
 //                matrix and thrust::replace relabels, dbscan.cu:60-125).
 //   k_comp, k_far, k_far_pairs   pairs of stencil cells in two components are
 //                decided exactly and united.
-//   k_roots_final / k_keys / k_border / rank scan / k_output
+//   k_roots_final / k_keys / k_border / rank scan / k_output (_split, _place)
 //                canonical labels:
 //                cluster id = rank of the component's minimum core input
 //                index; border = minimum id over adjacent cores; noise = 0
@@ -2084,14 +2084,19 @@ __global__ __launch_bounds__(256) void k_border(Dev d) {
 // ------------------------------------------------------------ rank + out --
 // Ranks of the clusters: the flags of their smallest core input indices are
 // bits, so rank(k) = the flags before k's word (a scan over N/64 words: small
-// enough to stay in L2 for the random reads of k_output, where one entry per
+// enough to stay in L2 for the random reads of the labels, where one entry per
 // point was not) + the bits below k in its word.
+constexpr int kOutWindows = 512;  // windows of the labels, at most
+constexpr int kOutPad = 16;       // a window's cursor has a cache line of its own
 constexpr int RK_T = 256;
 constexpr int RK_I = 4;
 constexpr int RK_TILE = RK_T * RK_I;  // words per workgroup
 
-__global__ __launch_bounds__(RK_T) void k_rank_count(Dev d) {
+// (`cursor`: k_output_split's, started here, or null)
+__global__ __launch_bounds__(RK_T) void k_rank_count(Dev d, uint32_t* cursor) {
   if (abandoned(d)) return;
+  if (cursor && blockIdx.x == 0)
+    for (int i = threadIdx.x; i < kOutWindows; i += RK_T) cursor[i * kOutPad] = 0;
   const int64_t nf = (d.n + 63) / 64, t0 = (int64_t)blockIdx.x * RK_TILE;
   int c = 0;
 #pragma unroll
@@ -2111,7 +2116,7 @@ __global__ __launch_bounds__(RK_T) void k_rank_write(Dev d) {
   const int64_t nf = (d.n + 63) / 64, t0 = (int64_t)blockIdx.x * RK_TILE;
   __shared__ int s_w[4];
   __shared__ int64_t s_p[4];
-  // flags of the workgroups before (at most 2^28 / 64 / 1024 = 4096 counts)
+  // flags of the workgroups before (a count for 65536 points)
   int64_t pre = 0;
   for (int i = threadIdx.x; i < (int)blockIdx.x; i += RK_T) pre += d.scan_tmp[i];
   pre = wave_sum(pre);
@@ -2145,38 +2150,144 @@ __device__ __forceinline__ int32_t rank_of(const Dev& d, int64_t k) {
   return d.rank[k >> 6] + __popcll(d.flag[k >> 6] & ((1ull << (k & 63)) - 1ull));
 }
 
+// Labels of NI points from i0 on, RS apart, and their input indices (an index
+// past the end reads point 0); returns the number of noise points.
+template <int NI, int RS>
+__device__ __forceinline__ int point_labels(const Dev& d, int64_t i0, int32_t (&o)[NI],
+                                            int32_t (&lab)[NI]) {
+  int32_t k[NI], rb[NI];
+  int64_t pb[NI];
+#pragma unroll
+  for (int u = 0; u < NI; ++u) {
+    const int64_t ic = i0 + u * RS < d.n ? i0 + u * RS : 0;
+    o[u] = d.orig[ic];
+    k[u] = d.keyv[ic];
+    pb[u] = inst_of_cell(d, d.ninst == 1 ? 0 : d.cell_of[ic])->pt_begin;
+  }
+#pragma unroll
+  for (int u = 0; u < NI; ++u) {
+    lab[u] = rank_of(d, k[u] == kNoKey ? 0 : k[u]);
+    rb[u] = d.ninst == 1 ? 0 : rank_of(d, pb[u]);
+  }
+  int noise = 0;
+#pragma unroll
+  for (int u = 0; u < NI; ++u) {
+    lab[u] = k[u] == kNoKey ? 0 : lab[u] - rb[u] + 1;
+    noise += i0 + u * RS < d.n && k[u] == kNoKey;
+  }
+  return noise;
+}
+
 __global__ __launch_bounds__(256) void k_output(Dev d) {
   if (abandoned(d)) return;
   int32_t* labels = out_labels(d);
   long long noise = 0;
-  for (int64_t i0 = blockIdx.x * (int64_t)(kRelU * 256); i0 < d.n;
+  for (int64_t i0 = blockIdx.x * (int64_t)(kRelU * 256) + threadIdx.x; i0 - threadIdx.x < d.n;
        i0 += (int64_t)gridDim.x * (kRelU * 256)) {
-    int32_t o[kRelU], k[kRelU], rk[kRelU], rb[kRelU];
-    int64_t pb[kRelU];
+    int32_t o[kRelU], lab[kRelU];
+    noise += point_labels<kRelU, 256>(d, i0, o, lab);
+#pragma unroll
+    for (int u = 0; u < kRelU; ++u)
+      if (i0 + u * 256 < d.n) labels[o[u]] = lab[u];
+  }
+  stat_add(d, C_NNOISE, noise);
+}
+
+// The labels of a large call in two steps.  Written one by one in sorted order
+// each 4-byte label is a partial line of its own (32 M points: 815 us, 2.5 TB/s
+// of 64-byte writes).  k_output_split sorts tiles of (input index, label) pairs
+// by window of the labels in LDS and appends them window by window (the input
+// indices are a permutation, so a window's place and size are known, and the
+// order inside it does not matter); k_output_place writes each window on one
+// XCD, whose L2 joins its lines.
+//
+// k_output against the two steps, us: 1 M points 14 / 20, 1.5 M 22 / 24, 4 M 74
+// / 41, 7 M in a batch 101 / 98, 32 M 815 / 289.  A part is gathered from its
+// whole window, so the windows stay below kOutWindow labels; larger calls
+// (above 67 M points) keep the one step.
+constexpr int kOutItems = 16;
+constexpr int64_t kOutSplit = 1 << 21;
+constexpr int64_t kOutWindow = 1 << 17;
+__global__ __launch_bounds__(512, 4) void k_output_split(Dev d, int shift, uint32_t* cursor,
+                                                      uint2* pairs) {
+  if (abandoned(d)) return;
+  constexpr int T = 512, NI = kOutItems;
+  static_assert(T == kOutWindows, "a thread per window");
+  __shared__ uint2 s_p[T * NI];
+  __shared__ uint32_t s_cnt[T], s_dst[T], s_w[T / 64];
+  const int tid = threadIdx.x, wv = tid >> 6;
+  s_cnt[tid] = 0;
+  const int64_t t0 = (int64_t)blockIdx.x * (T * NI);
+  int32_t o[NI], lab[NI];
+  int noise = 0;
+#pragma unroll
+  for (int h = 0; h < NI; h += kRelU) {
+    int32_t ho[kRelU], hl[kRelU];
+    noise += point_labels<kRelU, T>(d, t0 + tid + h * T, ho, hl);
 #pragma unroll
     for (int u = 0; u < kRelU; ++u) {
-      const int64_t i = i0 + u * 256 + threadIdx.x;
-      const int64_t ic = i < d.n ? i : 0;
-      o[u] = d.orig[ic];
-      k[u] = d.keyv[ic];
-      pb[u] = inst_of_cell(d, d.ninst == 1 ? 0 : d.cell_of[ic])->pt_begin;
-    }
-#pragma unroll
-    for (int u = 0; u < kRelU; ++u) {
-      rk[u] = rank_of(d, k[u] == kNoKey ? 0 : k[u]);
-      rb[u] = d.ninst == 1 ? 0 : rank_of(d, pb[u]);
-    }
-#pragma unroll
-    for (int u = 0; u < kRelU; ++u) {
-      const int64_t i = i0 + u * 256 + threadIdx.x;
-      if (i < d.n) {
-        const int32_t lab = k[u] == kNoKey ? 0 : rk[u] - rb[u] + 1;
-        labels[o[u]] = lab;
-        noise += lab == 0;
-      }
+      o[h + u] = ho[u];
+      lab[h + u] = hl[u];
     }
   }
   stat_add(d, C_NNOISE, noise);
+  __syncthreads();
+  uint32_t at[NI];
+#pragma unroll
+  for (int u = 0; u < NI; ++u)
+    at[u] = t0 + u * T + tid < d.n ? atomicAdd(&s_cnt[o[u] >> shift], 1u) : 0u;
+  __syncthreads();
+  const uint32_t c = s_cnt[tid];
+  const uint32_t base = c ? atomicAdd(&cursor[tid * kOutPad], c) : 0u;
+  const uint32_t inc = wave_incl_scan(c);
+  if (lane_id() == 63) s_w[wv] = inc;
+  __syncthreads();
+  uint32_t lst = inc - c;
+  for (int w = 0; w < wv; ++w) lst += s_w[w];
+  s_cnt[tid] = lst;
+  s_dst[tid] = ((uint32_t)tid << shift) + base - lst;
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < NI; ++u)
+    if (t0 + u * T + tid < d.n)
+      s_p[s_cnt[o[u] >> shift] + at[u]] = make_uint2((uint32_t)o[u], (uint32_t)lab[u]);
+  __syncthreads();
+  const int tn = (int)(d.n - t0 < T * NI ? d.n - t0 : T * NI);
+#pragma unroll 4
+  for (int u = 0; u < NI; ++u) {
+    const int l = u * T + tid;
+    if (l < tn) {
+      const uint2 p = s_p[l];
+      pairs[s_dst[p.x >> shift] + (uint32_t)l] = p;
+    }
+  }
+}
+
+// A workgroup gathers PART labels, a part of a window, in LDS and writes them
+// in order (written from the pairs directly, the scattered 4-byte requests took
+// 236 us on 32 M points).
+template <int PART, int T>
+__global__ __launch_bounds__(T) void k_output_place(Dev d, int shift, const uint2* pairs) {
+  if (abandoned(d)) return;
+  __shared__ int32_t s_l[PART];
+  constexpr int U = 8;
+  const int64_t first = (int64_t)xcd_runs<8>(blockIdx.x, gridDim.x) * PART;
+  const int64_t w0 = first >> shift << shift;
+  const int64_t w1 = w0 + (1LL << shift) < d.n ? w0 + (1LL << shift) : d.n;
+  for (int64_t i0 = w0 + threadIdx.x; i0 < w1; i0 += T * U) {
+    uint2 p[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) p[u] = pairs[i0 + u * T < w1 ? i0 + u * T : w0];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t l = p[u].x - (uint32_t)first;
+      if (i0 + u * T < w1 && l < (uint32_t)PART) s_l[l] = (int32_t)p[u].y;
+    }
+  }
+  __syncthreads();
+  int32_t* labels = out_labels(d) + first;
+  const int np = (int)(d.n - first < PART ? d.n - first : PART);
+  for (int l = threadIdx.x; l < np; l += T) labels[l] = s_l[l];
 }
 
 // ------------------------------------------------------------- launchers --
@@ -2292,12 +2403,28 @@ void launch_core_out(const uint8_t* core, const int32_t* orig, int64_t n, uint8_
 
 void launch_relabel(const Dev& d, int64_t n, hipStream_t s) {
   const int nb = (int)(((n + 63) / 64 + RK_TILE - 1) / RK_TILE);
-  hipLaunchKernelGGL(k_rank_count, dim3(nb), dim3(RK_T), 0, s, d);
+  const bool split = n >= kOutSplit && n <= kOutWindows * kOutWindow;
+  hipLaunchKernelGGL(k_rank_count, dim3(nb), dim3(RK_T), 0, s, d, split ? d.hist : nullptr);
   hipLaunchKernelGGL(k_rank_write, dim3(nb), dim3(RK_T), 0, s, d);
   int g2 = (int)((n + 255) / 256);
   if (g2 > 4096) g2 = 4096;
   if (g2 < 1) g2 = 1;
-  hipLaunchKernelGGL(k_output, dim3(g2), dim3(256), 0, s, d);
+  if (split) {
+    int shift = 0;
+    while ((n - 1) >> shift >= kOutWindows) ++shift;
+    uint2* pairs = reinterpret_cast<uint2*>(d.key[0]);  // (the representatives are done with)
+    hipLaunchKernelGGL(k_output_split, dim3((unsigned)((n + 512 * kOutItems - 1) / (512 * kOutItems))),
+                       dim3(512), 0, s, d, shift, d.hist, pairs);
+    // (a window smaller than the part it is gathered in shares its workgroup)
+    if (shift > 13)
+      hipLaunchKernelGGL((k_output_place<32768, 1024>), dim3((unsigned)((n + 32767) / 32768)),
+                         dim3(1024), 0, s, d, std::max(shift, 15), pairs);
+    else
+      hipLaunchKernelGGL((k_output_place<8192, 512>), dim3((unsigned)((n + 8191) / 8192)),
+                         dim3(512), 0, s, d, 13, pairs);
+  } else {
+    hipLaunchKernelGGL(k_output, dim3(g2), dim3(256), 0, s, d);
+  }
 }
 
 }  // namespace dclust
