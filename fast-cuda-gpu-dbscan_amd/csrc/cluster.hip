@@ -2088,6 +2088,7 @@ __global__ __launch_bounds__(256) void k_border(Dev d) {
 // point was not) + the bits below k in its word.
 constexpr int kOutWindows = 512;  // windows of the labels, at most
 constexpr int kOutPad = 16;       // a window's cursor has a cache line of its own
+constexpr int kRankOne = 1 << 13;  // words that one workgroup ranks
 constexpr int RK_T = 256;
 constexpr int RK_I = 4;
 constexpr int RK_TILE = RK_T * RK_I;  // words per workgroup
@@ -2143,6 +2144,31 @@ __global__ __launch_bounds__(RK_T) void k_rank_write(Dev d) {
     run += c[r];
     if (i == nf - 1) d.ctl[C_NCLUST] = run;
   }
+}
+
+// The two in one for at most 2^19 points, a launch less: 4 us for 100 k points
+// and 6 for 262 k where the two take 9, but 11 for 614 k and 16 for 1 M.
+__global__ __launch_bounds__(1024) void k_rank_one(Dev d) {
+  if (abandoned(d)) return;
+  constexpr int W = kRankOne / 1024;
+  const int nf = (int)((d.n + 63) / 64), w0 = threadIdx.x * W, wv = threadIdx.x >> 6;
+  __shared__ int s_w[16];
+  int c[W], sum = 0;
+#pragma unroll
+  for (int r = 0; r < W; ++r) c[r] = w0 + r < nf ? __popcll(d.flag[w0 + r]) : 0;
+#pragma unroll
+  for (int r = 0; r < W; ++r) sum += c[r];
+  const int incl = wave_incl_scan(sum);
+  if (lane_id() == 63) s_w[wv] = incl;
+  __syncthreads();
+  int run = incl - sum;
+  for (int w = 0; w < wv; ++w) run += s_w[w];
+#pragma unroll
+  for (int r = 0; r < W; ++r) {
+    if (w0 + r < nf) d.rank[w0 + r] = run;
+    run += c[r];
+  }
+  if (threadIdx.x == 1023) d.ctl[C_NCLUST] = run;
 }
 
 // flags before input index k
@@ -2404,8 +2430,12 @@ void launch_core_out(const uint8_t* core, const int32_t* orig, int64_t n, uint8_
 void launch_relabel(const Dev& d, int64_t n, hipStream_t s) {
   const int nb = (int)(((n + 63) / 64 + RK_TILE - 1) / RK_TILE);
   const bool split = n >= kOutSplit && n <= kOutWindows * kOutWindow;
-  hipLaunchKernelGGL(k_rank_count, dim3(nb), dim3(RK_T), 0, s, d, split ? d.hist : nullptr);
-  hipLaunchKernelGGL(k_rank_write, dim3(nb), dim3(RK_T), 0, s, d);
+  if ((n + 63) / 64 <= kRankOne) {
+    hipLaunchKernelGGL(k_rank_one, dim3(1), dim3(1024), 0, s, d);
+  } else {
+    hipLaunchKernelGGL(k_rank_count, dim3(nb), dim3(RK_T), 0, s, d, split ? d.hist : nullptr);
+    hipLaunchKernelGGL(k_rank_write, dim3(nb), dim3(RK_T), 0, s, d);
+  }
   int g2 = (int)((n + 255) / 256);
   if (g2 > 4096) g2 = 4096;
   if (g2 < 1) g2 = 1;

@@ -188,7 +188,8 @@ __global__ __launch_bounds__(256) void k_bbox(Dev d) {
         s_red[0][6] = fmax(s_red[0][6], s_red[w][6]);
       }
     unsigned long long* bb =
-        d.bbox + ((int64_t)ch.inst * kBoxStripes + blockIdx.x % kBoxStripes) * 8;
+        d.bbox + ((int64_t)ch.inst * kBoxStripes +
+                  (ch.begin - I.pt_begin) / kChunk % kBoxStripes) * 8;
     for (int k = 0; k < dim; ++k) {
       atomicMin(&bb[k], ord_d(s_red[0][k]));
       atomicMax(&bb[3 + k], ord_d(s_red[0][3 + k]));
@@ -380,8 +381,12 @@ __global__ __launch_bounds__(1024) void k_grid_setup(Dev d) {
         const unsigned long long* bs = d.bbox + (int64_t)i * kBoxStripes * 8;
 #pragma unroll
         for (int k = 0; k < 8; ++k) bb[k] = k < 3 ? ~0ull : 0ull;
+        // (as many stripes as the instance has chunks: with all 32 this read
+        // was most of the 33 us of 256 instances, 45 of 400 tiny ones)
+        const int64_t chunks = (I.pt_end - I.pt_begin + kChunk - 1) / kChunk;
+        const int ns = chunks < kBoxStripes ? (int)chunks : kBoxStripes;
 #pragma unroll 4
-        for (int st = 0; st < kBoxStripes; ++st)
+        for (int st = 0; st < ns; ++st)
 #pragma unroll
           for (int k = 0; k < 8; ++k) {
             const unsigned long long v = bs[st * 8 + k];
@@ -892,8 +897,7 @@ __global__ __launch_bounds__(1024) void k_scan_top(int64_t* v, int nb, long long
 }
 
 // instance owning a key: last i with key_base <= key
-__device__ __forceinline__ int32_t inst_of_key(const Dev& d, uint64_t key) {
-  int lo = 0, hi = d.ninst - 1;
+__device__ __forceinline__ int32_t inst_of_key(const Dev& d, uint64_t key, int lo, int hi) {
   while (lo < hi) {
     int mid = (lo + hi + 1) >> 1;
     if ((uint64_t)d.inst[mid].key_base <= key) lo = mid; else hi = mid - 1;
@@ -914,15 +918,6 @@ __device__ __forceinline__ void split_key(const Inst& I, uint64_t key, int64_t& 
     col = (int64_t)(rel / nzl);
     zl = (uint32_t)(rel - (uint64_t)col * nzl);
   }
-}
-
-// Column-table index of a key.
-__device__ __forceinline__ int64_t column_of(const Dev& d, uint64_t key) {
-  const Inst& I = d.inst[inst_of_key(d, key)];
-  int64_t col;
-  uint32_t zl;
-  split_key(I, key, col, zl);
-  return I.line_base + col;
 }
 
 // Sum of the block counts v[0..b) (`scanned` false: they are counts; true:
@@ -959,6 +954,18 @@ __global__ __launch_bounds__(CS_T) void k_csr_write(Dev d, bool scanned) {
   // instance table before the first store (the stores could alias it as far
   // as the compiler knows, which would hold each round's reads behind the
   // previous round's stores)
+  // (the tile's keys are sorted: they lie in the instances of its first and
+  // last key, in a batch mostly one; 7 M points in 256 instances 113 us with a
+  // search per cell, 71 now)
+  int i_lo = 0, i_hi = 0;
+  if (d.ninst != 1) {
+    const int64_t last = t0 + CS_TILE < d.n ? t0 + CS_TILE - 1 : d.n - 1;
+    const int par = sort_passes(d) & 1;
+    const SortKey<KF>* key = key_buf<KF>(d, par);
+    const int32_t* val = d.val[par];
+    i_lo = inst_of_key(d, entry_key<KF>(key[t0], KF == 36 ? val[t0] : 0), 0, d.ninst - 1);
+    i_hi = inst_of_key(d, entry_key<KF>(key[last], KF == 36 ? val[last] : 0), i_lo, d.ninst - 1);
+  }
   int32_t ir[CS_I];
   uint32_t zr[CS_I], cr[CS_I];
 #pragma unroll
@@ -968,7 +975,7 @@ __global__ __launch_bounds__(CS_T) void k_csr_write(Dev d, bool scanned) {
     cr[r] = 0;
     const int64_t i = t0 + r * CS_T + threadIdx.x;
     if (i < d.n && (i == 0 || kr[r] != kp[r])) {
-      ir[r] = inst_of_key(d, kr[r]);
+      ir[r] = inst_of_key(d, kr[r], i_lo, i_hi);
       const Inst& I = d.inst[ir[r]];
       int64_t col;
       split_key(I, kr[r], col, zr[r]);
@@ -1002,11 +1009,28 @@ __global__ __launch_bounds__(CS_T) void k_csr_write(Dev d, bool scanned) {
         d.cell_zl[cid] = zr[r];
         if (table && (i == 0 || kp[r] < k - zr[r])) {
           d.lines[cr[r]].x = (int32_t)cid;
-          if (i > 0) d.lines[column_of(d, kp[r])].y = (int32_t)cid;
+          if (i > 0) {
+            // (the previous key's instance: this one, or one before it)
+            const int32_t pi = kp[r] >= (uint64_t)d.inst[ir[r]].key_base
+                                   ? ir[r]
+                                   : inst_of_key(d, kp[r], 0, ir[r] - 1);
+            const Inst& I = d.inst[pi];
+            int64_t col;
+            uint32_t zl;
+            split_key(I, kp[r], col, zl);
+            d.lines[I.line_base + col].y = (int32_t)cid;
+          }
         }
       }
       if (i == d.n - 1) {
-        if (table) d.lines[column_of(d, k)].y = (int32_t)cid + 1;
+        // (the last point's cell started in this tile or before)
+        if (table) {
+          const Inst& I = d.inst[inst_of_key(d, k, i_lo, i_hi)];
+          int64_t col;
+          uint32_t zl;
+          split_key(I, k, col, zl);
+          d.lines[I.line_base + col].y = (int32_t)cid + 1;
+        }
         d.cell_start[cid + 1] = (int32_t)d.n;
         d.ctl[C_NCELL] = cid + 1;
       }
@@ -1073,27 +1097,34 @@ __global__ __launch_bounds__(256) void k_gather(Dev d, int64_t waves, uint32_t i
 
 // ------------------------------------------------------------------ rows --
 // Three lower bounds lo[j] = first index in [lo[j], hi[j]) with a[i] >= v[j],
-// in lockstep (the loads of the three searches overlap).
+// in lockstep (the loads of the three searches overlap), a quarter of the
+// range per step: a chain of loads half as long as by halves, which is what
+// the few columns left to k_rows_global take (22 us with halves, 18 now, on
+// calls of 262 k to 1.5 M points).
 template <typename T>
 __device__ __forceinline__ void lower_bound3(const T* a, int32_t (&lo)[3], int32_t (&hi)[3],
                                              const T (&v)[3]) {
+  const auto cut = [](int32_t l, int32_t h, int i) {  // pivot i of 1..3, in [l, h)
+    return l + (int32_t)(((uint64_t)(uint32_t)(h - l) * (uint32_t)i) >> 2);
+  };
   for (;;) {
-    T km[3];
+    T km[3][3];
     bool any = false;
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
-      km[j] = lo[j] < hi[j] ? a[(lo[j] + hi[j]) >> 1] : (T)0;
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+        km[j][i] = lo[j] < hi[j] ? a[cut(lo[j], hi[j], i + 1)] : (T)0;
       any |= lo[j] < hi[j];
     }
     if (!any) return;
 #pragma unroll
     for (int j = 0; j < 3; ++j)
       if (lo[j] < hi[j]) {
-        const int32_t mid = (lo[j] + hi[j]) >> 1;
-        if (km[j] < v[j])
-          lo[j] = mid + 1;
-        else
-          hi[j] = mid;
+        const int32_t l = lo[j], h = hi[j];
+        const int c = (km[j][0] < v[j]) + (km[j][1] < v[j]) + (km[j][2] < v[j]);
+        if (c > 0) lo[j] = cut(l, h, c) + 1;
+        if (c < 3) hi[j] = cut(l, h, c + 1);
       }
   }
 }

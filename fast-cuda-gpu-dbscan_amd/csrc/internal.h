@@ -289,7 +289,7 @@ struct PairList {
 // order and the buffers are not swapped).
 constexpr int kDigitBits = 9;  // of a radix pass, at most
 
-// Bounding-box partials: chunk b reduces into stripe b % kBoxStripes of its
+// Bounding-box partials: chunk b of an instance reduces into stripe b % kBoxStripes of its
 // instance (so that the atomics of many chunks do not meet on one address);
 // the grid set-up reduces the stripes.
 constexpr int kBoxStripes = 32;

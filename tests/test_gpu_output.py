@@ -34,3 +34,30 @@ def test_batch():
     assert not np.any(errs)
     for x, lab in zip(xs, labels):
         assert np.array_equal(lab, oracle.fast_dbscan(x, 0.5, 3)[0])
+
+
+# one workgroup ranks the clusters up to 2^19 points: the last size that it
+# takes and the first that it does not; a flag in the last bit of the last word
+@pytest.mark.parametrize("n", [1 << 19, (1 << 19) + 1, 64 * 1000 - 1])
+def test_cluster_ranks(devmem, n):
+    x = np.repeat(np.arange((n + 1) // 2, dtype=np.float64), 2)[:n, None] * [1.0, 0.0]
+    x = x[np.random.default_rng(n).permutation(n)]
+    ref = oracle.fast_dbscan(x, 0.5, 2)[0]
+    d_x, d_l = devmem.upload(x), devmem.alloc(4 * n)
+    with dclust.Handle(0) as h:
+        st = h.run_device(d_x, n, dclust.make_params(2, 0.5, 2), d_l)
+    assert np.array_equal(devmem.download(np.empty(n, dtype=np.int32), d_l), ref)
+    assert st["n_clusters"] == n // 2
+
+
+def test_batch_of_many_chunks_and_instances():
+    # instances of no point, one point, one chunk and more chunks than the
+    # bounding box has stripes
+    ns = [200000, 0, 1, 4096, 4097, 33] * 3
+    xs = [_pairs(max(n, 1), 7 + n)[:n] for n in ns]
+    with dclust.Handle(0) as h:
+        labels, errs = h.run_batched(xs, [dclust.make_params(2, 0.5, 3)] * len(ns))
+    assert not np.any(errs)
+    for x, lab in zip(xs, labels):
+        if len(x):
+            assert np.array_equal(lab, oracle.fast_dbscan(x, 0.5, 3)[0])
