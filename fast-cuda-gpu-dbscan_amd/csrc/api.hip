@@ -1005,8 +1005,7 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
     HIPCHK(upload());
     HIPCHK(mark(h, E_START, false));
     enqueue_head(d, nullptr, call, nchunks, s);
-    HIPCHK(hipMemcpyAsync(ctl_h, d.ctl, sizeof(ctl_h), hipMemcpyDeviceToHost, s));
-    HIPCHK(hipStreamSynchronize(s));
+    HIPCHK(read_counters(h, d, s, ctl_h));
     // more cells than the 63-bit sort key holds, over all instances
     if (ctl_h[C_KEYOVF]) {
       if (inst_err)

@@ -147,8 +147,16 @@ __device__ void setup_totals(const Dev& d, unsigned long long cells, unsigned lo
 // (a call of one instance has no separate grid set-up: the workgroup that
 // finishes last does it, from coherent loads of the stripes, which saves a
 // launch of one workgroup that took 11 to 19 us)
-__global__ __launch_bounds__(256) void k_bbox(Dev d) {
-  const Chunk ch = chunk_at(d, blockIdx.x);
+__global__ __launch_bounds__(256, 6) void k_bbox(Dev d) {
+  Chunk ch;
+  if (d.ninst != 1) {
+    ch = d.chunks[blockIdx.x];
+  } else {  // an equal share of the points
+    const int64_t per = (d.n + gridDim.x - 1) / gridDim.x, lo = blockIdx.x * per;
+    ch.inst = 0;
+    ch.begin = lo < d.n ? lo : d.n - 1;
+    ch.end = lo + per < d.n ? lo + per : d.n;
+  }
   const Inst& I = d.inst[ch.inst];
   const int dim = I.dim;
   double mn[3] = {INFINITY, INFINITY, INFINITY};
@@ -189,7 +197,7 @@ __global__ __launch_bounds__(256) void k_bbox(Dev d) {
       }
     unsigned long long* bb =
         d.bbox + ((int64_t)ch.inst * kBoxStripes +
-                  (ch.begin - I.pt_begin) / kChunk % kBoxStripes) * 8;
+                  (d.ninst != 1 ? (ch.begin - I.pt_begin) / kChunk : blockIdx.x) % kBoxStripes) * 8;
     for (int k = 0; k < dim; ++k) {
       atomicMin(&bb[k], ord_d(s_red[0][k]));
       atomicMax(&bb[3 + k], ord_d(s_red[0][3 + k]));
@@ -204,7 +212,13 @@ __global__ __launch_bounds__(256) void k_bbox(Dev d) {
     // so it is enough that they have completed (a device-wide fence per
     // workgroup writes L2 back: 4 M points 65 us with it, 22 without)
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    s_last = atomicAdd((unsigned long long*)&d.ctl[C_BOXES], 1ull) + 1 == gridDim.x;
+    // counted in stripes first: one address takes about 10 ns per workgroup
+    const unsigned G = gridDim.x, g = blockIdx.x % kStripes;
+    s_last = 0;
+    if (atomicAdd((unsigned long long*)&d.stat[g * kStatStride + C_BOXES], 1ull) + 1 ==
+        (G - g + kStripes - 1) / kStripes)
+      s_last = atomicAdd((unsigned long long*)&d.ctl[C_BOXES], 1ull) + 1 ==
+               (G < (unsigned)kStripes ? G : (unsigned)kStripes);
   }
   __syncthreads();
   if (!s_last || threadIdx.x >= 64) return;
@@ -266,18 +280,24 @@ __device__ void setup_instance(Inst& I, const unsigned long long (&bb)[8],
   double mn[3] = {0, 0, 0}, mx[3] = {0, 0, 0};
   double emin = INFINITY;
   bool empty = I.pt_end <= I.pt_begin;
-  for (int k = 0; k < dim; ++k) {
-    mn[k] = empty ? 0.0 : unord_d(bb[k]);
-    mx[k] = empty ? 0.0 : unord_d(bb[3 + k]);
-    emin = fmin(emin, mx[k] - mn[k]);
-  }
+  // (constant indexes throughout: the arrays stay in registers)
+#pragma unroll
+  for (int k = 0; k < 3; ++k)
+    if (k < dim && !empty) {
+      mn[k] = unord_d(bb[k]);
+      mx[k] = unord_d(bb[3 + k]);
+    }
+#pragma unroll
+  for (int k = 0; k < 3; ++k)
+    if (k < dim) emin = fmin(emin, mx[k] - mn[k]);
   I.maxabs = empty ? 0.0 : unord_d(bb[6]);
   if (bb[7]) {
     // DCLUST_E_PARAM: non-finite input.  The instance keeps a one-cell
     // grid (every point in cell 0) so that every kernel stays in bounds;
     // its result is discarded.
     I.err = -1;
-    for (int k = 0; k < dim; ++k) mn[k] = mx[k] = 0.0;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) mn[k] = mx[k] = 0.0;
     I.maxabs = 0.0;
   }
   if (I.r > 0) {
@@ -293,8 +313,9 @@ __device__ void setup_instance(Inst& I, const unsigned long long (&bb)[8],
     // kernel stays in bounds; its result is discarded (error set)
     double inv = 1.0 / w;
     bool ok = true;
-    for (int k = 0; k < dim; ++k)
-      if (floor((mx[k] - mn[k]) * inv) + 1.0 > cap) ok = false;
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      if (k < dim && floor((mx[k] - mn[k]) * inv) + 1.0 > cap) ok = false;
     if (ok) break;
     if (I.err == 0) I.err = -6;  // DCLUST_E_CAPACITY
     w *= 2.0;
@@ -302,6 +323,7 @@ __device__ void setup_instance(Inst& I, const unsigned long long (&bb)[8],
   I.w = w;
   I.inv_w = 1.0 / w;
   cells = 1;
+#pragma unroll
   for (int k = 0; k < 3; ++k) {
     I.mn[k] = k < dim ? mn[k] : 0.0;
     I.nk[k] = 1;
@@ -315,7 +337,8 @@ __device__ void setup_instance(Inst& I, const unsigned long long (&bb)[8],
   I.cstride = dim == 3 ? by + 1 : 1;
   lines = bx * I.cstride;
   I.nlines = lines;
-  I.nzl = (long long)I.nk[dim - 1] << (dim - 1);
+  I.nzl = dim == 3 ? (long long)I.nk[2] << 2 : (long long)I.nk[1] << 1;
+  I.inv_nzl = 1.0 / (double)I.nzl;
   keys = (unsigned long long)lines * (unsigned long long)I.nzl;
   // FP32 guard band (units of w * 2^-29)
   const double gs = I.inv_w * 0x1p29;
@@ -693,7 +716,7 @@ __device__ __forceinline__ uint32_t sort_scan(uint32_t v, uint32_t (&s_w)[RS_T /
 // their order.  The tile is staged in LDS in local digit order and written
 // out in runs per digit.  `inline_scan`: few workgroups, which add up the
 // counts before them here instead of in a launch of their own.
-constexpr int kSortInline = 32;
+constexpr int kSortInline = 128;
 template <int KF, int NI>
 __global__ __launch_bounds__(RS_T, 4) void k_rs_scatter(Dev d, int pass, int nblk,
                                                         bool inline_scan) {
@@ -721,7 +744,7 @@ __global__ __launch_bounds__(RS_T, 4) void k_rs_scatter(Dev d, int pass, int nbl
   // where this workgroup's next entry of digit tid goes
   uint32_t pre = 0, tot = 0;
   if (inline_scan) {
-#pragma unroll 8
+#pragma unroll 16
     for (int q = 0; q < nblk; ++q) {
       const uint32_t c = d.hist[(int64_t)q * RS_D + tid];
       tot += c;
@@ -906,18 +929,24 @@ __device__ __forceinline__ int32_t inst_of_key(const Dev& d, uint64_t key, int l
 }
 
 // Column (within the instance) and place in the column of a key, decoded once
-// per cell.
+// per cell.  By the stored reciprocal: an instance has fewer than 2^42 columns,
+// so the rounded quotient is off by less than 2^-9 and its floor by one at
+// most.  (With integer divisions, unrolled and 64-bit ones among them,
+// k_csr_write took 13 us on 100 k points, 37 on 4 M, 127 on 32 M; 12, 33, 115 now.)
 __device__ __forceinline__ void split_key(const Inst& I, uint64_t key, int64_t& col,
                                           uint32_t& zl) {
-  const uint64_t rel = key - (uint64_t)I.key_base, nzl = (uint64_t)I.nzl;
-  if ((rel >> 32) == 0 && (nzl >> 32) == 0) {
-    const uint32_t q = (uint32_t)rel / (uint32_t)nzl;
-    col = q;
-    zl = (uint32_t)rel - q * (uint32_t)nzl;
-  } else {
-    col = (int64_t)(rel / nzl);
-    zl = (uint32_t)(rel - (uint64_t)col * nzl);
+  const uint64_t rel = key - (uint64_t)I.key_base;
+  int64_t q = (int64_t)((double)(int64_t)rel * I.inv_nzl);
+  int64_t r = (int64_t)rel - q * I.nzl;
+  if (r < 0) {
+    --q;
+    r += I.nzl;
+  } else if (r >= I.nzl) {
+    ++q;
+    r -= I.nzl;
   }
+  col = q;
+  zl = (uint32_t)r;
 }
 
 // Sum of the block counts v[0..b) (`scanned` false: they are counts; true:
@@ -945,8 +974,7 @@ __global__ __launch_bounds__(CS_T) void k_csr_write(Dev d, bool scanned) {
   if (abandoned(d)) return;
   const bool table = d.ctl[C_NLINES] <= d.line_cap;
   const int64_t t0 = (int64_t)blockIdx.x * CS_TILE;
-  __shared__ int s_w[4];
-  __shared__ int64_t s_run;
+  __shared__ int s_w[CS_I][4];
   const int wv = threadIdx.x >> 6;
   uint64_t kr[CS_I], kp[CS_I];
   load_key_pairs<KF, CS_I>(d, t0, kr, kp);
@@ -982,10 +1010,14 @@ __global__ __launch_bounds__(CS_T) void k_csr_write(Dev d, bool scanned) {
       cr[r] = (uint32_t)(I.line_base + col);
     }
   }
-  {
-    const int64_t pre = block_prefix(d.scan_tmp, blockIdx.x, scanned);
-    if (threadIdx.x == 0) s_run = pre;
+  // flags of every round and wave first: one barrier, not three a round
+#pragma unroll
+  for (int r = 0; r < CS_I; ++r) {
+    const int64_t i = t0 + r * CS_T + threadIdx.x;
+    const unsigned long long m = ballot(i < d.n && (i == 0 || kr[r] != kp[r]));
+    if (lane_id() == 0) s_w[r][wv] = __popcll(m);
   }
+  int64_t run = block_prefix(d.scan_tmp, blockIdx.x, scanned);
   __syncthreads();
 #pragma unroll
   for (int r = 0; r < CS_I; ++r) {
@@ -993,12 +1025,13 @@ __global__ __launch_bounds__(CS_T) void k_csr_write(Dev d, bool scanned) {
     bool inr = i < d.n;
     const uint64_t k = kr[r];
     const bool f = inr && (i == 0 || k != kp[r]);
-    unsigned long long m = ballot(f);
-    if (lane_id() == 0) s_w[wv] = __popcll(m);
-    __syncthreads();
-    int64_t pre = s_run;
-    for (int w = 0; w < wv; ++w) pre += s_w[w];
-    int64_t cid = pre + mbcnt(m) + (f ? 1 : 0) - 1;  // inclusive - 1
+    int64_t pre = run;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      pre += w < wv ? s_w[r][w] : 0;
+      run += s_w[r][w];
+    }
+    int64_t cid = pre + mbcnt(ballot(f)) + (f ? 1 : 0) - 1;  // inclusive - 1
     if (inr) {
       d.cell_of[i] = (int32_t)cid;
       if (f) {
@@ -1035,9 +1068,6 @@ __global__ __launch_bounds__(CS_T) void k_csr_write(Dev d, bool scanned) {
         d.ctl[C_NCELL] = cid + 1;
       }
     }
-    __syncthreads();
-    if (threadIdx.x == 0) s_run += s_w[0] + s_w[1] + s_w[2] + s_w[3];
-    __syncthreads();
   }
 }
 
@@ -1518,7 +1548,9 @@ __global__ __launch_bounds__(256) void k_nbr_stats(Dev d) {
 
 // ------------------------------------------------------------- launchers --
 void launch_index_head(const Dev& d, int nchunks, hipStream_t s) {
-  hipLaunchKernelGGL(k_bbox, dim3(nchunks), dim3(256), 0, s, d);
+  // (one instance: 1024 points and more a workgroup, a step of its threads)
+  const int64_t shares = std::max<int64_t>(1, std::min<int64_t>(2048, (d.n + 1023) / 1024));
+  hipLaunchKernelGGL(k_bbox, dim3(d.ninst == 1 ? (unsigned)shares : nchunks), dim3(256), 0, s, d);
   if (d.ninst != 1) hipLaunchKernelGGL(k_grid_setup, dim3(1), dim3(1024), 0, s, d);
 }
 

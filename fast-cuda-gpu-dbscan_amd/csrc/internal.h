@@ -151,6 +151,7 @@ struct Inst {
   int64_t cstride;             // columns per step of the first axis' blocks (3-D: one
                                // more than there are, so that the column before the
                                // first and after the last of a step is always empty)
+  double inv_nzl;              // fl(1 / nzl)
   int64_t pt_begin, pt_end;    // global point-index range
   int64_t xyz_off;             // element offset of the first coordinate
 };
@@ -161,7 +162,7 @@ constexpr long long kMaxLineTable = 1LL << 26;  // 512 MiB at most
 
 // Chunk of at most kChunk points of one instance (work list of the per-point
 // kernels that need the instance, so no point->instance search is needed;
-// host-built for a batch, computed from the chunk's number for one instance).
+// host-built, for a batch).
 constexpr int64_t kChunk = 4096;
 struct Chunk {
   int32_t inst;
@@ -626,17 +627,6 @@ __device__ __forceinline__ uint2 make_row(int32_t first, uint32_t bits, int32_t 
 // cell in slot s of a row
 __device__ __forceinline__ int32_t slot_cell(uint2 row, int s) {
   return (int32_t)row.x + __popc(row.y & ((1u << s) - 1u));
-}
-
-// Chunk b of the call's points.
-__device__ __forceinline__ Chunk chunk_at(const Dev& d, int b) {
-  if (d.ninst != 1) return d.chunks[b];
-  Chunk ch;
-  ch.inst = 0;
-  ch.pad = 0;
-  ch.begin = b * kChunk;
-  ch.end = ch.begin + kChunk < d.n ? ch.begin + kChunk : d.n;
-  return ch;
 }
 
 // Instance of a cell (a run of one instance reads the table entry directly,
