@@ -679,10 +679,10 @@ def main():
     st = dict(sts[-1])
     ms_step = dt / args.steps * 1e3
     value = n * args.steps / dt / 1e6
-    # The timed leg's replays record only the events around the whole run and
-    # the neighbour-count kernel (every event inside a graph idles the device
-    # for a few microseconds); an untimed leg with every phase event gives the
-    # phase table and the other kernels' times.
+    # The timed leg's replays time the whole run by events around it and the
+    # neighbour count by the device clock (every event inside a graph idles the
+    # device for a few microseconds); an untimed leg with every phase event
+    # gives the phase table and the other kernels' times.
     sts_ph = sts
     if not args.profile_run:
         os.environ["DCLUST_PHASE_TIMES"] = "1"
@@ -698,7 +698,8 @@ def main():
     for k, tk in KERNEL_TIME.items():
         if k not in kb:
             continue
-        # live HIP events on the library's stream: k_core's from the timed leg
+        # measured in these runs: k_core's time from the timed leg's device clock,
+        # the others' from the phase leg's events
         t_k = float(np.mean([s[tk] for s in (sts if k == "k_core" else sts_ph)]))
         if t_k <= 0:
             continue  # (a profile run has no phase leg)
@@ -719,7 +720,7 @@ def main():
         "config": {"workload": desc, "n_points": n, "dim": dim, "eps": info["eps"],
                    "minpts": info["minpts"],
                    "precision": "fp32+fp64 guard band" if f32 else "fp64"},
-        # the longest single kernel of the run (live HIP events): its algorithmic
+        # the longest of these kernels (times as above): its algorithmic
         # bytes from the work it did, and the HBM bytes rocprofv3 measured
         "roofline": {"kernel": dom, "bound": "hbm", "achieved": kd["achieved"],
                      "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": kd["frac"],

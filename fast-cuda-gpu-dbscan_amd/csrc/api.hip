@@ -5,9 +5,10 @@
 // seed lists, collision matrix and all labels back and forth every
 // iteration (main.cu:369-403, dbscan.cu:25-187).  Here a handle owns a
 // device arena that grows on demand and is reused; a run is a fixed sequence
-// of kernel launches on the handle's stream with two small host reads (the
-// sort key width after the grid set-up, and the correction-queue length
-// after each expansion pass).
+// of kernel launches on the handle's stream with one small host read (the
+// sort key width after the grid set-up; with seed lists also the
+// correction-queue length after each expansion pass), or one captured graph
+// without any.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -56,11 +57,11 @@ struct dclust_handle {
   // launch shapes found by dclust_autotune_device, keyed by (dimension mix,
   // log2 of the total point count, precision form)
   std::map<std::tuple<int, int, int>, dclust_params> tuned;
-  // replay of repeated identical calls
+  // replay of repeated calls
   std::vector<uint8_t> prev_sig;   // launch state of the last eager run
-  int prev_npass = 0;              // its expansion passes
-  long long prev_nlines = 0;       // its neighbour-line count
-  int prev_key_bits = 0;           // its sort key width
+  int prev_npass = 0;              // most of its runs so far: expansion passes,
+  long long prev_nlines = 0;       // columns
+  int prev_key_bits = 0;           // and sort key width
   hipGraphExec_t gexec = nullptr;  // captured run
   std::vector<uint8_t> gsig;       // launch state it was captured for
   int gpasses = 0;                 // expansion passes it holds

@@ -6,8 +6,8 @@
 // 5^D stencil of cells around its cell.  The stencil is covered by windows of
 // 3^(D-1) neighbour columns of cells ("rows", internal.h).
 //
-//   k_core, k_core_rest, k_core_crowd   one lane per point (a wavefront where
-//                the candidates are many): neighbour count with early exit
+//   k_core, k_core_rest, k_core_crowd   one lane per point, then several (a
+//                wavefront where the candidates are many): neighbour count with early exit
 //                at minpts -> core flag.  (dbscan.cu:331-369 counts while it
 //                expands; here the count is its own pass, so every later
 //                kernel knows which points are core.)  A cell holding
@@ -15,15 +15,16 @@
 //                point that stays below minpts has seen all its neighbours
 //                and records them for the border pass.
 //   k_rep, k_adj   the near graph over core cells: two cells at most one
-//                apart along every axis are linked when their representatives (one core point each)
-//                are certainly joined.
+//                apart along every axis are linked when their representatives
+//                (one core point each) are certainly joined.
 //   k_link_local, k_link_cross   components of the near graph by union-find,
 //                in LDS over runs of cells, then in global memory.
 //   k_expand     the same components by persistent seed-list expansion
 //                (dbscan.cu:254-387) over cells, for calls that give the
 //                reference's launch values (MAX_SEEDS, THREAD_BLOCKS,
-//                THREAD_COUNT, EXTRA_COLLISION_SIZE): each wavefront owns a seed list of cells in LDS and
-//                pops up to 64 of them at once, one per lane; each lane
+//                THREAD_COUNT, EXTRA_COLLISION_SIZE): each wavefront owns a
+//                seed list of cells in LDS and pops up to 64 of them at once,
+//                one per lane; each lane
 //                claims the adjacent unclaimed cells of its cell with one CAS
 //                each (MarkAsCandidate, dbscan.cu:189-222) and pushes them;
 //                cells already claimed by another chain become collision

@@ -5,13 +5,14 @@
 //                 host, initialised to 0 / 999999999; here +-inf)
 //   k_grid_setup  cell width, cells per axis, key space per instance
 //                 (main.cu:184-207 bin width + eps check, main.cu:209-244 tree
-//                 metadata: replaced by a flat grid)
-//   k_cellkey     per-point cell key (insertData, indexing.cu:107-118)
+//                 metadata: replaced by a flat grid); with one instance done
+//                 by the last workgroup of k_bbox
+//   k_cellkey(_hist)  per-point cell key (insertData, indexing.cu:107-118)
 //   radix sort    LDS radix sort of (key, id), stable (thrust::sort_by_key,
 //                 main.cu:332-333)
 //   CSR           wavefront ballot/mbcnt compaction of key changes into cell
 //                 ranges (INDEXING_ADJUSTMENT's per-leaf equal_range,
-//                 indexing.cu:23-51)
+//                 indexing.cu:23-51), and the table of columns
 //   k_gather      cell-sorted SoA coordinates (FP64 + fixed-point)
 //   k_rows        the windows of each cell's 3^(D-1) neighbour columns that
 //                 cover its stencil (cells of side eps/2, a 5^D stencil;

@@ -3,7 +3,7 @@
 // Data layout in HBM (all arrays live in the handle's arena, sized for the
 // largest run seen so far and reused):
 //   input   xyz       caller's row-major FP64 rows, instances back to back
-//   sort    key[2]    u64 cell keys (ping-pong), val[2] i32 point ids
+//   sort    key[2]    u32 or u64 cell keys (ping-pong), val[2] i32 point ids
 //   CSR     cell_start[C+1], cell_key[C], cell_inst[C], cell_col[C], cell_zl[C],
 //           rows[3^(D-1)][C] (windows of the neighbour columns),
 //           cell_ncore[C], cell_label[C] (chain), amask[C] (near graph), rep[C]
@@ -12,7 +12,8 @@
 //           orig[N], cell_of[N], core[N] u8, rec[N][R] + rec_n[N] (the
 //           neighbours of each non-core point)
 //   merge   parent[] union-find over cells, compmin[N], pairs[waves][E] int2
-//   output  keyv[N] (component min input index), flag[N] u8, rank[N]
+//   output  keyv[N] (component min input index), a flag bit per input index,
+//           rank[N/64]
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -20,7 +21,6 @@
 
 namespace dclust {
 
-constexpr int kWave = 64;
 constexpr int32_t kUnclaimed = -1;
 constexpr int32_t kNoKey = 0x7fffffff;
 constexpr int kFixBits = 29;  // fixed-point fraction bits per cell width
@@ -400,9 +400,6 @@ __device__ __forceinline__ int rl_i(int v, int l) {
 __device__ __forceinline__ uint32_t rl_u(uint32_t v, int l) {
   return (uint32_t)__builtin_amdgcn_readlane((int)v, l);
 }
-__device__ __forceinline__ float rl_f(float v, int l) {
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
-}
 __device__ __forceinline__ double rl_d(double v, int l) {
   long long b = __double_as_longlong(v);
   int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffLL), l);
@@ -456,12 +453,6 @@ __device__ __forceinline__ T wave_incl_scan(T v) {
     if (l >= o) v += u;
   }
   return v;
-}
-
-// Aggregated atomic add of a wave-uniform sum (one atomic per wave).
-__device__ __forceinline__ void wave_add(long long* p, long long v) {
-  long long s = wave_sum(v);
-  if (lane_id() == 0 && s != 0) atomicAdd((unsigned long long*)p, (unsigned long long)s);
 }
 
 // chain ids are seed cell indices: the id space is the cell count

@@ -85,9 +85,9 @@ typedef struct dclust_params {
 
 /* Per-run diagnostics.  Times are HIP-event milliseconds on the handle's
  * stream (the reference's clock() buckets, main.cu:410-432).  A replay of a
- * captured run records only the events of t_total_ms, t_index_ms and
- * t_core_ms (each event inside a graph idles the device for a few
- * microseconds); t_rows_ms, t_adj_ms, t_expand_ms, t_merge_ms, t_far_ms,
+ * captured run holds no events (each one inside a graph idles the device for
+ * a few microseconds): t_total_ms comes from the events around it, t_index_ms
+ * and t_core_ms from the device clock; t_rows_ms, t_adj_ms, t_expand_ms, t_merge_ms, t_far_ms,
  * t_border_ms, t_relabel_ms and diag[4] are then 0, unless the environment
  * variable DCLUST_PHASE_TIMES=1 is set when the call is made. */
 typedef struct dclust_stats {
@@ -177,14 +177,15 @@ int dclust_run(dclust_handle* h, const double* xyz, int64_t n,
 
 /* Same with device-resident input and output (HIP device pointers).
  *
- * Repeated calls: a call whose sizes, parameters, pointers and environment
- * switches all equal the previous call's is captured once into a hipGraph
- * and replayed from then on (the coordinates may change between calls).
- * A replay launches the whole run at once with no host read in between:
- * the radix passes of the previous run's key width and a fixed number of
- * expansion passes, one more than the previous run needed.  When the
- * replay finds that the key or the expansion needed more, the call reruns
- * eagerly and the next identical call captures a new graph.  The
+ * Repeated calls: a call whose dimensions, sizes, launch shape, precision,
+ * record slots (minpts in steps of eight, up to 32) and environment switches
+ * equal the previous call's is captured once into a hipGraph and replayed from
+ * then on; coordinates, buffers, eps, minpts and r may change between calls.
+ * A replay launches the whole run at once with no host read in between: the
+ * radix passes and the column table of the largest such run so far, and with
+ * seed lists one expansion pass more than the previous run needed.  When the
+ * replay finds that it needs more, the call reruns eagerly and the next one
+ * captures a larger graph.  The
  * environment variable DCLUST_GRAPH=0 turns replay off.  This applies to
  * every entry point that runs a clustering (dclust_run, the batched ones). */
 int dclust_run_device(dclust_handle* h, const double* d_xyz, int64_t n,
@@ -197,10 +198,10 @@ int dclust_run_device(dclust_handle* h, const double* d_xyz, int64_t n,
  * Same arguments, labels and statistics as dclust_run_device; every buffer
  * of the run comes from one 64 MiB array per GPU that the library's code
  * object carries, so the call makes no hipMalloc / hipFree.  Limit: the run
- * must fit that array -- about 230,000 3-D points in the FP32 form with
- * minpts <= 10 (about 210,000 in the FP64 form or with minpts >= 16, more
- * in 2-D); larger inputs return DCLUST_E_CAPACITY before any work.  The run is eager (no graph
- * replay).  All calls on one GPU share its array and each leaves its
+ * must fit that array -- about 270,000 3-D points in the FP32 form with
+ * minpts <= 10 (about 235,000 in the FP64 form with minpts >= 16, more in
+ * 2-D); larger inputs return DCLUST_E_CAPACITY before any work.  The run is
+ * eager (no graph replay).  All calls on one GPU share its array and each leaves its
  * contents there (dclust_last_core_flags reads them): calls that overlap on
  * one GPU, from any handles or threads, race. */
 int dclust_run_device_noalloc(dclust_handle* h, const double* d_xyz, int64_t n,
