@@ -549,13 +549,13 @@ hipError_t enqueue_tail(dclust_handle* h, const Dev& d, bool f32, int grid_cells
   if ((e = mark(h, E_FAR, graph)) != hipSuccess) return e;
   launch_border(d, f32, s);
   if ((e = mark(h, E_BORDER, graph)) != hipSuccess) return e;
-  launch_relabel(d, d.n, s);
+  launch_relabel(d, d.n, h->pin ? h->pin_dev : nullptr, s);
   if ((e = mark(h, E_END, graph)) != hipSuccess) return e;
   return hipGetLastError();
 }
 
-// The control counters and their stripes into the handle's pinned buffer
-// (inside a capture this becomes the graph's last kernel).
+// The control counters and their stripes into the handle's pinned buffer (the
+// run's last kernel does the same).
 hipError_t enqueue_readback(dclust_handle* h, const Dev& d, hipStream_t s) {
   launch_readback(d, h->pin_dev, s);
   return hipGetLastError();
@@ -589,7 +589,6 @@ hipError_t capture_run(dclust_handle* h, const Dev& d, const Call& call, const R
     if (p == 0) body = mark(h, E_PASS0, true);
   }
   if (body == hipSuccess) body = enqueue_tail(h, d, f32, grid_cells, true);
-  if (body == hipSuccess && h->pin) body = enqueue_readback(h, d, s);
   e = hipStreamEndCapture(s, &g);
   if (body != hipSuccess) e = body;
   if (e == hipSuccess) e = hipGraphInstantiate(out, g, nullptr, nullptr, 0);
@@ -1057,7 +1056,7 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
     ++npass;
     HIPCHK(enqueue_tail(h, d, f32, grid_cells, false));
     HIPCHK(copy_labels());
-    HIPCHK(read_counters(h, d, s, ctl_h));
+    HIPCHK(read_counters(h, d, s, ctl_h, h->pin != nullptr));
     finish_run(h, d, shape, ctl_h, npass, false, stats);
     if (npass >= kMaxExpandPasses) return DCLUST_E_CAPACITY;
     if (graph_on) {

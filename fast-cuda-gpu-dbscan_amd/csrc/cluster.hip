@@ -1898,6 +1898,8 @@ __global__ __launch_bounds__(256) void k_flatten(Dev d) {
 // and nothing is stored until every load is done, so the latencies overlap.
 constexpr int kRelU = 4;
 
+// Keys of the core points (k_border, which reads them, gives the others
+// theirs).
 __global__ __launch_bounds__(256) void k_keys(Dev d) {
   if (abandoned(d)) return;
   for (int64_t i0 = blockIdx.x * (int64_t)(kRelU * 256); i0 < d.n;
@@ -1922,14 +1924,14 @@ __global__ __launch_bounds__(256) void k_keys(Dev d) {
     for (int u = 0; u < kRelU; ++u) k[u] = d.compmin[pr[u]];
 #pragma unroll
     for (int u = 0; u < kRelU; ++u) {
-      const int64_t i = i0 + u * 256 + threadIdx.x;
-      if (i < d.n) {
-        d.keyv[i] = cr[u] ? k[u] : kNoKey;
-        if (cr[u] && o[u] == k[u]) atomicOr(&d.flag[k[u] >> 6], 1ull << (k[u] & 63));
+      if (cr[u]) {
+        d.keyv[ic[u]] = k[u];
+        if (o[u] == k[u]) atomicOr(&d.flag[k[u] >> 6], 1ull << (k[u] & 63));
       }
     }
   }
 }
+
 // ---------------------------------------------------------------- border --
 // P(q -> p) for a core point q and a non-core point p, evaluated from the
 // core point's side as its expansion in the reference oracle would.
@@ -2064,7 +2066,7 @@ __global__ __launch_bounds__(256) void k_border(Dev d) {
   if (abandoned(d)) return;
   const Stripe L(d.border_pts);
   Tally t;
-  long long ovf = 0;
+  long long ovf = 0, noise = 0;
   for (int64_t i0 = L.first(256); i0 < L.n; i0 += L.step(256)) {
     const int64_t i = i0 + threadIdx.x;
     const bool act = i < L.n;
@@ -2082,10 +2084,12 @@ __global__ __launch_bounds__(256) void k_border(Dev d) {
     DCLUST_BY_DIM(act, dim, (best = border_lane<3, F32>(d, P, p, c, t, ovf)),
                   (best = border_lane<2, F32>(d, P, p, c, t, ovf)));
     if (act) d.keyv[p] = best;
+    noise += act && best == kNoKey;
   }
   stat_add(d, C_BAND, t.band);
   stat_add(d, C_FLIP, t.flip);
   stat_add(d, C_RECOVF, ovf);
+  stat_add(d, C_NNOISE, noise);
 }
 
 // ------------------------------------------------------------ rank + out --
@@ -2184,9 +2188,9 @@ __device__ __forceinline__ int32_t rank_of(const Dev& d, int64_t k) {
 }
 
 // Labels of NI points from i0 on, RS apart, and their input indices (an index
-// past the end reads point 0); returns the number of noise points.
+// past the end reads point 0).
 template <int NI, int RS>
-__device__ __forceinline__ int point_labels(const Dev& d, int64_t i0, int32_t (&o)[NI],
+__device__ __forceinline__ void point_labels(const Dev& d, int64_t i0, int32_t (&o)[NI],
                                             int32_t (&lab)[NI]) {
   int32_t k[NI], rb[NI];
   int64_t pb[NI];
@@ -2202,28 +2206,31 @@ __device__ __forceinline__ int point_labels(const Dev& d, int64_t i0, int32_t (&
     lab[u] = rank_of(d, k[u] == kNoKey ? 0 : k[u]);
     rb[u] = d.ninst == 1 ? 0 : rank_of(d, pb[u]);
   }
-  int noise = 0;
 #pragma unroll
-  for (int u = 0; u < NI; ++u) {
-    lab[u] = k[u] == kNoKey ? 0 : lab[u] - rb[u] + 1;
-    noise += i0 + u * RS < d.n && k[u] == kNoKey;
-  }
-  return noise;
+  for (int u = 0; u < NI; ++u) lab[u] = k[u] == kNoKey ? 0 : lab[u] - rb[u] + 1;
 }
 
-__global__ __launch_bounds__(256) void k_output(Dev d) {
-  if (abandoned(d)) return;
+// A run's last kernel has a workgroup more that reads the counters back (`out`
+// not null: in a launch of their own 5 us a call); it does so in an abandoned
+// run too, where it is the only one that works.
+__device__ __forceinline__ bool reads_back(const Dev& d, long long* out) {
+  if (!out || blockIdx.x != gridDim.x - 1) return false;
+  readback(d, out);
+  return true;
+}
+
+__global__ __launch_bounds__(256) void k_output(Dev d, long long* out) {
+  if (reads_back(d, out) || abandoned(d)) return;
   int32_t* labels = out_labels(d);
-  long long noise = 0;
+  const int G = out ? gridDim.x - 1 : gridDim.x;
   for (int64_t i0 = blockIdx.x * (int64_t)(kRelU * 256) + threadIdx.x; i0 - threadIdx.x < d.n;
-       i0 += (int64_t)gridDim.x * (kRelU * 256)) {
+       i0 += (int64_t)G * (kRelU * 256)) {
     int32_t o[kRelU], lab[kRelU];
-    noise += point_labels<kRelU, 256>(d, i0, o, lab);
+    point_labels<kRelU, 256>(d, i0, o, lab);
 #pragma unroll
     for (int u = 0; u < kRelU; ++u)
       if (i0 + u * 256 < d.n) labels[o[u]] = lab[u];
   }
-  stat_add(d, C_NNOISE, noise);
 }
 
 // The labels of a large call in two steps.  Written one by one in sorted order
@@ -2252,18 +2259,16 @@ __global__ __launch_bounds__(512, 4) void k_output_split(Dev d, int shift, uint3
   s_cnt[tid] = 0;
   const int64_t t0 = (int64_t)blockIdx.x * (T * NI);
   int32_t o[NI], lab[NI];
-  int noise = 0;
 #pragma unroll
   for (int h = 0; h < NI; h += kRelU) {
     int32_t ho[kRelU], hl[kRelU];
-    noise += point_labels<kRelU, T>(d, t0 + tid + h * T, ho, hl);
+    point_labels<kRelU, T>(d, t0 + tid + h * T, ho, hl);
 #pragma unroll
     for (int u = 0; u < kRelU; ++u) {
       o[h + u] = ho[u];
       lab[h + u] = hl[u];
     }
   }
-  stat_add(d, C_NNOISE, noise);
   __syncthreads();
   uint32_t at[NI];
 #pragma unroll
@@ -2300,11 +2305,12 @@ __global__ __launch_bounds__(512, 4) void k_output_split(Dev d, int shift, uint3
 // in order (written from the pairs directly, the scattered 4-byte requests took
 // 236 us on 32 M points).
 template <int PART, int T>
-__global__ __launch_bounds__(T) void k_output_place(Dev d, int shift, const uint2* pairs) {
-  if (abandoned(d)) return;
+__global__ __launch_bounds__(T) void k_output_place(Dev d, int shift, const uint2* pairs,
+                                                    long long* out) {
+  if (reads_back(d, out) || abandoned(d)) return;
   __shared__ int32_t s_l[PART];
   constexpr int U = 8;
-  const int64_t first = (int64_t)xcd_runs<8>(blockIdx.x, gridDim.x) * PART;
+  const int64_t first = (int64_t)xcd_runs<8>(blockIdx.x, out ? gridDim.x - 1 : gridDim.x) * PART;
   const int64_t w0 = first >> shift << shift;
   const int64_t w1 = w0 + (1LL << shift) < d.n ? w0 + (1LL << shift) : d.n;
   for (int64_t i0 = w0 + threadIdx.x; i0 < w1; i0 += T * U) {
@@ -2434,7 +2440,8 @@ void launch_core_out(const uint8_t* core, const int32_t* orig, int64_t n, uint8_
   hipLaunchKernelGGL(k_core_out, dim3(g), dim3(256), 0, s, core, orig, n, out);
 }
 
-void launch_relabel(const Dev& d, int64_t n, hipStream_t s) {
+void launch_relabel(const Dev& d, int64_t n, long long* out, hipStream_t s) {
+  const unsigned rb = out ? 1 : 0;  // (the workgroup that reads the counters back)
   const int nb = (int)(((n + 63) / 64 + RK_TILE - 1) / RK_TILE);
   const bool split = n >= kOutSplit && n <= kOutWindows * kOutWindow;
   if ((n + 63) / 64 <= kRankOne) {
@@ -2454,13 +2461,13 @@ void launch_relabel(const Dev& d, int64_t n, hipStream_t s) {
                        dim3(512), 0, s, d, shift, d.hist, pairs);
     // (a window smaller than the part it is gathered in shares its workgroup)
     if (shift > 13)
-      hipLaunchKernelGGL((k_output_place<32768, 1024>), dim3((unsigned)((n + 32767) / 32768)),
-                         dim3(1024), 0, s, d, std::max(shift, 15), pairs);
+      hipLaunchKernelGGL((k_output_place<32768, 1024>), dim3((unsigned)((n + 32767) / 32768) + rb),
+                         dim3(1024), 0, s, d, std::max(shift, 15), pairs, out);
     else
-      hipLaunchKernelGGL((k_output_place<8192, 512>), dim3((unsigned)((n + 8191) / 8192)),
-                         dim3(512), 0, s, d, 13, pairs);
+      hipLaunchKernelGGL((k_output_place<8192, 512>), dim3((unsigned)((n + 8191) / 8192) + rb),
+                         dim3(512), 0, s, d, 13, pairs, out);
   } else {
-    hipLaunchKernelGGL(k_output, dim3(g2), dim3(256), 0, s, d);
+    hipLaunchKernelGGL(k_output, dim3(g2 + rb), dim3(256), 0, s, d, out);
   }
 }
 

@@ -81,26 +81,9 @@ void launch_init_head(const Dev& d, const Call* src, const Call& v, hipStream_t 
   hipLaunchKernelGGL(k_init_head, dim3(fill_grid(tot)), dim3(256), 0, s, d, src, v);
 }
 
-// End of a run: the control counters, their stripes added, into a host buffer
-// (pinned and mapped): one workgroup, a wavefront per counter, a lane per
-// stripe.  Inside a captured run this follows the last kernel with no gap,
-// where copy nodes would each wait on a separate transfer.
-static_assert((C_NCTL + 15) / 16 * 16 <= kStatStride, "counters of a stripe");
-__global__ __launch_bounds__(1024) void k_readback(Dev d, long long* out) {
-  constexpr int R = (C_NCTL + 15) / 16;  // counters per wavefront
-  const int wv = threadIdx.x >> 6;
-  long long v[R], base[R];
-#pragma unroll
-  for (int r = 0; r < R; ++r) {  // (past the last counter: the stripe's padding)
-    v[r] = d.stat[lane_id() * kStatStride + wv + 16 * r];
-    base[r] = d.ctl[wv + 16 * r < C_NCTL ? wv + 16 * r : 0];
-  }
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    const long long s = wave_sum(v[r]);
-    if (lane_id() == 0 && wv + 16 * r < C_NCTL) out[wv + 16 * r] = base[r] + s;
-  }
-}
+// The counters after the grid set-up of an eager run (a run's last kernel
+// reads them back itself).
+__global__ __launch_bounds__(1024) void k_readback(Dev d, long long* out) { readback(d, out); }
 
 void launch_readback(const Dev& d, long long* out, hipStream_t s) {
   hipLaunchKernelGGL(k_readback, dim3(1), dim3(1024), 0, s, d, out);

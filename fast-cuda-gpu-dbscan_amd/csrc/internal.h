@@ -534,6 +534,27 @@ struct Stripe {
   }
 };
 
+// The control counters, their stripes added, into the handle's pinned buffer,
+// by one workgroup of at least four wavefronts: a lane per counter, a share of
+// the stripes per wavefront.
+static_assert(C_NCTL <= 64 && kStatStride == 64, "a lane per counter");
+__device__ __forceinline__ void readback(const Dev& d, long long* out) {
+  __shared__ long long s_sum[16][64];
+  const int l = lane_id(), wv = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  long long v[kStripes / 4], sum = wv == 0 && l < C_NCTL ? d.ctl[l] : 0;
+#pragma unroll
+  for (int r = 0; r < kStripes / 4; ++r)
+    v[r] = wv + r * nw < kStripes ? d.stat[(wv + r * nw) * kStatStride + l] : 0;
+#pragma unroll
+  for (int r = 0; r < kStripes / 4; ++r) sum += v[r];
+  s_sum[wv][l] = sum;
+  __syncthreads();
+  if (threadIdx.x >= C_NCTL) return;
+  sum = 0;
+  for (int w = 0; w < nw; ++w) sum += s_sum[w][l];
+  out[l] = sum;
+}
+
 // Prefix of the sub-list counts of L in LDS (s_pre[kStripes + 1]); returns
 // the list length.  Every thread of the workgroup calls it.
 __device__ __forceinline__ long long slist_prefix(const SList& L, long long* s_pre) {

@@ -41,7 +41,8 @@ int64_t cell_blocks(int64_t n);
 // stencil pairs across components, then final roots
 void launch_far(const Dev& d, bool f32, int grid, hipStream_t s);
 void launch_border(const Dev& d, bool f32, hipStream_t s);
-void launch_relabel(const Dev& d, int64_t n, hipStream_t s);
+// (`out`: the counters go there with the run's last kernel, or null)
+void launch_relabel(const Dev& d, int64_t n, long long* out, hipStream_t s);
 // core flags of the last run (cell-sorted core[], orig[]) to input order
 void launch_core_out(const uint8_t* core, const int32_t* orig, int64_t n, uint8_t* out,
                      hipStream_t s);
