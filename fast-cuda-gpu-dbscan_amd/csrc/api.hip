@@ -119,8 +119,8 @@ struct dclust_handle {
 namespace {
 
 enum Slot {
-  S_XYZ, S_INST, S_CHUNK, S_BBOX, S_CTL, S_KEY, S_VAL, S_HIST, S_OFFS,
-  S_DTOT, S_CSTART, S_CKEY, S_CINST, S_CM, S_ROWS, S_CELLOF, S_X,
+  S_XYZ, S_INST, S_CHUNK, S_BBOX, S_CTL, S_KEY, S_VAL, S_HIST, S_DGRP,
+  S_CSTART, S_CKEY, S_CINST, S_CM, S_ROWS, S_CELLOF, S_X,
   S_G, S_ORIG, S_CORE, S_LABEL, S_PARENT, S_COMPMIN, S_PAIRS, S_Q0, S_Q1,
   S_KEYV, S_FLAG, S_RANK, S_SCAN, S_LABOUT, S_COREOUT, S_PAIRCNT, S_SEGPOS, S_LINES, S_AMASK,
   S_REC, S_RECN, S_CCOL, S_CCOMP, S_BORDERPTS, S_CORECELLS, S_TUNELAB, S_STAT, S_GLINES,
@@ -842,8 +842,7 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
     d.far_heavy = PairList{(int2*)d.val[0] + cap_f * kStripes,
                            (unsigned long long*)(d.stat + C_NFARHEAVY), cap_f};
     d.hist = M.get<uint32_t>(S_HIST, sort_hist_entries(ntot));
-    d.offs = M.get<uint32_t>(S_OFFS, sort_hist_entries(ntot));
-    d.dtot = M.get<uint32_t>(S_DTOT, 1 << kDigitBits);
+    d.dgrp = M.get<uint32_t>(S_DGRP, (size_t)kSortPasses * kSortGroups << kDigitBits);
     d.cell_start = M.get<int32_t>(S_CSTART, ntot + 1);
     d.cell_key = M.get<uint64_t>(S_CKEY, ntot);
     d.cell_col = M.get<uint32_t>(S_CCOL, ntot);

@@ -34,19 +34,20 @@ static int fill_grid(int64_t n) {
   return (int)b;
 }
 
-// Start of a run, one launch: control counters, statistics stripes and the
-// bounding-box stripes (per instance and stripe: 0..2 min
+// Start of a run, one launch: control counters, statistics stripes, the sort's
+// group counts and the bounding-box stripes (per instance and stripe: 0..2 min
 // as ordered keys starting at the largest key, 3..5 max, 6 max |x|, 7
 // non-finite flag, all starting at 0).  What the call brings (input, output,
 // the parameters of a single instance) is taken from `src` (pinned host
 // memory) in a captured run, whose replays read what the host left there,
 // else from `v`.
+constexpr int64_t kGroupWords = ((int64_t)kSortPasses * kSortGroups << kDigitBits) / 2;
 __global__ __launch_bounds__(256) void k_init_head(Dev d, const Call* src, Call v) {
   constexpr int kInstWords = sizeof(Inst) / 8;
   const int64_t nb = (int64_t)d.ninst * kBoxStripes * 8;
   const int64_t ns = (int64_t)kStatStride * kStripes;
   const int64_t ni = d.ninst == 1 ? kInstWords : d.ninst;
-  const int64_t tot = nb + ns + C_NCTL + ni;
+  const int64_t tot = nb + ns + C_NCTL + ni + kGroupWords;
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < tot;
        i += (int64_t)gridDim.x * blockDim.x) {
     if (i < nb) {
@@ -60,6 +61,8 @@ __global__ __launch_bounds__(256) void k_init_head(Dev d, const Call* src, Call 
       if (c == C_LABELS) w = reinterpret_cast<long long>(src ? src->labels : v.labels);
       if (c == C_T_START) w = (long long)__builtin_amdgcn_s_memrealtime();
       d.ctl[c] = w;
+    } else if (i >= tot - kGroupWords) {
+      reinterpret_cast<unsigned long long*>(d.dgrp)[i - (tot - kGroupWords)] = 0ull;
     } else {
       const int64_t k = i - nb - ns - C_NCTL;
       if (d.ninst == 1) {
@@ -77,7 +80,7 @@ __global__ __launch_bounds__(256) void k_init_head(Dev d, const Call* src, Call 
 
 void launch_init_head(const Dev& d, const Call* src, const Call& v, hipStream_t s) {
   const int64_t tot = (int64_t)d.ninst * kBoxStripes * 8 + (int64_t)kStatStride * kStripes + C_NCTL +
-                      std::max<int64_t>(d.ninst, sizeof(Inst) / 8);
+                      std::max<int64_t>(d.ninst, sizeof(Inst) / 8) + kGroupWords;
   hipLaunchKernelGGL(k_init_head, dim3(fill_grid(tot)), dim3(256), 0, s, d, src, v);
 }
 
@@ -470,16 +473,16 @@ __device__ __forceinline__ int32_t cell_index(double x, const Inst& I, int k) {
 }
 
 // ------------------------------------------------------------ radix sort --
-// LSD radix sort by digits of at most 9 bits, three launches a pass.  Every
+// LSD radix sort by digits of at most 9 bits, two launches a pass.  Every
 // workgroup owns one contiguous range of the entries, so the digit counts are
-// few ([workgroups][512], a scan of a few microseconds), and its tiles write
-// one after the other to neighbouring places, whose partial lines its L2
+// few ([workgroups][512], added up in groups as they are made), and its tiles
+// write one after the other to neighbouring places, whose partial lines its L2
 // joins.  Buffer parity: the number of passes.
 //
 // Bound by the bytes it moves, in runs of a few dozen bytes, at the larger sizes
 // and by launches and each workgroup's chain of barriers at the smaller.  Per
-// pass, 32 M points of 33 bits: count 29 us, scan 6, scatter 147 to 177 (four
-// passes); 4 M of 32 bits 6 + 6 + 24 (four).  Before (8-bit digits, one tile of
+// pass, 32 M points of 33 bits: count 29 us, scatter 147 to 177 (four passes);
+// 4 M of 32 bits 6 + 26 (four).  Before (8-bit digits, one tile of
 // 2048 keys a workgroup, counts [256][n / 2048]) 88 + 43 + 233 (five passes of
 // 64-bit keys) and 15 + 6 + 22.  Interleaving the tiles of neighbouring
 // workgroups instead (one tile each) took longer, 225 us a scatter.
@@ -540,13 +543,16 @@ __device__ __forceinline__ void hist_clear(uint32_t (&h)[RS_D * kHistCopies]) {
   for (int c = 0; c < kHistCopies; ++c) h[c * RS_T + threadIdx.x] = 0;
   __syncthreads();
 }
+// (also to the counts of the workgroup's group, which start at zero)
 __device__ __forceinline__ void hist_store(const Dev& d, uint32_t (&h)[RS_D * kHistCopies],
-                                           int b) {
+                                           int pass, int b) {
   __syncthreads();
   uint32_t sum = 0;
 #pragma unroll
   for (int c = 0; c < kHistCopies; ++c) sum += h[threadIdx.x * kHistCopies + c];
   d.hist[(int64_t)b * RS_D + threadIdx.x] = sum;
+  if (sum)
+    atomicAdd(&d.dgrp[(pass * kSortGroups + b / kSortGroup) * RS_D + threadIdx.x], sum);
 }
 
 template <int D, int KF, int T, typename F>
@@ -617,7 +623,7 @@ __global__ __launch_bounds__(RS_T) void k_cellkey_hist(Dev d, int nblk) {
   const int copy = threadIdx.x & (kHistCopies - 1);
   cellkeys<KF, RS_T>(d, 0, lo, hi,
                      [&](uint32_t k) { atomicAdd(&h[(k & mask) * kHistCopies + copy], 1u); });
-  hist_store(d, h, b);
+  hist_store(d, h, 0, b);
 }
 
 template <int KF>
@@ -651,31 +657,7 @@ __global__ __launch_bounds__(RS_T) void k_rs_hist(Dev d, int pass, int nblk) {
       if (i0 + u * RS_T < hi) 
         atomicAdd(&h[entry_digit<KF>(k[u], v[u], shift, mask) * kHistCopies + copy], 1u);
   }
-  hist_store(d, h, b);
-}
-
-// Counts of the workgroups before each, and the digit totals: a workgroup
-// takes eight digits, 32 segments of the rows each.
-__global__ __launch_bounds__(256) void k_rs_rowscan(Dev d, int pass, int nblk) {
-  if (pass >= sort_passes(d)) return;
-  __shared__ uint32_t s_seg[32][8];
-  const int dg = blockIdx.x * 8 + (threadIdx.x & 7), sg = threadIdx.x >> 3;
-  const int per = (nblk + 31) / 32;
-  const int r0 = sg * per < nblk ? sg * per : nblk, r1 = r0 + per < nblk ? r0 + per : nblk;
-  uint32_t sum = 0;
-#pragma unroll 8
-  for (int r = r0; r < r1; ++r) sum += d.hist[(int64_t)r * RS_D + dg];
-  s_seg[sg][threadIdx.x & 7] = sum;
-  __syncthreads();
-  uint32_t pre = 0;
-  for (int s = 0; s < sg; ++s) pre += s_seg[s][threadIdx.x & 7];
-  if (sg == 31) d.dtot[dg] = pre + sum;
-#pragma unroll 8
-  for (int r = r0; r < r1; ++r) {
-    const uint32_t c = d.hist[(int64_t)r * RS_D + dg];
-    d.offs[(int64_t)r * RS_D + dg] = pre;
-    pre += c;
-  }
+  hist_store(d, h, pass, b);
 }
 
 // Exclusive scan over the workgroup's RS_T threads (a barrier inside; s_w is
@@ -698,12 +680,11 @@ __device__ __forceinline__ uint32_t sort_scan(uint32_t v, uint32_t (&s_w)[RS_T /
 // in order); one barrier later each digit's counts of the waves before it and
 // the tile's local starts turn the ranks into positions, so equal digits keep
 // their order.  The tile is staged in LDS in local digit order and written
-// out in runs per digit.  `inline_scan`: few workgroups, which add up the
-// counts before them here instead of in a launch of their own.
-constexpr int kSortInline = 128;
+// out in runs per digit.  The counts of the workgroups before come from the
+// groups and from the rows of the own group, at most 47 loads a thread (a scan
+// of all rows in a launch of its own took 5 us a pass).
 template <int KF, int NI>
-__global__ __launch_bounds__(RS_T, 4) void k_rs_scatter(Dev d, int pass, int nblk,
-                                                        bool inline_scan) {
+__global__ __launch_bounds__(RS_T, 4) void k_rs_scatter(Dev d, int pass, int nblk) {
   using KT = SortKey<KF>;
   constexpr int TILE = RS_T * NI, NW = RS_T / 64;
   const int np = sort_passes(d);
@@ -727,16 +708,19 @@ __global__ __launch_bounds__(RS_T, 4) void k_rs_scatter(Dev d, int pass, int nbl
   sort_range(d.n, b, nblk, lo, hi);
   // where this workgroup's next entry of digit tid goes
   uint32_t pre = 0, tot = 0;
-  if (inline_scan) {
-#pragma unroll 16
-    for (int q = 0; q < nblk; ++q) {
-      const uint32_t c = d.hist[(int64_t)q * RS_D + tid];
-      tot += c;
-      pre += q < b ? c : 0u;
-    }
-  } else {
-    pre = d.offs[(int64_t)b * RS_D + tid];
-    tot = d.dtot[tid];
+  const int grp = b / kSortGroup;
+#pragma unroll
+  for (int q = 0; q < kSortGroups; ++q) {
+    const uint32_t c = d.dgrp[(pass * kSortGroups + q) * RS_D + tid];
+    tot += c;
+    pre += q < grp ? c : 0u;
+  }
+  for (int q0 = grp * kSortGroup; q0 < b; q0 += 16) {
+    uint32_t c[16];  // (rows past the own one are read, not counted: one trip)
+#pragma unroll
+    for (int u = 0; u < 16; ++u) c[u] = d.hist[(int64_t)(q0 + u < b ? q0 + u : b) * RS_D + tid];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) pre += q0 + u < b ? c[u] : 0u;
   }
   uint32_t goff = sort_scan(tot, s_w1) + pre;
   // (32-bit places from here on: ids are 32-bit too)
@@ -1539,7 +1523,7 @@ void launch_index_head(const Dev& d, int nchunks, hipStream_t s) {
 }
 
 // Workgroups and entries per thread of the radix passes over n entries: at most
-// kSortGrid workgroups (two per CU; more of them only lengthen the scan), and
+// kSortGrid workgroups (two per CU; with 768 or 1024 the scatters of 4 M points took 129 and 134 us), and
 // the largest tile of which each still gets one and a half or more, so that one
 // tile's loads run beside another's write-out.  Scatter of all passes, us, at
 // 2 / 4 / 8 / 16 entries per thread: 10 k points 12 / 15 / 17 / -, 262 k
@@ -1547,7 +1531,6 @@ void launch_index_head(const Dev& d, int nchunks, hipStream_t s) {
 // 44 / 45 / 60 / 55, 4 M 152 / 112 / 96 / 126, 8 M (batch) 233 / 178 / 171 / 156,
 // 32 M - / 833 / 692 / 622.  (64-bit keys stop at 8: the tile has 12 bytes an
 // entry.)
-constexpr int kSortGrid = 512;
 struct SortShape {
   int blocks, items;
 };
@@ -1565,12 +1548,10 @@ constexpr int kClearGrid = 1024;
 
 template <int KF, int NI>
 static void radix_passes(const Dev& d, int passes, int nblk, hipStream_t s) {
-  const bool inl = nblk <= kSortInline;
   for (int p = 0; p < passes; ++p) {
     if (p > 0 || d.ninst != 1)
       hipLaunchKernelGGL(k_rs_hist<KF>, dim3(nblk), dim3(RS_T), 0, s, d, p, nblk);
-    if (!inl) hipLaunchKernelGGL(k_rs_rowscan, dim3(RS_D / 8), dim3(256), 0, s, d, p, nblk);
-    hipLaunchKernelGGL((k_rs_scatter<KF, NI>), dim3(nblk), dim3(RS_T), 0, s, d, p, nblk, inl);
+    hipLaunchKernelGGL((k_rs_scatter<KF, NI>), dim3(nblk), dim3(RS_T), 0, s, d, p, nblk);
   }
 }
 

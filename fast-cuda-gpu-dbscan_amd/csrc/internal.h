@@ -289,6 +289,10 @@ struct PairList {
 // runs unless every key has the same digit (then the data is already in
 // order and the buffers are not swapped).
 constexpr int kDigitBits = 9;  // of a radix pass, at most
+constexpr int kSortPasses = 8;  // of up to 64 bits
+constexpr int kSortGrid = 512;  // workgroups of the sort, at most
+constexpr int kSortGroup = 32;  // of which so many add to one group's counts
+constexpr int kSortGroups = kSortGrid / kSortGroup;
 
 // Bounding-box partials: chunk b of an instance reduces into stripe b % kBoxStripes of its
 // instance (so that the atomics of many chunks do not meet on one address);
@@ -324,8 +328,7 @@ struct Dev {
   uint64_t* key[2];
   int32_t* val[2];
   uint32_t* hist;   // [nblk][512] digit counts of the sort's workgroups
-  uint32_t* offs;   // [nblk][512] digit counts of the workgroups before
-  uint32_t* dtot;   // [512] digit totals of the current pass
+  uint32_t* dgrp;   // [kSortPasses][kSortGroups][512] digit counts of its groups
 
   // CSR
   int32_t* cell_start;  // [N+1]

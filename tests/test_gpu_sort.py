@@ -20,7 +20,7 @@ def _pairs(n, dim, span, eps, seed):
     return x
 
 
-# one workgroup and its edges; inline and separate scans (128 workgroups of 1024
+# one workgroup and its edges; four and five groups of 32 workgroups (128 of 1024
 # entries: 131072); the first sizes of 4 and 8 entries a thread
 @pytest.mark.parametrize("n", [1, 2, 511, 1024, 1025, 32768, 32769, 65537, 131072, 131073, 1572863, 1572865, 3145729])
 def test_sizes(devmem, n):
