@@ -573,14 +573,15 @@ __device__ __forceinline__ void cellkey_points(const Dev& d, const Inst& I, int6
       const int64_t i = i0 + u * T;
       if (i < np) {
         const int32_t cx = cell_index(v[u][0], I, 0), cl = cell_index(v[u][D - 1], I, D - 1);
-        int64_t lin;
+        uint64_t lin;  // (unsigned: an instance may have a few keys above 2^63)
         if (D == 3) {
           const int32_t cy = cell_index(v[u][1], I, 1);
-          lin = ((cx >> 1) * I.cstride + (cy >> 1)) * I.nzl + cl * 4LL + (cx & 1) * 2 + (cy & 1);
+          lin = (uint64_t)((cx >> 1) * I.cstride + (cy >> 1)) * (uint64_t)I.nzl +
+                (uint64_t)(cl * 4LL + (cx & 1) * 2 + (cy & 1));
         } else {
-          lin = (cx >> 1) * I.nzl + cl * 2LL + (cx & 1);
+          lin = (uint64_t)((cx >> 1) * I.nzl + cl * 2LL + (cx & 1));
         }
-        const uint64_t key = I.key_base + lin;
+        const uint64_t key = (uint64_t)I.key_base + lin;
         key_buf<KF>(d, 0)[begin + i] = (SortKey<KF>)(KF == 36 ? key >> 4 : key);
         // (the first pass knows the ids, which are the positions)
         if (KF == 36)
@@ -899,13 +900,14 @@ __device__ __forceinline__ int32_t inst_of_key(const Dev& d, uint64_t key, int l
 // Column (within the instance) and place in the column of a key, decoded once
 // per cell.  By the stored reciprocal: an instance has fewer than 2^42 columns,
 // so the rounded quotient is off by less than 2^-9 and its floor by one at
-// most.  (With integer divisions, unrolled and 64-bit ones among them,
+// most.  Unsigned up to the remainder: 2^21 cells along each of three axes have
+// keys up to 2^63 + 2^43.  (With integer divisions, unrolled and 64-bit ones among them,
 // k_csr_write took 13 us on 100 k points, 37 on 4 M, 127 on 32 M; 12, 33, 115 now.)
 __device__ __forceinline__ void split_key(const Inst& I, uint64_t key, int64_t& col,
                                           uint32_t& zl) {
   const uint64_t rel = key - (uint64_t)I.key_base;
-  int64_t q = (int64_t)((double)(int64_t)rel * I.inv_nzl);
-  int64_t r = (int64_t)rel - q * I.nzl;
+  int64_t q = (int64_t)((double)rel * I.inv_nzl);
+  int64_t r = (int64_t)(rel - (uint64_t)q * (uint64_t)I.nzl);
   if (r < 0) {
     --q;
     r += I.nzl;
