@@ -106,6 +106,7 @@ struct dclust_handle {
         want = bytes;
       }
       if (e != hipSuccess) {
+        (void)hipGetLastError();  // (else the next call's launch check finds it)
         *err = e;
         b.p = nullptr;
         return nullptr;
