@@ -84,10 +84,15 @@ struct dclust_handle {
   bool stage_failed = false;
   hipEvent_t stage_ev[2] = {};
   // the instance table and chunk list last copied to the device, and where
-  // (a replay with the same bytes at the same place skips the copies)
+  // (a replay with the same bytes at the same place skips the copies; memory
+  // that is freed takes them with it, whatever later has its address)
   std::vector<uint8_t> up_bytes;
   const void* up_inst = nullptr;
   const void* up_chunks = nullptr;
+  void forget_upload() {
+    up_bytes.clear();
+    up_inst = up_chunks = nullptr;
+  }
 
   template <class T>
   T* get(int slot, size_t count, hipError_t* err) {
@@ -95,6 +100,7 @@ struct dclust_handle {
     Buf& b = bufs[slot];
     size_t bytes = std::max<size_t>(count, 1) * sizeof(T);
     if (b.cap < bytes) {
+      if (b.p && (b.p == up_inst || b.p == up_chunks)) forget_upload();
       if (b.p) (void)hipFree(b.p);
       b.p = nullptr;
       b.cap = 0;
@@ -949,7 +955,7 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
     // error codes; a single instance comes with the first kernel)
     auto upload = [&]() -> hipError_t {
       if (ninst == 1) {
-        h->up_bytes.clear();  // (the arena's table is overwritten)
+        h->forget_upload();  // (the arena's table is overwritten)
         return hipSuccess;
       }
       std::vector<uint8_t> up(sizeof(Inst) * ninst + sizeof(Chunk) * nchunks);
@@ -963,8 +969,7 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
         ue = hipMemcpyAsync((void*)d.chunks, chunks.data(), sizeof(Chunk) * nchunks,
                             hipMemcpyHostToDevice, s);
       if (fixed_mem || ue != hipSuccess) {
-        h->up_bytes.clear();  // (a fixed region is not the arena)
-        h->up_inst = h->up_chunks = nullptr;
+        h->forget_upload();  // (a fixed region is not the arena)
       } else {
         h->up_bytes.swap(up);
         h->up_inst = d.inst;
@@ -1075,6 +1080,7 @@ fail:
   if (stats) stats->hip_error = (int32_t)herr;
   h->last_err = (int)herr;
   h->prev_sig.clear();
+  h->forget_upload();  // (its copies may not have completed)
   return DCLUST_E_HIP;
 }
 

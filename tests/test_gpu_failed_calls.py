@@ -34,3 +34,28 @@ def test_call_after_one_out_of_memory(devmem, replays):
             devmem.h2d(d_l, np.full(n, -7, dtype=np.int32))
             h.run_device(d_x, n, p, d_l)
             assert np.array_equal(devmem.download(np.empty(n, dtype=np.int32), d_l), ref)
+
+
+def test_batch_after_a_call_out_of_memory(devmem):
+    # the instance table and the chunk list of a repeated batch stay on the
+    # device; a batch of more instances takes new ones and then finds no memory
+    # (2^47 bytes of collision pairs), so the next batch has to bring its own
+    xs = [_blobs(n, d, n) for n, d in ((700, 2), (5000, 3), (300, 2))]
+    ps = [dclust.make_params(x.shape[1], 0.02, 4) for x in xs]
+    ns = np.array([len(x) for x in xs], dtype=np.int64)
+    refs = np.concatenate([oracle.fast_dbscan(x, 0.02, 4)[0] for x in xs])
+    d_x = devmem.upload(np.concatenate([x.ravel() for x in xs]))
+    d_l = devmem.alloc(4 * int(ns.sum()))
+    more = np.full(3000, 2, dtype=np.int64)
+    d_m, d_ml = devmem.upload(np.zeros(3000 * 2 * 2)), devmem.alloc(4 * 6000)
+    huge = [dclust.make_params(2, 0.02, 4, seeds=64, blocks=8192, threads=256,
+                               extra=2 ** 31 - 1)] * 3000
+    with dclust.Handle(0) as h:
+        for fail in (False, False, True, True, False):
+            if fail:
+                with pytest.raises(dclust.DclustError) as e:
+                    h.run_batched_device(d_m, more, huge, d_ml)
+                assert e.value.code == dclust.E_OOM
+            devmem.h2d(d_l, np.full(int(ns.sum()), -7, dtype=np.int32))
+            assert not np.any(h.run_batched_device(d_x, ns, ps, d_l))
+            assert np.array_equal(devmem.download(np.empty_like(refs), d_l), refs)
