@@ -49,7 +49,7 @@ struct dclust_handle {
   hipStream_t stream = nullptr;
   hipEvent_t ev[E_N] = {};
   std::vector<Buf> bufs;
-  int64_t last_n = -1;
+  int64_t last_n = -1;  // points of the last run (-1: none, or its arrays are gone)
   uint8_t* last_core = nullptr;        // device, cell-sorted core flags of the last run
   const int32_t* last_orig = nullptr;  // device, cell-sorted input indices
   uint8_t* last_core_out = nullptr;    // device, input-order staging
@@ -101,6 +101,10 @@ struct dclust_handle {
     size_t bytes = std::max<size_t>(count, 1) * sizeof(T);
     if (b.cap < bytes) {
       if (b.p && (b.p == up_inst || b.p == up_chunks)) forget_upload();
+      if (b.p && (b.p == last_core || b.p == last_orig || b.p == last_core_out)) {
+        last_n = -1;
+        last_core = nullptr;
+      }
       if (b.p) (void)hipFree(b.p);
       b.p = nullptr;
       b.cap = 0;

@@ -59,3 +59,19 @@ def test_batch_after_a_call_out_of_memory(devmem):
             devmem.h2d(d_l, np.full(int(ns.sum()), -7, dtype=np.int32))
             assert not np.any(h.run_batched_device(d_x, ns, ps, d_l))
             assert np.array_equal(devmem.download(np.empty_like(refs), d_l), refs)
+
+
+def test_core_flags_after_a_larger_call_that_failed(devmem):
+    # the larger call takes new arrays before it finds its bin width too small
+    x, big = _blobs(3000, 3, 2), _blobs(200000, 3, 3)
+    with dclust.Handle(0) as h:
+        h.run(x, 0.02, 4)
+        assert np.array_equal(h.core_flags(len(x)), oracle.fast_dbscan(x, 0.02, 4)[1])
+        with pytest.raises(dclust.DclustError) as e:
+            h.run(big, 0.02, 4, r=10 ** 6)
+        assert e.value.code == dclust.E_BINWIDTH
+        with pytest.raises(dclust.DclustError) as e:
+            h.core_flags(len(x))
+        assert e.value.code == dclust.E_PARAM
+        h.run(x, 0.02, 4)
+        assert np.array_equal(h.core_flags(len(x)), oracle.fast_dbscan(x, 0.02, 4)[1])
