@@ -811,7 +811,7 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
   std::memset(&d, 0, sizeof(d));
   d.n = ntot;
   d.ninst = ninst;
-  d.nchunks = nchunks;
+  d.err_stops = ninst == 1 || !inst_err;
   const Call call{d_xyz, d_labels, inst[0]};
   d.chains = shape.chains ? 1 : 0;
   // (without seed lists the expansion's buffers stay unused and minimal)
@@ -994,11 +994,13 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
       HIPCHK(hipEventRecord(h->ev[E_END], s));  // (after the counters' readback)
       HIPCHK(copy_labels());
       HIPCHK(read_counters(h, d, s, ctl_h, h->greadback));
-      if (!ctl_h[C_ABANDON]) {
+      // (an error that fails the call has abandoned the run, which has written
+      // neither labels nor core flags: an eager one returns before it does)
+      if (!ctl_h[C_ABANDON] || (ctl_h[C_ERR] && !ctl_h[C_KEYOVF] && d.err_stops)) {
         if (ctl_h[C_ERR]) {
           int first = 0;
           HIPCHK(read_inst_errors(d, ninst, inst_err, &first));
-          if (ninst == 1 || !inst_err) return first ? first : DCLUST_E_PARAM;
+          if (d.err_stops) return first ? first : DCLUST_E_PARAM;
           rc = first;
         }
         finish_run(h, d, shape, ctl_h, (int)std::max<long long>(1, ctl_h[C_LASTPASS]),
@@ -1024,7 +1026,7 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
     if (ctl_h[C_ERR]) {
       int first = 0;
       HIPCHK(read_inst_errors(d, ninst, inst_err, &first));
-      if (ninst == 1 || !inst_err) return first ? first : DCLUST_E_PARAM;
+      if (d.err_stops) return first ? first : DCLUST_E_PARAM;
       rc = first;  // batched with per-instance errors: keep going
     }
     const int bits = (int)ctl_h[C_KEYBITS];

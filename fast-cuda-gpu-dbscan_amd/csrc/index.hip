@@ -360,6 +360,7 @@ __device__ void setup_totals(const Dev& d, unsigned long long cells, unsigned lo
     d.ctl[C_KEYBITS] = 8;
   } else {
     d.ctl[C_KEYBITS] = key_bits_for(keys);
+    if (err && d.err_stops) d.ctl[C_ABANDON] = 1;
   }
 }
 

@@ -316,7 +316,7 @@ constexpr int kClockMHz = 100;  // of the constant device clock
 struct Dev {
   int64_t n;
   int32_t ninst;
-  int32_t nchunks;
+  int32_t err_stops;  // 1: an instance's error fails the call, which then writes nothing
   Inst* inst;
   const Chunk* chunks;
   unsigned long long* bbox;  // [ninst][kBoxStripes][8] ordered-u64 min0..2 max0..2,

@@ -1,5 +1,7 @@
 """Calls that fail leave the handle fit for the next ones: what the library
 remembers of earlier calls goes with the memory it lay in."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -75,3 +77,75 @@ def test_core_flags_after_a_larger_call_that_failed(devmem):
         assert e.value.code == dclust.E_PARAM
         h.run(x, 0.02, 4)
         assert np.array_equal(h.core_flags(len(x)), oracle.fast_dbscan(x, 0.02, 4)[1])
+
+
+@pytest.mark.parametrize("prec", [dclust.FP64, dclust.FP32_GUARD])
+def test_failed_replay_writes_nothing(devmem, prec, monkeypatch):
+    # a captured run replays for other parameters and other data; when those
+    # fail the call, labels and core flags stay as an eager call leaves them
+    monkeypatch.delenv("DCLUST_GRAPH", raising=False)
+    x = _blobs(7001, 3, 4)
+    n = len(x)
+    bad = x.copy()
+    bad[1234, 1] = np.nan
+    ref, core, _ = oracle.fast_dbscan(x, 0.02, 4)
+    d_x, d_bad, d_l = devmem.upload(x), devmem.upload(bad), devmem.alloc(4 * n)
+
+    def params(eps=0.02, r=0):
+        return dclust.make_params(3, eps, 4, r=r, precision=prec)
+
+    with dclust.Handle(0) as h:
+        for _ in range(3):
+            st = h.run_device(d_x, n, params(), d_l)
+        assert st["diag"][14] == 1
+        devmem.h2d(d_l, np.full(n, -7, dtype=np.int32))
+        for buf, p, code in ((d_x, params(r=10 ** 6), dclust.E_BINWIDTH),
+                             (d_bad, params(), dclust.E_PARAM),
+                             (d_x, params(eps=1e-13), dclust.E_PARAM),
+                             (d_x, params(eps=1e-9), dclust.E_CAPACITY)):
+            with pytest.raises(dclust.DclustError) as e:
+                h.run_device(buf, n, p, d_l)
+            assert e.value.code == code
+            assert np.all(devmem.download(np.empty(n, dtype=np.int32), d_l) == -7)
+            assert np.array_equal(h.core_flags(n), core)
+        st = h.run_device(d_x, n, params(), d_l)
+        assert np.array_equal(devmem.download(np.empty(n, dtype=np.int32), d_l), ref)
+
+
+@pytest.mark.parametrize("errors_wanted", [False, True])
+def test_failed_replay_of_a_batch(devmem, errors_wanted, monkeypatch):
+    # without inst_err one bad instance fails the whole call; with it the
+    # others are clustered
+    monkeypatch.delenv("DCLUST_GRAPH", raising=False)
+    xs = [_blobs(900, 2, 5), _blobs(1100, 3, 6)]
+    ns = np.array([len(x) for x in xs], dtype=np.int64)
+    tot = int(ns.sum())
+    refs = [oracle.fast_dbscan(x, 0.02, 4)[0] for x in xs]
+    bad = [xs[0], np.where(np.arange(1100)[:, None] == 7, np.inf, xs[1])]
+    d_x = devmem.upload(np.concatenate([x.ravel() for x in xs]))
+    d_bad = devmem.upload(np.concatenate([x.ravel() for x in bad]))
+    d_l = devmem.alloc(4 * tot)
+    parr = (dclust.Params * 2)(*[dclust.make_params(x.shape[1], 0.02, 4) for x in xs])
+    errs, st = np.zeros(2, dtype=np.int32), dclust.Stats()
+
+    with dclust.Handle(0) as h:
+        def call(buf):
+            devmem.h2d(d_l, np.full(tot, -7, dtype=np.int32))
+            rc = dclust._lib().dclust_run_batched_device(
+                h._h, 2, C.c_void_p(buf), ns.ctypes.data, parr, C.c_void_p(d_l),
+                errs.ctypes.data if errors_wanted else None, C.byref(st))
+            return rc, devmem.download(np.empty(tot, dtype=np.int32), d_l)
+
+        for k in range(3):
+            rc, lab = call(d_x)
+            assert rc == 0 and np.array_equal(lab, np.concatenate(refs))
+        assert st.diag[14] == 1
+        rc, lab = call(d_bad)
+        assert rc == dclust.E_PARAM
+        if errors_wanted:
+            assert errs.tolist() == [0, dclust.E_PARAM]
+            assert np.array_equal(lab[:900], refs[0])
+        else:
+            assert np.all(lab == -7)
+        rc, lab = call(d_x)
+        assert rc == 0 and np.array_equal(lab, np.concatenate(refs)) and st.diag[14] == 1
