@@ -848,6 +848,9 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
     // the sort's point ids, then (from k_far on) the listed pairs of cells
     d.val[0] = M.get<int32_t>(S_VAL, 2 * (size_t)ntot);
     d.val[1] = d.val[0] + ntot;
+    // (as many pairs as that memory holds: a quarter to a half of the points.
+    // Only lattices and the like list more, and what finds no room is decided
+    // cell by cell, where the first unions settle most of the rest)
     const int64_t cap_f = ntot / 2 / kStripes;
     d.far_light = PairList{(int2*)d.val[0], (unsigned long long*)(d.stat + C_NFARLIGHT), cap_f};
     d.far_heavy = PairList{(int2*)d.val[0] + cap_f * kStripes,
@@ -899,9 +902,11 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
     d.near_roots = SList{d.q[0], (unsigned long long*)(d.stat + C_NROOTS),
                          cap_c};
     // the component keys, before them the list of points the first count pass
-    // leaves
+    // leaves, then that of cells whose border pairs found no room (listed by
+    // workgroup, as the points are, and no more of them)
     d.keyv = M.get<int32_t>(S_KEYV, (size_t)std::max(ntot, cap_p * kStripes));
     d.core_rest = SList{d.keyv, (unsigned long long*)(d.stat + C_NCOREREST), cap_p};
+    d.far_over = SList{d.keyv, (unsigned long long*)(d.stat + C_NFAROVER), cap_p};
     d.flag = M.get<unsigned long long>(S_FLAG, ntot / 64 + 1);
     d.rank = M.get<int32_t>(S_RANK, ntot / 64 + 1);
     d.scan_tmp = M.get<int64_t>(S_SCAN, scan_tmp_entries(ntot));

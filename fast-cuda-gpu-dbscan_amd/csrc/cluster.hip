@@ -1141,19 +1141,25 @@ __device__ bool cells_joined(const Dev& d, const Par& P, int32_t qs, int32_t qe,
 }
 
 // Core cell A, one lane: the stencil cells above A (each unordered pair is
-// taken by its lower cell) with core points in another component are listed,
-// pairs with a heavy cell apart.  (Deciding them here held the lanes of the
-// listing at 5 waves per SIMD with 32 spilled registers: 158 us on the 4 M
-// point 3-D workload, against 65 + 24 with k_far_pairs.)
+// taken by its lower cell) with core points in another component, `sel`, and
+// which of those pairs have a heavy cell, `heavy`, by slot of A's own row and
+// the rows above it.  (Deciding them here held the lanes of the listing at 5
+// waves per SIMD with 32 spilled registers: 158 us on the 4 M point 3-D
+// workload, against 65 + 24 with k_far_pairs.)
+constexpr int kFarRows = Win<3>::rows - Win<3>::own;
+struct FarCell {
+  uint2 row[kFarRows];
+  uint32_t sel[kFarRows], heavy[kFarRows];
+};
 template <int D>
-__device__ __forceinline__ void far_cell(const Dev& d, int32_t A, int32_t compA, bool heavyA) {
+__device__ __forceinline__ void far_cell(const Dev& d, int32_t A, int32_t compA, bool heavyA,
+                                         FarCell& f) {
   constexpr int NU = Win<D>::rows - Win<D>::own;  // own row and those above
   constexpr int nl = Win<D>::nl;
   const int local = (int)(d.cell_zl[A] & (nl - 1));
   const RowsOf rows = rows_of(d, A);
-  uint2 row[NU];
 #pragma unroll
-  for (int j = 0; j < NU; ++j) row[j] = rows[Win<D>::own + j];
+  for (int j = 0; j < NU; ++j) f.row[j] = rows[Win<D>::own + j];
   // cells with core points in another component, by place in each window's
   // cells (cell_comp is -1 for a cell without core points); the windows'
   // cells are consecutive, so their components are loaded four at a time (up
@@ -1161,8 +1167,8 @@ __device__ __forceinline__ void far_cell(const Dev& d, int32_t A, int32_t compA,
   uint32_t other[NU];
 #pragma unroll
   for (int j = 0; j < NU; ++j) {
-    const int n = row_cells(row[j]);
-    const int32_t* cp = d.cell_comp + (int64_t)row[j].x;
+    const int n = row_cells(f.row[j]);
+    const int32_t* cp = d.cell_comp + (int64_t)f.row[j].x;
     other[j] = 0u;
 #pragma unroll
     for (int q = 0; q < Win<D>::slots; q += 4)
@@ -1179,22 +1185,73 @@ __device__ __forceinline__ void far_cell(const Dev& d, int32_t A, int32_t compA,
     if (!other[j]) continue;
     const int r = Win<D>::own + j;
     const int a = D == 3 ? r / 3 - 1 : r - 1, b = D == 3 ? r % 3 - 1 : 0;
-    uint32_t todo = row[j].y & row_valid<D>(a, b, local);
+    uint32_t todo = f.row[j].y & row_valid<D>(a, b, local);
     if (j == 0) todo &= ~0u << (2 * nl + local + 1);  // above A in its own column
     while (todo) {
       const int s = __ffs(todo) - 1;
       todo &= todo - 1;
-      const int place = __popc(row[j].y & ((1u << s) - 1u));
+      const int place = __popc(f.row[j].y & ((1u << s) - 1u));
       if (!((other[j] >> place) & 1u)) continue;
-      const int32_t B = (int32_t)row[j].x + place;
-      const bool heavy = heavyA || d.cell_start[B + 1] - d.cell_start[B] > kHeavy;
-      const PairList& L = heavy ? d.far_heavy : d.far_light;
-      const int st = blockIdx.x & (kStripes - 1);
-      const unsigned long long at = atomicAdd(&L.cnt[st * kStatStride], 1ull);
-      if (at < (unsigned long long)L.cap) L.data[st * L.cap + (int64_t)at] = make_int2(A, B);
+      const int32_t B = (int32_t)f.row[j].x + place;
+      f.sel[j] |= 1u << s;
+      if (heavyA || d.cell_start[B + 1] - d.cell_start[B] > kHeavy) f.heavy[j] |= 1u << s;
     }
   }
 }
+
+// Stores the pairs of a wavefront's cells, `tot` in all, this lane's `mine` of
+// them from number `first` on (its light or its heavy ones), and returns how
+// many found room.  One atomic for the wavefront's pairs: the sub-list of its
+// own first, then whichever have room, so that a list takes as many pairs as it
+// holds from however few wavefronts, and a full one costs a single look at its
+// counters.  k_far with an atomic for each pair, on the sub-list of the
+// workgroup, and now: 2566 and 184 us on a 3-D lattice of 1 M points with eps
+// 1.5 spacings, 948 and 115 on a 2-D one with eps one spacing, 61 and 45 on the
+// 4 M point 3-D workload.
+__device__ __forceinline__ int far_store(const PairList& L, const FarCell& f, int32_t A,
+                                         bool heavy, int first, int mine, int tot) {
+  const int lane = lane_id();
+  int done = 0;
+  int st = (int)((blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) & (kStripes - 1));
+  unsigned long long tried = 0;
+  for (;;) {
+    long long at = 0;
+    if (lane == 0)
+      at = (long long)atomicAdd(&L.cnt[st * kStatStride], (unsigned long long)(tot - done));
+    at = rl_l(at, 0);
+    const long long room = (long long)L.cap - at;
+    const int take = room <= 0 ? 0 : (room < tot - done ? (int)room : tot - done);
+    if (take > 0 && mine > 0 && first < done + take && first + mine > done) {
+      int2* to = L.data + st * L.cap + at;
+      int k = first - done;
+#pragma unroll
+      for (int j = 0; j < kFarRows; ++j) {
+        uint32_t m = f.sel[j] & (heavy ? f.heavy[j] : ~f.heavy[j]);
+        while (m) {
+          const int s = __ffs(m) - 1;
+          m &= m - 1;
+          if (k >= 0 && k < take) to[k] = make_int2(A, slot_cell(f.row[j], s));
+          ++k;
+        }
+      }
+    }
+    done += take;
+    if (done == tot) break;
+    tried |= 1ull << st;
+    const unsigned long long open =
+        ballot((long long)__hip_atomic_load(&L.cnt[lane * kStatStride], __ATOMIC_RELAXED,
+                                            __HIP_MEMORY_SCOPE_AGENT) < (long long)L.cap) &
+        ~tried;
+    if (!open) break;
+    const unsigned long long above = open & (~0ull << st);  // (st itself is not open)
+    st = __ffsll((long long)(above ? above : open)) - 1;
+  }
+  return done;
+}
+
+// A listed cell of Dev::far_over: its index, and which pairs were not stored.
+constexpr int32_t kOverLight = 1 << 28, kOverHeavy = 1 << 29, kOverCell = kOverLight - 1;
+static_assert(kMaxCells <= (1LL << 28), "a cell index has 28 bits");
 
 __global__ __launch_bounds__(256, 8) void k_far(Dev d) {
   if (abandoned(d)) return;
@@ -1212,7 +1269,38 @@ __global__ __launch_bounds__(256, 8) void k_far(Dev d) {
       comp = d.cell_comp[A];
       heavy = d.cell_start[A + 1] - d.cell_start[A] > kHeavy;
     }
-    DCLUST_BY_DIM(act, dim, far_cell<3>(d, A, comp, heavy), far_cell<2>(d, A, comp, heavy));
+    FarCell f;
+#pragma unroll
+    for (int j = 0; j < kFarRows; ++j) {
+      f.row[j] = make_uint2(0u, 0u);
+      f.sel[j] = f.heavy[j] = 0u;
+    }
+    DCLUST_BY_DIM(act, dim, far_cell<3>(d, A, comp, heavy, f), far_cell<2>(d, A, comp, heavy, f));
+    int nl = 0, nh = 0;
+#pragma unroll
+    for (int j = 0; j < kFarRows; ++j) {
+      nl += __popc(f.sel[j] & ~f.heavy[j]);
+      nh += __popc(f.heavy[j]);
+    }
+    if (!ballot((nl | nh) != 0)) continue;
+    // (a lane has at most 100 pairs, so both counts of the wave fit one word)
+    const uint32_t both = (uint32_t)nl | (uint32_t)nh << 16;
+    const uint32_t incl = wave_incl_scan(both), before = incl - both, all = rl_u(incl, 63);
+    const int tl = (int)(all & 0xffffu), th = (int)(all >> 16);
+    const int fl = (int)(before & 0xffffu), fh = (int)(before >> 16);
+    const int sl = tl ? far_store(d.far_light, f, A, false, fl, nl, tl) : 0;
+    const int sh = th ? far_store(d.far_heavy, f, A, true, fh, nh, th) : 0;
+    // cells with pairs that found no room
+    const int32_t left = (nl && fl + nl > sl ? kOverLight : 0) | (nh && fh + nh > sh ? kOverHeavy : 0);
+    if (const unsigned long long m = ballot(left != 0)) {
+      const int st = blockIdx.x & (kStripes - 1);
+      long long at = 0;
+      if (lane_id() == 0)
+        at = (long long)atomicAdd(&d.far_over.cnt[st * kStatStride],
+                                  (unsigned long long)__popcll(m));
+      at = rl_l(at, 0);
+      if (left) d.far_over.data[st * d.far_over.cap + at + mbcnt(m)] = A | left;
+    }
   }
 }
 
@@ -1293,11 +1381,6 @@ __device__ __forceinline__ long long pairs_prefix(const PairList& L, long long* 
   __syncthreads();
   return s_pre[kStripes];
 }
-// this thread's sub-list took more pairs than it holds
-__device__ __forceinline__ bool pairs_over(const PairList& L) {
-  return threadIdx.x < kStripes &&
-         (long long)L.cnt[threadIdx.x * kStatStride] > (long long)L.cap;
-}
 __device__ __forceinline__ int2 pairs_at(const PairList& L, const long long* s_pre, long long i) {
   int lo = 0, hi = kStripes - 1;  // last sub-list whose range starts at or before i
   while (lo < hi) {
@@ -1340,12 +1423,32 @@ __device__ __forceinline__ void far_light(const Dev& d, int32_t A, int32_t B, Ta
   }
 }
 
-// Every pair of core cell A's, decided by one lane (when a list of pairs was
-// too short).
-template <int D, bool F32>
-__device__ void far_cell_all(const Dev& d, const Par& P, int32_t A, Tally& t, long long& freeb,
-                             long long& joins) {
+// One pair, the whole wavefront (wave-uniform: every lane walks the same path,
+// lane 0's roots are taken).
+template <bool F32>
+__device__ __forceinline__ void far_heavy(const Dev& d, int32_t A, int32_t B, Tally& t,
+                                          long long& joins) {
+  const int32_t ra = rfl_i(uf_find_cached(d.parent, d.cell_comp[A]));
+  const int32_t rb = rfl_i(uf_find_cached(d.parent, d.cell_comp[B]));
+  if (ra == rb) return;
+  const Inst& I = *inst_of_cell(d, A);
+  const Par P(I);
+  const bool j = I.dim == 3 ? wave_joined<3, F32>(d, P, A, B, t)
+                            : wave_joined<2, F32>(d, P, A, B, t);
+  if (j && lane_id() == 0) {
+    uf_union(d.parent, ra, rb);
+    ++joins;
+  }
+}
+
+// The light or the heavy pairs of core cell A (when a list had no room for
+// all of them), in turn.
+template <int D, typename F>
+__device__ __forceinline__ void far_cell_pairs(const Dev& d, int32_t A, bool heavy,
+                                               const F& decide) {
   const int local = (int)(d.cell_zl[A] & (Win<D>::nl - 1));
+  const int32_t comp = d.cell_comp[A];
+  const bool heavyA = d.cell_start[A + 1] - d.cell_start[A] > kHeavy;
   for (int r = Win<D>::own; r < Win<D>::rows; ++r) {
     const uint2 row = rows_of(d, A)[r];
     uint32_t todo = row.y & (D == 3 ? row_valid<3>(r / 3 - 1, r % 3 - 1, local)
@@ -1353,15 +1456,18 @@ __device__ void far_cell_all(const Dev& d, const Par& P, int32_t A, Tally& t, lo
     while (todo) {
       const int32_t B = slot_cell(row, __ffs(todo) - 1);
       todo &= todo - 1;
-      if (B > A && d.cell_comp[B] >= 0 && d.cell_comp[B] != d.cell_comp[A])
-        far_light<F32>(d, A, B, t, freeb, joins);
+      if (B <= A || d.cell_comp[B] < 0 || d.cell_comp[B] == comp) continue;
+      if ((heavyA || d.cell_start[B + 1] - d.cell_start[B] > kHeavy) == heavy) decide(B);
     }
   }
 }
 
 // The listed pairs: light ones one lane each, those with a heavy cell one
-// wavefront each (wave-uniform: every lane walks the same path, lane 0's
-// roots are taken).
+// wavefront each.  Then the cells whose pairs found their list full, in the
+// same way, a cell's pairs one after the other: the unions of the first then
+// settle most of the rest.  (Two sheets of 100 k points in 288 cells, just over
+// eps apart: 2.1 s when few sub-lists took all pairs and a lane each decided
+// those of a cell again, 69 us now.)
 template <bool F32>
 __global__ __launch_bounds__(256, 4) void k_far_pairs(Dev d) {
   if (abandoned(d)) return;
@@ -1379,34 +1485,29 @@ __global__ __launch_bounds__(256, 4) void k_far_pairs(Dev d) {
   for (long long i = (long long)blockIdx.x * 4 + (threadIdx.x >> 6); i < nh;
        i += (long long)gridDim.x * 4) {
     const int2 pr = pairs_at(d.far_heavy, s_pre, i);
-    const int32_t A = rfl_i(pr.x), B = rfl_i(pr.y);
-    const int32_t ra = rfl_i(uf_find_cached(d.parent, d.cell_comp[A]));
-    const int32_t rb = rfl_i(uf_find_cached(d.parent, d.cell_comp[B]));
-    if (ra == rb) continue;
-    const Inst& I = *inst_of_cell(d, A);
-    const Par P(I);
-    const bool j = I.dim == 3 ? wave_joined<3, F32>(d, P, A, B, t)
-                              : wave_joined<2, F32>(d, P, A, B, t);
-    if (j && lane_id() == 0) {
-      uf_union(d.parent, ra, rb);
-      ++joins;
-    }
+    far_heavy<F32>(d, rfl_i(pr.x), rfl_i(pr.y), t, joins);
   }
-  // pairs that found their list full: all pairs again (those decided above
-  // are skipped or decided the same)
-  const bool over = pairs_over(d.far_light) || pairs_over(d.far_heavy);
-  if (__syncthreads_or(over)) {
-    const long long nc = slist_prefix(d.core_cells, s_pre);
-    for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < nc;
-         i += (long long)gridDim.x * 256) {
-      const int32_t A = slist_at(d.core_cells, s_pre, i);
-      const Inst& I = *inst_of_cell(d, A);
-      const Par P(I);
-      if (I.dim == 3)
-        far_cell_all<3, F32>(d, P, A, t, freeb, joins);
-      else
-        far_cell_all<2, F32>(d, P, A, t, freeb, joins);
-    }
+  __syncthreads();
+  const long long no = slist_prefix(d.far_over, s_pre);
+  for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < no;
+       i += (long long)gridDim.x * 256) {
+    const int32_t e = slist_at(d.far_over, s_pre, i), A = e & kOverCell;
+    if (!(e & kOverLight)) continue;
+    const auto light = [&](int32_t B) { far_light<F32>(d, A, B, t, freeb, joins); };
+    if (inst_of_cell(d, A)->dim == 3)
+      far_cell_pairs<3>(d, A, false, light);
+    else
+      far_cell_pairs<2>(d, A, false, light);
+  }
+  for (long long i = (long long)blockIdx.x * 4 + (threadIdx.x >> 6); i < no;
+       i += (long long)gridDim.x * 4) {
+    const int32_t e = rfl_i(slist_at(d.far_over, s_pre, i)), A = e & kOverCell;
+    if (!(e & kOverHeavy)) continue;
+    const auto heavy = [&](int32_t B) { far_heavy<F32>(d, A, rfl_i(B), t, joins); };
+    if (inst_of_cell(d, A)->dim == 3)
+      far_cell_pairs<3>(d, A, true, heavy);
+    else
+      far_cell_pairs<2>(d, A, true, heavy);
   }
   stat_add(d, C_BAND, t.band);
   stat_add(d, C_ASYM, t.asym);

@@ -191,7 +191,6 @@ enum Ctl : int {
   C_EVAL,
   C_OVF,
   C_ERR,
-  C_SORTPAR,  // number of executed radix scatters (buffer parity)
   C_BAND_CORE,
   C_POPS,       // cells expanded
   C_BUSY_SUM,  // expansion: sum over waves of their lifetime (us)
@@ -226,6 +225,7 @@ enum Ctl : int {
   C_NROOTS,       // near components (listed in Dev::near_roots)
   C_NFARLIGHT,    // pairs across components (listed in Dev::far_light)
   C_NFARHEAVY,    // those with a heavy cell (listed in Dev::far_heavy)
+  C_NFAROVER,     // cells with pairs that found no room there (Dev::far_over)
   C_BOXES,        // chunks whose bounding box is done (one instance)
   // this call's input and output (addresses), written by the run's first kernel
   C_XYZ,
@@ -351,6 +351,7 @@ struct Dev {
   PairList far_light;   // pairs of cells across components without a heavy cell and
   PairList far_heavy;   // with one (over the sort's point ids, which the gather is the
                         // last to read)
+  SList far_over;       // cells with pairs that neither had room for (over keyv)
   uint2* rows;          // [kMaxRows][rstride] neighbour windows (first cell, slot bits and
                         // point count), row-major so that consecutive cells are adjacent
   int64_t rstride;      // >= number of cells
