@@ -176,8 +176,11 @@ __device__ __forceinline__ bool edge_pair(const Dev& d, const Par& P, int32_t a,
 //                 points write neighbouring words).
 //   k_core_crowd  one wavefront per listed point with more than kCoreCrowd
 //                 candidates (a few lanes would take as long as the rest of the
-//                 launch), and in the FP32 form per point that a pair inside the
-//                 guard band decides.
+//                 launch); in the FP32 form first four lanes per point that a pair
+//                 inside the guard band may decide, by the exact predicate.  (Few
+//                 of those in most data, but every point of a lattice whose
+//                 spacing is eps: a wavefront each took 1538 of the 1894 us of a
+//                 call on 1 M such points, 110 of 505 now.)
 //
 // Both passes over points are bound by the rows and coordinates they fetch at
 // random: neighbouring points name the same ones, so each XCD takes runs of
@@ -416,10 +419,10 @@ __device__ __forceinline__ void row_points_in(const Dev& d, uint2 row, uint32_t 
 }
 
 // Count of p over all of its rows by the Q lanes that share it.  0:
-// not core, 1: core, 2: left to a wavefront (many candidates, or in the FP32
-// form a pair inside the guard band that the others do not make up for: the
-// exact test costs 20 registers).
-template <int D, bool F32, int Q>
+// not core, 1: core, 2: left to a wavefront (many candidates), 3: in the FP32
+// form, left to the exact test (`exact`) for a pair inside the guard band that
+// the others do not make up for: it costs 20 registers.
+template <int D, bool F32, int Q, bool exact>
 __device__ int core_rest(const Dev& d, const Par& P, int32_t p, int R,
                          int2* ranges, int32_t* lrec, Tally& t) {
   constexpr int NR = Win<D>::rows, NK = (NR + Q - 1) / Q;
@@ -507,7 +510,7 @@ __device__ int core_rest(const Dev& d, const Par& P, int32_t p, int R,
     for (int u = 0; u < B; ++u) {
       bool sym = false, fwd = false;
       if ((uint32_t)(qi[u] - qs) >= (uint32_t)own) {
-        if (F32) {
+        if (F32 && !exact) {
           const float sd = d2fix<D>(pg, cg[u]);
           sym = fwd = sd < P.d2_in;
           band |= !(sd < P.d2_in) && !(sd > P.d2_out);
@@ -521,19 +524,22 @@ __device__ int core_rest(const Dev& d, const Par& P, int32_t p, int R,
       if (sym && slot < R) lrec[slot] = qi[u];
       nrec += __popc(m);
       cnt += __popc(m);
-      if (!F32)
+      if (!F32 || exact)
         if (const unsigned long long one = ballot(sym && !fwd)) cnt -= __popc(mine(one));
     }
   }
   if (cnt >= P.minpts) return 1;
-  if (F32 && mine(ballot(band))) return 2;
+  if (F32 && !exact && mine(ballot(band))) return 3;
   wave_sync();
   for (int i = sub; i < nrec && i < R; i += Q) d.rec[(int64_t)i * d.n + p] = lrec[i];
   if (sub == 0) d.rec_n[p] = (uint8_t)(nrec <= R ? nrec : kRecNone);
   return 0;
 }
 
-// LDS of a k_core_rest workgroup: per point nine ranges, and R record slots
+// Entry of Dev::core_crowd: a point, and whether four lanes take it.
+constexpr int32_t kBandPoint = 1 << 28;
+
+// LDS of a k_core_rest workgroup (k_core_crowd: Q = 4): per point nine ranges, and R record slots
 // (one more: fewer bank conflicts)
 static size_t core_lds(int R, int Q) {
   return 256 / Q * (kMaxRows * sizeof(int2) + (R + 1) * 4);
@@ -563,11 +569,11 @@ __global__ __launch_bounds__(256, (F32 ? 7 : 5) + (Q == 4)) void k_core_rest(Dev
     }
     const Par P(*I);
     int res = 0;
-    DCLUST_BY_DIM(act, dim, (res = core_rest<3, F32, Q>(d, P, p, R, ranges, lrec, t)),
-                  (res = core_rest<2, F32, Q>(d, P, p, R, ranges, lrec, t)));
+    DCLUST_BY_DIM(act, dim, (res = core_rest<3, F32, Q, false>(d, P, p, R, ranges, lrec, t)),
+                  (res = core_rest<2, F32, Q, false>(d, P, p, R, ranges, lrec, t)));
     if (act && lead && res == 1) d.core[p] = 1;
     block_append(act && lead && res == 0, p, d.border_pts);
-    block_append(act && lead && res == 2, p, d.core_crowd);
+    block_append(act && lead && res >= 2, p | (res == 3 ? kBandPoint : 0), d.core_crowd);
   }
   stat_add(d, C_EVAL, t.eval);
   stat_add(d, C_CORE_ROWS, t.rows);
@@ -620,25 +626,61 @@ __device__ bool core_wave(const Dev& d, const Par& P, int32_t p, int R, Tally& t
   return cnt >= P.minpts;
 }
 
+// The listed points that a pair inside the guard band may decide.
+__device__ __forceinline__ void core_band(const Dev& d, const Stripe& L, int2* s_core, Tally& t) {
+  constexpr int Q = 4, PB = 256 / Q;
+  const int R = d.rec_stride;
+  const int pt = threadIdx.x / Q;
+  const bool lead = threadIdx.x % Q == 0;
+  int2* ranges = s_core + pt * kMaxRows;
+  int32_t* lrec = reinterpret_cast<int32_t*>(s_core + PB * kMaxRows) + pt * (R + 1);
+  for (int64_t i0 = L.first(PB); i0 < L.n; i0 += L.step(PB)) {
+    const int32_t e = i0 + pt < L.n ? L.data[i0 + pt] : 0;
+    const bool act = (e & kBandPoint) != 0;
+    if (!__syncthreads_or(act)) continue;
+    const int32_t p = act ? e & ~kBandPoint : 0;
+    const Inst* I = d.inst;
+    int dim = 0;
+    if (act) {
+      if (d.ninst != 1) I = inst_of_cell(d, d.cell_of[p]);
+      dim = I->dim;
+    }
+    const Par P(*I);
+    int res = 0;
+    DCLUST_BY_DIM(act, dim, (res = core_rest<3, true, Q, true>(d, P, p, R, ranges, lrec, t)),
+                  (res = core_rest<2, true, Q, true>(d, P, p, R, ranges, lrec, t)));
+    if (act && lead && res == 1) d.core[p] = 1;
+    block_append(act && lead && res == 0, p, d.border_pts);
+  }
+}
+
 template <bool F32>
 __global__ __launch_bounds__(256) void k_core_crowd(Dev d) {
   if (abandoned(d)) return;
+  extern __shared__ int2 s_core[];
   const Stripe L(d.core_crowd);
   const int R = d.rec_stride;
   Tally t;
-  for (int64_t i = L.first(4) + (threadIdx.x >> 6); i < L.n; i += L.step(4)) {
-    const int32_t p = rfl_i(L.data[i]);
-    const Inst& I = *inst_of_cell(d, d.ninst == 1 ? 0 : d.cell_of[p]);
-    const Par P(I);
-    const bool isc = I.dim == 3 ? core_wave<3, F32>(d, P, p, R, t)
-                                : core_wave<2, F32>(d, P, p, R, t);
-    if (lane_id() == 0) {
-      if (isc) {
-        d.core[p] = 1;
-      } else {
-        const SList& B = d.border_pts;
-        const int s = blockIdx.x & (kStripes - 1);
-        B.data[s * B.cap + (int64_t)atomicAdd(&B.cnt[s * kStatStride], 1ull)] = p;
+  if constexpr (F32) core_band(d, L, s_core, t);
+  // (a wavefront's next 64 entries at once)
+  const int64_t step = L.step(4);
+  for (int64_t i = L.first(4) + (threadIdx.x >> 6); i < L.n; i += 64 * step) {
+    const int64_t il = i + lane_id() * step;
+    const int32_t el = il < L.n ? L.data[il] : kBandPoint;
+    for (unsigned long long m = ballot(!(el & kBandPoint)); m; m &= m - 1) {
+      const int32_t p = rl_i(el, __ffsll((long long)m) - 1);
+      const Inst& I = *inst_of_cell(d, d.ninst == 1 ? 0 : d.cell_of[p]);
+      const Par P(I);
+      const bool isc = I.dim == 3 ? core_wave<3, F32>(d, P, p, R, t)
+                                  : core_wave<2, F32>(d, P, p, R, t);
+      if (lane_id() == 0) {
+        if (isc) {
+          d.core[p] = 1;
+        } else {
+          const SList& B = d.border_pts;
+          const int s = blockIdx.x & (kStripes - 1);
+          B.data[s * B.cap + (int64_t)atomicAdd(&B.cnt[s * kStatStride], 1ull)] = p;
+        }
       }
     }
   }
@@ -2451,7 +2493,8 @@ static void core_kernels(const Dev& d, hipStream_t s) {
   hipLaunchKernelGGL(k_core<F32>, dim3(point_grid(d.n)), dim3(256), 0, s, d);
   hipLaunchKernelGGL((k_core_rest<F32, Q>), dim3(list_grid(d.n * Q)), dim3(256),
                      core_lds(d.rec_stride, Q), s, d);
-  hipLaunchKernelGGL(k_core_crowd<F32>, dim3(list_grid(d.n)), dim3(256), 0, s, d);
+  hipLaunchKernelGGL(k_core_crowd<F32>, dim3(list_grid(d.n)), dim3(256),
+                     F32 ? core_lds(d.rec_stride, 4) : 0, s, d);
 }
 
 void launch_core(const Dev& d, bool f32, hipStream_t s) {

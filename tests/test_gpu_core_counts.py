@@ -56,3 +56,18 @@ def test_pairs_at_eps(devmem, prec, dim, step):
     st = _check(devmem, x, 0.5, max(2, full // 2), prec)
     if prec == dclust.FP32_GUARD and step == 0.5:  # (no nearer neighbour makes up for them)
         assert st["band_rechecks"] > 0
+
+
+@pytest.mark.parametrize("prec", [dclust.FP64, dclust.FP32_GUARD])
+@pytest.mark.parametrize("dim,minpts", [(2, 3), (2, 5), (2, 6), (3, 7), (3, 8)])
+def test_every_point_at_eps(devmem, prec, dim, minpts):
+    # a lattice with eps its spacing: each point's neighbours are all exactly
+    # eps away (2 dim of them inside the lattice); beside it a crowd of more
+    # than 512 candidates a point, whose points share the same list
+    m = 150 if dim == 2 else 30
+    g = np.stack(np.meshgrid(*[np.arange(m)] * dim, indexing="ij"), -1).reshape(-1, dim) * 0.5
+    rng = np.random.default_rng(dim + minpts)
+    x = np.concatenate([g, 200.0 + rng.normal(0, 0.25, (2500, dim))])
+    st = _check(devmem, x[rng.permutation(len(x))], 0.5, minpts, prec)
+    if prec == dclust.FP32_GUARD:
+        assert st["band_rechecks"] > len(g)
