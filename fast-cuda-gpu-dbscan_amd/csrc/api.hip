@@ -12,12 +12,14 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <set>
 #include <tuple>
 #include <vector>
 
@@ -57,6 +59,10 @@ struct dclust_handle {
   // launch shapes found by dclust_autotune_device, keyed by (dimension mix,
   // log2 of the total point count, precision form)
   std::map<std::tuple<int, int, int>, dclust_params> tuned;
+  // launch values that the autotuners of this handle gave out in place of
+  // zeros where the union-find is the faster one: a call that brings them
+  // is run as the call with the zeros (shape_values)
+  std::set<std::array<int32_t, 4>> stands_for_zeros;
   // replay of repeated calls
   std::vector<uint8_t> prev_sig;   // launch state of the last eager run
   int prev_npass = 0;              // most of its runs so far: expansion passes,
@@ -388,9 +394,16 @@ const ShapeRow* shape_row(int dims, int64_t n) {
   return nullptr;
 }
 
+// The launch values of a call.
+std::array<int32_t, 4> shape_values(const dclust_params& p) {
+  return {p.seed_list_size, p.blocks, p.block_threads, p.extra_collision};
+}
+constexpr std::array<int32_t, 4> kNoShape = {0, 0, 0, 0};
+
 // Near components: a call that names any value of the expansion's shape
 // (MAX_SEEDS, THREAD_BLOCKS, THREAD_COUNT, EXTRA_COLLISION_SIZE) runs the
-// seed-list expansion with that shape.  A call that leaves them all 0 unites
+// seed-list expansion with that shape (unless the values are ones that the
+// handle's autotuner gave out for zeros).  A call that leaves them all 0 unites
 // the near graph's pairs in a parallel union-find instead (k_link_*): the
 // expansion's time is the serial rounds of its longest wavefront, 435 us of
 // 2.45 ms on 4 M 3-D points (plus 64 us to merge its chains) and 79 (+ 24) of
@@ -401,7 +414,8 @@ const ShapeRow* shape_row(int dims, int64_t n) {
 // entries, 256 threads, blocks at resident occupancy, at most 8 per CU).
 RunShape pick_shape(dclust_handle* h, const dclust_params& p, int64_t n, bool f32, int dims) {
   RunShape r;
-  r.chains = p.seed_list_size > 0 || p.blocks > 0 || p.block_threads > 0 || p.extra_collision > 0;
+  const std::array<int32_t, 4> values = shape_values(p);
+  r.chains = values != kNoShape && !h->stands_for_zeros.count(values);
   const ShapeRow* row = (p.seed_list_size == 0 && p.block_threads == 0 && p.blocks == 0)
                             ? shape_row(dims, n)
                             : nullptr;
@@ -1514,8 +1528,9 @@ int dclust_autotune_device(dclust_handle* h, int32_t count, const double* d_xyz,
   hipError_t herr = hipSuccess;
   int32_t* lab = h->get<int32_t>(S_TUNELAB, std::max<int64_t>(tot, 1), &herr);
   if (!lab) return DCLUST_E_OOM;
-  // candidates: seed-list length x workgroup size x workgroups per CU; each
-  // is run twice and scored by its faster run
+  // candidates: seed-list length x workgroup size x workgroups per CU, and no
+  // launch values at all (the union-find); each is run twice and scored by its
+  // faster run
   const int seeds_c[] = {256, 512, 1024, 2048};
   const int threads_c[] = {128, 256};
   const int per_cu_c[] = {4, 8, 16};
@@ -1526,6 +1541,22 @@ int dclust_autotune_device(dclust_handle* h, int32_t count, const double* d_xyz,
     ~Eager() { h->graph_off = false; }
   } eager{h};
   h->graph_off = true;
+  auto timed = [&](int seeds, int threads, int blocks, double* t) {
+    for (auto& q : trial) {
+      q.seed_list_size = seeds;
+      q.block_threads = threads;
+      q.blocks = blocks;
+      q.extra_collision = 0;
+    }
+    *t = 1e30;
+    int rc = DCLUST_OK;
+    for (int rep = 0; rep < 2 && rc == DCLUST_OK; ++rep) {
+      dclust_stats st;
+      rc = run_device(h, count, d_xyz, n, trial.data(), lab, nullptr, &st);
+      *t = std::min(*t, st.t_total_ms);
+    }
+    return rc;
+  };
   double best = 1e30;
   dclust_params best_p = params[0];
   for (int sd : seeds_c)
@@ -1533,24 +1564,25 @@ int dclust_autotune_device(dclust_handle* h, int32_t count, const double* d_xyz,
       for (int pc : per_cu_c) {
         const int waves_per_cu = pc * th / 64;
         if (waves_per_cu > 32) continue;  // beyond what a CU holds
-        for (auto& q : trial) {
-          q.seed_list_size = sd;
-          q.block_threads = th;
-          q.blocks = h->num_cu * pc;
-          q.extra_collision = 0;
-        }
-        double t = 1e30;
-        for (int rep = 0; rep < 2; ++rep) {
-          dclust_stats st;
-          int rc = run_device(h, count, d_xyz, n, trial.data(), lab, nullptr, &st);
-          if (rc != DCLUST_OK) return rc;
-          t = std::min(t, st.t_total_ms);
-        }
+        // (a shape given out for zeros earlier is measured as itself)
+        double t = 0.0;
+        const std::array<int32_t, 4> values = {sd, h->num_cu * pc, th, 0};
+        const bool stood = h->stands_for_zeros.erase(values) > 0;
+        const int rc = timed(sd, th, h->num_cu * pc, &t);
+        if (stood) h->stands_for_zeros.insert(values);
+        if (rc != DCLUST_OK) return rc;
         if (t < best) {
           best = t;
           best_p = trial[0];
         }
       }
+  double zeros = 0.0;
+  const int rc = timed(0, 0, 0, &zeros);
+  if (rc != DCLUST_OK) return rc;
+  if (zeros <= best)
+    h->stands_for_zeros.insert(shape_values(best_p));
+  else
+    h->stands_for_zeros.erase(shape_values(best_p));
   for (int32_t i = 0; i < count; ++i) {
     params[i].seed_list_size = best_p.seed_list_size;
     params[i].block_threads = best_p.block_threads;
@@ -1571,11 +1603,13 @@ int dclust_autotune(dclust_handle* h, int64_t n, dclust_params* p) {
     if (p->blocks == 0) p->blocks = it->second.blocks;
     return DCLUST_OK;
   }
+  const bool zeros = shape_values(*p) == kNoShape;
   RunShape r = pick_shape(h, *p, n, f32, p->dim == 3 ? 2 : 1);
   if (p->seed_list_size == 0) p->seed_list_size = r.seeds;
   if (p->block_threads == 0) p->block_threads = r.threads;
   if (p->blocks == 0) p->blocks = r.blocks;
   if (p->extra_collision == 0) p->extra_collision = r.pair_per * (r.threads / 64);
+  if (zeros) h->stands_for_zeros.insert(shape_values(*p));
   return DCLUST_OK;
 }
 

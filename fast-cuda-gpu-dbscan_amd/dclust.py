@@ -323,7 +323,9 @@ class Handle:
 
     def autotune_device(self, d_xyz: int, ns, params_list):
         """Measure the candidate launch shapes on device-resident instances
-        and return the params with the fastest shape filled in."""
+        and return the params with the fastest shape filled in.  (Where a call
+        without launch values is faster, the shape stands for them on this
+        handle.)"""
         k = len(ns)
         ns = np.ascontiguousarray(ns, dtype=np.int64)
         parr = (Params * k)(*params_list)

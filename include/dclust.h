@@ -69,7 +69,9 @@ extern "C" {
  * blocks, block_threads and extra_collision all 0 finds the near components
  * by a parallel union-find without seed lists (faster than any shape; eff_*
  * then hold the shape an expansion of that size would take); a call that
- * gives any of them runs the seed-list expansion with that shape.
+ * gives any of them runs the seed-list expansion with that shape, except for
+ * values that dclust_autotune or dclust_autotune_device wrote for zeros on
+ * the same handle where the zeros are faster: those stand for the zeros.
  */
 typedef struct dclust_params {
   int32_t dim;
@@ -255,18 +257,22 @@ int dclust_last_core_flags(dclust_handle* h, uint8_t* core_out, int64_t n);
  * collision buffer): fills the zero fields of *p from the shapes that
  * dclust_autotune_device has measured on this handle for the same dimension,
  * size class (log2 n) and precision, else from the library's built-in table
- * (shapes measured on an MI355X per dimension mix and size class; a run
- * whose seed list, blocks and threads are all 0 uses it too). */
+ * (shapes measured on an MI355X per dimension mix and size class).  If all
+ * four launch values of *p are 0, the built-in shape stands for those zeros on
+ * this handle: a call that brings it runs without seed lists, as fast as one
+ * that brings the zeros. */
 int dclust_autotune(dclust_handle* h, int64_t n, dclust_params* p);
 
 /* Empirical autotuner (no counterpart in the reference, whose launch shape is
  * fixed at compile time, common.h:6-25): clusters the given device-resident
  * instances (layout of dclust_run_batched_device; count = 1 for one dataset)
  * with every candidate shape -- seed-list length {256, 512, 1024, 2048} x
- * workgroup size {128, 256} x workgroups per CU {4, 8, 16} -- keeps the
- * fastest, writes it into params[0..count) and remembers it for
- * dclust_autotune.  Optional: the built-in table holds the shapes this sweep
- * found for representative problems.  The grid does not depend on
+ * workgroup size {128, 256} x workgroups per CU {4, 8, 16} -- and with no
+ * launch values (no seed lists).  The fastest shape is written into
+ * params[0..count) and remembered for dclust_autotune; where the run without
+ * seed lists was faster still, that shape stands for the zeros from then on:
+ * calls of this handle that bring it run without seed lists too.  Optional: a
+ * call that leaves the launch values 0 does so by itself.  The grid does not depend on
  * PARTITION_SIZE (the cell width is fixed by eps; r only validates the bin
  * width), so r is not a tuning dimension: labels and times are the same for
  * every valid r. */
