@@ -64,3 +64,56 @@ def test_batch_of_wide_keys(devmem):
         assert not np.any(errs) and 32 < h.last_stats["key_bits"] <= 36
     for x, lab in zip(xs, labels):
         assert np.array_equal(lab, oracle.fast_dbscan(x, eps, 3)[0])
+
+
+# the wider forms at the first sizes of 4 and 8 entries a thread, whose last
+# tiles hold one entry: 33 and 36 bits (four of them in the ids), 37 and 60
+@pytest.mark.parametrize("span,bits", [(2000, 33), (3900, 36), (5000, 37), (900000, 60)])
+@pytest.mark.parametrize("n", [1572865, 3145729])
+def test_wide_keys_of_large_calls(devmem, span, bits, n):
+    eps = 0.5
+    x = _pairs(n, 3, span, eps, span)
+    d_x, d_l = devmem.upload(x), devmem.alloc(4 * n)
+    ref = oracle.fast_dbscan(x, eps, 3)
+    with dclust.Handle(0) as h:
+        st = h.run_device(d_x, n, dclust.make_params(3, eps, 3, precision=dclust.FP32_GUARD), d_l)
+        assert st["key_bits"] == bits
+        assert np.array_equal(devmem.download(np.empty(n, dtype=np.int32), d_l), ref[0])
+        assert np.array_equal(h.core_flags(n), ref[1])
+
+
+@pytest.mark.parametrize("span,lo,hi", [(1400, 33, 36), (4200, 37, 40)])
+@pytest.mark.parametrize("n", [1572865, 3145729])
+def test_large_batch_of_wide_keys(devmem, span, lo, hi, n):
+    eps = 0.5
+    ns = np.array([n - 500003, 400000, 3, 100000], dtype=np.int64)
+    xs = [_pairs(k, 3, span, eps, k) for k in ns]
+    d_x = devmem.upload(np.concatenate([x.ravel() for x in xs]))
+    d_l = devmem.alloc(4 * n)
+    with dclust.Handle(0) as h:
+        assert not np.any(h.run_batched_device(d_x, ns, [dclust.make_params(3, eps, 3)] * 4, d_l))
+        assert lo <= h.last_stats["key_bits"] <= hi
+    lab = devmem.download(np.empty(n, dtype=np.int32), d_l)
+    for x, part in zip(xs, np.split(lab, np.cumsum(ns)[:-1])):
+        assert np.array_equal(part, oracle.fast_dbscan(x, eps, 3)[0])
+
+
+@pytest.mark.parametrize("n", [5000, 70001])
+def test_replay_widens_through_the_forms(devmem, n, monkeypatch):
+    # a captured run of 32-, 36- or 64-bit keys meets a wider key: the call is
+    # run again with the wider form, which then serves the narrower keys too
+    monkeypatch.delenv("DCLUST_GRAPH", raising=False)
+    x = _pairs(n, 3, 1500, 0.5, 1)
+    d_x, d_l = devmem.upload(x), devmem.alloc(4 * n)
+    seen = []
+    with dclust.Handle(0) as h:
+        for eps in (0.5, 0.5, 0.25, 0.25, 0.2, 0.15, 0.15, 0.01, 0.01, 0.2, 0.5):
+            devmem.h2d(d_l, np.full(n, -7, dtype=np.int32))
+            st = h.run_device(d_x, n, dclust.make_params(3, eps, 3), d_l)
+            ref = oracle.fast_dbscan(x, eps, 3)
+            assert np.array_equal(devmem.download(np.empty(n, dtype=np.int32), d_l), ref[0])
+            assert np.array_equal(h.core_flags(n), ref[1])
+            seen.append((st["key_bits"], st["diag"][14]))
+    bits = [b for b, _ in seen]
+    assert bits[0] <= 32 < bits[2] <= 36 and bits[4] <= 36 < bits[5] <= 45 < bits[7]
+    assert [r for _, r in seen] == [0, 1, 0, 1, 1, 0, 1, 0, 1, 1, 1]
