@@ -505,12 +505,13 @@ def tune_table(hip, h, reps=10):
     """Measures the launch shapes behind the library's built-in shape table:
     dclust_autotune_device's sweep (seed-list length x workgroup size x
     workgroups per CU) on representative problems of each dimension mix and
-    size class, each best shape timed against the library's default shape;
+    size class, each best shape timed (on a handle of its own, where it does not
+    stand for the zeros) against the call without launch values;
     then clusterings of the same points at several PARTITION_SIZE values
     (r only validates the bin width: the grid is fixed by eps)."""
     rows = []
 
-    def timed(d_x, ns, params, d_l):
+    def timed(d_x, ns, params, d_l, h=h):
         for _ in range(2):
             h.run_batched_device(d_x, ns, params, d_l)
         hip.sync()
@@ -537,7 +538,8 @@ def tune_table(hip, h, reps=10):
                 for i in infos]
         t_def = timed(d_x, ns, base, d_l)
         tuned = h.autotune_device(d_x, ns, base)
-        t_best = timed(d_x, ns, tuned, d_l)
+        with dclust.Handle(0) as own:
+            t_best = timed(d_x, ns, tuned, d_l, own)
         dims = sorted({int(i["dim"]) for i in infos})
         row = {"case": name, "dims": dims, "points": int(ns.sum()),
                "log2_points": int(np.floor(np.log2(max(1, ns.sum())))),

@@ -799,7 +799,6 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
     ntot += n[i];
     off += n[i] * I.dim;
   }
-  // cell indices are packed into 28 bits in the neighbour-line table
   if (ntot >= kMaxCells) return DCLUST_E_CAPACITY;
   if (inst_err)
     for (int32_t i = 0; i < ninst; ++i) inst_err[i] = 0;
@@ -833,7 +832,7 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
   d.pair_per = shape.pair_per;
   d.rstride = ntot;
   // neighbourhood sizes (stats.cand_total / nbr_cells_total) cost an extra
-  // dependent load per stencil line; they are summed only on request
+  // dependent load per row; they are summed only on request
   {
     const char* e = std::getenv("DCLUST_NBR_STATS");
     d.nbr_stats = (e && e[0] == '1') ? 1 : 0;
@@ -1051,7 +1050,7 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
     const int bits = (int)ctl_h[C_KEYBITS];
     const long long nlines = ctl_h[C_NLINES];
     if (stats) stats->key_bits = (int32_t)ctl_h[C_KEYBITS];
-    // dense line table when it is small enough, else binary search
+    // dense column table when it is small enough, else binary search
     d.line_cap = 0;
     if (nlines <= kMaxLineTable) {
       d.lines = mem.get<int2>(S_LINES, (size_t)std::max<long long>(nlines, 1));

@@ -711,7 +711,9 @@ __global__ __launch_bounds__(1024) void k_rep(Dev d) {
   const int64_t cc = in ? c : 0;
   const int32_t q0 = d.cell_start[cc], q1 = d.cell_start[cc + 1];
   const int minpts = inst_of_cell(d, cc)->minpts;
-  // core points: all of a cell of minpts points, else few flags to count
+  // core points: all of a cell of minpts points, else its fewer than minpts
+  // flags, one after the other (262 k 3-D points: 11 us with minpts 32, 13 with
+  // 64, 53 with 512, 188 with 2000, a thirtieth of such a call)
   int32_t ncore = q1 - q0, first = q0;
   if (ncore < minpts) {
     ncore = 0;

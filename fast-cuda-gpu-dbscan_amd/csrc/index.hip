@@ -197,7 +197,12 @@ __global__ __launch_bounds__(256, 6) void k_bbox(Dev d) {
   if (threadIdx.x == 0) {
     // the stripes' atomics before the count: both are done at device scope,
     // so it is enough that they have completed (a device-wide fence per
-    // workgroup writes L2 back: 4 M points 65 us with it, 22 without)
+    // workgroup writes L2 back: 4 M points 65 us with it, 22 without).  The
+    // wait orders nothing but accesses that bypass the XCD's L2, so within this
+    // kernel the stripes may be written by device-scope atomics and read by
+    // device-scope atomic loads only: a plain store would stay in one XCD's L2.
+    // (The language gives no such order; this relies on gfx950's vmcnt, which
+    // counts an atomic without a result until it is done at its scope.)
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     // counted in stripes first: one address takes about 10 ns per workgroup
     const unsigned G = gridDim.x, g = blockIdx.x % kStripes;
@@ -456,6 +461,7 @@ __device__ __forceinline__ SortKey<KF>* key_buf(const Dev& d, int b) {
   return reinterpret_cast<SortKey<KF>*>(d.key[b]);
 }
 constexpr uint32_t kIdMask = (1u << 28) - 1;  // of the 36-bit form
+static_assert(kMaxCells <= (int64_t)kIdMask + 1, "every id fits the 36-bit form");
 // the whole key of a sort entry
 template <int KF>
 __device__ __forceinline__ uint64_t entry_key(SortKey<KF> k, int32_t v) {
@@ -683,7 +689,7 @@ __device__ __forceinline__ uint32_t sort_scan(uint32_t v, uint32_t (&s_w)[RS_T /
 // the tile's local starts turn the ranks into positions, so equal digits keep
 // their order.  The tile is staged in LDS in local digit order and written
 // out in runs per digit.  The counts of the workgroups before come from the
-// groups and from the rows of the own group, at most 47 loads a thread (a scan
+// groups and from the rows of the own group, at most 48 loads a thread (a scan
 // of all rows in a launch of its own took 5 us a pass).
 template <int KF, int NI>
 __global__ __launch_bounds__(RS_T, 4) void k_rs_scatter(Dev d, int pass, int nblk) {
@@ -862,9 +868,8 @@ __global__ __launch_bounds__(CS_T) void k_csr_count(Dev d, int bits) {
   if (threadIdx.x == 0) d.scan_tmp[blockIdx.x] = s[0] + s[1] + s[2] + s[3];
 }
 
-// exclusive scan of nb int64 values in place by one block; writes the total
-// to *total (may be null)
-__global__ __launch_bounds__(1024) void k_scan_top(int64_t* v, int nb, long long* total) {
+// exclusive scan of nb int64 values in place by one block
+__global__ __launch_bounds__(1024) void k_scan_top(int64_t* v, int nb) {
   __shared__ int64_t s[1024];
   const int per = (nb + 1023) / 1024;
   const int b0 = threadIdx.x * per;
@@ -886,7 +891,6 @@ __global__ __launch_bounds__(1024) void k_scan_top(int64_t* v, int nb, long long
       v[b0 + j] = run;
       run += x;
     }
-  if (threadIdx.x == 1023 && total) *total = s[1023];
 }
 
 // instance owning a key: last i with key_base <= key
@@ -1581,8 +1585,7 @@ static void index_sort(const Dev& d, int64_t n, int nchunks, int bits, hipStream
                      std::min(KF, kDigitBits * passes));
   const bool scan = ncs > kScanInline;
   if (scan)
-    hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(1024), 0, s, d.scan_tmp, ncs,
-                       (long long*)nullptr);
+    hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(1024), 0, s, d.scan_tmp, ncs);
   hipLaunchKernelGGL(k_csr_write<KF>, dim3(ncs), dim3(CS_T), 0, s, d, scan);
 }
 

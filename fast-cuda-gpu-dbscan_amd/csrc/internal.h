@@ -25,10 +25,19 @@ constexpr int32_t kUnclaimed = -1;
 constexpr int32_t kNoKey = 0x7fffffff;
 constexpr int kFixBits = 29;  // fixed-point fraction bits per cell width
 constexpr int kMaxRows = 9;   // 3^(D-1) neighbour columns for D <= 3
-constexpr int64_t kMaxCells = 1LL << 28;  // points (and so cells) of a call
+// points (and so cells) of a call: below this, because the 36-bit sort form
+// keeps point ids in 28 bits
+constexpr int64_t kMaxCells = 1LL << 28;
 constexpr int kHeavy = 32;    // cells with more points are "heavy" (a wavefront per border pair)
-constexpr int kRecSlots = 32;  // neighbour records kept per non-core point (at most)
-constexpr int kRecSlotsFixed = 16;  // the same in the fixed region of no-allocation runs
+// Neighbour records kept per non-core point, at most.  A bound on memory, not a
+// measured optimum: 32 slots are 128 of the 400 or so bytes a point takes, and
+// 16 keep the fixed region's capacity.  A non-core point has fewer than minpts
+// neighbours, so records cover minpts up to 33 (17); above that the points with
+// more neighbours are scanned again by k_border: 262 k 3-D points 37 us with
+// minpts 33, 352 with 64, 701 with 128; without allocation, 100 k points 9 us
+// with minpts 16, 81 with 24.
+constexpr int kRecSlots = 32;
+constexpr int kRecSlotsFixed = 16;  // in the fixed region of no-allocation runs
 // rec_n of a point without records, whose rows are scanned instead: fewer
 // than minpts points in all, or more neighbours than slots
 constexpr int kRecFew = 254;
@@ -285,9 +294,8 @@ struct PairList {
   int64_t cap;
 };
 
-// Sort-pass bookkeeping: pass p is active when p*8 < key bits; its scatter
-// runs unless every key has the same digit (then the data is already in
-// order and the buffers are not swapped).
+// Radix sort: the fewest passes of digits of at most kDigitBits bits that cover
+// the key, each of which scatters (index.hip).
 constexpr int kDigitBits = 9;  // of a radix pass, at most
 constexpr int kSortPasses = 8;  // of up to 64 bits
 constexpr int kSortGrid = 512;  // workgroups of the sort, at most

@@ -31,7 +31,6 @@ void launch_link(const Dev& d, hipStream_t s);
 void launch_comp(const Dev& d, hipStream_t s);
 void launch_pass_prep(const Dev& d, int pass, hipStream_t s);
 void launch_pass_carry(const Dev& d, int pass, int check, hipStream_t s);
-// after `passes` expansion passes: pending work abandons the rest of the run
 void launch_expand(const Dev& d, int pass, int grid, int seeds, int threads, int budget,
                    hipStream_t s);
 void launch_merge(const Dev& d, int grid, hipStream_t s);

@@ -276,7 +276,9 @@ class Handle:
 
     def run_batched(self, arrays, params_list):
         """Cluster independent instances in one pass; returns (labels list,
-        per-instance error codes)."""
+        per-instance error codes).  The labels are views of one array for the
+        whole batch: keeping one instance's keeps all of it, so copy() what is
+        to outlive the others."""
         k = len(arrays)
         xs = [np.ascontiguousarray(a, dtype=np.float64) for a in arrays]
         ns = np.array([a.shape[0] for a in xs], dtype=np.int64)

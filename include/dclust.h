@@ -144,7 +144,7 @@ typedef struct dclust_stats {
   int32_t eff_block_threads;
   int32_t eff_seed_list_size;
   int32_t eff_extra_collision;
-  double t_rows_ms;       /* the neighbour-line kernel alone (inside t_index) */
+  double t_rows_ms;       /* the neighbour-window kernels alone (in t_index) */
   int64_t n_core_cells;   /* cells holding core points                       */
   int64_t n_adj_points;   /* core points of light cells                      */
   int64_t n_lines;        /* possible grid columns (column-table entries)    */
@@ -235,7 +235,11 @@ int dclust_run_onestep_device(dclust_handle* h, const double* d_xyz, int64_t n,
  * (no counterpart in the reference, which clusters one dataset per process).
  * xyz[i]: n[i] rows of params[i].dim doubles on the host; labels[i]: n[i]
  * int32 on the host, numbered per instance.  inst_err (may be NULL)
- * receives a per-instance error code.  stats aggregates the batch. */
+ * receives a per-instance error code.  stats aggregates the batch.
+ * DCLUST_E_CAPACITY if the cells of all instances number more than 2^63, or
+ * their sort keys 2^64 or more (in 3-D the cells with the first two axes
+ * rounded up to even and the second one two cells longer; it takes a million
+ * instances for the keys to reach their limit before the cells reach theirs). */
 int dclust_run_batched(dclust_handle* h, int32_t count,
                        const double* const* xyz, const int64_t* n,
                        const dclust_params* params, int32_t* const* labels,
