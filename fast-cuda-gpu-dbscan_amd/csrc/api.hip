@@ -861,9 +861,9 @@ int run_device(dclust_handle* h, int32_t ninst, const double* d_xyz, const int64
     // the sort's point ids, then (from k_far on) the listed pairs of cells
     d.val[0] = M.get<int32_t>(S_VAL, 2 * (size_t)ntot);
     d.val[1] = d.val[0] + ntot;
-    // (as many pairs as that memory holds: a quarter to a half of the points.
-    // Only lattices and the like list more, and what finds no room is decided
-    // cell by cell, where the first unions settle most of the rest)
+    // (as many pairs as that memory holds: half as many in each list as there
+    // are points.  Only lattices and the like list more, and what finds no room
+    // is decided cell by cell, where the first unions settle most of the rest)
     const int64_t cap_f = ntot / 2 / kStripes;
     d.far_light = PairList{(int2*)d.val[0], (unsigned long long*)(d.stat + C_NFARLIGHT), cap_f};
     d.far_heavy = PairList{(int2*)d.val[0] + cap_f * kStripes,

@@ -186,7 +186,7 @@ __device__ __forceinline__ bool edge_pair(const Dev& d, const Par& P, int32_t a,
 // random: neighbouring points name the same ones, so each XCD takes runs of
 // kXcdRun workgroups of points, and the lists of k_core are walked on the XCD
 // that filled them.  k_core / k_core_rest / k_core_crowd, us: 4 M 3-D points,
-// FP32 form, 147 / 145 / 18 (with whole eighths of the points per XCD, lists
+// FP32 form, 144 / 123 / 15 (with whole eighths of the points per XCD, lists
 // walked in order and a lane per listed point 162 / 204 / 5); the batch of 7 M
 // points 198 / 179 / 18 (233 / 270 / 33); 262 k dense 3-D points, FP64 form,
 // 29 / 47 / 10 (31 / 110 / 18); 100 k 3-D points, FP32 form, 14 / 15 / 4 (13 /
