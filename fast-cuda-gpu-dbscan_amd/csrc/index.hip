@@ -349,6 +349,14 @@ __device__ void setup_instance(Inst& I, const unsigned long long (&bb)[8],
   I.d2_in = fin;
   I.d2_out = fout;
   I.d2_mid = (float)e2;
+  // The FP64 predicate compares squares: where eps^2 rounds to infinity or has
+  // lost bits to underflow (0 below 1.6e-162, where only the box test is left),
+  // the fixed-point distances say nothing about it.  Then every pair is inside
+  // the band, so that nothing is joined or left out by them.
+  if (!(I.eps2 >= 0x1p-1000 && I.eps2 <= 0x1.fffffffffffffp1023)) {
+    I.d2_in = -1.f;
+    I.d2_out = INFINITY;
+  }
 }
 
 // The call's totals: key width, columns, errors.
